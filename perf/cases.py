@@ -71,7 +71,7 @@ def draw(rng):
         role, n = rng.choice(("full", "segment", "last")), _log(rng, 1, 64)
         longest = _log(rng, 20, min(2000 if model == "small-llama" else 4000 if model == "llama2-7b" else 7000, 72000 // n))
         return _case("step", model, 0, rng.randint(2, 4), role, n, max(1, longest // 3), longest,
-                     weights="fp8" if fp8 else "bf16", sample=role != "segment" and n >= 8 and rng.random() < 0.5)
+                     weights="fp8" if fp8 else "bf16", sample=role != "segment" and n >= 16 and rng.random() < 0.5)
     if kind == "prompt":
         model, n = rng.choice(("small-llama", "llama2-7b", "llama3-8b")), _log(rng, 1, 40)
         longest = _log(rng, 4, min(1900 if model == "small-llama" else 4000 if model == "llama2-7b" else 7900, 7900 // n))
@@ -111,7 +111,25 @@ def _weights(case, seed, cfg):
                              device="cuda:0", seed=seed % 10007, fp8=case["weights"] == "fp8")
     if case["sample"]:  # a trained head is decided: few tokens share most of the probability
         w.lm_head = w.lm_head * 4
+    if cfg.hybrid:
+        _decide(w, cfg, torch.Generator().manual_seed(seed))
     return w
+
+
+def _decide(w, cfg, gen):
+    """Tokens lean towards some experts of every block, of as many groups as are kept: a trained router is decided, and its
+    choices do not turn on the last bit of a sum."""
+    lean = torch.zeros_like(w.embed, dtype=torch.float32)
+    for sp, lay in zip(cfg.layers, w.layers):
+        if sp.moe is None:
+            continue
+        m, size = sp.moe, sp.moe.experts // sp.moe.groups
+        score = torch.rand(cfg.vocab_size, m.groups, size, generator=gen)
+        drop = torch.topk(torch.rand(cfg.vocab_size, m.groups, generator=gen), m.groups - m.keep).indices
+        wish = torch.topk(score.scatter_(1, drop[:, :, None].expand(-1, -1, size), -1.0).flatten(1), m.top).indices.cuda()
+        for k in range(m.top):
+            lean += (16.0 / cfg.embed_scale) * lay.w_r.float()[wish[:, k]]
+    w.embed = (w.embed.float() + lean).to(w.embed.dtype)
 
 
 def _rows(n, case, cfg, gen):
@@ -124,8 +142,7 @@ def _rows(n, case, cfg, gen):
 
 
 def _decided(x, w, gen):
-    """Rows that lean towards some experts of every block, popular ones more often: a trained router is decided, and its
-    choices do not turn on the last bit of a sum."""
+    """Rows that lean towards some experts of every block, popular ones more often (see ``_decide``)."""
     for lay in w.layers if w.cfg.is_moe else ():
         r = lay.router.float()
         wish = torch.multinomial(torch.linspace(1.0, 0.3, r.shape[0]).expand(x.shape[0], -1), w.cfg.num_experts_per_tok,
@@ -267,7 +284,7 @@ def tolerance(case):
     """bf16 activations between 32-bit sums.  Against ``exact`` the uniform families are 0.003 to 0.02 off (a bf16 stream), the
     hybrid decoders 0.0035 to 0.011 (a 32-bit one); a token sampled from such logits may be another one."""
     out = {"rel": 0.06 if not _config(case).hybrid else 0.04}
-    return {**out, "differ": 0.5} if case["sample"] else out
+    return {**out, "differ": 0.6} if case["sample"] else out
 
 
 # ------------------------------------------------------------------ the same in 64 bits, plain torch
