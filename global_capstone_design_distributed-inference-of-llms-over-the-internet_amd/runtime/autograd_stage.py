@@ -12,12 +12,16 @@ Reference (vendored upstream server):
   adapters on their side.
 
 The inference hot path (paged KV, HIP kernels, hipGraphs) is not differentiable and does not
-need to be. This module is the training-time path: plain PyTorch ops on the stage's resident
-weights (the same tensors the executor uses; no copies).
-* GEMMs go through rocBLAS / hipBLASLt.
-* Attention is an explicit causal softmax in fp32.
-* Backward = recompute forward + ``torch.autograd.grad``, as upstream, so no activations are
-  held between the two RPCs.
+need to be. This module is the training-time path on the stage's resident weights (the same
+tensors the executor uses; no copies), in two forms:
+* kernels (``ops/train.py``): bf16 LLaMA / Mistral blocks on the GPU. The weights are frozen, so a
+  block's backward is written out: the forward of the span is made again, keeping per block its
+  input, q / k / v, the attention's output and gate / up rows, then the blocks are run backwards.
+  Attention never holds a [heads, T, T] tensor.
+* plain PyTorch ops for everything else (CPU, fp32, experts, GPT-2, callers that differentiate
+  ``forward`` themselves): attention is an explicit causal softmax in fp32, backward = recompute
+  forward + ``torch.autograd.grad``, as upstream.
+Either way GEMMs go through rocBLAS / hipBLASLt and no activations are held between the two RPCs.
 """
 from __future__ import annotations
 
@@ -27,7 +31,9 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
+from .. import ops
 from ..models.weights import split_gate_up
+from ..ops import train
 from ..ops.moe import moe_mlp_torch
 from ..ops.reference import rope_cos_sin
 
@@ -35,6 +41,23 @@ from ..ops.reference import rope_cos_sin
 def _rms(x, w, eps):
     xf = x.float()
     return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)).to(x.dtype) * w
+
+
+def _plain(*tensors) -> bool:
+    """Are these ordinary tensors in an ordinary call: no subclass, no transform (vmap, grad, forward mode), no tracing and
+    no dispatch mode that has to see every operation?"""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors) and
+            not torch.compiler.is_compiling() and not torch.jit.is_tracing() and
+            torch._C._functorch.peek_interpreter_stack() is None and
+            torch.autograd.forward_ad._current_level < 0 and
+            torch._C._len_torch_dispatch_stack() == 0 and
+            torch.overrides._get_current_function_mode() is None)
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """[B, T, H] as rows that the kernels read: contiguous and 16-byte aligned."""
+    t = t.reshape(-1, t.shape[-1]).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 class AutogradStage:
@@ -101,6 +124,65 @@ class AutogradStage:
         m = F.gelu(m @ lay.fc_w.t() + lay.fc_b, approximate="tanh")
         return x + m @ lay.fc2_w.t() + lay.fc2_b
 
+    # ------------------------------------------------------------------ blocks on kernels
+    def _kernels(self, hidden, prompts, *more) -> bool:
+        """Does the kernel form cover this call?  bf16 blocks it knows the shape of, whole weights on one GPU, at least one
+        token; a caller that differentiates the call itself (``backward`` does it without autograd) takes the other."""
+        given = [t for t in (hidden, prompts) + more if t is not None]
+        if self.device.type != "cuda" or self.dtype != torch.bfloat16 or not train.shape_ok(self.cfg) or not self.w.layers:
+            return False
+        if not _plain(*given) or hidden.dim() != 3 or not hidden.numel() or hidden.shape[2] != self.cfg.hidden_size:
+            return False
+        for lay in self.w.layers:
+            mats = [getattr(lay, n, None) for n in ("input_norm", "qkv", "o", "post_norm", "gate_up", "down")]
+            if any(m is None or m.dtype != torch.bfloat16 or not m.is_contiguous() or m.data_ptr() % 16 or m.requires_grad or
+                   m.device.type != "cuda" or m.device != mats[0].device for m in mats):
+                return False
+        ops.require_native()
+        return True
+
+    def _kernel_blocks(self, x, prompts, B, T, table, keep: bool):
+        """The span's blocks over the rows ``x`` [B T, H]: (rows out, what ``_kernel_grads`` reads of every block).  With
+        ``keep`` the last block ends at its gate / up rows: nothing of a gradient depends on what follows."""
+        cfg = self.cfg
+        nh, nkv, D, eps = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, cfg.rms_norm_eps
+        kept, y = [], None
+        for i, lay in enumerate(self.w.layers):
+            if prompts is not None and prompts.shape[2]:
+                x, y = (x.clone() if y is None else x + y), None
+                x.view(B, T, -1)[:, :prompts.shape[2]] += prompts[i]
+            x, h = train.norm(x, lay.input_norm, eps, y)
+            qkv = train.rope_(torch.mm(h, lay.qkv.t()), table, nh + nkv, D)
+            a, a32, lse = train.attention(qkv, B, nh, nkv, D, keep)
+            x2, h = train.norm(x, lay.post_norm, eps, torch.mm(a, lay.o.t()))
+            gu = torch.mm(h, lay.gate_up.t())
+            if keep:
+                kept.append((x, qkv, a32, lse, x2, gu))
+                if i == len(self.w.layers) - 1:
+                    return None, kept
+            x, y = x2, torch.mm(ops.swiglu(gu), lay.down.t())
+        return x + y, kept
+
+    def _kernel_grads(self, g, kept, prompts, B, T, table):
+        """Gradients of the blocks' input and of the prompts from the gradient ``g`` [B T, H] of their output."""
+        cfg = self.cfg
+        nh, nkv, D, eps = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, cfg.rms_norm_eps
+        gp = None if prompts is None else torch.empty_like(prompts)
+        for i in reversed(range(len(kept))):
+            lay, (x, qkv, a32, lse, x2, gu) = self.w.layers[i], kept.pop()
+            dgu = train.glu_grad_(gu, torch.mm(g, lay.down))
+            g = train.norm_grad(x2, torch.mm(dgu, lay.gate_up), lay.post_norm, eps, g)
+            dqkv = train.attention_grad(qkv, B, nh, nkv, D, a32, lse, torch.mm(g, lay.o), table)
+            g = train.norm_grad(x, torch.mm(dqkv, lay.qkv), lay.input_norm, eps, g)
+            if gp is not None:
+                d = g.view(B, T, -1)[:, :gp.shape[2]]
+                gp[i] = d.sum(0, keepdim=True) if gp.shape[1] == 1 else d
+        return g, gp
+
+    def _angles(self, T: int):
+        cfg = self.cfg
+        return train.angle_table(*rope_cos_sin(cfg.head_dim, T, cfg.rope_theta, self.device, cfg.rope_scaling))
+
     # ------------------------------------------------------------------ public API
     def forward(self, hidden: torch.Tensor, prompts: Optional[torch.Tensor] = None) -> torch.Tensor:
         """hidden [B, T, H]; prompts None or [n_blocks, B|1, P, H] (P <= T). Returns [B, T, H]."""
@@ -110,6 +192,11 @@ class AutogradStage:
             if prompts.dim() != 4 or prompts.shape[0] != self.n_blocks or prompts.shape[2] > x.shape[1]:
                 raise ValueError(f"prompts must be [{self.n_blocks}, B, P<=T, H], got {tuple(prompts.shape)}")
         T = x.shape[1]
+        if self._kernels(x, prompts) and not (torch.is_grad_enabled() and (
+                x.requires_grad or (prompts is not None and prompts.requires_grad))):
+            B = x.shape[0]
+            y, _ = self._kernel_blocks(_rows(x), prompts, B, T, self._angles(T), False)
+            return y.view(B, T, -1)
         cos = sin = None
         if self.cfg.model_type != "gpt2":
             cos, sin = rope_cos_sin(self.cfg.head_dim, T, self.cfg.rope_theta, self.device, self.cfg.rope_scaling)
@@ -122,7 +209,10 @@ class AutogradStage:
 
     def backward(self, hidden: torch.Tensor, grad_output: torch.Tensor,
                  prompts: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
-        """Recompute the forward with autograd and return (grad_hidden, grad_prompts)."""
+        """Recompute the forward and return (grad_hidden, grad_prompts)."""
+        got = self._backward_kernels(hidden, grad_output, prompts)
+        if got is not None:
+            return got
         with torch.enable_grad():
             x = hidden.detach().to(self.device, self.dtype).requires_grad_(True)
             p = None
@@ -135,3 +225,21 @@ class AutogradStage:
         if p is not None:
             gp = grads[1] if grads[1] is not None else torch.zeros_like(p)
         return grads[0], gp
+
+    def _backward_kernels(self, hidden, grad_output, prompts):
+        """``backward`` on the kernels, or None where they do not cover the call (the other form then raises what is to be
+        raised)."""
+        if not self._kernels(hidden, prompts, grad_output) or grad_output.shape != hidden.shape:
+            return None
+        B, T, H = hidden.shape
+        if prompts is not None and (prompts.dim() != 4 or prompts.shape[0] != self.n_blocks or prompts.shape[2] > T or
+                                    prompts.shape[1] not in (1, B) or prompts.shape[3] != H):
+            return None
+        with torch.no_grad():
+            x = _rows(hidden.to(self.device, self.dtype))
+            g = _rows(grad_output.to(self.device, self.dtype))
+            p = prompts.to(self.device, self.dtype) if prompts is not None else None
+            table = self._angles(T)
+            _, kept = self._kernel_blocks(x, p, B, T, table, True)
+            gx, gp = self._kernel_grads(g, kept, p, B, T, table)
+            return gx.view(B, T, H), gp
