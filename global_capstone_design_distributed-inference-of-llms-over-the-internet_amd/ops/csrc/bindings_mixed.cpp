@@ -28,6 +28,8 @@ int mp_moe_router_splits(int T, int W, int E, int f32);
 int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, const int32_t* ctx, float* part, int S, float* ew,
                  int32_t* idx, int32_t* slot, int32_t* lists, int32_t* tok, int T, int E, int W, int top, int groups,
                  int keep, float scale, int f32, hipStream_t stream);
+int mp_moe_combine(const void* y, int f32, const float* ew, const int32_t* slot, void* out, int64_t T, int top, int H,
+                   hipStream_t stream);
 int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt, const int32_t* tok, const int32_t* lists,
                 const void* w, void* out, int out_f32, int rows, int E, int N, int K, int block, float limit, int f32,
                 hipStream_t stream);
@@ -239,6 +241,20 @@ void moe_gemm(int64_t form, const at::Tensor& x, const opt_tensor& tok, const at
                "moe_gemm");
 }
 
+void moe_combine(const at::Tensor& y, const at::Tensor& ew, const at::Tensor& slot, at::Tensor& out) {
+  const int f32 = act_type(y, "y");
+  MP_CHECK(slot.dim() == 2 && out.dim() == 2 && out.is_cuda() && out.scalar_type() == at::kBFloat16 && out.is_contiguous() &&
+               out.size(0) == slot.size(0) && out.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0,
+           "out bf16 [T, H], H a multiple of 8");
+  const int64_t T = slot.size(0), top = slot.size(1);
+  MP_CHECK(top >= 1, "at least one choice");
+  check_rows(y, T * top, out.size(1), "y");
+  MP_CHECK(y.is_contiguous(), "y contiguous");
+  check_launch(mp_moe_combine(y.data_ptr(), f32, f32_vec(ew, T * top, "ew"), i32_vec(slot, T * top, "slot"), out.data_ptr(), T,
+                              top, out.size(1), cur_stream()),
+               "moe_combine");
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(mpamd, m) {
@@ -257,6 +273,7 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def(
       "moe_route(Tensor x, Tensor w, Tensor ctx, Tensor(a!) part, Tensor(b!) ew, Tensor(c!) idx, Tensor(d!) slot, "
       "Tensor(e!) lists, Tensor(f!) tok, int groups, int keep, float scale, int packed) -> ()");
+  m.def("moe_combine(Tensor y, Tensor ew, Tensor slot, Tensor(a!) out) -> ()");
   m.def(
       "moe_gemm(int form, Tensor x, Tensor? tok, Tensor lists, Tensor w, Tensor(a!) out, int rows, int tokens, int glu, "
       "int block, float limit, int packed) -> ()");
@@ -267,5 +284,6 @@ TORCH_LIBRARY_IMPL(mpamd, CUDA, m) {
   m.impl("ffn_act", &ffn_act);
   m.impl("mixed_attention", &mixed_attention);
   m.impl("moe_route", &moe_route);
+  m.impl("moe_combine", &moe_combine);
   m.impl("moe_gemm", &moe_gemm);
 }

@@ -1,16 +1,18 @@
-// Routed experts of the hybrid decoders: router, choice, and the experts' gated feed-forwards as grouped products.
+// Routed experts (hybrid decoders, Mixtral): router, choice, and the experts' gated feed-forwards as grouped products.
 //
 //   moe_router       logits[t, e] = x[t] . router[e] in 32-bit, over K slices
 //   moe_choose       softmax over all experts; a group of neighbouring experts counts as its best one; the ``top``
 //                    experts with the largest scores among the ``keep`` best groups; weights = scores / (sum + 1e-20)
 //                    * scale.  Every choice also gets its place among its expert's rows
 //   moe_place        rows sorted by expert: first row of every expert, the token of every row, the row of every choice
+//   moe_combine      every token's rows, weighed and added
 //   moe_gemm_any     any shape and both element types
 //   moe_gemm_rows    bf16, few rows per expert: weights stream once through registers in fragment order
 //   moe_gemm_tile    bf16, many rows per expert: 128 x 128 or 256 x 256 tiles through LDS
 //
 // The products come in two kinds: gathered rows x gate/up weights with the clamped gated form as epilogue
-// (GLU: out = g sigmoid(1.702 g) (u + 1), g <= limit, |u| <= limit), and sorted rows x down weights.
+// (GLU: out = g sigmoid(1.702 g) (u + 1), g <= limit, |u| <= limit; without a limit silu(g) u), and sorted rows x down
+// weights.
 #include "common.h"
 #include "act_io.h"
 
@@ -38,10 +40,12 @@ __device__ __forceinline__ int64_t act_at(int row, int col, int64_t xs, int mt) 
 }
 
 __device__ __forceinline__ float moe_glu(float g, float u, float limit) {
+  if (limit <= 0.f) return g / (1.f + __expf(-g)) * u;  // (uniform)
   const float a = fminf(g, limit), b = fminf(fmaxf(u, -limit), limit);
   return a / (1.f + __expf(-MOE_ALPHA * a)) * (b + 1.f);
 }
 __device__ __forceinline__ float moe_glu_exact(float g, float u, float limit) {
+  if (limit <= 0.f) return g / (1.f + expf(-g)) * u;
   const float a = fminf(g, limit), b = fminf(fmaxf(u, -limit), limit);
   return a / (1.f + expf(-MOE_ALPHA * a)) * (b + 1.f);
 }
@@ -563,6 +567,34 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
   }
 }
 
+// out[t] = sum over its choices of weight * row; a token without choices: 0.  A thread has 8 columns of a token; the rows of
+// its choices are read at once.  Bound by the rows' bytes in prompts (2700 tokens of two 4096-wide rows: 18 us for 66 MB) and
+// by its launch in decode steps (4.7 us, where one add per expert took 8 x 6).
+template <typename T>
+__global__ __launch_bounds__(256) void moe_combine_kernel(const T* __restrict__ y, const float* __restrict__ ew,
+                                                          const int32_t* __restrict__ slot, bf16_t* __restrict__ out, int top,
+                                                          int H, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int64_t t = i / (H / 8);
+  const int c = (int)(i % (H / 8)) * 8;
+  float acc[8] = {};
+  for (int k = 0; k < top; k += 4) {
+    float v[4][8], w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int32_t r = slot[t * top + min(k + j, top - 1)];
+      w[j] = k + j < top && r >= 0 ? ew[t * top + k + j] : 0.f;
+      ld_vec<8>(y + (int64_t)max(r, 0) * H + c, v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += w[j] == 0.f ? 0.f : w[j] * v[j][e];  // (rows never written are not counted)
+  }
+  st_vec<8>(out + t * H + c, acc);
+}
+
 template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
 static int launch_moe_tile(const MoeGemm& a, int rows, int act, hipStream_t stream) {
   constexpr int BM = 16 * MW * WM, BN = 16 * NW * WN, LDS = MG_P * (BM + BN) * 64;
@@ -623,6 +655,21 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
   const int per = (T + 256 * nw - 1) / (256 * nw), nb = (T + nw * per - 1) / (nw * per);
   hipLaunchKernelGGL(moe_choose_kernel, dim3(nb), dim3(nw * 64), lds, stream, a, per);
   if (nb > 1) hipLaunchKernelGGL(moe_place_kernel, dim3((T * top + 255) / 256), dim3(256), 0, stream, a);
+  return (int)hipGetLastError();
+}
+
+extern "C" int mp_moe_combine(const void* y, int f32, const float* ew, const int32_t* slot, void* out, int64_t T, int top,
+                              int H, hipStream_t stream) {
+  using namespace mp;
+  (void)hipGetLastError();
+  if (H % 8 || top < 1) return -1;
+  if (T == 0) return 0;
+  const int64_t n = T * (H / 8);
+  const dim3 g((unsigned)((n + 255) / 256));
+  if (f32)
+    hipLaunchKernelGGL((moe_combine_kernel<float>), g, dim3(256), 0, stream, (const float*)y, ew, slot, (bf16_t*)out, top, H, n);
+  else
+    hipLaunchKernelGGL((moe_combine_kernel<bf16_t>), g, dim3(256), 0, stream, (const bf16_t*)y, ew, slot, (bf16_t*)out, top, H, n);
   return (int)hipGetLastError();
 }
 

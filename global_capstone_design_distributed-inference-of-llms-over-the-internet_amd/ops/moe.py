@@ -8,20 +8,14 @@ framework's engine:
   renormalise the kept weights to sum to 1;
 * expert j: ``down_j(silu(gate_j h) * up_j h)``; token output = sum_j w_j * expert_j(h).
 
-MI355X execution strategy (runtime/executor.py ``_moe_mlp``):
+MI355X execution strategy: choice, sorting and grouped products run on kernels (csrc/moe.hip) and stay on the device at
+every size, so a step has no host sync, graphs capture it and only experts that were chosen are read.  The hybrid
+decoders' experts (group-limited routing, clamped gate) and Mixtral's (``mixtral_mlp``: plain top-k, silu gate) are the
+same kernels.
 
-* decode steps (T <= 64 rows) run EVERY expert on the whole (tiny) batch through the packed
-  weight-streaming GEMMs and combine with a dense [T, E] weight matrix whose unrouted
-  entries are zero.  A decode step is HBM-bound: at batch 64 with top-2 of 8 experts every
-  expert is routed to by some token (P(unused) = (6/8 * 5/7)^64 ~ 1e-10), so the bytes read
-  equal the sparse schedule's, the extra MFMA work is free at M <= 64, and the step has no
-  data-dependent shapes - it stays inside the hipGraph;
-* prefill (T > 64) groups tokens by expert (one host sync per layer, outside any graph),
-  runs each expert's GEMMs on its gathered rows and scatter-adds the weighted result.
-
-The hybrid decoders' experts (``choose`` / ``experts``: group-limited softmax routing, clamped gated experts) run on
-kernels of their own (csrc/moe.hip): choice, sorting and grouped products stay on the device at every size, so a step
-has no host sync and only experts that were chosen are read.
+Mixtral stages that these do not cover (the CPU, expert widths not in steps of 32, library GEMMs forced) keep the plain
+form (runtime/executor.py ``_moe_mlp``): decode steps run every expert on the whole batch and combine with a dense weight
+matrix, prompts group tokens by expert on the host.
 """
 from __future__ import annotations
 
@@ -170,6 +164,15 @@ def experts(x, c: Choice, up, down, up_p, down_p, block, e, packed=False):
                              int(packed))
     torch.ops.mpamd.moe_gemm(form, act, None, c.lists, down_p if form else down, y, R, c.tokens, 0, 1, 0.0, 0)
     return y
+
+
+def mixtral_mlp(x, ctx, router, up_p, down_p, spec, out, e, packed=False):
+    """Mixtral's sparse MLP of the rows ``x`` (row-major or packed) into ``out`` [T, W] bf16 (0 on padding rows, ``ctx`` 0).
+    ``spec``: a ``MoESpec`` without a limit; weights in packed form."""
+    c = choose(x, router, ctx, spec, e, packed=packed)
+    y = experts(x, c, None, None, up_p, down_p, GU_BLOCK, e, packed=packed)
+    torch.ops.mpamd.moe_combine(y, c.weights, c.slot, out)
+    return out
 
 
 # mean rows per expert from which the tiled products (128 and 256 rows a tile) run instead of the weight-streaming one

@@ -35,7 +35,7 @@ import torch
 
 from .. import native, ops
 from ..ops import moe
-from ..models.config import ModelConfig
+from ..models.config import ModelConfig, MoESpec
 from ..models.weights import StageWeights
 from .graphs import capture
 from .hybrid import HybridStage
@@ -757,7 +757,7 @@ class StageExecutor:
                 self._ar(o)
                 ops.rmsnorm(o, g_post, eps, out=xn, residual=res, mode=1, packed=True)
                 if L.moe:
-                    self._moe_mlp(L, xn, T, mlp, act, e, packed=True)
+                    self._moe_mlp(L, xn, T, mlp, act, e, q_ctx, packed=True)
                     continue
                 ops.linear(xn, L.gate_up, out=act, epilogue=1, wp=L.gate_up_p, a_rows=T, out_packed=True)
                 ops.linear(act, L.down, out=mlp, wp=L.down_p, a_rows=T)
@@ -793,7 +793,7 @@ class StageExecutor:
                 self._ar(o)
                 ops.rmsnorm(o, g_post, eps, out=xn, residual=res, mode=1)
                 if L.moe:
-                    self._moe_mlp(L, xn, T, mlp, act, e, packed=False)
+                    self._moe_mlp(L, xn, T, mlp, act, e, q_ctx, packed=False)
                     continue
                 ops.linear(xn, L.dense("gate_up"), out=act, epilogue=1, wp=gu_p)
                 ops.linear(act, L.dense("down"), out=mlp, wp=L.down_p)
@@ -990,12 +990,23 @@ class StageExecutor:
             u = self._ones = torch.ones(self.cfg.hidden_size, dtype=self.dtype, device=self.device)
         return u
 
-    def _moe_mlp(self, L, xn, T, mlp, act, e, packed: bool) -> None:
-        """Mixtral sparse-MoE MLP into ``mlp`` (ops/moe.py has the routing math and the
-        decode-vs-prefill strategy).  Decode steps run every expert on the whole batch with a
-        dense combine matrix: no host sync, so the step stays graph-capturable."""
+    def _moe_grouped(self, L) -> bool:
+        """Do the grouped expert kernels cover this Mixtral layer?"""
+        return (self.device.type == "cuda" and L.gate_up_p is not None and L.router.is_contiguous() and
+                ops.gemm_policy() != "hipblaslt" and
+                moe.expert_mfma_ok(self.cfg.intermediate_size, self.cfg.hidden_size, L.router.dtype))
+
+    def _moe_mlp(self, L, xn, T, mlp, act, e, q_ctx, packed: bool) -> None:
+        """Mixtral sparse-MoE MLP into ``mlp``: grouped expert kernels (ops/moe.py), else the plain form, whose
+        decode steps run every expert on the whole batch with a dense combine matrix: no host sync, so the step
+        stays graph-capturable."""
         cfg = self.cfg
         E, k, H = cfg.num_local_experts, cfg.num_experts_per_tok, cfg.hidden_size
+        if self._moe_grouped(L):
+            moe.mixtral_mlp(xn, q_ctx, L.router, L.gate_up_p, L.down_p, MoESpec(E, k, cfg.intermediate_size, 0.0), mlp, e,
+                            packed=packed)
+            self._ar(mlp)
+            return
         if packed:
             logits = ops.linear(xn, None, out=e("moe_logits", (T, 16 * L.router_p.shape[0])), wp=L.router_p,
                                 a_rows=T)[:, :E]

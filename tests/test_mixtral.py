@@ -153,3 +153,42 @@ def test_mixtral_gpu_matches_fp32_reference(graphs):
         nxt = torch.argmax(logits.float(), -1)
         seqs = [torch.cat([s, nxt[i:i + 1].cpu()]) for i, s in enumerate(seqs)]
         logits = ex.forward([("a", 1), ("b", 1)], nxt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,packed", [(1, True), (5, True), (16, True), (17, True), (64, True), (3, False), (65, False), (200, False),
+                                      (700, False)])
+@pytest.mark.parametrize("E,k,H,F", [(8, 2, 256, 96), (4, 1, 128, 512), (5, 3, 264 - 8, 64), (8, 8, 128, 32)])
+def test_grouped_experts_match_64_bits(T, packed, E, k, H, F):
+    """Router, choice, products of every form and the weighed sum.  bf16: inner activation and (long steps) rows are rounded
+    once each, 2^-9 root mean square at most, so 2^-7 covers the sum; choices are made decided by wide router logits."""
+    from src import ops
+    from src.models.config import MoESpec
+    from src.models.weights import interleave_gate_up
+
+    ops.require_native()
+    g = torch.Generator().manual_seed(T * 31 + E)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    router = torch.randn(E, H, generator=g).to(torch.bfloat16)
+    gate, up = (torch.randn(E, F, H, generator=g).div(H ** 0.5).to(torch.bfloat16) for _ in range(2))
+    down = torch.randn(E, H, F, generator=g).div(F ** 0.5).to(torch.bfloat16)
+    ctx = torch.ones(T, dtype=torch.int32)
+    if T > 2:
+        ctx[T // 2] = 0  # a padding row of a graph
+    xd = x.double()
+    p, idx = torch.softmax(xd @ router.double().t(), -1).topk(k, -1)
+    p = p / p.sum(-1, keepdim=True)
+    want = torch.zeros(T, H, dtype=torch.float64)
+    for j in range(E):
+        t, c = (idx == j).nonzero(as_tuple=True)
+        a = torch.nn.functional.silu(xd[t] @ gate[j].double().t()) * (xd[t] @ up[j].double().t())
+        want[t] += (a @ down[j].double().t()) * p[t, c, None]
+    want[ctx == 0] = 0
+    pack = lambda w: torch.stack([ops.pack_weight(m.contiguous()) for m in w.cuda()])  # noqa: E731
+    gu = torch.stack([interleave_gate_up(a, b) for a, b in zip(gate, up)])
+    rows = ops.pack_act(x.cuda()) if packed else x.cuda()
+    out = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+    moe.mixtral_mlp(rows, ctx.cuda(), router.cuda(), pack(gu), pack(down), MoESpec(E, k, F, 0.0), out,
+                    lambda n, s, d=torch.bfloat16: torch.empty(s, dtype=d, device="cuda"), packed=packed)
+    assert float((out.double().cpu() - want).norm() / want.norm()) < 2 ** -7
+    assert not out[ctx == 0].any()
