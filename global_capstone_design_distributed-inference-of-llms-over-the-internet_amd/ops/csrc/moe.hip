@@ -8,13 +8,15 @@
 //   moe_combine      every token's rows, weighed and added
 //   moe_gemm_any     any shape and both element types
 //   moe_gemm_rows    bf16, few rows per expert: weights stream once through registers in fragment order
-//   moe_gemm_tile    bf16, many rows per expert: 128 x 128 or 256 x 256 tiles through LDS
+//   moe_gemm_tile    bf16, many rows per expert: 128 x 128 or 256 x 256 tiles through an LDS ring
+//   moe_gemm_wide    bf16, many rows per expert, K in steps of 64: 256 x 256 tiles, whole cache lines of the rows
 //
 // The products come in two kinds: gathered rows x gate/up weights with the clamped gated form as epilogue
 // (GLU: out = g sigmoid(1.702 g) (u + 1), g <= limit, |u| <= limit; without a limit silu(g) u), and sorted rows x down
 // weights.
 #include "common.h"
 #include "act_io.h"
+#include <type_traits>
 
 namespace mp {
 
@@ -456,10 +458,43 @@ __global__ __launch_bounds__(256) void moe_gemm_rows_kernel(MoeGemm a) {
 // Many rows per expert: WM x WN waves of MW x NW fragment tiles (rows x weight rows), 32 columns a stage.  Both operands
 // arrive in LDS in fragment order (global_load_lds, 1 KiB a wave: packed weights as they lie, rows gathered by lane)
 // through a ring of MG_P slots, MG_P - 1 of them in flight.
+constexpr int MG_BAND = 8;
 constexpr int MG_P = 4;
 
 __device__ __forceinline__ int moe_tile_count(const MoeLists& l, int E, int i, int lane, int bm) {
   return i + lane < E ? (l.cnt[i + lane] + bm - 1) / bm : 0;
+}
+
+// which tile this workgroup makes (one wave): experts' row tiles in order, an expert's tiles in bands of MG_BAND row tiles, a
+// band's by weight rows, then rows; a contiguous run of them per XCD, whose 32 CUs then share few rows and few weights.  pick: expert (-1: none), weight tile, row tile
+__device__ __forceinline__ void moe_pick(const MoeLists& l, int E, int ntn, int bm, int* pick) {
+  const int lane = threadIdx.x & 63;
+  int total = 0;
+  for (int i = 0; i < E; i += 64) total += moe_tile_count(l, E, i, lane, bm);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, 64);
+  const int all = total * ntn, per = (all + 7) / 8;
+  const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  const bool on = ((int)blockIdx.x >> 3) < per && id < all;
+  if (lane == 0) pick[0] = -1;
+  int base = 0;
+  for (int i = 0; i < E && on; i += 64) {
+    const int c = moe_tile_count(l, E, i, lane, bm);
+    int x = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(x, d, 64);
+      if (lane >= d) x += y;
+    }
+    const int lo = (base + x - c) * ntn, hi = (base + x) * ntn;
+    if (id >= lo && id < hi) {
+      const int q = id - lo, band = q / (MG_BAND * ntn), h = min(MG_BAND, c - MG_BAND * band), r = q - band * MG_BAND * ntn;
+      pick[0] = i + lane;
+      pick[1] = r / h;
+      pick[2] = MG_BAND * band + r % h;
+    }
+    base += __shfl(x, 63, 64);
+  }
 }
 
 template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
@@ -471,34 +506,7 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
   const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ntn = (a.N + BN - 1) / BN;
-  if (wv == 0) {  // which tile: experts' row tiles in order, an expert's tiles by weight rows, then rows
-    int total = 0;
-    for (int i = 0; i < a.E; i += 64) total += moe_tile_count(l, a.E, i, lane, BM);
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, 64);
-    const int all = total * ntn, per = (all + 7) / 8;  // a contiguous run of tiles per XCD
-    const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-    const bool on = ((int)blockIdx.x >> 3) < per && id < all;
-    if (lane == 0) pick[0] = -1;
-    int base = 0;
-    for (int i = 0; i < a.E && on; i += 64) {
-      const int c = moe_tile_count(l, a.E, i, lane, BM);
-      int x = c;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-      }
-      const int lo = (base + x - c) * ntn, hi = (base + x) * ntn;
-      if (id >= lo && id < hi) {
-        pick[0] = i + lane;
-        pick[1] = (id - lo) / c;
-        pick[2] = (id - lo) % c;
-      }
-      base += __shfl(x, 63, 64);
-    }
-  }
+  if (wv == 0) moe_pick(l, a.E, (a.N + BN - 1) / BN, BM, pick);
   __syncthreads();
   const int e = pick[0];
   if (e < 0) return;
@@ -565,6 +573,154 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
       st_vec<4>((TO*)a.out + (int64_t)(r0 + m) * (GLU ? a.N / 2 : a.N) + (GLU ? o / 2 : o) + 4 * g4, y);
     }
   }
+}
+
+// Many rows per expert, K in steps of 64: 256 x 256 tiles, eight waves of 64 rows x 128 weight rows, 64 columns a stage in
+// two LDS slots.
+//   * Rows arrive 128 bytes at a time (8 rows an instruction), whole cache lines: 32-column stages fetch every line twice,
+//     and 256 rows of lines are the whole L1, so the second half came from L2 again.  The 16-byte chunks of a row are
+//     permuted by its low bits on the way in, which leaves the operand reads free of bank conflicts (none counted).
+//   * The operands of a half stage are read from LDS while the MFMAs of the half before it run, across the one barrier a
+//     stage has: behind it the other slot has landed for all waves and this one is free.
+//   * A wave whose 64 rows are past the expert's last only loads; the two waves of a SIMD have different rows, so a tile of
+//     up to 128 rows takes half the time.
+// Bound by MFMA issue and, in part, by waits for the next stage.  8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s;
+// the ring of 32-column stages took 687 us.  2700 tokens of two of eight 14336-wide experts of width 4096: up 1502 ->
+// 1253 us, down 803 -> 667 us; 4298 tokens of four of 32 1408-wide ones of 2048: 260 -> 208 us, 151 -> 128 us.  Measured and
+// left: four waves of 128 x 128 (the same time where the tiles are full, 5-10 % more elsewhere), a second barrier that
+// frees the slot sooner (6 % more), loads spread over the whole half stage (6 % more).
+template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * 64) void moe_gemm_wide_kernel(MoeGemm a) {
+  constexpr int BM = 16 * MW * WM, BN = 16 * NW * WN, XB = BM * 128, SLOT = XB + BN * 128;
+  constexpr int JX = BM / 8 / (WM * WN), JW = BN / 8 / (WM * WN);
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  __shared__ int pick[4];
+  const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (wv == 0) moe_pick(l, a.E, (a.N + BN - 1) / BN, BM, pick);
+  __syncthreads();
+  const int e = pick[0];
+  if (e < 0) return;
+  const int n0 = pick[1] * BN, m0 = pick[2] * BM, r0 = l.off[e], n = l.cnt[e], nt = a.N / 16, ks = a.K / 64;
+  const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * a.N * a.K;
+  uint32_t xo[JX], wo[JW];  // byte offsets of this wave's pieces of a stage (the launcher checks that they fit)
+#pragma unroll
+  for (int j = 0; j < JX; ++j) {
+    const int m = r0 + min(m0 + 8 * (JX * wv + j) + (lane >> 3), n - 1), row = a.tok ? a.tok[m] : m;
+    xo[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + 16 * ((lane & 7) ^ (lane >> 3));
+  }
+#pragma unroll
+  for (int j = 0; j < JW; ++j)
+    wo[j] = (uint32_t)min(n0 / 16 + (JW * wv + j) / 2, nt - 1) * (uint32_t)(a.K * 32) + 1024 * (j & 1) + lane * 16;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  typedef __attribute__((address_space(1))) const void* gptr_t;
+  auto issue = [&](int st) {
+    char* b = smem + (st & 1) * SLOT;
+    const char *xb_ = (const char*)a.x + st * 128, *wb_ = (const char*)w + (int64_t)st * 2048;
+#pragma unroll
+    for (int j = 0; j < JX; ++j)
+      __builtin_amdgcn_global_load_lds((gptr_t)(xb_ + xo[j]), (lptr_t)(b + (JX * wv + j) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < JW; ++j)
+      __builtin_amdgcn_global_load_lds((gptr_t)(wb_ + wo[j]), (lptr_t)(b + XB + (JW * wv + j) * 1024), 16, 0, 0);
+  };
+  const int wn = wv % WN, wm = wv / WN;  // (the waves of a SIMD, 4 apart, have different rows)
+  const int xrow = (16 * MW * wm + c16) * 128, x0 = xrow + 16 * (g4 ^ (c16 & 7)), x1 = xrow + 16 * ((4 + g4) ^ (c16 & 7));
+  const int w0 = XB + 2 * NW * wn * 1024 + lane * 16;
+  f32x4 acc[NW][MW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i)
+#pragma unroll
+    for (int j = 0; j < MW; ++j) acc[i][j] = (f32x4)(0.f);
+  u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
+  auto take = [&](int st, int h, u16x8(&xr)[MW], u16x8(&wr)[NW]) {
+    const char* b = smem + (st & 1) * SLOT;
+#pragma unroll
+    for (int j = 0; j < MW; ++j) xr[j] = *reinterpret_cast<const u16x8*>(b + (h ? x1 : x0) + j * 2048);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) wr[i] = *reinterpret_cast<const u16x8*>(b + w0 + (2 * i + h) * 1024);
+  };
+  auto multiply = [&](const u16x8(&xr)[MW], const u16x8(&wr)[NW]) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int j = 0; j < MW; ++j) acc[i][j] = mfma_bf(wr[i], xr[j], acc[i][j]);
+  };
+  issue(0);
+  if (ks > 1) issue(1);
+  if (ks > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(JX + JW) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_wait_barrier();
+  if (m0 + 16 * MW * wm >= n) {  // no rows: such a wave only loads, its SIMD is the other one's
+    for (int st = 0; st + 1 < ks; ++st) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_wait_barrier();
+      if (st + 2 < ks) issue(st + 2);
+    }
+    return;
+  }
+  take(0, 0, xa, wa);
+  auto half = [&](auto reads, auto loads) {
+    constexpr int R = decltype(reads)::value ? NW + MW : 0, L = decltype(loads)::value ? JX + JW : 0, M = MW * NW;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < (M - L) / 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      if (i < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto stage = [&](int st, auto next, auto load) {
+    __builtin_amdgcn_sched_barrier(0);
+    take(st, 1, xb, wb);
+    multiply(xa, wa);
+    half(std::true_type{}, std::false_type{});
+    if constexpr (decltype(next)::value) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_wait_barrier();  // stage st + 1 has landed for all waves, and all have read stage st
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(load)::value) issue(st + 2);
+      take(st + 1, 0, xa, wa);
+    }
+    multiply(xb, wb);
+    half(next, load);
+  };
+  typedef std::true_type yes;
+  typedef std::false_type no;
+  int st = 0;
+  for (; st + 2 < ks; ++st) stage(st, yes{}, yes{});
+  if (st + 1 < ks) stage(st++, yes{}, no{});
+  stage(st, no{}, no{});
+#pragma unroll
+  for (int j = 0; j < MW; ++j) {
+    const int m = m0 + 16 * (MW * wm + j) + c16;
+    if (m >= n) continue;
+#pragma unroll
+    for (int i = 0; i < NW; i += GLU ? 2 : 1) {
+      const int o = n0 + 16 * (NW * wn + i);
+      if (o >= a.N) continue;
+      float y[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = GLU ? moe_glu(acc[i][j][r], acc[GLU ? i + 1 : i][j][r], a.limit) : acc[i][j][r];
+      st_vec<4>((TO*)a.out + (int64_t)(r0 + m) * (GLU ? a.N / 2 : a.N) + (GLU ? o / 2 : o) + 4 * g4, y);
+    }
+  }
+}
+
+template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
+static int launch_moe_wide(const MoeGemm& a, int rows, int act, hipStream_t stream) {
+  constexpr int BM = 16 * MW * WM, BN = 16 * NW * WN, LDS = 2 * (BM + BN) * 128;
+  const int tiles = (rows / BM + act) * ((a.N + BN - 1) / BN);
+  (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO, MW, NW, WM, WN>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO, MW, NW, WM, WN>), dim3((tiles + 7) / 8 * 8), dim3(WM * WN * 64), LDS,
+                     stream, a);
+  return (int)hipGetLastError();
 }
 
 // out[t] = sum over its choices of weight * row; a token without choices: 0.  A thread has 8 columns of a token; the rows of
@@ -693,11 +849,14 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
       return (int)hipGetLastError();
     }
     if (mt > 0) return -1;
-    // 256 x 256 tiles where an expert's rows fill them, else 128 x 128
-    const bool big = form == 3;
-#define MP_MT(GLU_, TO_)                                                       \
-  return big ? launch_moe_tile<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
-             : launch_moe_tile<GLU_, TO_, 4, 4, 2, 2>(a, rows, act, stream);
+    // 256 x 256 tiles from 128 rows an expert on (ops/moe.py expert_form); where K is not in steps of 64, or a piece's
+    // byte offset does not fit 32 bits, the ring of 32-column stages: its 256 x 256 form from 384 rows on, else 128 x 128
+    const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31);
+    const bool big = form == 3 && rows >= 384 * E;
+#define MP_MT(GLU_, TO_)                                                        \
+  return wide  ? launch_moe_wide<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
+         : big ? launch_moe_tile<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
+               : launch_moe_tile<GLU_, TO_, 4, 4, 2, 2>(a, rows, act, stream);
     if (glu) MP_MT(true, bf16_t)
     if (out_f32) MP_MT(false, float)
     MP_MT(false, bf16_t)

@@ -159,7 +159,7 @@ def experts(x, c: Choice, up, down, up_p, down_p, block, e, packed=False):
             at += n
         return y
     form = 0 if up_p is None else expert_form(R, m.experts, packed)
-    y = e("moe_y", (R, W), dt if form > 1 else torch.float32)
+    y = e("moe_y", (R, W), dt if form > 1 and R >= NARROW_ROWS * m.experts else torch.float32)
     torch.ops.mpamd.moe_gemm(form, x, c.tok, c.lists, up_p if form else up, act, R, c.tokens, 1, block, float(m.limit),
                              int(packed))
     torch.ops.mpamd.moe_gemm(form, act, None, c.lists, down_p if form else down, y, R, c.tokens, 0, 1, 0.0, 0)
@@ -175,8 +175,13 @@ def mixtral_mlp(x, ctx, router, up_p, down_p, spec, out, e, packed=False):
     return out
 
 
-# mean rows per expert from which the tiled products (128 and 256 rows a tile) run instead of the weight-streaming one
-TILE_ROWS, BIG_TILE_ROWS = 48, 384
+# mean rows per expert from which the tiled products (128 and 256 rows a tile) run instead of the weight-streaming one.
+# 256-row tiles: at 160 rows 452 + 332 us against 717 + 417 us (8 experts of 4096 x 14336) and 108 + 40 against 144 + 74 us
+# (32 of 2048 x 1408); at 96 rows 411 + 299 against 446 + 216 us and 102 + 34 against 92 + 37 us.
+# The streaming product reads an expert's weights once per 64 rows but multiplies few rows with each: at 24 rows 410 + 212 us
+# against 347 + 219 us (8 experts) and 78 + 40 against 74 + 32 us (32), at 16 rows 357 + 185 against 358 + 234 us and 71 + 36
+# against 74 + 31 us.  Rows go out in the activations' type from NARROW_ROWS on, below that in 32 bits.
+TILE_ROWS, BIG_TILE_ROWS, NARROW_ROWS = 24, 128, 48
 
 
 def expert_form(rows: int, experts: int, packed: bool) -> int:

@@ -1,0 +1,54 @@
+"""Tiled expert products (csrc/moe.hip) at the edges of their tiles against 64-bit products."""
+import pytest
+import torch
+
+from src import ops
+from src.ops import moe
+
+pytestmark = pytest.mark.gpu
+
+# rows of the experts: none, one, ends of a wave's 64 rows, of half a tile, of a tile, of a band of 8 tiles
+COUNTS = {"small": [0, 1, 63, 64, 65], "tile": [127, 128, 129, 0, 255], "whole": [256, 257, 511], "band": [2049]}
+
+
+def _lists(counts):
+    E = len(counts)
+    off = [sum(counts[:i]) for i in range(E + 1)]
+    act = [e for e in range(E) if counts[e]]
+    return torch.tensor(counts + off + act + [0] * (E - len(act)) + [len(act)], dtype=torch.int32, device="cuda")
+
+
+@pytest.mark.parametrize("rows", COUNTS)
+@pytest.mark.parametrize("N,K", [(32, 64), (256, 128), (288, 192), (544, 320), (96, 96)])
+@pytest.mark.parametrize("form", [2, 3])
+def test_products(rows, N, K, form):
+    """Every output is one sum of K exact products in 32 bits, rounded to bf16: half a unit of 2^-7 at most; gated forms
+    round the gate's exponential too, far below that."""
+    ops.require_native()
+    counts = COUNTS[rows]
+    E, R = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(N + K + R)
+    T = R + 3
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16)
+    tok = torch.randint(0, T, (R,), generator=g, dtype=torch.int32)
+    w = torch.randn(E, N, K, generator=g).div(K ** 0.5).to(torch.bfloat16)
+    wp = torch.stack([ops.pack_weight(m) for m in w.cuda()])
+    lists, owner = _lists(counts), torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    z = torch.einsum("rk,rnk->rn", x.double()[tok.long()], w.double()[owner]) if R < 400 else \
+        torch.cat([x.double()[tok[owner == e].long()] @ w[e].double().t() for e in range(E)])
+    for glu, limit in ((0, 0.0), (1, 0.0), (1, 1.5)):
+        out = torch.full((R, N // 2 if glu else N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        torch.ops.mpamd.moe_gemm(form, x.cuda(), tok.cuda(), lists, wp, out, R, T, glu, 16, limit, 0)
+        want = z
+        if glu:
+            v = z.view(R, N // 32, 2, 16)
+            a, b = v[:, :, 0].reshape(R, -1), v[:, :, 1].reshape(R, -1)
+            want = torch.nn.functional.silu(a) * b if not limit else moe._glu(z, 16, limit)
+        assert float((out.double().cpu() - want).norm() / want.norm()) < 2.0 ** -8
+        again = torch.empty_like(out)
+        torch.ops.mpamd.moe_gemm(form, x.cuda(), tok.cuda(), lists, wp, again, R, T, glu, 16, limit, 0)
+        assert torch.equal(out, again)
+    rows_in = x.cuda()[tok.long().cuda()].contiguous()  # sorted rows, fp32 out
+    out = torch.full((R, N), float("nan"), device="cuda")
+    torch.ops.mpamd.moe_gemm(form, rows_in, None, lists, wp, out, R, T, 0, 1, 0.0, 0)
+    assert float((out.double().cpu() - z).norm() / z.norm()) < 1e-5
