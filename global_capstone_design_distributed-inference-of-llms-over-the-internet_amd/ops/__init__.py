@@ -1033,6 +1033,8 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
         raise RuntimeError(f"packed activations need the native decode GEMM (M={M}, N={N}, K={K})")
     if w is None:
         raise RuntimeError(f"no row-major weight for the hipBLASLt path (M={M}, N={N}, K={K})")
+    if policy != "hipblaslt" and prompt.ok(x, w, epilogue):
+        return prompt.gemm(x, w, out, epilogue, glu_limit)
     if epilogue == 0 and out is not None and out.is_contiguous() and out.dtype == x.dtype and \
             out.shape == (M, N) and x.dim() == 2:
         return torch.mm(x, w.t(), out=out)  # hipBLASLt straight into the caller's buffer (no copy)
@@ -1470,5 +1472,5 @@ def autotune_w8(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 12, rounds:
 
 
 # the hybrid decoders' ops (imported last: they dispatch through this module)
-from . import hybrid, mixers  # noqa: E402,F401
+from . import hybrid, mixers, prompt  # noqa: E402,F401
 from .moe import expert_mfma_ok  # noqa: E402,F401

@@ -1,0 +1,48 @@
+// torch custom-op registrations (namespace `mpamd`) of the prompt product (gemm_prompt.hip).  Same rules as bindings.cpp:
+// outputs come from the caller, launches go to the current stream, shapes and dtypes are checked here.
+#include <c10/hip/HIPGuard.h>
+
+#include "bind_check.h"
+
+extern "C" {
+int64_t mp_gemm_prompt_ws(int M, int N, int K);
+int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit, float* ws,
+                 hipStream_t stream);
+}
+
+namespace {
+
+int64_t gemm_prompt_ws(int64_t M, int64_t N, int64_t K) { return mp_gemm_prompt_ws((int)M, (int)N, (int)K); }
+
+// out[M, N'] = epilogue(x[M, K] w[N, K]^T)
+void gemm_prompt(const at::Tensor& x, const at::Tensor& w, at::Tensor& out, const c10::optional<at::Tensor>& ws, int64_t epi,
+               double limit) {
+  MP_CHECK(x.is_cuda() && w.is_cuda() && out.is_cuda() && x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "2-d GPU tensors");
+  MP_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16, "bf16");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  MP_CHECK(M >= 1 && K >= 64 && K % 64 == 0 && N >= 16 && N % 16 == 0 && w.size(1) == K, "K in steps of 64, N in steps of 16");
+  check_rows(x, M, K, "x");
+  check_rows(w, N, K, "w");
+  check_rows(out, M, epi == 1 ? N / 2 : N, "out");
+  MP_CHECK(w.is_contiguous() && out.is_contiguous() && out.size(0) == M && x.stride(0) % 8 == 0 && x.stride(0) >= K, "strides");
+  MP_CHECK(M * x.stride(0) < (1ll << 31) && N * K < (1ll << 31), "operands of at most 4 GiB");
+  const int64_t need = mp_gemm_prompt_ws((int)M, (int)N, (int)K);
+  MP_CHECK(need == 0 || ws.has_value(), "this shape needs a workspace");
+  const c10::hip::HIPGuard guard(x.device().index());
+  float* p = nullptr;
+  if (need) {
+    MP_CHECK(ws->is_cuda() && ws->scalar_type() == at::kFloat && ws->is_contiguous() && ws->numel() >= need, "workspace");
+    p = ws->data_ptr<float>();
+  }
+  check_launch(mp_gemm_prompt(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), M, N, K, epi, (float)limit, p, cur_stream()),
+               "gemm_prompt");
+}
+
+}  // namespace
+
+TORCH_LIBRARY_FRAGMENT(mpamd, m) {
+  m.def("gemm_prompt_ws(int M, int N, int K) -> int", &gemm_prompt_ws);
+  m.def("gemm_prompt(Tensor x, Tensor w, Tensor(a!) out, Tensor(b!)? ws, int epi, float limit) -> ()");
+}
+
+TORCH_LIBRARY_IMPL(mpamd, CUDA, m) { m.impl("gemm_prompt", &gemm_prompt); }

@@ -1,0 +1,185 @@
+// Products of prompt-sized steps: y[M, N'] = epilogue(x[M, K] w[N, K]^T), both operands row-major, 256 x 256 tiles of
+// wide_tile.h.  Epilogues: none; the gated forms over gate / up rows in blocks of 16 (silu(g) u, or with a limit
+// g sigmoid(1.702 g) (u + 1) on clamped inputs), N' = N / 2; max(y, 0)^2.  Everything up to the one store is 32 bits: next to
+// a library product and an activation kernel, the product's rows are neither written, read back nor rounded.
+//
+// Tiles that fill the 256 CUs go out whole, in bands of 8 row tiles and contiguous runs per XCD.  What is left over would
+// hold the chip for another whole tile's time with some of its CUs: up to 128 such tiles have their K cut into 2 or more
+// equal parts, one per CU, fp32 parts go to a workspace and a second kernel adds a tile's parts in order and stores it.
+// Workgroups of the same part are neighbours, so that an XCD's CUs still walk the same columns of shared rows (ranges that
+// begin anywhere, as many as CUs, lost that: 176 left-over tiles of K 11008 took 310 us, made whole 216 us).
+#include "act_io.h"
+#include "wide_tile.h"
+
+namespace mp {
+
+constexpr int GW_CUS = 256, GW_BAND = 8;
+constexpr int64_t GW_SLAB = 256 * 256;  // fp32 elements of a part
+// stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
+// tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
+constexpr int GW_SPLIT_STAGES = 24;
+
+struct GemmPrompt {
+  const bf16_t* x;
+  int64_t xs;
+  const bf16_t* w;
+  bf16_t* out;
+  int M, N, K;
+  float limit;
+  int mt, nt;      // row and weight tiles
+  int full, rest, parts;  // tiles made whole; tiles cut into parts
+  float* slabs;           // [parts][rest][8 waves][8][4][64 lanes][4]
+};
+
+__device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, int& n0) {
+  const int band = id / (GW_BAND * a.nt), h = min(GW_BAND, a.mt - GW_BAND * band), r = id - band * GW_BAND * a.nt;
+  m0 = (GW_BAND * band + r % h) * WideTile::BM;
+  n0 = r / h * WideTile::BN;
+}
+template <int EPI>
+__device__ __forceinline__ void gw_store(const GemmPrompt& a, int m, int o, const f32x4& v, const f32x4& u, int g4) {
+  float y[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (EPI == 1 && a.limit > 0.f) {
+      const float g = fminf(v[r], a.limit), w = fminf(fmaxf(u[r], -a.limit), a.limit);
+      y[r] = g / (1.f + __expf(-1.702f * g)) * (w + 1.f);
+    } else if (EPI == 1) {
+      y[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
+    } else if (EPI == 4) {
+      const float p = v[r] < 0.f ? 0.f : v[r];  // (not a number stays one)
+      y[r] = p * p;
+    } else {
+      y[r] = v[r];
+    }
+  }
+  st_vec<4>(a.out + (int64_t)m * (EPI == 1 ? a.N / 2 : a.N) + (EPI == 1 ? o / 2 : o) + 4 * g4, y);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_prompt_kernel(GemmPrompt a) {
+  typedef WideTile W;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4, ks = a.K / 64, b = blockIdx.x;
+  const int blocks = (a.full + 7) / 8 * 8;  // of whole tiles
+  int id, s0 = 0, n = ks, part = 0;
+  if (b < blocks) {
+    id = (b & 7) * (blocks / 8) + (b >> 3);
+    if (id >= a.full) return;
+  } else {
+    const int all = a.rest * a.parts, g = ((b - blocks) & 7) * ((all + 7) / 8) + ((b - blocks) >> 3);
+    if (g >= all) return;
+    part = g / a.rest, id = a.full + g % a.rest;
+    s0 = part * ks / a.parts, n = (part + 1) * ks / a.parts - s0;
+  }
+  int m0, n0;
+  gw_tile(a, id, m0, n0);
+  uint32_t xo[4], wo[4];  // (the launcher checks that they fit)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    xo[j] = (uint32_t)min(m0 + W::piece_row(j), a.M - 1) * (uint32_t)(a.xs * 2) + W::piece_byte();
+    wo[j] = (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
+  }
+  f32x4 acc[W::NW][W::MW];
+#pragma unroll
+  for (int i = 0; i < W::NW; ++i)
+#pragma unroll
+    for (int j = 0; j < W::MW; ++j) acc[i][j] = (f32x4)(0.f);
+  const int mw = m0 + 16 * W::MW * W::wm(), nw = n0 + 16 * W::NW * W::wn();
+  const char *x = (const char*)a.x + s0 * 128, *w = (const char*)a.w + s0 * 128;
+  W::run<false>(smem, x, w, xo, wo, n, mw < a.M, acc);
+  if (mw >= a.M) return;
+  if (n == ks) {
+#pragma unroll
+    for (int j = 0; j < W::MW; ++j) {
+      const int m = mw + 16 * j + c16;
+      if (m >= a.M) continue;
+#pragma unroll
+      for (int i = 0; i < W::NW; i += EPI == 1 ? 2 : 1)
+        if (nw + 16 * i < a.N) gw_store<EPI>(a, m, nw + 16 * i, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], g4);
+    }
+  } else {
+    float* s = a.slabs + (part * a.rest + id - a.full) * GW_SLAB + (W::wave() * 32 * 64 + lane) * 4;
+#pragma unroll
+    for (int i = 0; i < W::NW; ++i)
+#pragma unroll
+      for (int j = 0; j < W::MW; ++j) *reinterpret_cast<f32x4*>(s + (i * 4 + j) * 256) = acc[i][j];
+  }
+}
+
+// a left-over tile's parts added and stored; blockIdx.y: two of the eight row groups of weights, two of the four of rows
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_prompt_close_kernel(GemmPrompt a) {
+  typedef WideTile W;
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4, r = blockIdx.x;
+  const int i0 = 2 * (blockIdx.y >> 1), j0 = 2 * (blockIdx.y & 1);
+  int m0, n0;
+  gw_tile(a, a.full + r, m0, n0);
+  const int m = m0 + 16 * (W::MW * W::wm() + j0) + c16, o = n0 + 16 * (W::NW * W::wn() + i0);
+  if (m0 + 16 * W::MW * W::wm() >= a.M || o >= a.N) return;
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4)(0.f);
+  for (int p = 0; p < a.parts; ++p) {
+    const float* s = a.slabs + (p * a.rest + r) * GW_SLAB + ((W::wave() * 32 + i0 * 4 + j0) * 64 + lane) * 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += *reinterpret_cast<const f32x4*>(s + (i * 4 + j) * 256);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (m + 16 * j >= a.M) continue;
+#pragma unroll
+    for (int i = 0; i < 2; i += EPI == 1 ? 2 : 1)
+      if (o + 16 * i < a.N) gw_store<EPI>(a, m + 16 * j, o + 16 * i, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], g4);
+  }
+}
+
+// into how many parts the tiles past the last whole wave of CUs are cut (1: they are made whole like the others): where
+// the stages that a CU saves are worth the parts' way through memory
+static int gw_parts(int tiles, int ks) {
+  const int rest = tiles % GW_CUS;
+  if (!rest || ks < 8) return 1;
+  const int parts = GW_CUS / rest < ks / 4 ? GW_CUS / rest : ks / 4;  // (at least four stages a part)
+  return ks - (ks + parts - 1) / parts >= GW_SPLIT_STAGES ? parts : 1;
+}
+
+}  // namespace mp
+
+// fp32 elements of the workspace
+extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K) {
+  using namespace mp;
+  const int tiles = ((M + 255) / 256) * ((N + 255) / 256), parts = gw_parts(tiles, K / 64);
+  return parts > 1 ? parts * (tiles % GW_CUS) * GW_SLAB : 0;
+}
+
+extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit,
+                            float* ws, hipStream_t stream) {
+  (void)hipGetLastError();
+  using namespace mp;
+  if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31))
+    return -1;
+  if (epi == 1 && N % 32) return -2;
+  GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, (M + 255) / 256, (N + 255) / 256, 0, 0, 1, ws};
+  const int tiles = a.mt * a.nt;
+  a.parts = gw_parts(tiles, K / 64);
+  a.rest = a.parts > 1 ? tiles % GW_CUS : 0;
+  if (a.rest && ws == nullptr) return -3;
+  a.full = tiles - a.rest;
+  const dim3 grid((a.full + 7) / 8 * 8 + (a.rest * a.parts + 7) / 8 * 8);
+#define MP_GW(E_)                                                                                                          \
+  {                                                                                                                        \
+    (void)hipFuncSetAttribute((const void*)gemm_prompt_kernel<E_>, hipFuncAttributeMaxDynamicSharedMemorySize, WideTile::LDS); \
+    hipLaunchKernelGGL((gemm_prompt_kernel<E_>), grid, dim3(512), WideTile::LDS, stream, a);                                  \
+    if (a.rest) hipLaunchKernelGGL((gemm_prompt_close_kernel<E_>), dim3(a.rest, 8), dim3(512), 0, stream, a);                 \
+  }
+  if (epi == 0) MP_GW(0)
+  else if (epi == 1) MP_GW(1)
+  else if (epi == 4) MP_GW(4)
+  else return -4;
+#undef MP_GW
+  return (int)hipGetLastError();
+}

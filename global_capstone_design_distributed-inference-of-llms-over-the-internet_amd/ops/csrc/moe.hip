@@ -16,7 +16,7 @@
 // weights.
 #include "common.h"
 #include "act_io.h"
-#include <type_traits>
+#include "wide_tile.h"
 
 namespace mp {
 
@@ -575,134 +575,44 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
   }
 }
 
-// Many rows per expert, K in steps of 64: 256 x 256 tiles, eight waves of 64 rows x 128 weight rows, 64 columns a stage in
-// two LDS slots.
-//   * Rows arrive 128 bytes at a time (8 rows an instruction), whole cache lines: 32-column stages fetch every line twice,
-//     and 256 rows of lines are the whole L1, so the second half came from L2 again.  The 16-byte chunks of a row are
-//     permuted by its low bits on the way in, which leaves the operand reads free of bank conflicts (none counted).
-//   * The operands of a half stage are read from LDS while the MFMAs of the half before it run, across the one barrier a
-//     stage has: behind it the other slot has landed for all waves and this one is free.
-//   * A wave whose 64 rows are past the expert's last only loads; the two waves of a SIMD have different rows, so a tile of
-//     up to 128 rows takes half the time.
-// Bound by MFMA issue and, in part, by waits for the next stage.  8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s;
-// the ring of 32-column stages took 687 us.  2700 tokens of two of eight 14336-wide experts of width 4096: up 1502 ->
-// 1253 us, down 803 -> 667 us; 4298 tokens of four of 32 1408-wide ones of 2048: 260 -> 208 us, 151 -> 128 us.  Measured and
-// left: four waves of 128 x 128 (the same time where the tiles are full, 5-10 % more elsewhere), a second barrier that
-// frees the slot sooner (6 % more), loads spread over the whole half stage (6 % more).
-template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void moe_gemm_wide_kernel(MoeGemm a) {
-  constexpr int BM = 16 * MW * WM, BN = 16 * NW * WN, XB = BM * 128, SLOT = XB + BN * 128;
-  constexpr int JX = BM / 8 / (WM * WN), JW = BN / 8 / (WM * WN);
+// Many rows per expert, K in steps of 64: 256 x 256 tiles (wide_tile.h) of gathered rows and packed weights.
+// 8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s; the ring of 32-column stages took 687 us.  2700 tokens of two of
+// eight 14336-wide experts of width 4096: up 1502 -> 1253 us, down 803 -> 667 us; 4298 tokens of four of 32 1408-wide ones of
+// 2048: 260 -> 208 us, 151 -> 128 us.
+template <bool GLU, typename TO>
+__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a) {
+  typedef WideTile W;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ int pick[4];
   const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
-  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (wv == 0) moe_pick(l, a.E, (a.N + BN - 1) / BN, BM, pick);
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+  if (W::wave() == 0) moe_pick(l, a.E, (a.N + W::BN - 1) / W::BN, W::BM, pick);
   __syncthreads();
   const int e = pick[0];
   if (e < 0) return;
-  const int n0 = pick[1] * BN, m0 = pick[2] * BM, r0 = l.off[e], n = l.cnt[e], nt = a.N / 16, ks = a.K / 64;
+  const int n0 = pick[1] * W::BN, m0 = pick[2] * W::BM, r0 = l.off[e], n = l.cnt[e], nt = a.N / 16;
   const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * a.N * a.K;
-  uint32_t xo[JX], wo[JW];  // byte offsets of this wave's pieces of a stage (the launcher checks that they fit)
+  uint32_t xo[4], wo[4];  // (the launcher checks that they fit)
 #pragma unroll
-  for (int j = 0; j < JX; ++j) {
-    const int m = r0 + min(m0 + 8 * (JX * wv + j) + (lane >> 3), n - 1), row = a.tok ? a.tok[m] : m;
-    xo[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + 16 * ((lane & 7) ^ (lane >> 3));
+  for (int j = 0; j < 4; ++j) {
+    const int m = r0 + min(m0 + W::piece_row(j), n - 1), row = a.tok ? a.tok[m] : m;
+    xo[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + W::piece_byte();
+    wo[j] = (uint32_t)min(n0 / 16 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
   }
+  f32x4 acc[W::NW][W::MW];
 #pragma unroll
-  for (int j = 0; j < JW; ++j)
-    wo[j] = (uint32_t)min(n0 / 16 + (JW * wv + j) / 2, nt - 1) * (uint32_t)(a.K * 32) + 1024 * (j & 1) + lane * 16;
-  typedef __attribute__((address_space(3))) void* lptr_t;
-  typedef __attribute__((address_space(1))) const void* gptr_t;
-  auto issue = [&](int st) {
-    char* b = smem + (st & 1) * SLOT;
-    const char *xb_ = (const char*)a.x + st * 128, *wb_ = (const char*)w + (int64_t)st * 2048;
+  for (int i = 0; i < W::NW; ++i)
 #pragma unroll
-    for (int j = 0; j < JX; ++j)
-      __builtin_amdgcn_global_load_lds((gptr_t)(xb_ + xo[j]), (lptr_t)(b + (JX * wv + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < W::MW; ++j) acc[i][j] = (f32x4)(0.f);
+  const int mw = m0 + 16 * W::MW * W::wm(), nw = n0 + 16 * W::NW * W::wn();
+  W::run<true>(smem, (const char*)a.x, (const char*)w, xo, wo, a.K / 64, mw < n, acc);
 #pragma unroll
-    for (int j = 0; j < JW; ++j)
-      __builtin_amdgcn_global_load_lds((gptr_t)(wb_ + wo[j]), (lptr_t)(b + XB + (JW * wv + j) * 1024), 16, 0, 0);
-  };
-  const int wn = wv % WN, wm = wv / WN;  // (the waves of a SIMD, 4 apart, have different rows)
-  const int xrow = (16 * MW * wm + c16) * 128, x0 = xrow + 16 * (g4 ^ (c16 & 7)), x1 = xrow + 16 * ((4 + g4) ^ (c16 & 7));
-  const int w0 = XB + 2 * NW * wn * 1024 + lane * 16;
-  f32x4 acc[NW][MW];
-#pragma unroll
-  for (int i = 0; i < NW; ++i)
-#pragma unroll
-    for (int j = 0; j < MW; ++j) acc[i][j] = (f32x4)(0.f);
-  u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
-  auto take = [&](int st, int h, u16x8(&xr)[MW], u16x8(&wr)[NW]) {
-    const char* b = smem + (st & 1) * SLOT;
-#pragma unroll
-    for (int j = 0; j < MW; ++j) xr[j] = *reinterpret_cast<const u16x8*>(b + (h ? x1 : x0) + j * 2048);
-#pragma unroll
-    for (int i = 0; i < NW; ++i) wr[i] = *reinterpret_cast<const u16x8*>(b + w0 + (2 * i + h) * 1024);
-  };
-  auto multiply = [&](const u16x8(&xr)[MW], const u16x8(&wr)[NW]) {
-#pragma unroll
-    for (int i = 0; i < NW; ++i)
-#pragma unroll
-      for (int j = 0; j < MW; ++j) acc[i][j] = mfma_bf(wr[i], xr[j], acc[i][j]);
-  };
-  issue(0);
-  if (ks > 1) issue(1);
-  if (ks > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(JX + JW) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  lds_wait_barrier();
-  if (m0 + 16 * MW * wm >= n) {  // no rows: such a wave only loads, its SIMD is the other one's
-    for (int st = 0; st + 1 < ks; ++st) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      lds_wait_barrier();
-      if (st + 2 < ks) issue(st + 2);
-    }
-    return;
-  }
-  take(0, 0, xa, wa);
-  auto half = [&](auto reads, auto loads) {
-    constexpr int R = decltype(reads)::value ? NW + MW : 0, L = decltype(loads)::value ? JX + JW : 0, M = MW * NW;
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < (M - L) / 2; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-      if (i < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto stage = [&](int st, auto next, auto load) {
-    __builtin_amdgcn_sched_barrier(0);
-    take(st, 1, xb, wb);
-    multiply(xa, wa);
-    half(std::true_type{}, std::false_type{});
-    if constexpr (decltype(next)::value) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      lds_wait_barrier();  // stage st + 1 has landed for all waves, and all have read stage st
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (decltype(load)::value) issue(st + 2);
-      take(st + 1, 0, xa, wa);
-    }
-    multiply(xb, wb);
-    half(next, load);
-  };
-  typedef std::true_type yes;
-  typedef std::false_type no;
-  int st = 0;
-  for (; st + 2 < ks; ++st) stage(st, yes{}, yes{});
-  if (st + 1 < ks) stage(st++, yes{}, no{});
-  stage(st, no{}, no{});
-#pragma unroll
-  for (int j = 0; j < MW; ++j) {
-    const int m = m0 + 16 * (MW * wm + j) + c16;
+  for (int j = 0; j < W::MW; ++j) {
+    const int m = mw + 16 * j + c16;
     if (m >= n) continue;
 #pragma unroll
-    for (int i = 0; i < NW; i += GLU ? 2 : 1) {
-      const int o = n0 + 16 * (NW * wn + i);
+    for (int i = 0; i < W::NW; i += GLU ? 2 : 1) {
+      const int o = nw + 16 * i;
       if (o >= a.N) continue;
       float y[4];
 #pragma unroll
@@ -712,14 +622,12 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_wide_kernel(MoeGemm a) 
   }
 }
 
-template <bool GLU, typename TO, int MW, int NW, int WM, int WN>
+template <bool GLU, typename TO>
 static int launch_moe_wide(const MoeGemm& a, int rows, int act, hipStream_t stream) {
-  constexpr int BM = 16 * MW * WM, BN = 16 * NW * WN, LDS = 2 * (BM + BN) * 128;
-  const int tiles = (rows / BM + act) * ((a.N + BN - 1) / BN);
-  (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO, MW, NW, WM, WN>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO, MW, NW, WM, WN>), dim3((tiles + 7) / 8 * 8), dim3(WM * WN * 64), LDS,
-                     stream, a);
+  const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN);
+  (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            WideTile::LDS);
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3((tiles + 7) / 8 * 8), dim3(512), WideTile::LDS, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -854,7 +762,7 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
     const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31);
     const bool big = form == 3 && rows >= 384 * E;
 #define MP_MT(GLU_, TO_)                                                        \
-  return wide  ? launch_moe_wide<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
+  return wide  ? launch_moe_wide<GLU_, TO_>(a, rows, act, stream) \
          : big ? launch_moe_tile<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
                : launch_moe_tile<GLU_, TO_, 4, 4, 2, 2>(a, rows, act, stream);
     if (glu) MP_MT(true, bf16_t)

@@ -1,0 +1,169 @@
+"""Products of prompt-sized steps (csrc/gemm_prompt.hip) and when they run in place of the library's.
+
+``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel.
+The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
+on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs:
+
+* shapes in the committed table (``python -m src.ops.tune --prompt``: every projection of every preset, steps of up to 8192
+  rows) run here at the row-tile counts where this kernel was at least as fast at all three row counts timed inside the
+  tile, and 3 % faster on average;
+* other shapes run here where even the library's best rate loses: no whole wave of tiles, a long K (160 stages of 64) whose
+  parts fill the CUs.  4096 x 14336: 400 rows 599 against 799 TFLOP/s, 1030 rows 958 / 1090, 1800 rows 1153 / 1251;
+  8192 x 28672, 131 rows 203 / 479.  With fewer parts than 218 on the 256 CUs it loses (8192 x 28672, 520 rows: 962 / 710).
+"""
+from __future__ import annotations
+
+import json
+import os
+import threading
+from typing import Dict, FrozenSet, Iterable, Optional, Tuple
+
+import torch
+
+TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "prompt_gemm_gfx950.json")
+EPILOGUES = (0, 1, 4)
+TILE, CUS, MAX_ROWS = 256, 256, 8192
+Shape = Tuple[int, int, int]  # N, K, epilogue
+
+_LOCK = threading.Lock()
+_STATE: dict = {"table": None}
+
+
+def _key(shape: Shape) -> str:
+    return "N%dxK%de%d" % shape
+
+
+def _load(path: str) -> Dict[Shape, FrozenSet[int]]:
+    with open(path) as f:
+        t = json.load(f)
+    out = {}
+    for s, tiles in t.get("tiles", {}).items():
+        n, rest = s[1:].split("xK")
+        k, e = rest.split("e")
+        out[(int(n), int(k), int(e))] = frozenset(tiles)
+    return out
+
+
+def table() -> Dict[Shape, FrozenSet[int]]:
+    """(N, K, epilogue) -> row-tile counts at which the kernel runs (read once; MPAMD_KERNEL_TABLE=0: none)."""
+    with _LOCK:
+        if _STATE["table"] is None:
+            on = os.environ.get("MPAMD_KERNEL_TABLE") != "0" and os.path.exists(TABLE)
+            _STATE["table"] = _load(TABLE) if on else {}
+        return _STATE["table"]
+
+
+def shape_ok(M: int, N: int, K: int, epilogue: int) -> bool:
+    """Does the kernel cover the shape?  (Byte offsets of a piece are 32 bits.)"""
+    return (epilogue in EPILOGUES and M >= 1 and K >= 64 and K % 64 == 0 and N % (32 if epilogue == 1 else 16) == 0 and
+            N >= 16 and M * K < 1 << 31 and N * K < 1 << 31)
+
+
+def chosen(M: int, N: int, K: int, epilogue: int) -> bool:
+    """Does a step of M rows run this product here?"""
+    if M <= TILE or M > MAX_ROWS or not shape_ok(M, N, K, epilogue):
+        return False
+    m = -(-M // TILE)
+    tiles = table().get((N, K, epilogue))
+    if tiles is not None:
+        return m in tiles
+    n = m * -(-N // TILE)
+    return K >= 160 * 64 and n < CUS and CUS // n >= 2 and CUS // n * n >= 218
+
+
+def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
+    """Is this product of rows [M, K] with weights [N, K] one that runs here?  Callers that differentiate it, and operands
+    the kernel does not read (other types, strides, alignments), keep the library's."""
+    if w is None or x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        return False
+    if not (chosen(x.shape[0], w.shape[0], w.shape[1], epilogue) and x.shape[1] == w.shape[1] and x.is_cuda and
+            w.device == x.device and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0 and
+            x.stride(0) >= x.shape[1] and x.shape[0] * x.stride(0) < 1 << 31):
+        return False
+    return x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not (
+        torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+
+
+def gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, epilogue: int = 0, limit: float = 0.0):
+    """epilogue 0: x w^T; 1: the gated forms over gate / up rows in blocks of 16 (``limit`` 0: silu); 4: max(., 0)^2."""
+    M, (N, K) = x.shape[0], w.shape
+    cols = N // 2 if epilogue == 1 else N
+    y = out if out is not None and out.is_contiguous() and out.dtype == x.dtype and out.data_ptr() % 16 == 0 else \
+        torch.empty(M, cols, dtype=x.dtype, device=x.device)
+    need = torch.ops.mpamd.gemm_prompt_ws(M, N, K)
+    ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+    torch.ops.mpamd.gemm_prompt(x, w, y, ws, epilogue, limit)
+    return y if out is None or y is out else out.copy_(y)
+
+
+# ------------------------------------------------------------------ the table
+def shapes(cfg) -> Iterable[Shape]:
+    """Row-major projections of a model's prompts."""
+    H = cfg.hidden_size
+    out = set()
+    if cfg.hybrid:
+        for sp in cfg.layers:
+            out |= {(sp.in_rows, H, 0), (H, sp.o_cols, 0)}
+            if sp.mixer == "latent_attention":
+                out.add((sp.q_rows, sp.q_rank, 0))
+            if sp.ff and not sp.parallel:
+                out |= {(sp.ff_rows, H, 1 if sp.glu else 4 if sp.ffn == "relu2" else 0), (H, sp.ff, 0)}
+        if cfg.injects:
+            out.add((H, 2 * H, 0))
+    elif cfg.model_type != "gpt2":
+        out = {(cfg.q_dim + 2 * cfg.kv_dim, H, 0), (H, cfg.q_dim, 0)}
+        if not cfg.is_moe:
+            out |= {(2 * cfg.intermediate_size, H, 1), (H, cfg.intermediate_size, 0)}
+    return sorted(s for s in out if shape_ok(MAX_ROWS, *s) and s[0] * s[1] >= 1 << 22)
+
+
+def tune(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
+    """Time both products over the row-tile counts of every shape, best of three rounds in turn."""
+    from . import hybrid, require_native, swiglu, use_tuned_gemms
+
+    require_native()
+    use_tuned_gemms()
+
+    def ms(f, n=4):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        f()
+        a.record()
+        for _ in range(n):
+            f()
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) / n
+
+    got = {}
+    for N, K, epi in todo:
+        w = torch.empty(N, K, device=device).normal_(0, 0.02).to(torch.bfloat16)
+        tiles = []
+        for m in range(2, MAX_ROWS // TILE + 1):
+            ratios = []
+            for M in (TILE * m - 251, TILE * m - 124, TILE * m):
+                x = torch.randn(M, K, device=device).to(torch.bfloat16)
+                z = torch.empty(M, N, dtype=x.dtype, device=device)
+                y = torch.empty(M, N // 2 if epi == 1 else N, dtype=x.dtype, device=device)
+
+                def lib():
+                    torch.mm(x, w.t(), out=z)
+                    if epi == 1:
+                        swiglu(z, out=y)
+                    elif epi == 4:
+                        hybrid.relu2(z, y)
+
+                t = [min(v) for v in zip(*[(ms(lib), ms(lambda: gemm(x, w, y, epi))) for _ in range(3)])]
+                ratios.append(t[0] / t[1])
+            if min(ratios) >= 1.0 and sum(ratios) / 3 >= 1.03:
+                tiles.append(m)
+        got[(N, K, epi)] = tiles
+        if log:
+            log(f"{_key((N, K, epi))}: {tiles}")
+    return got
+
+
+def save(path: str, got: Dict[Shape, list]) -> None:
+    with open(path, "w") as f:
+        f.write('{\n "arch": "gfx950",\n "tiles": {\n')
+        f.write(",\n".join(f'  "{_key(s)}": {json.dumps(got[s])}' for s in sorted(got)))
+        f.write("\n }\n}\n")

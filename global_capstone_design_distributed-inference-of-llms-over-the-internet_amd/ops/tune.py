@@ -10,6 +10,9 @@ end-to-end qkv-fold A/B of each decode batch in ``--batches``.  The resulting ch
 per (row bucket, N, K, epilogue) and one fold decision per (graph batch bucket, N, K) - are
 written as JSON.  Executors load that file by default, so every box running the tree runs the
 same kernel mix (``ops.load_kernel_table``) and bench records carry its sha.
+
+``--prompt`` writes the table of prompt products (``ops.prompt.TABLE``) instead: every projection of every preset, both
+kernels timed over the row-tile counts of steps of up to 8192 rows.
 """
 from __future__ import annotations
 
@@ -20,6 +23,20 @@ import sys
 import time
 
 
+def tune_prompt(out=None) -> int:
+    import torch
+
+    from ..models.config import PRESETS
+    from . import prompt
+
+    if not torch.cuda.is_available():
+        print("tune: needs an MI355X", file=sys.stderr)
+        return 2
+    todo = sorted({s for cfg in PRESETS.values() for s in prompt.shapes(cfg)})
+    prompt.save(out or prompt.TABLE, prompt.tune(todo, log=lambda m: print(f"tune: {m}", file=sys.stderr, flush=True)))
+    return 0
+
+
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description=__doc__.split("\n\n")[0])
     ap.add_argument("--models", default="small-llama,tiny-llama,llama2-7b,llama3-8b,llama3-70b:fp8",
@@ -27,7 +44,10 @@ def main(argv=None) -> int:
     ap.add_argument("--batches", default="64", help="decode batches whose qkv-fold A/B is pinned")
     ap.add_argument("--prompt-len", type=int, default=128)
     ap.add_argument("--out", default=None, help="default: the committed table path")
+    ap.add_argument("--prompt", action="store_true", help="time the prompt products of every preset")
     a = ap.parse_args(argv)
+    if a.prompt:
+        return tune_prompt(a.out)
     os.environ["MPAMD_KERNEL_TABLE"] = "0"   # time everything: nothing pre-loaded
     os.environ.setdefault("MPAMD_GEMM_AUTOTUNE", "1")
     import torch

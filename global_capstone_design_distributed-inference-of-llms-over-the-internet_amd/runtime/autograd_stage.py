@@ -18,10 +18,10 @@ tensors the executor uses; no copies), in two forms:
   block's backward is written out: the forward of the span is made again, keeping per block its
   input, q / k / v, the attention's output and gate / up rows, then the blocks are run backwards.
   Attention never holds a [heads, T, T] tensor.
-* plain PyTorch ops for everything else (CPU, fp32, experts, GPT-2, callers that differentiate
+* plain PyTorch ops and library GEMMs for everything else (CPU, fp32, experts, GPT-2, callers that differentiate
   ``forward`` themselves): attention is an explicit causal softmax in fp32, backward = recompute
   forward + ``torch.autograd.grad``, as upstream.
-Either way GEMMs go through rocBLAS / hipBLASLt and no activations are held between the two RPCs.
+Either way no activations are held between the two RPCs.
 """
 from __future__ import annotations
 
@@ -152,15 +152,18 @@ class AutogradStage:
                 x, y = (x.clone() if y is None else x + y), None
                 x.view(B, T, -1)[:, :prompts.shape[2]] += prompts[i]
             x, h = train.norm(x, lay.input_norm, eps, y)
-            qkv = train.rope_(torch.mm(h, lay.qkv.t()), table, nh + nkv, D)
+            qkv = train.rope_(ops.linear(h, lay.qkv), table, nh + nkv, D)
             a, a32, lse = train.attention(qkv, B, nh, nkv, D, keep)
-            x2, h = train.norm(x, lay.post_norm, eps, torch.mm(a, lay.o.t()))
-            gu = torch.mm(h, lay.gate_up.t())
+            x2, h = train.norm(x, lay.post_norm, eps, ops.linear(a, lay.o))
             if keep:
+                gu = ops.linear(h, lay.gate_up)
                 kept.append((x, qkv, a32, lse, x2, gu))
                 if i == len(self.w.layers) - 1:
                     return None, kept
-            x, y = x2, torch.mm(ops.swiglu(gu), lay.down.t())
+                act = ops.swiglu(gu)
+            else:
+                act = ops.linear(h, lay.gate_up, epilogue=1)
+            x, y = x2, ops.linear(act, lay.down)
         return x + y, kept
 
     def _kernel_grads(self, g, kept, prompts, B, T, table):

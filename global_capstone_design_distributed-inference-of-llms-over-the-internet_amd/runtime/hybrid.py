@@ -369,6 +369,9 @@ class HybridStage:
                 ops.native_gemm_ok(T, rows, self.W, fused["epilogue"], pkd):
             ops.linear(xu, None, wp=lay.w_up_p, a_rows=T, out=a, out_packed=pkd, **fused)  # in the GEMM's epilogue
             return a, pkd
+        if not pku and not pkd and (not glu or lay.ffn_block == ops.GU_BLOCK) and \
+                ops.gemm_policy() != "hipblaslt" and ops.prompt.ok(xu, lay.w_up, fused["epilogue"]):
+            return ops.linear(xu, lay.w_up, out=a, **fused), False
         u = self._mm(xu, lay.w_up, lay.w_up_p, T, pku, e(f"u{rows}", (T, rows)))
         if glu:
             mops.clamped_glu(u, a, lay.ffn_block, sp.limit, packed=pkd)

@@ -1,0 +1,92 @@
+"""Prompt products (csrc/gemm_prompt.hip) at the edges of their tiles and parts, and which products take them."""
+import pytest
+import torch
+
+from src import ops
+from src.ops import prompt
+
+# bf16 has 7 stored bits: a value in [1, 2) is rounded by at most half a unit of 2^-7, so by 2^-8 of itself
+BF16 = 2.0 ** -8
+
+
+def _want(z, epi, limit):
+    if epi == 4:
+        return z.clamp_min(0) ** 2
+    if epi == 0:
+        return z
+    v = z.view(z.shape[0], -1, 2, 16)
+    g, u = v[:, :, 0].flatten(1), v[:, :, 1].flatten(1)
+    if not limit:
+        return torch.nn.functional.silu(g) * u
+    g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+    return g * torch.sigmoid(1.702 * g) * (u + 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 64, 65, 255, 256, 257, 640])
+@pytest.mark.parametrize("N,K", [(16, 64), (32, 128), (256, 192), (288, 320), (544, 2048), (4096, 1664)])
+def test_products(M, N, K):
+    """One sum of K exact products in 32 bits (in parts or whole), rounded to bf16 once."""
+    ops.require_native()
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16)[:, :K]
+    w = torch.randn(N, K, generator=g).div(K ** 0.5).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    xd = torch.empty(M, K + 8, dtype=x.dtype, device="cuda")[:, :K].copy_(x)  # rows apart, as in a wider matrix
+    for epi, limit in ((0, 0.0), (1, 0.0), (1, 1.5), (4, 0.0)):
+        if epi == 1 and N % 32:
+            continue
+        out = torch.full((M, N // 2 if epi == 1 else N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        got = prompt.gemm(xd, w.cuda(), out, epi, limit)
+        want = _want(z, epi, limit)
+        assert got is out and float((out.double().cpu() - want).norm() / want.norm()) < BF16
+        assert torch.equal(out, prompt.gemm(xd, w.cuda(), None, epi, limit))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4100, 4096, 2048), (300, 4096, 11008), (1030, 4096, 10240), (2049, 2304, 4096)])
+def test_left_over_tiles_in_parts(M, N, K):
+    ops.require_native()
+    assert torch.ops.mpamd.gemm_prompt_ws(M, N, K) > 0
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    want = x.double() @ w.double().t()
+    for epi in (0, 1):
+        r = _want(want, epi, 0.0)
+        assert float((prompt.gemm(x, w, None, epi).double() - r).norm() / r.norm()) < BF16
+
+
+@pytest.mark.gpu
+def test_not_a_number_and_infinity_pass():
+    ops.require_native()
+    x = torch.ones(260, 64, dtype=torch.bfloat16, device="cuda")
+    x[3, 5], x[4, 6] = float("nan"), float("inf")
+    w = torch.ones(32, 64, dtype=torch.bfloat16, device="cuda")
+    for epi in (0, 4):
+        y = prompt.gemm(x, w, None, epi)
+        assert y[3].isnan().all() and y[4].isinf().all() and y[5:].isfinite().all() and y[:3].isfinite().all()
+
+
+def test_table_and_rule(monkeypatch):
+    """Tabled shapes by their row tiles, others only with a long K whose parts fill the CUs; never outside the kernel."""
+    monkeypatch.setitem(prompt._STATE, "table", {(4096, 4096, 0): frozenset({3})})
+    assert prompt.chosen(513, 4096, 4096, 0) and prompt.chosen(768, 4096, 4096, 0)
+    assert not prompt.chosen(512, 4096, 4096, 0) and not prompt.chosen(769, 4096, 4096, 0)
+    assert not prompt.chosen(768, 4096, 4096, 1)
+    assert prompt.chosen(400, 4096, 14336, 0) and prompt.chosen(1800, 4096, 14336, 0)
+    assert not prompt.chosen(400, 4096, 8192, 0) and not prompt.chosen(520, 8192, 28672, 0)
+    assert not prompt.chosen(4298, 4096, 14336, 0)
+    for M in (1, 256, 8193, 20000):
+        assert not prompt.chosen(M, 4096, 14336, 0)
+    assert not prompt.chosen(400, 4096 + 8, 14336, 0) and not prompt.chosen(400, 4096, 14336 + 32, 0)
+    assert not prompt.chosen(400, 4096, 14336, 2) and not prompt.chosen(400, 4096, 14336, 3)
+    x, w = torch.zeros(400, 14336, dtype=torch.bfloat16), torch.zeros(4096, 14336, dtype=torch.bfloat16)
+    assert not prompt.ok(x, w, 0)  # the CPU
+    assert prompt.shapes(__import__("src.models.config", fromlist=["PRESETS"]).PRESETS["llama2-7b"]) == \
+        [(4096, 4096, 0), (4096, 11008, 0), (12288, 4096, 0), (22016, 4096, 1)]
+
+
+def test_committed_table_reads():
+    t = prompt._load(prompt.TABLE)
+    assert t and all(prompt.shape_ok(8192, *s) and all(2 <= m <= 32 for m in v) for s, v in t.items())
