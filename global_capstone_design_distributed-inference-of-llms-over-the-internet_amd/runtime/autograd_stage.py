@@ -152,18 +152,18 @@ class AutogradStage:
                 x, y = (x.clone() if y is None else x + y), None
                 x.view(B, T, -1)[:, :prompts.shape[2]] += prompts[i]
             x, h = train.norm(x, lay.input_norm, eps, y)
-            qkv = train.rope_(ops.linear(h, lay.qkv), table, nh + nkv, D)
+            qkv = train.rope_(ops.linear(h, lay.qkv, tiles=True), table, nh + nkv, D)
             a, a32, lse = train.attention(qkv, B, nh, nkv, D, keep)
-            x2, h = train.norm(x, lay.post_norm, eps, ops.linear(a, lay.o))
+            x2, h = train.norm(x, lay.post_norm, eps, ops.linear(a, lay.o, tiles=True))
             if keep:
-                gu = ops.linear(h, lay.gate_up)
+                gu = ops.linear(h, lay.gate_up, tiles=True)
                 kept.append((x, qkv, a32, lse, x2, gu))
                 if i == len(self.w.layers) - 1:
                     return None, kept
                 act = ops.swiglu(gu)
             else:
-                act = ops.linear(h, lay.gate_up, epilogue=1)
-            x, y = x2, ops.linear(act, lay.down)
+                act = ops.linear(h, lay.gate_up, epilogue=1, tiles=True)
+            x, y = x2, ops.linear(act, lay.down, tiles=True)
         return x + y, kept
 
     def _kernel_grads(self, g, kept, prompts, B, T, table):

@@ -143,7 +143,7 @@ class HybridStage:
     def _mm(self, x, w, wp, T: int, packed: bool, out):
         if packed:
             return ops.linear(x, None, wp=wp, a_rows=T, out=out)
-        return ops.linear(x, w, out=out)
+        return ops.linear(x, w, out=out, tiles=True)
 
     def _add(self, y_in, w, wp, packed: bool, T: int, res, gain, nxt, e, experts=None, join=None, keep=True):
         """Close a sublayer: add y = y_in w^T to the stream (``keep`` False: replace it) and write the next sublayer's
@@ -371,7 +371,7 @@ class HybridStage:
             return a, pkd
         if not pku and not pkd and (not glu or lay.ffn_block == ops.GU_BLOCK) and \
                 ops.gemm_policy() != "hipblaslt" and ops.prompt.ok(xu, lay.w_up, fused["epilogue"]):
-            return ops.linear(xu, lay.w_up, out=a, **fused), False
+            return ops.linear(xu, lay.w_up, out=a, tiles=True, **fused), False
         u = self._mm(xu, lay.w_up, lay.w_up_p, T, pku, e(f"u{rows}", (T, rows)))
         if glu:
             mops.clamped_glu(u, a, lay.ffn_block, sp.limit, packed=pkd)
