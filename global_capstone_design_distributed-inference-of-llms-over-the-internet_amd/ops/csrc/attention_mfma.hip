@@ -16,21 +16,26 @@
 //   O[row][d] += P[row][tok] . V[tok][d]            D/16 MFMAs
 //       A = P straight from the S^T accumulators: lane (q, c) holds row c at tokens
 //       {4q..4q+3, 16+4q..16+4q+3}, used as the MFMA k order,
-//       B = V^T read from a per-wave LDS tile [d][32 tok] (row pitch 36 bf16) that the
-//       wave fills from the contiguous 8 KiB of V (the tile never straddles a 64-token page;
-//       tokens past the context are zeroed so stale cache bytes never meet a p = 0)
-//       -> two ds_read_b64 per fragment, in the same permuted k order.
+//       B = V^T: the wave copies its 32 rows of V, whole rows a load, into an LDS tile of its own
+//       (the tile never straddles a 64-token page; tokens past the context are zeroed so stale
+//       cache bytes never meet a p = 0) and reads 4 tokens x 16 columns transposed at a time
+//       (ds_read_b64_tr_b16), two per fragment, in the same permuted k order.
 // The 4 waves' (m, l, O) are merged through LDS; with num_parts > 1 the merged partials go
 // to the split-K workspace reduced by paged_attn_reduce_kernel (attention.hip).
 //
 // ROPE = true (GQA decode: every block is ONE token of one sequence, the last of its context):
-// `q` is the unrotated fused qkv row and the kernel also does rope_kv.hip's work.  The partner
-// of a lane's q chunk kd (rotate_half, D/2 away) is its own chunk kd ^ KD/2, so q rotates in
-// registers; the new token's k is rotated the same way, its score q.k_new is summed over the
-// 4 lanes of the row with two xor shuffles and replaces the (stale) cache score of token
-// ctx - 1, and its v chunk overwrites that token's column of the wave's LDS V tile.  The cache
-// loads stay exactly as without ROPE.  Wave 0 of the first block of the kv head whose slice
-// holds the token writes k / v to the page slot (slots[t] < 0: nothing written).
+// `q` is the unrotated fused qkv row and the kernel also does rope_kv.hip's work.  The block's
+// heads and the new token's k are turned once, by a thread each pair of 8-column chunks, and go
+// to the waves through LDS; the score q.k_new is summed over the 4 lanes of the row with two xor
+// shuffles and replaces the (stale) cache score of token ctx - 1, and the new v row replaces that
+// token's in the wave's LDS V tile.  The cache loads stay exactly as without ROPE.  Wave 0 of the
+// first block of the kv head whose slice holds the token writes k / v to the page slot (slots[t] < 0:
+// nothing written).
+// Decode reads K and V once and is bound by them, long contexts by how many workgroups share a CU:
+// with 160 registers and 35 KB (V in rows, transposed by the read; the queries turned once) 3 fit, so
+// the 640 slices of 12 sessions of 1.7k to 5.8k tokens (32 / 8 heads) run at once - 45 us for 184 MB
+// where 2 to a CU took 58 in a full round and a quarter one; 64 sessions up to 512: 25.0 -> 20.6 us,
+// one of 900: 12.3 -> 10.1.
 // (K/V loads keep the default cache policy here: non-temporal loads, a win for the MHA decode
 // kernel in attention.hip, measured 12-14 % SLOWER on this kernel at 64 / 256 sessions, cold
 // caches - profiles/r3_i/attn_nt.jsonl vs attn_def.jsonl.)
@@ -58,6 +63,14 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u16x8& a, const u16x8& b, const
                                                  0, 0, 0);
 }
 
+typedef short s16x4_mf __attribute__((ext_vector_type(4)));
+// each group of 16 lanes reads 4 rows x 16 columns and gets them transposed: lane i column i, 4 rows
+__device__ __forceinline__ u16x4 tr_read16(const unsigned char* p) {
+  const s16x4_mf v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4_mf*)(const_cast<unsigned char*>(p)));
+  return __builtin_bit_cast(u16x4, v);
+}
+
 constexpr int VT_PITCH = 36;  // bf16 per LDS row of the transposed V tile (32 tokens + pad; 8-B aligned rows)
 
 // FOLD (ROPE only): q / k / v come from the qkv GEMM's split-K slabs through LDS (s_fold).  A
@@ -65,7 +78,7 @@ constexpr int VT_PITCH = 36;  // bf16 per LDS row of the transposed V tile (32 t
 // loads, which count against vmcnt, so the RoPE prologue waited for the K / V stream issued
 // before them.
 template <int D, int HB, bool ROPE, bool FOLD = false>
-__global__ __launch_bounds__(256, 2) void attn_mfma_kernel(
+__global__ __launch_bounds__(256, 3) void attn_mfma_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int bt_stride, const int32_t* __restrict__ q_seq,
     const int32_t* __restrict__ q_ctx, const int32_t* __restrict__ qb_tok0, const int32_t* __restrict__ qb_ntok,
@@ -74,14 +87,15 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(
   constexpr int TB = 16 / HB;
   constexpr int KD = D / 32;  // k-chunks of the QK^T product
   constexpr int DT = D / 16;  // 16-column tiles of O
-  __shared__ __attribute__((aligned(16))) bf16_t s_vt[4][D * VT_PITCH];
+  // a wave's V tile [32][D] bf16 in its steps, its O rows [16][D + 1] fp32 for the merge after them
+  constexpr int OP = D + 1, WB = (16 * OP * 4 + 255) / 256 * 256;
+  __shared__ __attribute__((aligned(256))) unsigned char s_wave[4][WB];
   __shared__ float s_m[4][16], s_l[4][16];
-  __shared__ __attribute__((aligned(16))) float s_o[4][16][D + 1];
 
   const int b = blockIdx.x, p = blockIdx.z;
   const int hbase = blockIdx.y * HB;
   const int g = hbase / (nh / nkv);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, qd = lane >> 4;
   // ROPE (decode): block b is token b (``decode_qblocks``: one token per block, in order), so the
   // block-table walk starts from q_seq / q_ctx directly - one dependent global load fewer in the
@@ -102,265 +116,237 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(
   const int start = p * PS, end = min(start + PS, blk_ctx);
 
   constexpr int NV = (32 * D * 2) / 1024;  // 16-B V chunks per lane per step
+  // (a page's base is the same in the whole wave: scalar bases, 32-bit lane offsets)
+  const unsigned klane = c * D + qd * 8;
   auto load_k = [&](int bs, int64_t pg, u16x8 (&kr)[2][KD]) {
     const bf16_t* kpage = kc + pg * page_stride + head_off + (int64_t)(bs & (page_size - 1)) * D;
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int kd = 0; kd < KD; ++kd)
-        kr[sub][kd] = *reinterpret_cast<const u16x8*>(kpage + (int64_t)(sub * 16 + c) * D + kd * 32 + qd * 8);
+        kr[sub][kd] = *reinterpret_cast<const u16x8*>(kpage + kd * 32 + (klane + sub * 16 * D));
   };
   auto load_v = [&](int bs, int64_t pg, u16x8 (&vr)[NV]) {
     const bf16_t* vpage = vc + pg * page_stride + head_off + (int64_t)(bs & (page_size - 1)) * D;
+    unsigned vlane = lane;
+    asm volatile("" : "+v"(vlane));  // (two offsets formed at each use instead of held)
+    vlane *= 8;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int ci = i * 64 + lane;
-      vr[i] = *reinterpret_cast<const u16x8*>(vpage + (int64_t)(ci % 32) * D + (ci / 32) * 8);
-    }
+    for (int i = 0; i < NV; ++i) vr[i] = *reinterpret_cast<const u16x8*>(vpage + (i & 3) * 512 + (vlane + (i >> 2) * 2048));
   };
-  // K in ping-pong register buffers one step ahead (no register copies: a copy of in-flight
-  // loads would force a vmcnt(0) early); a step's V is issued at its top, ahead of the next
-  // step's K and the page id two steps ahead, so waiting for it leaves those in flight
-  u16x8 ka[2][KD], kb[2][KD], vr[NV];
-  int64_t pg_cur = 0, pg_next = 0;
-  const int b_first = start + w * 32;
-  // The first step's page ids, then (below) the query / RoPE loads, then this step's K AND V:
-  // the page-table round trip and the K / V stream overlap the query and rotary-table loads
-  // instead of following the whole RoPE prologue (decode blocks have one or two steps per wave:
-  // these dependent round trips, not the bytes, set the kernel time).
-  if (b_first < end) pg_cur = bt[b_first >> page_log2];
-  if (b_first + 128 < end) pg_next = bt[(b_first + 128) >> page_log2];
-
-  // ROPE with qkv partials (decode blocks, one token): the block's HB query heads, its key and its
-  // value summed from the split-K slabs, row-scaled and rounded (common.h qkv_part_finish8: the
-  // reduce launch's bits) ONCE per block into LDS - every slab element read once, not once per
-  // lane group of every wave; the RoPE below then reads them as it would the bf16 qkv row.
-  // Issue order = need order (vmcnt retires in order): row-statistics shards and slab loads, the
-  // rotary table, then the first step's K / V - so the fold's and the RoPE's waits leave the K / V
-  // stream in flight, and its round trip overlaps theirs instead of following the fold's barrier.
-  constexpr int CK = D / 8;  // 8-column chunks per head
-  constexpr int NFOLD = (HB + 2) * CK;
-  constexpr int NI = (NFOLD + 255) / 256;  // fold items per thread (256 threads)
-  __shared__ u16x8 s_fold[NFOLD];
-  constexpr bool from_part = ROPE && FOLD;
-  int fcol[NI];
-#pragma unroll
-  for (int j = 0; j < NI; ++j) {
-    const int fi = min(tid + 256 * j, NFOLD - 1);  // (threads past the items fetch the last one again, unused)
-    fcol[j] = (fi / CK < HB ? (hbase + fi / CK) * D : fi / CK == HB ? (nh + g) * D : (nh + nkv + g) * D) +
-              (fi % CK) * 8;
-  }
-  unsigned long long ssv = 0;
-  QkvPart8 ff[NI];
-  if constexpr (from_part) {
-    ssv = qkv_part_ss_load(rf.qp, tok0);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) qkv_part_fetch8(rf.qp, tok0, fcol[j], ff[j]);
-  }
-  u16x8 qf[KD], kr[KD];
-  u16x8 vn = (u16x8)(0);
-  if constexpr (!from_part) {
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-      qf[kd] = row_ok ? *reinterpret_cast<const u16x8*>(q + (int64_t)(tok0 + my_t) * q_stride + (int64_t)my_h * D +
-                                                        kd * 32 + qd * 8)
-                      : (u16x8)(0);
-    if constexpr (ROPE) {  // the new token's key and value from the bf16 qkv row
-      const bf16_t* qrow = q + (int64_t)tok0 * q_stride;
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) kr[kd] = *reinterpret_cast<const u16x8*>(qrow + (nh + g) * D + kd * 32 + qd * 8);
-      vn = *reinterpret_cast<const u16x8*>(qrow + (nh + nkv + g) * D + ((lane * 8) % D));
-    }
-  }
-  constexpr int HK = KD / 2, HALF = D / 2;
-  f32x4 cs[ROPE ? HK : 1][2], sn[ROPE ? HK : 1][2];
-  int64_t kv_slot = -1;
-  if constexpr (ROPE) {
-    kv_slot = rf.slots[tok0];
-    const int64_t ps_ = rf.pos[tok0];
-#pragma unroll
-    for (int h = 0; h < HK; ++h) {
-      const int64_t ci = ps_ * HALF + h * 32 + qd * 8;
-      cs[h][0] = *reinterpret_cast<const f32x4*>(rf.cos_t + ci);
-      cs[h][1] = *reinterpret_cast<const f32x4*>(rf.cos_t + ci + 4);
-      sn[h][0] = *reinterpret_cast<const f32x4*>(rf.sin_t + ci);
-      sn[h][1] = *reinterpret_cast<const f32x4*>(rf.sin_t + ci + 4);
-    }
-  }
-
-  if (b_first < end) {
-    load_k(b_first, pg_cur, ka);
-    load_v(b_first, pg_cur, vr);
-  }
-
-  if constexpr (from_part) {
-    const float qrs = qkv_part_ss_scale(rf.qp, ssv);
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-      if (tid + 256 * j < NFOLD) s_fold[tid + 256 * j] = qkv_part_finish8(rf.qp, tok0, fcol[j], ff[j], qrs);
-    lds_wait_barrier();  // (lgkmcnt only: the K / V loads stay in flight)
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd) qf[kd] = row_ok ? s_fold[(my_h - hbase) * CK + kd * 4 + qd] : (u16x8)(0);
-  }
-
-  int tnew = -1;
-  float qk_new = 0.f;
-  if constexpr (ROPE) {
-    if constexpr (from_part) {
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) kr[kd] = s_fold[HB * CK + kd * 4 + qd];
-      vn = s_fold[(HB + 1) * CK + ((lane * 8) % D) / 8];
-    }
-    auto rot = [&](const u16x8 (&a)[KD], u16x8 (&r)[KD]) {
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) {
-        const int h = kd % HK;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float c_ = cs[h][j >> 2][j & 3], s_ = sn[h][j >> 2][j & 3];
-          const float x = bf2f(a[kd][j]), y = bf2f(a[kd ^ HK][j]);
-          r[kd][j] = kd < HK ? f2bf(x * c_ - y * s_) : f2bf(x * c_ + y * s_);
-        }
-      }
-    };
-    u16x8 qr[KD], kn[KD];
-    rot(qf, qr);
-    rot(kr, kn);
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd) qf[kd] = row_ok ? qr[kd] : (u16x8)(0);
-    float part = 0.f;
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) part += bf2f(qf[kd][j]) * bf2f(kn[kd][j]);
-    part += __shfl_xor(part, 16, 64);
-    part += __shfl_xor(part, 32, 64);
-    qk_new = part;
-    tnew = blk_ctx - 1;
-    const int64_t slot = kv_slot;
-    if (w == 0 && tnew >= start && tnew < end && slot >= 0 && hbase % (nh / nkv) == 0) {
-      const int64_t dst = (slot >> page_log2) * page_stride + head_off + (slot & (page_size - 1)) * D;
-      if (c == 0) {
-#pragma unroll
-        for (int kd = 0; kd < KD; ++kd) *reinterpret_cast<u16x8*>(rf.kw + dst + kd * 32 + qd * 8) = kn[kd];
-      }
-      if (lane * 8 < D) *reinterpret_cast<u16x8*>(rf.vw + dst + lane * 8) = vn;
-    }
-  }
-
   f32x4 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = (f32x4)(0.f);
   float m = -INFINITY, l = 0.f;
-  bf16_t* vt = s_vt[w];
+  if (start < end) {  // (a slice past the context: an empty partial)
+    // One register set each for a step's K and V: the next step's K is requested as soon as this
+    // step's scores are formed, the next V as soon as this V is in LDS, so both are in flight through
+    // the rest of the step, and 3 workgroups fit a CU
+    u16x8 ka[2][KD], vr[NV];
+    const int b_first = start + w * 32;
+    const int b_load = min(b_first, (end - 1) & ~31);  // (a wave with no step of its own reads the last one, unused)
+    // Issue order = need order (vmcnt retires in order): what the RoPE needs, then the first step's K
+    // and V - the page-table round trip and the K / V stream overlap the rotary prologue instead of
+    // following it (decode blocks have one or two steps per wave: these dependent round trips, not
+    // the bytes, set the kernel time).
+    const int64_t pg_first = bt[b_load >> page_log2];
+    int64_t pg_next = b_first + 128 < end ? bt[(b_first + 128) >> page_log2] : 0;
 
-  // Software-pipelined walk over this wave's 32-token steps (b0 = start + 32 w + 128 i): the K
-  // fragments of step i+1 (and the page id of step i+2) are loaded while step i computes, so a
-  // step exposes one memory round trip (its V) instead of three dependent ones (page id -> K -> V).
-  // At decode sizes every wave has one or two steps: the chain, not the bytes, set the time
-  // (Llama-3-70B, 64 sessions: 16.9 us per layer for 37 MB of K/V).
-  // one 32-token step over K / V fragments already in registers
-  auto step = [&](int b0, const u16x8 (&kr)[2][KD], const u16x8 (&vr)[NV]) {
-    // ---- S^T = K . Q^T for tokens b0 .. b0+31 (two 16-token subtiles) ----
-    f32x4 st[2];
+    constexpr int CK = D / 8;    // 8-column chunks per head
+    constexpr int HK = CK / 2;   // chunk e of a head turns with chunk e + HK (rotate_half)
+    constexpr bool from_part = ROPE && FOLD;
+    u16x8 qf[KD];
+    u16x8 vn = (u16x8)(0);
+    int tnew = -1;
+    float qk_new = 0.f;
+    if constexpr (!ROPE) {
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-      st[sub] = (f32x4)(0.f);
+      for (int kd = 0; kd < KD; ++kd)
+        qf[kd] = row_ok ? *reinterpret_cast<const u16x8*>(q + (int64_t)(tok0 + my_t) * q_stride + (int64_t)my_h * D +
+                                                          kd * 32 + qd * 8)
+                        : (u16x8)(0);
+      load_k(b_load, pg_first, ka);
+      load_v(b_load, pg_first, vr);
+    } else {
+      // The block's HB query heads and its new key are turned ONCE, a pair of chunks a thread, and
+      // reach every wave through LDS (each wave turning them for itself held 96 more registers at the
+      // time the first K and V are in flight: 244, two workgroups a CU).
+      constexpr int NROT = (HB + 1) * HK;
+      static_assert(NROT <= 256, "one pair of chunks a thread");
+      __shared__ u16x8 s_rot[(HB + 1) * CK];
+      const int ri = min(tid, NROT - 1), rh = ri / HK, re = ri % HK;  // (threads past the pairs: the last one again)
+      const int rcol = (rh < HB ? hbase + rh : nh + g) * D + re * 8;
+      const int64_t kv_slot = rf.slots[tok0];
+      const int64_t ci = rf.pos[tok0] * (D / 2) + re * 8;
+      u16x8 xa, xb;
+      f32x4 cs[2], sn[2];
+      // FOLD: the heads, the key and the value summed from the split-K slabs, row-scaled and rounded
+      // (common.h qkv_part_finish8: the reduce launch's bits) once per block into LDS - every slab
+      // element read once, not once per lane group of every wave
+      constexpr int NFOLD = (HB + 2) * CK;
+      constexpr int NI = (NFOLD + 255) / 256;  // fold items per thread (256 threads)
+      __shared__ u16x8 s_fold[FOLD ? NFOLD : 1];
+      int fcol[NI];
+      unsigned long long ssv = 0;
+      QkvPart8 ff[NI];
+      if constexpr (from_part) {
 #pragma unroll
-      for (int kd = 0; kd < KD; ++kd) st[sub] = mfma_bf16(kr[sub][kd], qf[kd], st[sub]);
-    }
-    // ---- V tile -> LDS transposed [d][tok] (this wave only; in-order LDS needs no barrier) ----
-    // tokens vary fastest across lanes: each half-wave's transposed stores are 32 consecutive
-    // bf16 of one d row (token-major lanes would put 16 lanes on 4 banks, sub-dword)
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int ci = i * 64 + lane;
-      const int tk = ci % 32, d0 = (ci / 32) * 8;
-      u16x8 vv = vr[i];
-      if (b0 + tk >= end) vv = (u16x8)(0);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[(d0 + e) * VT_PITCH + tk] = vv[e];
-    }
-    if constexpr (ROPE) {  // the new token: its score and its V column come from registers
-      const int rel = tnew - b0;
-      if (rel >= 0 && rel < 32) {
-        if (lane * 8 < D) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) vt[(lane * 8 + e) * VT_PITCH + rel] = vn[e];
+        for (int j = 0; j < NI; ++j) {
+          const int fi = min(tid + 256 * j, NFOLD - 1);
+          fcol[j] = (fi / CK < HB ? (hbase + fi / CK) * D : fi / CK == HB ? (nh + g) * D : (nh + nkv + g) * D) +
+                    (fi % CK) * 8;
         }
-        if (qd == ((rel & 15) >> 2)) {
+        ssv = qkv_part_ss_load(rf.qp, tok0);
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (r == (rel & 3)) {
-              if (rel < 16) st[0][r] = qk_new;
-              else st[1][r] = qk_new;
-            }
-        }
+        for (int j = 0; j < NI; ++j) qkv_part_fetch8(rf.qp, tok0, fcol[j], ff[j]);
+      } else {
+        const bf16_t* qrow = q + (int64_t)tok0 * q_stride;
+        xa = *reinterpret_cast<const u16x8*>(qrow + rcol);
+        xb = *reinterpret_cast<const u16x8*>(qrow + rcol + D / 2);
+        vn = *reinterpret_cast<const u16x8*>(qrow + (nh + nkv + g) * D + (lane % CK) * 8);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        cs[i] = *reinterpret_cast<const f32x4*>(rf.cos_t + ci + 4 * i);
+        sn[i] = *reinterpret_cast<const f32x4*>(rf.sin_t + ci + 4 * i);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (as written: the RoPE waits for its own loads only)
+      load_k(b_load, pg_first, ka);
+      load_v(b_load, pg_first, vr);
+      if constexpr (from_part) {
+        const float qrs = qkv_part_ss_scale(rf.qp, ssv);
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          if (tid + 256 * j < NFOLD) s_fold[tid + 256 * j] = qkv_part_finish8(rf.qp, tok0, fcol[j], ff[j], qrs);
+        lds_wait_barrier();  // (lgkmcnt only: the K / V loads stay in flight)
+        xa = s_fold[rh * CK + re];
+        xb = s_fold[rh * CK + re + HK];
+        vn = s_fold[(HB + 1) * CK + lane % CK];
+      }
+      u16x8 ra, rb;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float c_ = cs[j >> 2][j & 3], s_ = sn[j >> 2][j & 3];
+        const float x = bf2f(xa[j]), y = bf2f(xb[j]);
+        ra[j] = f2bf(fmaf(x, c_, -(y * s_)));  // (which product is rounded first is fixed)
+        rb[j] = f2bf(fmaf(x, s_, y * c_));
+      }
+      s_rot[rh * CK + re] = ra;
+      s_rot[rh * CK + re + HK] = rb;
+      lds_wait_barrier();
+      float part = 0.f;
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd) {
+        qf[kd] = row_ok ? s_rot[(my_h - hbase) * CK + kd * 4 + qd] : (u16x8)(0);
+        const u16x8 kn = s_rot[HB * CK + kd * 4 + qd];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) part += bf2f(qf[kd][j]) * bf2f(kn[j]);
+      }
+      part += __shfl_xor(part, 16, 64);
+      part += __shfl_xor(part, 32, 64);
+      qk_new = part;
+      tnew = blk_ctx - 1;
+      if (w == 0 && tnew >= start && tnew < end && kv_slot >= 0 && hbase % (nh / nkv) == 0 && lane < CK) {
+        const int64_t dst =
+            (kv_slot >> page_log2) * page_stride + head_off + (kv_slot & (page_size - 1)) * D + lane * 8;
+        *reinterpret_cast<u16x8*>(rf.kw + dst) = s_rot[HB * CK + lane];
+        *reinterpret_cast<u16x8*>(rf.vw + dst) = vn;
       }
     }
-    // ---- online softmax for row c over this lane's 8 tokens {4qd + r, 16 + 4qd + r} ----
-    float s8[8];
-    float lm = -INFINITY;
+
+    // 16-byte chunk ch of V row tk lies at tk 2 D + 16 (ch ^ 2 (tk & 7)) (mod the row): the 4 rows that a
+    // transposed read touches fall on different banks.  This lane's write and read offsets, up to a xor
+    // with constants:
+    unsigned char* vt = s_wave[w];
+    const int tr = qd * 4 + (c >> 2);
+    int vw_off = (lane / CK) * (2 * D) + ((lane % CK) ^ (((lane / CK) << 1) & (CK - 1))) * 16;
+    int vr_off = tr * (2 * D) + (((c >> 1) & 1) ^ (((tr & 7) << 1) & (CK - 1))) * 16 + (c & 1) * 8;
+
+    const int my_end = min(my_ctx, end);
+    // One 32-token step; MORE: the wave has another one 128 tokens on, so all of this one lies inside the
+    // slice.  (A compile-time choice: with loads in a branch the waits before V would cover them too.)
+    auto step = [&](int b0, auto more) {
+      constexpr bool MORE = decltype(more)::value;
+      asm volatile("" : "+v"(vw_off), "+v"(vr_off));  // (their xors formed in each step: 12 registers fewer)
+      // ---- S^T = K . Q^T for tokens b0 .. b0+31 (two 16-token subtiles) ----
+      f32x4 st[2];
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+      for (int sub = 0; sub < 2; ++sub) {
+        st[sub] = (f32x4)(0.f);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int tk = b0 + sub * 16 + qd * 4 + r;
-        const float v = (tk < my_ctx && tk < end) ? st[sub][r] * scale_log2 : -INFINITY;
-        s8[sub * 4 + r] = v;
-        lm = fmaxf(lm, v);
+        for (int kd = 0; kd < KD; ++kd) st[sub] = mfma_bf16(ka[sub][kd], qf[kd], st[sub]);
       }
-    lm = fmaxf(lm, __shfl_xor(lm, 16, 64));
-    lm = fmaxf(lm, __shfl_xor(lm, 32, 64));
-    const float m_new = fmaxf(m, lm);
-    const float alpha = (m_new == -INFINITY) ? 1.f : exp2f(m - m_new);
-    u16x8 pa;
-    float ps = 0.f;
+      if constexpr (MORE) load_k(b0 + 128, pg_next, ka);
+      // ---- V tile -> LDS (this wave only; in-order LDS needs no barrier); the new token's row from registers ----
+      if constexpr (!MORE) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float pv = (m_new == -INFINITY) ? 0.f : exp2f(s8[j] - m_new);
-      const bf16_t pb = f2bf(pv);
-      pa[j] = pb;
-      ps += bf2f(pb);  // l accumulates the rounded p that the MFMA uses
-    }
-    l = l * alpha + ps;
-    m = m_new;
-    // O rows are 4qd + r: fetch those rows' alpha from lanes 4qd + r (row == lane & 15)
-    float ar[4];
+        for (int i = 0; i < NV; ++i) {
+          const int tk = b0 + (i * 64 + lane) / CK;
+          if (tk >= end) vr[i] = (u16x8)(0);
+          if (ROPE && tk == tnew) vr[i] = vn;
+        }
+      }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, qd * 4 + r, 64);
-    // ---- O += P . V ----
+      for (int i = 0; i < NV; ++i) *reinterpret_cast<u16x8*>(vt + i * 1024 + (vw_off ^ (D == 128 ? (i & 1) * 128 : 0))) = vr[i];
+      if constexpr (MORE) {
+        load_v(b0 + 128, pg_next, vr);
+        if (b0 + 256 < end) pg_next = bt[(b0 + 256) >> page_log2];
+      }
+      if constexpr (ROPE && !MORE) {  // the new token's score comes from registers
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const bf16_t* vrow = vt + (dt * 16 + c) * VT_PITCH;
-      const u16x4 lo = *reinterpret_cast<const u16x4*>(vrow + qd * 4);
-      const u16x4 hi = *reinterpret_cast<const u16x4*>(vrow + 16 + qd * 4);
-      const u16x8 vfrag = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][r] *= ar[r];
-      o[dt] = mfma_bf16(pa, vfrag, o[dt]);
+          for (int r = 0; r < 4; ++r) st[sub][r] = b0 + sub * 16 + qd * 4 + r == tnew ? qk_new : st[sub][r];
+      }
+      // ---- online softmax for row c over this lane's 8 tokens {4qd + r, 16 + 4qd + r} ----
+      float s8[8];
+      float lm = -INFINITY;
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma clang fp contract(off)  // (scores are scaled and rounded before the maximum is taken off)
+          const int tk = b0 + sub * 16 + qd * 4 + r;
+          const float v = (ROPE && MORE) || tk < my_end ? st[sub][r] * scale_log2 : -INFINITY;
+          s8[sub * 4 + r] = v;
+          lm = fmaxf(lm, v);
+        }
+      lm = fmaxf(lm, __shfl_xor(lm, 16, 64));
+      lm = fmaxf(lm, __shfl_xor(lm, 32, 64));
+      const float m_new = fmaxf(m, lm);
+      const float alpha = (m_new == -INFINITY) ? 1.f : exp2f(m - m_new);
+      u16x8 pa;
+      float ps = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float pv = (m_new == -INFINITY) ? 0.f : exp2f(s8[j] - m_new);
+        const bf16_t pb = f2bf(pv);
+        pa[j] = pb;
+        ps += bf2f(pb);  // l accumulates the rounded p that the MFMA uses
+      }
+      l = l * alpha + ps;
+      m = m_new;
+      // O rows are 4qd + r: fetch those rows' alpha from lanes 4qd + r (row == lane & 15)
+      float ar[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, qd * 4 + r, 64);
+      // ---- O += P . V ----
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u16x4 lo = tr_read16(vt + (vr_off ^ (dt * 32)));
+        const u16x4 hi = tr_read16(vt + 16 * 2 * D + (vr_off ^ (dt * 32)));
+        const u16x8 vfrag = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[dt][r] *= ar[r];
+        o[dt] = mfma_bf16(pa, vfrag, o[dt]);
+      }
+    };
+    // the walk over this wave's steps b0 = start + 32 w + 128 i
+    if (b_first < end) {
+      int b0 = b_first;
+      for (; b0 + 128 < end; b0 += 128) step(b0, std::true_type{});
+      step(b0, std::false_type{});
     }
-  };
-  for (int b0 = b_first; b0 < end; b0 += 256) {
-    const bool more1 = b0 + 128 < end;
-    if (b0 != b_first) load_v(b0, pg_cur, vr);
-    int64_t pg2 = 0;
-    if (more1) {
-      load_k(b0 + 128, pg_next, kb);
-      if (b0 + 256 < end) pg2 = bt[(b0 + 256) >> page_log2];
-    }
-    step(b0, ka, vr);
-    if (!more1) break;
-    const bool more2 = b0 + 256 < end;
-    load_v(b0 + 128, pg_next, vr);
-    int64_t pg3 = 0;
-    if (more2) {
-      load_k(b0 + 256, pg2, ka);
-      if (b0 + 384 < end) pg3 = bt[(b0 + 384) >> page_log2];
-    }
-    step(b0 + 128, kb, vr);
-    pg_cur = pg2;
-    pg_next = pg3;
   }
   // row sums of l over the 4 lanes of each row
   l += __shfl_xor(l, 16, 64);
@@ -372,7 +358,7 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s_o[w][qd * 4 + r][dt * 16 + c] = o[dt][r];
+    for (int r = 0; r < 4; ++r) reinterpret_cast<float*>(s_wave[w])[(qd * 4 + r) * OP + dt * 16 + c] = o[dt][r];
   __syncthreads();
   // ---- merge the 4 waves; thread -> (row, d) ----
   for (int i = tid; i < 16 * D; i += 256) {
@@ -387,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(
 #pragma unroll
       for (int ww = 0; ww < 4; ++ww) {
         const float f = exp2f(s_m[ww][row] - M);
-        num += f * s_o[ww][row][d];
+        num += f * reinterpret_cast<const float*>(s_wave[ww])[row * OP + d];
         den += f * s_l[ww][row];
       }
     }
