@@ -505,9 +505,9 @@ class HybridStage:
         p["mixed"] = {}
         for tb in {t for t, _ in self.mixed_ok.values() if t}:
             blk = xops.mixed_blocks(ntoks, starts, tb)
-            span = int((np.asarray(starts) + np.asarray(ntoks)).max())
-            p["mixed"][tb] = {"blocks": up(blk), "sums": xops.sum_splits(blk.shape[1], span, self.ex._n_cu),
-                              "parts": xops.mixed_parts(blk.shape[1], span, self.ex._n_cu, 256)}
+            cus = self.ex._n_cu  # (two of the denominators' workgroups share a CU, the values' have one to themselves)
+            p["mixed"][tb] = {"blocks": up(blk), "sums": xops.prompt_splits(ntoks, starts, tb, 2 * cus),
+                              "parts": xops.prompt_splits(ntoks, starts, tb, 3 * cus // 2)}
         p["latent"] = {key: self._latent_plan(key, tb, ntoks, starts, rows, up)
                        for key, tb in self.latent_block.items() if tb}
         return p
