@@ -48,12 +48,15 @@ __device__ __forceinline__ float turned(const T* x, int d, int rot, const float*
 }
 
 // seg == null: blockIdx.y is one row of one token (q_ctx 0: a padding row).  seg: [2+, nseg] (tok0, ntok, ..)
-template <typename T, int VEC, int KIND>
-__global__ __launch_bounds__(256) void linear_scan_kernel(LinArgs a, const int32_t* __restrict__ seg, int nseg) {
-  constexpr int PRE = 16;
-  extern __shared__ float sm[];  // q[D], k[D], red[256 * VEC], red16[16]
+// NT threads: a state of more than 16 rows a thread of 256 (mLSTM's 256 x 256, a workgroup to a (sequence, head) and 64
+// of them for 4 sequences) was 16 rows and then 12 round trips of 4 behind them; 1024 take it in two:
+// 24.2 -> 16.0 us (16 sessions 47.9 -> 37.0).  From 512 workgroups on every CU has several and the gain is gone.
+template <typename T, int VEC, int KIND, int NT>
+__global__ __launch_bounds__(NT) void linear_scan_kernel(LinArgs a, const int32_t* __restrict__ seg, int nseg) {
+  constexpr int PRE = NT > 256 ? 8 : 16;
+  extern __shared__ float sm[];  // q[D], k[D], red[NT * VEC], red16[16]
   const int h = blockIdx.x, H = a.H, D = a.D, V = a.V, tid = threadIdx.x;
-  float *sq = sm, *sk = sm + D, *red = sm + 2 * D, *r16 = red + 256 * VEC;
+  float *sq = sm, *sk = sm + D, *red = sm + 2 * D, *r16 = red + NT * VEC;
   const int tok0 = seg ? seg[blockIdx.y] : (int)blockIdx.y;
   const int ntok = seg ? seg[nseg + blockIdx.y] : 1;
   const int ctx0 = a.q_ctx[tok0];
@@ -61,17 +64,26 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(LinArgs a, const int32
   const int64_t sh = (int64_t)a.q_seq[tok0] * H + h;
   float* S = a.state + sh * D * V;
   float* nm = KIND == MLSTM ? a.aux + sh * (D + 1) : nullptr;
-  const int nv = V / VEC, ng = 256 / nv;
+  const int nv = V / VEC, ng = NT / nv;
   const int g = tid / nv, c = (tid - g * nv) * VEC;
   const bool act = g < ng;
+  unsigned at = g * V + c;  // this thread's place in ng rows: row g + i ng is there after a scalar step
   float m = KIND == MLSTM && ctx0 > 1 ? nm[D] : 0.f;
   for (int t = tok0; t < tok0 + ntok; ++t) {
     const T* z = (const T*)a.z + (int64_t)t * a.zs;
     // the first PRE state rows of this thread are on their way while q, k and the gates are made
     float pre[PRE][VEC];
+    if constexpr (NT > 256) asm volatile("" : "+v"(at));  // (addresses formed here, not held: 128 registers)
+    auto ld = [&](int i) {
+      if constexpr (NT > 256) {
+        if (g + i * ng < D) ld_vec<VEC>(S + (int64_t)i * ng * V + at, pre[i % PRE]);
+      } else {
+        ld_vec<VEC>(S + (int64_t)min(g + i * ng, D - 1) * V + c, pre[i % PRE]);
+      }
+    };
     if (act) {
 #pragma unroll
-      for (int i = 0; i < PRE; ++i) ld_vec<VEC>(S + (int64_t)min(g + i * ng, D - 1) * V + c, pre[i]);
+      for (int i = 0; i < PRE; ++i) ld(i);
     }
     const bool fresh = t == tok0 && ctx0 == 1;  // a sequence's first token: the slot's old state does not count
     float fa, fb;                               // a_t, b_t
@@ -88,7 +100,7 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(LinArgs a, const int32
       fb = 1.f;
     }
     float nq = 0.f;
-    for (int d = tid; d < D; d += 256) {
+    for (int d = tid; d < D; d += NT) {
       float q, k;
       if constexpr (KIND == MLSTM) {
         q = to_f(z[h * D + d]) * a.qs;
@@ -113,30 +125,43 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(LinArgs a, const int32
     if (act) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) v[j] = ld_f(z, (int64_t)2 * H * D + h * V + c + j);
-      auto row = [&](int d, float (&s)[VEC]) {
+      auto row = [&](int d, float* to, float (&s)[VEC]) {
         const float k = sk[d], qd = sq[d];
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
           s[j] = (fresh ? 0.f : fa * s[j]) + k * v[j];
           o[j] += qd * s[j];
         }
-        st_vec<VEC>(S + (int64_t)d * V + c, s);
+        st_vec<VEC>(to, s);
       };
+      if constexpr (NT > 256) {
+        for (int i0 = 0; i0 * ng < D; i0 += PRE) {
+          if (i0) {
 #pragma unroll
-      for (int i = 0; i < PRE; ++i)
-        if (g + i * ng < D) row(g + i * ng, pre[i]);
+            for (int i = 0; i < PRE; ++i)
+              if (g + (i0 + i) * ng < D) ld_vec<VEC>(S + (int64_t)(i0 + i) * ng * V + at, pre[i]);
+          }
+#pragma unroll
+          for (int i = 0; i < PRE; ++i)
+            if (g + (i0 + i) * ng < D) row(g + (i0 + i) * ng, S + (int64_t)(i0 + i) * ng * V + at, pre[i]);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < PRE; ++i)
+          if (g + i * ng < D) row(g + i * ng, S + (int64_t)(g + i * ng) * V + c, pre[i]);
 #pragma unroll 4
-      for (int d = g + PRE * ng; d < D; d += ng) {
-        float s[VEC];
-        ld_vec<VEC>(S + (int64_t)d * V + c, s);
-        row(d, s);
+        for (int d = g + PRE * ng; d < D; d += ng) {
+          float s[VEC];
+          ld_vec<VEC>(S + (int64_t)d * V + c, s);
+          row(d, S + (int64_t)d * V + c, s);
+        }
       }
 #pragma unroll
       for (int j = 0; j < VEC; ++j) red[g * V + c + j] = o[j];
     }
     __syncthreads();
     float ss = 0.f;
-    for (int e = tid; e < V; e += 256) {
+    for (int e = tid; e < V; e += NT) {
       float x = 0.f;
       for (int i = 0; i < ng; ++i) x += red[i * V + e];
       x *= den;
@@ -145,7 +170,7 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(LinArgs a, const int32
     }
     const float sc = 1.f / sqrtf(block_sum(ss, r16) / (float)V + a.eps);
     const T* zg = z + 2 * H * D + H * V + h * V;
-    for (int e = tid; e < V; e += 256) {
+    for (int e = tid; e < V; e += NT) {
       const float gz = to_f(zg[e]), s = 1.f / (1.f + expf(-gz));
       const float w = KIND == MLSTM ? a.norm[h * V + e] * s : gz * s;
       st_act((T*)a.out, t, h * V + e, H * V, a.packed_mt, red[e] * sc * w);
@@ -159,11 +184,12 @@ template <typename T, int KIND>
 static int launch_scan(const LinArgs& a, const int32_t* seg, int nseg, int n, hipStream_t stream) {
   const int vec = a.V % 4 == 0 ? 4 : 1;
   if (a.V / vec > 256) return -1;
-  const size_t lds = (2 * a.D + 256 * vec + 16) * sizeof(float);
+  const int nt = vec == 4 && a.D <= 4096 && (int64_t)a.D * a.V > 16 * 256 * 4 && (int64_t)a.H * n <= 512 ? 1024 : 256;
+  const size_t lds = (2 * a.D + nt * vec + 16) * sizeof(float);
   if (lds > 60000) return -1;
-#define MP_LS(VEC_) \
-  hipLaunchKernelGGL((linear_scan_kernel<T, VEC_, KIND>), dim3(a.H, n), dim3(256), lds, stream, a, seg, nseg)
-  if (vec == 4) MP_LS(4); else MP_LS(1);
+#define MP_LS(VEC_, NT_) \
+  hipLaunchKernelGGL((linear_scan_kernel<T, VEC_, KIND, NT_>), dim3(a.H, n), dim3(NT_), lds, stream, a, seg, nseg)
+  if (nt == 1024) MP_LS(4, 1024); else if (vec == 4) MP_LS(4, 256); else MP_LS(1, 256);
 #undef MP_LS
   return (int)hipGetLastError();
 }
