@@ -2,7 +2,8 @@
 
 ``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel.
 The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
-on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs:
+on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs, for
+the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning; its docstring has why the others do not):
 
 * shapes in the committed table (``python -m src.ops.tune --prompt``: every projection of every preset, steps of up to 8192
   rows) run here at the row-tile counts where this kernel was at least as fast at all three row counts timed inside the
