@@ -8,7 +8,9 @@
 //
 // Attention.  All products are 16x16x32 bf16 MFMA over exact bf16 operands (q, k, v, and the incoming gradient), their
 // accumulators fp32.  What is fp32 in between - probabilities P and score gradients dS - enters the next product as
-// hi + lo bf16 pairs (16 mantissa bits, against the 8 of the bf16 result), so no step is held in 16 bits.
+// three bf16 terms, 8 significant bits each, whose sum is the fp32 number: no step is held in fewer bits than 32-bit
+// products of 32-bit operands would.  (With two terms, 16 bits, the output was 7 to 11 times as far from 64-bit attention
+// as with those, for 10 to 15 % less time.)
 // Orientation: a wave makes scores with the dimension it reduces over LATER in the accumulator's rows; P and dS are then
 // operands of the next product as they lie in the registers (k order permuted: 4 rows of one 16-row subtile, 4 of the
 // next), the other operand comes from the same row-major LDS tile through the transposing LDS read, and the outputs have
@@ -86,19 +88,23 @@ __device__ __forceinline__ u16x8 col_frag(const unsigned char* t, int row0, int 
   const u16x4 a = tr_read(p), b = tr_read(p + 16 * Tile<D, 64>::LD);
   return (u16x8){a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
-// 8 fp32 (two subtiles' 4) as hi + lo operands
-__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u16x8& hi, u16x8& lo) {
+// 8 fp32 (two subtiles' 4) as three operands; the remainders are exact, so is their sum
+__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u16x8 (&t)[3]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    hi[j] = f2bf(a[j]), lo[j] = f2bf(a[j] - bf2f(hi[j]));
-    hi[j + 4] = f2bf(b[j]), lo[j + 4] = f2bf(b[j] - bf2f(hi[j + 4]));
+  for (int j = 0; j < 8; ++j) {
+    float r = j < 4 ? a[j & 3] : b[j & 3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      t[i][j] = f2bf(r);
+      r -= bf2f(t[i][j]);
+    }
   }
 }
 
 // Forward and dQ: a workgroup has 64 queries of one head, 16 a wave, and walks the keys 64 at a time.
-// 2 x 777 tokens, 32 heads of 128 (8 kv heads): forward 53 us, dQ 66 us.  Bound by the chain of a tile's steps and by LDS
-// reads (24 KiB a wave and tile), not by MFMA, which is 8 and 14 us of it.  The fp32 batched products, softmax passes and
-// copies that it replaced were most of 12.3 ms for two blocks' forward and backward requests, 5.6 ms with these kernels.
+// 2 x 777 tokens, 32 heads of 128 (8 kv heads): forward 59 us, dQ 74 us.  Bound by the chain of a tile's steps and by LDS
+// reads (24 KiB a wave and tile), not by MFMA, which is 10 and 12 us of it.  The fp32 batched products, softmax passes and
+// copies that it replaced were most of 12.3 ms for two blocks' forward and backward requests, 5.1 ms with these kernels.
 template <int D, bool GRAD>
 __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
   constexpr int KS = D / 32, DT = D / 16;
@@ -198,13 +204,13 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
       const unsigned char* R = GRAD ? K : V;
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        u16x8 hi, lo;
-        split8(s[2 * half], s[2 * half + 1], hi, lo);
+        u16x8 t[3];
+        split8(s[2 * half], s[2 * half + 1], t);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const u16x8 f = col_frag<D>(R, 32 * half, dt);
-          o[dt] = mfma16(f, hi, o[dt]);
-          o[dt] = mfma16(f, lo, o[dt]);
+#pragma unroll
+          for (int i = 2; i >= 0; --i) o[dt] = mfma16(f, t[i], o[dt]);
         }
       }
     }
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
 // dK and dV: a workgroup has 64 keys of one query head, 16 a wave, and walks the queries from the diagonal on, 32 at a
 // time.  A query head's part goes out in fp32; the heads of a group are added by train_kv_close_kernel: a workgroup per
 // kv head would leave most CUs idle (13 x 8 blocks a sequence of 777 tokens) and atomics would make the sum's order,
-// and so its bits, change from run to run.  97 us for the tokens above, bound as the kernel above, and 11 us to close.
+// and so its bits, change from run to run.  114 us for the tokens above, bound as the kernel above, and 11 us to close.
 template <int D>
 __global__ __launch_bounds__(256) void train_attn_kv_kernel(TrainAttn a) {
   constexpr int KS = D / 32, DT = D / 16;
@@ -315,16 +321,17 @@ __global__ __launch_bounds__(256) void train_attn_kv_kernel(TrainAttn a) {
           ds[st][j] = p[st][j] == 0.f ? 0.f : p[st][j] * (dp[j] - del[j]) * a.scale;
         }
       }
-      u16x8 ph, pl, sh, sl;
-      split8(p[0], p[1], ph, pl);
-      split8(ds[0], ds[1], sh, sl);
+      u16x8 pt[3], st[3];
+      split8(p[0], p[1], pt);
+      split8(ds[0], ds[1], st);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const u16x8 gc = col_frag<D>(G, 0, dt), qc = col_frag<D>(Q, 0, dt);
-        dv[dt] = mfma16(gc, ph, dv[dt]);
-        dk[dt] = mfma16(qc, sh, dk[dt]);
-        dv[dt] = mfma16(gc, pl, dv[dt]);
-        dk[dt] = mfma16(qc, sl, dk[dt]);
+#pragma unroll
+        for (int i = 2; i >= 0; --i) {
+          dv[dt] = mfma16(gc, pt[i], dv[dt]);
+          dk[dt] = mfma16(qc, st[i], dk[dt]);
+        }
       }
     }
     if (more) stash(cur ^ 1);
@@ -451,7 +458,7 @@ __global__ __launch_bounds__(256) void train_glu_grad_kernel(bf16_t* gu, const b
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float g = bf2f(gv[j]), u = bf2f(uv[j]), d = bf2f(dv[j]);
-      const float s = 1.f / (1.f + __expf(-g));
+      const float s = 1.f / (1.f + expf(-g));
       gv[j] = f2bf(d * u * s * (1.f + g * (1.f - s)));
       uv[j] = f2bf(d * g * s);
     }
