@@ -432,31 +432,45 @@ __global__ __launch_bounds__(NW * 64, MP_ATTN_MINW) void paged_attn1_kernel(
 }
 
 // Combine split-K partials: one workgroup (D threads) per (query row, head).  A few kilobytes a
-// workgroup, so round trips set its time: the maximum is taken by the lanes over the parts at once,
-// and 8 parts are in flight together; the sums stay in slice order.  (Part after part, a branch
-// between its loads: 63 parts of one 8000-token session took 36.8 us with their attention, now 20.8.)
+// workgroup: round trips set its time where rows are few (decode), the loads it issues where they are
+// many (prompts).  N: up to 2, 4 or 8 parts are loaded at once and no more than there are to the next
+// of these; 0: any number, the maximum taken by the lanes over the parts at once, 8 in flight.  The
+// sums stay in slice order in every form.  With its attention, 32 / 8 heads: a prompt of 300 tokens (2
+// parts) 20.7 us, of 1500 72.1 us, one 8000-token session (63 parts) 18.8 us.  (Part after part, a
+// branch between the loads: 20.6, 77.0 and 37.1; 8 parts' loads whatever there are: 26.2, 94.1, 18.7.)
+template <int N>
 __global__ void paged_attn_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                          bf16_t* __restrict__ out, int NP, int D, int nh, int packed_mt) {
-  constexpr int AHEAD = 8;
+  constexpr int AHEAD = N ? N : 8;
   const int64_t h = blockIdx.x;
   const float* ml = part_ml + h * NP * 2;
-  float M = -INFINITY;
-  for (int p = threadIdx.x & 63; p < NP; p += 64) {
-    const float m = ml[2 * p], l = ml[2 * p + 1];
-    if (l > 0.f) M = fmaxf(M, m);
-  }
+  float m[AHEAD], l[AHEAD], o[AHEAD];
+  auto load = [&](int p0, int d) {
 #pragma unroll
-  for (int x = 1; x < 64; x <<= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
+    for (int j = 0; j < AHEAD; ++j) {
+      const int p = min(p0 + j, NP - 1);  // (past the last part: read again, not summed)
+      m[j] = ml[2 * p];
+      l[j] = ml[2 * p + 1];
+      o[j] = part_o[(h * NP + p) * D + d];
+    }
+  };
+  float M = -INFINITY;
+  if constexpr (N == 0) {
+    for (int p = threadIdx.x & 63; p < NP; p += 64) {
+      const float pm = ml[2 * p], pl = ml[2 * p + 1];
+      if (pl > 0.f) M = fmaxf(M, pm);
+    }
+#pragma unroll
+    for (int x = 1; x < 64; x <<= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
+  }
   for (int d = threadIdx.x; d < D; d += blockDim.x) {
     float num = 0.f, den = 0.f;
-    for (int p0 = 0; p0 < NP; p0 += AHEAD) {
-      float m[AHEAD], l[AHEAD], o[AHEAD];
+    for (int p0 = 0; p0 < (N ? 1 : NP); p0 += AHEAD) {
+      load(p0, d);
+      if constexpr (N > 0) {
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) {
-        const int p = min(p0 + j, NP - 1);  // (past the last part: read again, not summed)
-        m[j] = ml[2 * p];
-        l[j] = ml[2 * p + 1];
-        o[j] = part_o[(h * NP + p) * D + d];
+        for (int j = 0; j < N; ++j)
+          if (l[j] > 0.f) M = fmaxf(M, m[j]);
       }
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j)
@@ -472,6 +486,18 @@ __global__ void paged_attn_reduce_kernel(const float* __restrict__ part_o, const
     else
       out[h * D + d] = f2bf(v);
   }
+}
+
+// D in whole wavefronts (64 or 128)
+void launch_attn_reduce(const float* part_o, const float* part_ml, void* out, int rows, int NP, int D, int nh, int packed_mt,
+                        hipStream_t stream) {
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(rows), dim3(D), 0, stream, part_o, part_ml, (bf16_t*)out, NP, D, nh, packed_mt);
+  };
+  if (NP <= 2) go(paged_attn_reduce_kernel<2>);
+  else if (NP <= 4) go(paged_attn_reduce_kernel<4>);
+  else if (NP <= 8) go(paged_attn_reduce_kernel<8>);
+  else go(paged_attn_reduce_kernel<0>);
 }
 
 template <int D, int NREP, int NW>
@@ -560,8 +586,7 @@ extern "C" int mp_paged_attention(const void* q, int64_t q_stride, const void* k
   return -3;
 launched:
   if (NP > 1 && cnt == nullptr) {
-    hipLaunchKernelGGL(paged_attn_reduce_kernel, dim3(T * nh), dim3(D), 0, stream, ws_o, ws_ml, (bf16_t*)out, NP,
-                       D, nh, packed_mt);
+    launch_attn_reduce(ws_o, ws_ml, out, T * nh, NP, D, nh, packed_mt, stream);
   }
   return (int)hipGetLastError();
 }

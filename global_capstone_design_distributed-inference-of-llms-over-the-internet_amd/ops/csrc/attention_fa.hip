@@ -22,7 +22,7 @@
 //     O^T's column is the query row too, so the softmax rescale is a per-lane scalar.
 //   * causal skipping: a wave stops computing at its own rows' context (the diagonal steps
 //     of the earlier waves), workgroups are launched longest-context first.
-// Splits of the context (NP > 1) write (m, l, O) partials reduced by paged_attn_reduce_kernel.
+// Splits of the context (NP > 1) write (m, l, O) partials reduced by launch_attn_reduce (attention.hip).
 #include "common.h"
 
 namespace mp {
@@ -292,8 +292,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fa_kernel(
   }  // pass
 }
 
-__global__ void paged_attn_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                         bf16_t* __restrict__ out, int NP, int D, int nh, int packed_mt);
+void launch_attn_reduce(const float* part_o, const float* part_ml, void* out, int rows, int NP, int D, int nh, int packed_mt,
+                        hipStream_t stream);  // attention.hip
 
 }  // namespace mp
 
@@ -335,7 +335,6 @@ extern "C" int mp_attention_fa(const void* q, int64_t q_stride, const void* kc, 
 #undef MP_FA_NW
 #undef MP_FA
   if (NP > 1)
-    hipLaunchKernelGGL(paged_attn_reduce_kernel, dim3(T * nh), dim3(D), 0, stream, ws_o, ws_ml, (bf16_t*)out, NP, D,
-                       nh, 0);
+    launch_attn_reduce(ws_o, ws_ml, out, T * nh, NP, D, nh, 0, stream);
   return (int)hipGetLastError();
 }

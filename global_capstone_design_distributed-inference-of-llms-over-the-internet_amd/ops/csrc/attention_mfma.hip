@@ -21,7 +21,7 @@
 //       cache bytes never meet a p = 0) and reads 4 tokens x 16 columns transposed at a time
 //       (ds_read_b64_tr_b16), two per fragment, in the same permuted k order.
 // The 4 waves' (m, l, O) are merged through LDS; with num_parts > 1 the merged partials go
-// to the split-K workspace reduced by paged_attn_reduce_kernel (attention.hip).
+// to the split-K workspace reduced by launch_attn_reduce (attention.hip).
 //
 // ROPE = true (GQA decode: every block is ONE token of one sequence, the last of its context):
 // `q` is the unrotated fused qkv row and the kernel also does rope_kv.hip's work.  The block's
@@ -610,8 +610,8 @@ static void launch_attn_mfma(const void* q, int64_t q_stride, const void* kc, co
   else go(attn_mfma_kernel<D, HB, false, false>);
 }
 
-__global__ void paged_attn_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                         bf16_t* __restrict__ out, int NP, int D, int nh, int packed_mt);
+void launch_attn_reduce(const float* part_o, const float* part_ml, void* out, int rows, int NP, int D, int nh, int packed_mt,
+                        hipStream_t stream);  // attention.hip
 
 }  // namespace mp
 
@@ -674,7 +674,6 @@ extern "C" int mp_attention_mfma(const void* q, int64_t q_stride, const void* kc
   return -4;
 launched:
   if (NP > 1)
-    hipLaunchKernelGGL(paged_attn_reduce_kernel, dim3(T * nh), dim3(D), 0, stream, ws_o, ws_ml, (bf16_t*)out, NP, D,
-                       nh, packed_mt);
+    launch_attn_reduce(ws_o, ws_ml, out, T * nh, NP, D, nh, packed_mt, stream);
   return (int)hipGetLastError();
 }

@@ -1,4 +1,5 @@
-"""GQA decode attention (csrc/attention_mfma.hip) at the edges of its steps, waves and slices, against fp64.
+"""GQA decode attention (csrc/attention_mfma.hip) at the edges of its steps, waves and slices, and the sum of a prompt's
+slices (csrc/attention.hip), against fp64.
 
 The references start from the queries and keys that the kernels multiply, bit for bit, so all that is left between the two
 is bf16: weights p are rounded to 8 bits, in the sum of values and in its denominator, and so is the result.  A unit of that
@@ -105,3 +106,26 @@ def test_bound_sees_every_slice(D, nh, nkv, ctx, part):
         w = torch.ones(ctx, dtype=torch.float64)
         w[ctx - 1 if s is None else slice(s * part, (s + 1) * part)] = n
         assert ((_attend(q, k, v, w)[0] - want).abs() > 2 * bound).any(), (s, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(4, 1), (4, 4)])
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 7, 8, 9, 17])
+def test_slices_of_a_prompt_are_added(parts, nh, nkv):
+    """Every form of the sum (2, 4, 8 at once, any number) over many rows, of which early ones have empty slices."""
+    ops.require_native()
+    D, T = 128, 64 * parts - 5
+    g = torch.Generator().manual_seed(parts + nkv)
+    q, k = torch.randn(T, nh, D, generator=g).to(torch.bfloat16), torch.randn(T, nkv, D, generator=g).to(torch.bfloat16)
+    v = _values(T, nkv, D, 64, True, g, new=False)
+    kc, vc = (torch.zeros(parts, PAGE, nkv, D, dtype=x.dtype).view(-1, nkv, D).index_copy(0, torch.arange(T), x)
+              .view(parts, PAGE, nkv, D).transpose(1, 2).contiguous().cuda() for x in (k, v))
+    bt = torch.arange(parts, dtype=torch.int32)[None].cuda()
+    ctx = torch.arange(1, T + 1, dtype=torch.int32)
+    blocks = torch.from_numpy(ops.fa_blocks([T], nh // nkv, 4)).cuda()
+    got = ops.attention_fa(q.view(T, -1).cuda(), kc, vc, bt, torch.zeros(T, dtype=torch.int32).cuda(), ctx.cuda(), blocks, nh,
+                           nkv, D ** -0.5, max_ctx=T, waves=4, num_parts=parts)
+    for t in sorted({0, 1, 62, 63, 64, T // 2, T - 65, T - 2, T - 1} & set(range(T))):
+        want, bound = _attend(q[t], k[:t + 1], v[:t + 1])
+        err = (got[t].cpu().double().view(nh, D) - want).abs()
+        assert (err <= bound + 1e-9).all(), (t, (err / bound).nan_to_num().max())
