@@ -48,9 +48,9 @@ __device__ __forceinline__ float turned(const T* x, int d, int rot, const float*
 }
 
 // seg == null: blockIdx.y is one row of one token (q_ctx 0: a padding row).  seg: [2+, nseg] (tok0, ntok, ..)
-// NT threads: a state of more than 16 rows a thread of 256 (mLSTM's 256 x 256, a workgroup to a (sequence, head) and 64
-// of them for 4 sequences) was 16 rows and then 12 round trips of 4 behind them; 1024 take it in two:
-// 24.2 -> 16.0 us (16 sessions 47.9 -> 37.0).  From 512 workgroups on every CU has several and the gain is gone.
+// NT threads: a state of many more than 16 rows a thread of 256 is 16 rows and then a round trip for every 4 behind them;
+// 1024 threads take 256 x 256 in two: 24.2 -> 16.0 us for 4 sequences of 16 heads.  They pay from 48 rows a thread on
+// and while a workgroup has a CU to itself (launch_scan).
 template <typename T, int VEC, int KIND, int NT>
 __global__ __launch_bounds__(NT) void linear_scan_kernel(LinArgs a, const int32_t* __restrict__ seg, int nseg) {
   constexpr int PRE = NT > 256 ? 8 : 16;
@@ -184,7 +184,10 @@ template <typename T, int KIND>
 static int launch_scan(const LinArgs& a, const int32_t* seg, int nseg, int n, hipStream_t stream) {
   const int vec = a.V % 4 == 0 ? 4 : 1;
   if (a.V / vec > 256) return -1;
-  const int nt = vec == 4 && a.D <= 4096 && (int64_t)a.D * a.V > 16 * 256 * 4 && (int64_t)a.H * n <= 512 ? 1024 : 256;
+  // us with 256 and 1024 threads, 4 heads, bf16 mLSTM: 4 sequences of 192 x 192 11.6 / 11.8, 224 x 224 14.6 / 12.5,
+  // 256 x 256 16.4 / 13.8, 256 x 512 28.2 / 19.0; 32 sequences 13.5 / 14.0, 16.8 / 16.1, 24.1 / 20.3, 48.3 / 34.1;
+  // 64 sequences 19.5 / 22.7, 25.3 / 26.7, 29.7 / 32.2, 53.2 / 52.3
+  const int nt = vec == 4 && a.D <= 4096 && (int64_t)a.D * a.V >= 48 * 256 * 4 && (int64_t)a.H * n <= 128 ? 1024 : 256;
   const size_t lds = (2 * a.D + nt * vec + 16) * sizeof(float);
   if (lds > 60000) return -1;
 #define MP_LS(VEC_, NT_) \
