@@ -156,11 +156,13 @@ __device__ __forceinline__ void moe_active(const int32_t* cnt, const MoeLists& l
   if (lane == 0) *l.nact = base;
 }
 
-// ``per`` tokens a wave; one workgroup (gridDim.x == 1, one token a wave): places the rows as well.  Round trips set its
+// ``per`` tokens a wave; ALONE: one workgroup, one token a wave, places the rows as well.  Round trips set its
 // time: all slices of the logits are asked for at once, the rows are placed from registers, and up to
-// 64 experts take code of an eighth the size, which is fetched cold in every launch: 12.9 -> 9.3 -> 5.2 us for 6 tokens
-template <int CH_PER>
+// 64 experts take code of an eighth the size, which is fetched cold in every launch: 12.9 -> 9.3 -> 5.2 us for 6 tokens.
+// (Above that a lane has 8 logits to ask for, and 8 slices of each are enough.)
+template <int CH_PER, bool ALONE>
 __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a, int per) {
+  constexpr int AHEAD = CH_PER == 1 ? 16 : 8;
   extern __shared__ float sm[];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, E = a.E, gs = E / a.groups;
   const int nw = blockDim.x >> 6;
@@ -180,21 +182,19 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
       const int e = lane + 64 * j;
       nx[j] = 0.f;
       if (64 * j < E) {  // (uniform)
-        for (int s = 0; s < a.S; s += 16) {  // 16 slices' loads in flight, added in order
-          float p[16];
+        for (int s = 0; s < a.S; s += AHEAD) {  // so many slices' loads in flight, added in order
+          float p[AHEAD];
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
+          for (int i = 0; i < AHEAD; ++i)
             p[i] = a.part[((int64_t)min(s + i, a.S - 1) * a.T + min(t, a.T - 1)) * E + min(e, E - 1)];
 #pragma unroll
-          for (int i = 0; i < 16; ++i) nx[j] += s + i < a.S ? p[i] : 0.f;
+          for (int i = 0; i < AHEAD; ++i) nx[j] += s + i < a.S ? p[i] : 0.f;
         }
       }
     }
   };
   fetch(t0);
-  // a single workgroup has one token a wave: its picks stay in registers until their rows are known
-  const bool alone = gridDim.x == 1;
-  int pick[CH_PER], place[CH_PER];
+  int pick[CH_PER], place[CH_PER];  // (ALONE: a wave's one token's choices, until their rows are known)
 #pragma unroll
   for (int j = 0; j < CH_PER; ++j) pick[j] = -1;
   for (int i = 0; i < per; ++i) {
@@ -274,13 +274,13 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
           a.ew[at] = s[j] / (cs + 1e-20f) * a.scale;
           a.idx[at] = e;
           const int n = atomicAdd(&hist[e], 1);
-          if (alone) pick[j] = rank[j], place[j] = n;
+          if (ALONE) pick[j] = rank[j], place[j] = n;
           else a.slot[at] = n;
         }
     }
   }
   __syncthreads();
-  if (!alone) {  // places become places among all workgroups' rows
+  if constexpr (!ALONE) {  // places become places among all workgroups' rows
     for (int e = tid; e < E; e += blockDim.x) base[e] = hist[e] > 0 ? atomicAdd(&l.cnt[e], hist[e]) : 0;
     __syncthreads();
     for (int i = lane; i < per * a.top; i += 64) {
@@ -726,8 +726,9 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
   const size_t lds = (2 * E + 1 + nw * 2 * E) * sizeof(float);
   // one token a wave as long as that fills no more than the chip; a single workgroup also places the rows
   const int per = (T + 256 * nw - 1) / (256 * nw), nb = (T + nw * per - 1) / (nw * per);
-  if (E <= 64) hipLaunchKernelGGL(moe_choose_kernel<1>, dim3(nb), dim3(nw * 64), lds, stream, a, per);
-  else hipLaunchKernelGGL(moe_choose_kernel<MOE_EXPERTS / 64>, dim3(nb), dim3(nw * 64), lds, stream, a, per);
+  auto choose = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(nw * 64), lds, stream, a, per); };
+  if (E <= 64) nb > 1 ? choose(moe_choose_kernel<1, false>) : choose(moe_choose_kernel<1, true>);
+  else nb > 1 ? choose(moe_choose_kernel<MOE_EXPERTS / 64, false>) : choose(moe_choose_kernel<MOE_EXPERTS / 64, true>);
   if (nb > 1) hipLaunchKernelGGL(moe_place_kernel, dim3((T * top + 255) / 256), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
