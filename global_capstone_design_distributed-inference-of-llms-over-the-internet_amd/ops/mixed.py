@@ -65,6 +65,19 @@ def prompt_splits(ntoks, starts, tokens: int, slots: int, least: int = 256, most
     return ps, -(-span // ps)
 
 
+def fit_splits(parts, size: int, limit: int):
+    """``parts`` (keys per split, splits), or fewer and longer ones whose scratch of ``size`` bytes a split keeps within
+    ``limit``; (0, 1) where not even two do."""
+    ps, n = parts
+    most = limit // max(1, size)
+    if n <= most:
+        return ps, n
+    if most < 2:
+        return 0, 1
+    longer = KEYS * -(-ps * n // (KEYS * most))
+    return longer, -(-ps * n // longer)
+
+
 def mixed_blocks(ntoks, starts, tokens: int):
     """Query blocks of a ragged step: int32 [2, n] (first flat token, tokens; 0: a filler).  Workgroup i runs on XCD
     i % 8, and every XCD has an L2 of its own: a sequence's blocks stay on one XCD as long as that leaves none with more

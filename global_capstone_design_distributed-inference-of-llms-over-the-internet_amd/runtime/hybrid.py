@@ -279,7 +279,7 @@ class HybridStage:
         H, V = sp.heads, sp.vdim
         if plan is not None and tb:
             mp = plan["mixed"][tb]
-            parts = mp["parts"] if mp["parts"][1] * T * H * V * 4 <= MIXED_WS_BYTES else (0, 1)
+            parts = xops.fit_splits(mp["parts"], T * H * V * 4, MIXED_WS_BYTES)
             kw = dict(form=1, blocks=mp["blocks"], parts=parts, sum_parts=mp["sums"],
                       sums=e("mix_sums", (mp["sums"][1] * T * H,), f32))
             if parts[1] > 1:

@@ -20,8 +20,21 @@ def test_splits_follow_the_work(ntoks, starts, tokens, slots):
     assert ps - xops.KEYS < max(256, -(-span // 16), keys // slots)
 
 
+@pytest.mark.parametrize("parts", [(256, 1), (256, 16), (288, 9), (32, 11)])
+@pytest.mark.parametrize("most", [0, 1, 2, 3, 5, 8, 16, 100])
+def test_as_many_splits_as_fit(parts, most):
+    """Splits whose scratch is over its limit give way to fewer and longer ones, not to a single one."""
+    ps, n = xops.fit_splits(parts, 1000, 1000 * most + 999)
+    if parts[1] <= most:
+        assert (ps, n) == parts
+    elif most < 2:
+        assert (ps, n) == (0, 1)
+    else:
+        assert ps % xops.KEYS == 0 and 2 <= n <= most and ps * n >= parts[0] * parts[1] > ps * (n - 1)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("splits", [7, 8, 9, 17])
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 5, 7, 8, 9, 17])
 def test_decode_merges_any_number_of_splits(splits):
     from tests.test_nuvorax_gpu import DEV, near, run_attn
 
