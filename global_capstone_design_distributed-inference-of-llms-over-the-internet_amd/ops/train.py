@@ -15,7 +15,13 @@ MAX_WIDTH = 16384  # of a norm's row
 def shape_ok(cfg) -> bool:
     """Do the kernels cover the blocks of this model?"""
     return (cfg.model_type in ("llama", "mistral") and not cfg.is_moe and cfg.head_dim in (64, 128) and
-            cfg.hidden_size % 8 == 0 and cfg.hidden_size <= MAX_WIDTH and cfg.intermediate_size % 16 == 0)
+            cfg.hidden_size % 8 == 0 and cfg.hidden_size <= MAX_WIDTH and cfg.intermediate_size % 16 == 0 and
+            cfg.num_attention_heads <= 65535)
+
+
+def rows_ok(B: int, T: int) -> bool:
+    """Do they cover B sequences of T tokens?  (A sequence is a grid's z, a block of 64 tokens its x.)"""
+    return 1 <= B <= 65535 and 1 <= T <= 1 << 24
 
 
 def angle_table(cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:

@@ -131,7 +131,8 @@ class AutogradStage:
         given = [t for t in (hidden, prompts) + more if t is not None]
         if self.device.type != "cuda" or self.dtype != torch.bfloat16 or not train.shape_ok(self.cfg) or not self.w.layers:
             return False
-        if not _plain(*given) or hidden.dim() != 3 or not hidden.numel() or hidden.shape[2] != self.cfg.hidden_size:
+        if not _plain(*given) or hidden.dim() != 3 or not train.rows_ok(*hidden.shape[:2]) or \
+                hidden.shape[2] != self.cfg.hidden_size:
             return False
         for lay in self.w.layers:
             mats = [getattr(lay, n, None) for n in ("input_norm", "qkv", "o", "post_norm", "gate_up", "down")]

@@ -213,6 +213,8 @@ def test_which_calls_take_the_kernels(monkeypatch):
     assert not train.shape_ok(resolve_model("mixtral-8x7b")) and not train.shape_ok(resolve_model("gpt2"))
     cfg = resolve_model("tiny-llama")
     assert not train.shape_ok(dataclasses.replace(cfg, head_dim=96))
+    assert train.rows_ok(1, 1) and train.rows_ok(65535, 7) and not train.rows_ok(65536, 1) and not train.rows_ok(0, 5)
+    assert not train.rows_ok(1, 0) and not train.rows_ok(1, (1 << 24) + 1)
     w = random_stage_weights(cfg, 0, 2, has_embed=False, has_head=False, device="cpu")
     ag = AutogradStage(cfg, w, "cpu")
     h = torch.randn(1, 4, cfg.hidden_size, dtype=torch.bfloat16)
