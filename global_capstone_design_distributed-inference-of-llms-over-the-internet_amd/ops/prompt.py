@@ -3,14 +3,12 @@
 ``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel.
 The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
 on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs, for
-the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning; its docstring has why the others do not):
+the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning): shapes in the committed table
+(``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows) run here at the row-tile
+counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average.
 
-* shapes in the committed table (``python -m src.ops.tune --prompt``: every projection of every preset, steps of up to 8192
-  rows) run here at the row-tile counts where this kernel was at least as fast at all three row counts timed inside the
-  tile, and 3 % faster on average;
-* other shapes run here where even the library's best rate loses: no whole wave of tiles, a long K (160 stages of 64) whose
-  parts fill the CUs.  4096 x 14336: 400 rows 599 against 799 TFLOP/s, 1030 rows 958 / 1090, 1800 rows 1153 / 1251;
-  8192 x 28672, 131 rows 203 / 479.  With fewer parts than 218 on the 256 CUs it loses (8192 x 28672, 520 rows: 962 / 710).
+Everything else keeps the library.  (No rule on the shape alone holds at the shapes that were timed: "less than a wave of
+tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at 10 of 31 row-tile counts.)
 """
 from __future__ import annotations
 
@@ -23,7 +21,7 @@ import torch
 
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "prompt_gemm_gfx950.json")
 EPILOGUES = (0, 1, 4)
-TILE, CUS, MAX_ROWS = 256, 256, 8192
+TILE, MAX_ROWS = 256, 8192
 Shape = Tuple[int, int, int]  # N, K, epilogue
 
 _LOCK = threading.Lock()
@@ -62,14 +60,7 @@ def shape_ok(M: int, N: int, K: int, epilogue: int) -> bool:
 
 def chosen(M: int, N: int, K: int, epilogue: int) -> bool:
     """Does a step of M rows run this product here?"""
-    if M <= TILE or M > MAX_ROWS or not shape_ok(M, N, K, epilogue):
-        return False
-    m = -(-M // TILE)
-    tiles = table().get((N, K, epilogue))
-    if tiles is not None:
-        return m in tiles
-    n = m * -(-N // TILE)
-    return K >= 160 * 64 and n < CUS and CUS // n >= 2 and CUS // n * n >= 218
+    return TILE < M <= MAX_ROWS and shape_ok(M, N, K, epilogue) and -(-M // TILE) in table().get((N, K, epilogue), ())
 
 
 def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:

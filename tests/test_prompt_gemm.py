@@ -63,20 +63,25 @@ def test_not_a_number_and_infinity_pass():
     x = torch.ones(260, 64, dtype=torch.bfloat16, device="cuda")
     x[3, 5], x[4, 6] = float("nan"), float("inf")
     w = torch.ones(32, 64, dtype=torch.bfloat16, device="cuda")
-    for epi in (0, 4):
+    for epi in (0, 1, 4):
         y = prompt.gemm(x, w, None, epi)
         assert y[3].isnan().all() and y[4].isinf().all() and y[5:].isfinite().all() and y[:3].isfinite().all()
+    # a limit takes a number that is not one for itself, in the epilogue as in the pass over a product's rows
+    y, z = prompt.gemm(x, w, None, 1, 1.5), torch.empty(260, 16, dtype=torch.bfloat16, device="cuda")
+    ops.mixers.clamped_glu(prompt.gemm(x, w), z, 16, 1.5)
+    assert torch.equal(y.isfinite(), z.isfinite()) and y[5:].isfinite().all() and y[:3].isfinite().all()
 
 
 def test_table_and_rule(monkeypatch):
-    """Tabled shapes by their row tiles, others only with a long K whose parts fill the CUs; never outside the kernel."""
+    """Tabled shapes by their row tiles, nothing else; never outside the kernel."""
     monkeypatch.setitem(prompt._STATE, "table", {(4096, 4096, 0): frozenset({3})})
     assert prompt.chosen(513, 4096, 4096, 0) and prompt.chosen(768, 4096, 4096, 0)
     assert not prompt.chosen(512, 4096, 4096, 0) and not prompt.chosen(769, 4096, 4096, 0)
     assert not prompt.chosen(768, 4096, 4096, 1)
-    assert prompt.chosen(400, 4096, 14336, 0) and prompt.chosen(1800, 4096, 14336, 0)
-    assert not prompt.chosen(400, 4096, 8192, 0) and not prompt.chosen(520, 8192, 28672, 0)
-    assert not prompt.chosen(4298, 4096, 14336, 0)
+    for M in (400, 1030, 1800, 4298):  # a shape that was not timed
+        assert not prompt.chosen(M, 4096, 14336, 0)
+    monkeypatch.setitem(prompt._STATE, "table", {(4096, 14336, 0): frozenset(range(1, 40)), (4096, 14336 + 32, 0): frozenset({2})})
+    assert prompt.chosen(400, 4096, 14336, 0) and prompt.chosen(8192, 4096, 14336, 0)
     for M in (1, 256, 8193, 20000):
         assert not prompt.chosen(M, 4096, 14336, 0)
     assert not prompt.chosen(400, 4096 + 8, 14336, 0) and not prompt.chosen(400, 4096, 14336 + 32, 0)
@@ -85,6 +90,19 @@ def test_table_and_rule(monkeypatch):
     assert not prompt.ok(x, w, 0)  # the CPU
     assert prompt.shapes(__import__("src.models.config", fromlist=["PRESETS"]).PRESETS["llama2-7b"]) == \
         [(4096, 4096, 0), (4096, 11008, 0), (12288, 4096, 0), (22016, 4096, 1)]
+
+
+def test_table_switched_off(monkeypatch):
+    monkeypatch.setenv("MPAMD_KERNEL_TABLE", "0")
+    monkeypatch.setitem(prompt._STATE, "table", None)
+    assert prompt.table() == {} and not any(prompt.chosen(M, *s) for s in prompt._load(prompt.TABLE) for M in (400, 1800, 4298))
+
+
+def test_committed_table_decides():
+    """At every shape that was timed the choice is the table's."""
+    for s, tiles in prompt._load(prompt.TABLE).items():
+        for m in range(1, 34):
+            assert prompt.chosen(256 * m, *s) == prompt.chosen(256 * m - 100, *s) == (m in tiles)
 
 
 def test_committed_table_reads():
