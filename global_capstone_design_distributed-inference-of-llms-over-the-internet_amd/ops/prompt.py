@@ -5,7 +5,8 @@ The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s 
 on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs, for
 the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning): shapes in the committed table
 (``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows) run here at the row-tile
-counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average.
+counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
+both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
 
 Everything else keeps the library.  (No rule on the shape alone holds at the shapes that were timed: "less than a wave of
 tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at 10 of 31 row-tile counts.)
@@ -109,7 +110,19 @@ def shapes(cfg) -> Iterable[Shape]:
     return sorted(s for s in out if shape_ok(MAX_ROWS, *s) and s[0] * s[1] >= 1 << 22)
 
 
+def agreed(sweeps: Iterable[Dict[Shape, list]]) -> Dict[Shape, list]:
+    """The row-tile counts that all sweeps give."""
+    first, *rest = sweeps
+    return {s: [m for m in v if all(m in r[s] for r in rest)] for s, v in first.items()}
+
+
 def tune(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
+    """The row-tile counts of every shape at which the kernel is faster, in both of two sweeps."""
+    todo = list(todo)
+    return agreed([sweep(todo, device, log) for _ in range(2)])
+
+
+def sweep(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
     """Time both products over the row-tile counts of every shape, best of three rounds in turn."""
     from . import hybrid, require_native, swiglu, use_tuned_gemms
 

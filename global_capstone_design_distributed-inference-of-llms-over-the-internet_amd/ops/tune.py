@@ -12,7 +12,7 @@ written as JSON.  Executors load that file by default, so every box running the 
 same kernel mix (``ops.load_kernel_table``) and bench records carry its sha.
 
 ``--prompt`` writes the table of prompt products (``ops.prompt.TABLE``) instead: every projection of every preset, both
-kernels timed over the row-tile counts of steps of up to 8192 rows.
+kernels timed over the row-tile counts of steps of 257 to 8192 rows, twice; a count enters where both sweeps agree.
 """
 from __future__ import annotations
 

@@ -105,6 +105,11 @@ def test_committed_table_decides():
             assert prompt.chosen(256 * m, *s) == prompt.chosen(256 * m - 100, *s) == (m in tiles)
 
 
+def test_sweeps_have_to_agree():
+    a, b = {(64, 64, 0): [2, 3, 7], (32, 64, 1): []}, {(64, 64, 0): [3, 4, 7], (32, 64, 1): [5]}
+    assert prompt.agreed([a, b]) == {(64, 64, 0): [3, 7], (32, 64, 1): []}
+
+
 def test_committed_table_reads():
     t = prompt._load(prompt.TABLE)
     assert t and all(prompt.shape_ok(8192, *s) and all(2 <= m <= 32 for m in v) for s, v in t.items())
