@@ -79,7 +79,6 @@ class LlamaLayer:
     # Mixtral sparse-MoE block (HF MixtralSparseMoeBlock): ``router`` [E, H]; gate_up / down
     # (and their packed copies) are then stacked per expert: [E, 2F, H] / [E, H, F]
     router: Optional[torch.Tensor] = None
-    router_p: Optional[torch.Tensor] = None  # router padded to 16 rows, packed (decode GEMM)
     folded: bool = False  # qkv_p / gate_up_p carry the input / post-attention norm weights
 
     PROJ = ("qkv", "o", "gate_up", "down")
@@ -244,8 +243,7 @@ class StageWeights:
                 if lay.moe:
                     lay.gate_up_p = torch.stack([ops.pack_weight(w) for w in lay.gate_up])
                     lay.down_p = torch.stack([ops.pack_weight(w) for w in lay.down])
-                    E, H = lay.router.shape
-                    lay.router_p = ops.pack_weight(torch.cat([lay.router, lay.router.new_zeros((-E) % 16, H)]))
+                    lay.router = lay.router.contiguous()
                 else:
                     lay.gate_up_p = ops.pack_weight(lay.gate_up)
                     lay.down_p = ops.pack_weight(lay.down)

@@ -978,7 +978,7 @@ def unpack_weight(wp: torch.Tensor) -> torch.Tensor:
 
 
 def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_rows=None, out_packed=False,
-           gate=None, ss_in=None, eps=0.0, ap_out=None, ss_out=None, ss_zero=None, glu_limit=0.0, tiles=False):
+           ss_in=None, eps=0.0, ap_out=None, ss_out=None, ss_zero=None, glu_limit=0.0, tiles=False):
     """y = epilogue(x @ w^T). epilogue 0: none; 1: SwiGLU (16-row interleaved gate/up w), or with ``glu_limit`` > 0
     the clamped gate g sigmoid(1.702 g) (u + 1), g <= limit, |u| <= limit; 2: + residual;
     3: fused-norm producer (``residual`` updated in place to bf16(y + residual), also written packed to
@@ -1018,9 +1018,7 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
         if out is None:
             out = (torch.empty(packed_numel(M, ncols), dtype=x.dtype, device=x.device) if out_packed
                    else torch.empty(M, ncols, dtype=x.dtype, device=x.device))
-        if gate is not None:
-            kern = "pk"
-        elif M > 64 and t2d_rows(M) and t2d_ok(M, N, K, epilogue, out_packed):
+        if M > 64 and t2d_rows(M) and t2d_ok(M, N, K, epilogue, out_packed):
             kern = "t2d"  # row blocks x column groups (129..256 rows)
         elif M > 64:  # 65..256 rows: split-K ring where it applies (o, down), else the ring kernel
             kern = "rwk" if (not out_packed and _covered("rwk", M, N, K, epilogue)) else "rw"
@@ -1028,7 +1026,7 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
             kern = _kernel_for(M, N, K, epilogue)
         flags = 1 | (2 if out_packed else 0) | _kflags(kern) | (262144 if kern == "t2d" and T2D_GL else 0)
         ws = gemm_workspace(x.device) if _base(kern) in ("sk", "rwk", "rwki", "t2d") else None
-        torch.ops.mpamd.gemm(x, wp, out, residual, int(epilogue), M, flags, ws, gate, ap_out, ss_out, ss_zero, ss_in,
+        torch.ops.mpamd.gemm(x, wp, out, residual, int(epilogue), M, flags, ws, ap_out, ss_out, ss_zero, ss_in,
                              1.0 / K, float(eps), float(glu_limit))
         return out
     if epilogue == 3 or ss_in is not None:
@@ -1106,7 +1104,7 @@ def linear_partials(x, M: int, wp=None, w8=None, w_scale=None, out=None, rot: bo
     if f8:
         torch.ops.mpamd.gemm_w8(x, w8, w_scale, out, None, 0, M, flags, ws, None, None, None, None, 1.0 / K, 0.0)
     else:
-        torch.ops.mpamd.gemm(x, wp, out, None, 0, M, flags, ws, None, None, None, None, None, 1.0 / K, 0.0)
+        torch.ops.mpamd.gemm(x, wp, out, None, 0, M, flags, ws, None, None, None, None, 1.0 / K, 0.0)
     return _slab_view(x.device, S, M, N)
 
 

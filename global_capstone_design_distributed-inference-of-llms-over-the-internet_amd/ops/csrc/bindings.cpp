@@ -55,8 +55,8 @@ int mp_gemm_rw_ok(int M, int N, int K, int epilogue, int out_packed);
 int mp_gemm_t2d_ok(int M, int N, int K, int epilogue, int out_packed, int with_ws);
 int mp_quant_rows_fp8(const void* x, int64_t xs, void* a8, float* scale, int M, int K, hipStream_t stream);
 int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void* y, int64_t y_stride, const void* res,
-                 int64_t res_stride, int M, int N, int K, int epilogue, int flags, void* ws, const int* gate,
-                 void* ap, void* ss_out, void* ss_zero, const void* ss_in, float inv_k, float eps, float glu_limit,
+                 int64_t res_stride, int M, int N, int K, int epilogue, int flags, void* ws, void* ap,
+                 void* ss_out, void* ss_zero, const void* ss_in, float inv_k, float eps, float glu_limit,
                  hipStream_t stream);
 int mp_gemm_ss_elems();
 int mp_gemm_w8(const void* x, const void* wq, const float* wsc, void* y, int64_t y_stride, const void* res,
@@ -511,9 +511,9 @@ void sample(const at::Tensor& logits, const at::Tensor& temps, const at::Tensor&
 // flags bit 0: x is packed (holds ceil(M/16)*16*K elements, M given); bit 1: packed SwiGLU output
 void gemm(const at::Tensor& x, const at::Tensor& wp, at::Tensor& y, const c10::optional<at::Tensor>& residual,
           int64_t epilogue, int64_t M_, int64_t flags, const c10::optional<at::Tensor>& workspace,
-          const c10::optional<at::Tensor>& gate, const c10::optional<at::Tensor>& ap,
-          const c10::optional<at::Tensor>& ss_out, const c10::optional<at::Tensor>& ss_zero,
-          const c10::optional<at::Tensor>& ss_in, double inv_k, double eps, double glu_limit) {
+          const c10::optional<at::Tensor>& ap, const c10::optional<at::Tensor>& ss_out,
+          const c10::optional<at::Tensor>& ss_zero, const c10::optional<at::Tensor>& ss_in, double inv_k, double eps,
+          double glu_limit) {
   check_bf16_cuda(x, "x");
   check_bf16_cuda(wp, "wp");
   check_bf16_cuda(y, "y");
@@ -565,13 +565,8 @@ void gemm(const at::Tensor& x, const at::Tensor& wp, at::Tensor& y, const c10::o
              "gemm workspace too small (ops.gemm_workspace)");
     ws = workspace->data_ptr();
   }
-  const int* gp = nullptr;
-  if (gate.has_value()) {  // MoE expert gate: one int32 on the device (0 -> the GEMM is skipped)
-    MP_CHECK(gate->is_cuda() && gate->scalar_type() == at::kInt && gate->numel() == 1, "gate must be one cuda int32");
-    gp = gate->data_ptr<int>();
-  }
   check_launch(mp_gemm_bf16(x.data_ptr(), apk ? 0 : x.stride(0), wp.data_ptr(), y.data_ptr(), opk ? 0 : y.stride(0),
-                            rp, rs, M, N, K, (int)epilogue, (int)flags, ws, gp, app, sso, ssz, ssi, (float)inv_k,
+                            rp, rs, M, N, K, (int)epilogue, (int)flags, ws, app, sso, ssz, ssi, (float)inv_k,
                             (float)eps, (float)glu_limit, cur_stream()),
                "gemm");
 }
@@ -853,7 +848,7 @@ TORCH_LIBRARY(mpamd, m) {
       "Tensor(d!) recent_len, Tensor seeds, Tensor(a!) workspace, Tensor(b!) out, int update=0) -> ()");
   m.def(
       "gemm(Tensor x, Tensor wp, Tensor(a!) y, Tensor? residual, int epilogue, int M, int flags, "
-      "Tensor(b!)? workspace=None, Tensor? gate=None, Tensor(c!)? ap=None, Tensor(d!)? ss_out=None, "
+      "Tensor(b!)? workspace=None, Tensor(c!)? ap=None, Tensor(d!)? ss_out=None, "
       "Tensor(e!)? ss_zero=None, Tensor? ss_in=None, float inv_k=0., float eps=0., float glu_limit=0.) -> ()");
   m.def(
       "gemm_w8(Tensor x, Tensor wq, Tensor wsc, Tensor(a!) y, Tensor? residual, int epilogue, int M, int flags, "

@@ -73,7 +73,7 @@ extern "C" int64_t mp_gemm_workspace_bytes() {
 //        ss_in may be null when unused).
 extern "C" int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void* y, int64_t y_stride,
                             const void* res, int64_t res_stride, int M, int N, int K, int epilogue, int flags,
-                            void* ws, const int* gate, void* ap, void* ss_out, void* ss_zero, const void* ss_in,
+                            void* ws, void* ap, void* ss_out, void* ss_zero, const void* ss_in,
                             float inv_k, float eps, float glu_limit, hipStream_t stream) {
   (void)hipGetLastError();  // an earlier non-mpamd HIP call's stale error is not this launch's
   using namespace mp;
@@ -84,11 +84,11 @@ extern "C" int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void
   ep.glu_limit = glu_limit;
   if (M > 256 || K % (32 * GU_MAX) || N % 16 || ((flags & 1) == 0 && x_stride % 8)) return -1;
   int rc;
-  if (M > 64) {  // 65..256 rows: gemm_wide.hip (split-K ring / balanced ring, packed A, no gate)
-    if (!(flags & 1) || gate != nullptr) return -1;
+  if (M > 64) {  // 65..256 rows: gemm_wide.hip (split-K ring / balanced ring, packed A)
+    if (!(flags & 1)) return -1;
     return mp_gemm_bf16_wide(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ws, ep, stream);
   }
-  if ((flags & 1) && (flags & 4096) && !(flags & 2) && gate == nullptr) {  // row-split ring
+  if ((flags & 1) && (flags & 4096) && !(flags & 2)) {  // row-split ring
     switch ((M + 15) / 16) {
       case 2: rc = launch_gemm_rwr<2>(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream); break;
       case 4: rc = launch_gemm_rwr<4>(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream); break;
@@ -97,7 +97,7 @@ extern "C" int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void
     if (rc < 0) return rc;
     if (rc == 0) return (int)hipGetLastError();
   }
-  if ((flags & 1) && (flags & 256) && !(flags & 2) && gate == nullptr && ws != nullptr) {  // split-K ring
+  if ((flags & 1) && (flags & 256) && !(flags & 2) && ws != nullptr) {  // split-K ring
 #define MP_RWK(MT_) \
   rc = launch_gemm_rwk<MT_>(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, ep, ws, stream, rwk_comb(flags))
     switch ((M + 15) / 16) {  // the packed layout's row-tile count is part of its strides
@@ -111,7 +111,6 @@ extern "C" int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void
     if (rc == 0) return (int)hipGetLastError();
   }
   if (flags & 16384) return -6;  // partials only: nothing else writes them
-  if (gate != nullptr) flags &= ~(4 | 16 | 128);  // gated (MoE expert) GEMMs use the one-group kernel
   if ((flags & 1) && (flags & 128) && !(flags & 8)) {  // balanced ring kernel
     if (M <= 16) rc = launch_gemm_rw<1>(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
     else if (M <= 32) rc = launch_gemm_rw<2>(x, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
@@ -139,13 +138,10 @@ extern "C" int mp_gemm_bf16(const void* x, int64_t x_stride, const void* w, void
     if (rc == 0) return (int)hipGetLastError();
     // rc == 1: shape not covered by the stream-K form -> one-group-per-workgroup kernel
   }
-  if (M <= 16) rc = launch_gemm<1>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, gate, ep,
-                                   stream);
-  else if (M <= 32) rc = launch_gemm<2>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, gate,
-                                        ep, stream);
-  else if (M <= 48) rc = launch_gemm<3>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, gate,
-                                        ep, stream);
-  else rc = launch_gemm<4>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, gate, ep, stream);
+  if (M <= 16) rc = launch_gemm<1>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
+  else if (M <= 32) rc = launch_gemm<2>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
+  else if (M <= 48) rc = launch_gemm<3>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
+  else rc = launch_gemm<4>(x, x_stride, w, y, y_stride, res, res_stride, M, N, K, epilogue, flags, ep, stream);
   if (rc) return rc;
   return (int)hipGetLastError();
 }

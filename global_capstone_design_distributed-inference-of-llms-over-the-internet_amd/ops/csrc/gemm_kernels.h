@@ -263,15 +263,11 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
                                                           const bf16_t* __restrict__ wp, bf16_t* __restrict__ y,
                                                           int64_t y_stride, const bf16_t* __restrict__ res,
                                                           int64_t res_stride, int M, int N, int K,
-                                                          const int* __restrict__ gate, const EpiArgs ep) {
+                                                          const EpiArgs ep) {
   clear_other(ep);
   __shared__ u64 rs_part[SS_PG][SS_ROWS];
   __shared__ float rs_lds[SS_ROWS];
   RowScale<EPI < 2> rsc;
-  // MoE expert gate (ops/moe.py): a device-side count of tokens routed to this expert; 0 ->
-  // the whole grid exits before streaming any weight (output left as is, combine weight 0).
-  // One uniform scalar load per workgroup keeps hipGraph-captured decode steps shape-static.
-  if (gate != nullptr && *gate == 0) return;
   // fewer k-slices per group for the widest tiles keeps A + 2 x B + acc inside 256 VGPRs
   constexpr int GU = (MT * NT >= 6) ? 2 : 4;
   __shared__ __attribute__((aligned(16))) float red[8][MT * NT * 4][64];
@@ -412,8 +408,7 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
 
 template <int MT>
 static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_t ys, const void* res, int64_t rs,
-                       int M, int N, int K, int epi, int flags, const int* gate, const EpiArgs& ep,
-                       hipStream_t stream) {
+                       int M, int N, int K, int epi, int flags, const EpiArgs& ep, hipStream_t stream) {
   const int ntiles = N / 16;
   // two column tiles per wave when there are enough workgroups to fill the 256 CUs
   const bool two = epi == 1 || (ntiles % 2 == 0 && ntiles / 2 >= 256);
@@ -421,7 +416,7 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
 #define MP_LAUNCH(NT_, EPI_, APK_, OPK_)                                                                       \
   hipLaunchKernelGGL((gemm_packed_kernel<MT, NT_, EPI_, APK_, OPK_>), dim3(ntiles / NT_), dim3(512), 0, stream, \
                      (const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)y, ys, (const bf16_t*)res, rs, M, N, K, \
-                     gate, ep)
+                     ep)
   // Only the packed-activation form is instantiated: row-major callers pack x first
   // (mp_pack_act).  The row-major-A variant miscompiled at MT=1/NT=1 (ROCm 7.2, wrong
   // results with several k-groups per wave) and loses to the packed form anyway.

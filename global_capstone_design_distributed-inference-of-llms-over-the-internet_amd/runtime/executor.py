@@ -46,7 +46,7 @@ from .state_cache import RecurrentState
 logger = logging.getLogger(__name__)
 
 # per-path weight tensors a layer loop reads (what CPU offload streams)
-_PACKED_FIELDS = ("input_norm", "post_norm", "qkv_p", "o_p", "gate_up_p", "down_p", "router_p")
+_PACKED_FIELDS = ("input_norm", "post_norm", "qkv_p", "o_p", "gate_up_p", "down_p")
 _DENSE_FIELDS = ("input_norm", "post_norm", "qkv", "o", "gate_up", "down", "router")
 _GPT2_FIELDS = ("ln1_w", "ln1_b", "attn_w", "attn_b", "proj_w", "proj_b", "ln2_w", "ln2_b", "fc_w", "fc_b",
                 "fc2_w", "fc2_b")
@@ -245,7 +245,6 @@ class StageExecutor:
         # shortest split-K context slice (ops.attention_partition): longer on the MFMA GQA kernel
         self._attn_min_part = 256 if self.gqa_decode_mfma else 64
         self._decode_qb: Dict[int, torch.Tensor] = {}
-        self._moe_y: Dict[int, torch.Tensor] = {}
         self.timing = False
         # one executor may be driven by the TCP handler's GPU worker AND a device-channel
         # engine thread: every device step (incl. hipGraph capture) runs under this lock
@@ -297,11 +296,10 @@ class StageExecutor:
                 elif ops.autotune_mode() != "off":
                     H, F = cfg.hidden_size, cfg.intermediate_size
                     shapes = [] if (weights.fp8 or not weights.layers) else \
-                        [(cfg.q_dim + 2 * cfg.kv_dim, H, 0), (H, cfg.q_dim, 0), (2 * F, H, 1), (H, F, 0)]
+                        [(cfg.q_dim + 2 * cfg.kv_dim, H, 0), (H, cfg.q_dim, 0)] + \
+                        ([] if cfg.is_moe else [(2 * F, H, 1), (H, F, 0)])  # (experts: products of their own)
                     if self._fused and shapes:
                         shapes += [(H, cfg.q_dim, 3), (H, F, 3)]
-                    if cfg.is_moe and shapes:
-                        shapes.append((16 * ((cfg.num_local_experts + 15) // 16), H, 0))  # router
                     if weights.lm_head_p is not None:
                         shapes.append((16 * weights.lm_head_p.shape[0], H, 0))
                     ops.autotune_gemm(shapes, self.device)
@@ -997,9 +995,9 @@ class StageExecutor:
                 moe.expert_mfma_ok(self.cfg.intermediate_size, self.cfg.hidden_size, L.router.dtype))
 
     def _moe_mlp(self, L, xn, T, mlp, act, e, q_ctx, packed: bool) -> None:
-        """Mixtral sparse-MoE MLP into ``mlp``: grouped expert kernels (ops/moe.py), else the plain form, whose
-        decode steps run every expert on the whole batch with a dense combine matrix: no host sync, so the step
-        stays graph-capturable."""
+        """Mixtral sparse-MoE MLP into ``mlp``: grouped expert kernels (ops/moe.py; every packed step), else the
+        plain form (the CPU, library GEMMs forced), whose decode steps run every expert on the whole batch with a
+        dense combine matrix: no host sync, so the step stays graph-capturable."""
         cfg = self.cfg
         E, k, H = cfg.num_local_experts, cfg.num_experts_per_tok, cfg.hidden_size
         if self._moe_grouped(L):
@@ -1007,35 +1005,18 @@ class StageExecutor:
                             packed=packed)
             self._ar(mlp)
             return
-        if packed:
-            logits = ops.linear(xn, None, out=e("moe_logits", (T, 16 * L.router_p.shape[0])), wp=L.router_p,
-                                a_rows=T)[:, :E]
-        else:
-            logits = ops.linear(xn, L.router)
-        w, idx = moe.route(logits, k)
+        w, idx = moe.route(ops.linear(xn, L.router), k)
         acc = e("moe_acc", (T, H), torch.float32)
         acc.zero_()
         gp = (lambda j: L.gate_up_p[j]) if L.gate_up_p is not None else (lambda j: None)  # noqa: E731
         dp = (lambda j: L.down_p[j]) if L.down_p is not None else (lambda j: None)  # noqa: E731
         capturing = self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()
-        if packed or T <= 64 or capturing:
+        if T <= 64 or capturing:
             wd = moe.dense_weights(w, idx, E, out=e("moe_w", (T, E), torch.float32))
-            # small decode batches leave experts unrouted: their GEMMs are skipped on the device
-            # (gate = routed-token count) so a 1-session step streams ~k/E of the expert bytes.
-            # y persists per T and starts zeroed: a skipped GEMM leaves finite values * weight 0.
-            gated = packed and T * k <= 2 * E
-            cnt = (wd > 0).sum(0, dtype=torch.int32) if gated else None
-            y = self._moe_y.get(T)
-            if y is None:
-                y = self._moe_y[T] = torch.zeros(T, H, dtype=self.dtype, device=self.device)
+            y = e("moe_out", (T, H))
             for j in range(E):
-                if packed:
-                    g = cnt[j:j + 1] if gated else None
-                    ops.linear(xn, L.gate_up[j], out=act, epilogue=1, wp=gp(j), a_rows=T, out_packed=True, gate=g)
-                    ops.linear(act, L.down[j], out=y, wp=dp(j), a_rows=T, gate=g)
-                else:
-                    ops.linear(xn, L.gate_up[j], out=act, epilogue=1, wp=gp(j))
-                    ops.linear(act, L.down[j], out=y, wp=dp(j))
+                ops.linear(xn, L.gate_up[j], out=act, epilogue=1, wp=gp(j))
+                ops.linear(act, L.down[j], out=y, wp=dp(j))
                 acc.addcmul_(y, wd[:, j:j + 1])
         else:
             # prefill: group the T*k (token, expert) pairs by expert (one host sync per layer)

@@ -91,7 +91,7 @@ int main(int argc, char** argv) {
     const int fl = 1 | (M > 32 ? s.f64 : s.f32);
     const int nc = s.epi == 1 ? s.N / 2 : s.N;
     const int rc = mp_gemm_bf16(x[lane], s.K, wts + off, s.epi == 1 ? ap[lane] : y[lane], nc, nullptr, 0, M, s.N,
-                                s.K, s.epi, fl, ws[lane], nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f,
+                                s.K, s.epi, fl, ws[lane], nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f,
                                 st[lane]);
     if (rc) {
       fprintf(stderr, "gemm rc=%d (N=%d K=%d M=%d)\n", rc, s.N, s.K, M);

@@ -110,7 +110,7 @@ int main(int argc, char** argv) {
         auto run = [&](int i, unsigned short* out) {
           const unsigned short* w = pool + (size_t)(i % copies) * (wbytes / 2);
           return mp_gemm_bf16(x, s.K, w, out, ncols, nullptr, 0, M, s.N, s.K, s.epi, flags, ws, nullptr, nullptr,
-                              nullptr, nullptr, nullptr, 0.f, 0.f, 0);
+                              nullptr, nullptr, 0.f, 0.f, 0.f, 0);
         };
         int rc = run(0, kind == 0 ? yref : y);
         if (rc) {

@@ -112,7 +112,7 @@ int main(int argc, char** argv) {
           const unsigned short* w = pool + (size_t)(i % copies) * (wbytes / 2);
           if (S < 0)
             return mp_gemm_bf16(x, s.K, w, y, Nout, s.epi == 3 ? res : nullptr, s.N, M, s.N, s.K, s.epi, s.base_flags,
-                                ws, nullptr, ap, ss, ss2, s.epi < 2 ? ss_in : nullptr, 1.f / s.K, 1e-5f, 0);
+                                ws, ap, ss, ss2, s.epi < 2 ? ss_in : nullptr, 1.f / s.K, 1e-5f, 0.f, 0);
           const int fl = (s.epi == 1 ? 2 : 0) | (S > 1 ? (S << 16) : 0);
           int rc;
           switch (MT) {

@@ -108,7 +108,7 @@ int main(int argc, char** argv) {
           unsigned short* y = s.epi == 3 ? res : yref + 0;  // EPI 3 updates the residual in place
           if (s.epi == 0) y = res;
           return mp_gemm_bf16(x, s.K, w, y, s.N, s.epi == 3 ? res : nullptr, s.N, M, s.N, s.K, s.epi, 1 | kd.flags,
-                              ws, nullptr, ap, ss, ss2, nullptr, 1.f / s.K, 1e-5f, 0);
+                              ws, ap, ss, ss2, nullptr, 1.f / s.K, 1e-5f, 0.f, 0);
         };
         // correctness: one call from the saved residual with zeroed statistics
         CK(hipMemcpy(res, res0, (size_t)64 * 12288 * 2, hipMemcpyDeviceToDevice));

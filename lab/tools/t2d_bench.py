@@ -81,7 +81,7 @@ def main():
                 cands.append(("ring", flags0 | ring))
             for kname, flags in cands:
                 def run(i, flags=flags):
-                    torch.ops.mpamd.gemm(xp, wps[i % nw], out, res if epi == 3 else None, epi, M, flags, ws_buf, None,
+                    torch.ops.mpamd.gemm(xp, wps[i % nw], out, res if epi == 3 else None, epi, M, flags, ws_buf,
                                          apo if epi == 3 else None, ss[0] if epi == 3 else None,
                                          ss[1] if epi == 3 else None, ss_in, 1.0 / K, 1e-5)
                 try:

@@ -141,7 +141,7 @@ def test_mixtral_gpu_matches_fp32_reference(graphs):
     cfg = resolve_model("tiny-mixtral")
     w = _w(cfg, 0, cfg.num_hidden_layers, True, True, device="cuda", dtype=torch.bfloat16, seed=4)
     ex = StageExecutor(cfg, w, "cuda", kv_cache_bytes=128 << 20, max_sessions=4, max_seq_len=256, use_graphs=graphs)
-    assert w.layers[0].router_p is not None and w.layers[0].gate_up_p.shape[0] == cfg.num_local_experts
+    assert w.layers[0].gate_up_p.shape[0] == cfg.num_local_experts
     g = torch.Generator().manual_seed(0)
     prompts = [torch.randint(0, cfg.vocab_size, (n,), generator=g) for n in (80, 9)]
     logits = ex.forward([("a", 80), ("b", 9)], torch.cat(prompts).cuda())
