@@ -50,21 +50,6 @@ def mfma_ok(H, G, D, V, page, cap):
     return (r >> 8 if r & 1 else 0), bool(r & 2)
 
 
-def prompt_splits(ntoks, starts, tokens: int, slots: int, least: int = 256, most: int = 16):
-    """(keys per split, splits) of a prompt's blocks of ``tokens`` queries, ``slots`` workgroups at a time: a workgroup's
-    time is its keys, and under a causal mask the longest block has several times the average, so a split is the keys of
-    all blocks over the slots.  (Prompts of 1900 and 300 tokens through 3 blocks of Nuvorax-7B: 2455 us uncut, 2255 with
-    as many slots as CUs, 2166 with half as many again; 4 of 350 to 1801: 3011, 2942, 2879.)"""
-    work = span = 0
-    for n, s in zip(np.asarray(ntoks).tolist(), np.asarray(starts).tolist()):
-        full, rest = divmod(n, tokens)
-        work += full * s + tokens * full * (full + 1) // 2 + (s + n if rest else 0)
-        span = max(span, s + n)
-    span = max(1, span)
-    ps = KEYS * -(-max(least, -(-span // most), work // max(1, slots)) // KEYS)
-    return ps, -(-span // ps)
-
-
 def fit_splits(parts, size: int, limit: int):
     """``parts`` (keys per split, splits), or fewer and longer ones whose scratch of ``size`` bytes a split keeps within
     ``limit``; (0, 1) where not even two do."""
@@ -112,6 +97,46 @@ def mixed_blocks(ntoks, starts, tokens: int):
         for k, (_, t, n) in enumerate(b):
             out[:, k, i] = t, n
     return np.ascontiguousarray(out.reshape(2, -1))
+
+
+def prompt_splits(blk, ntoks, starts, n_cu: int = 256, least: int = 256, most: int = 16):
+    """(keys per split, splits) of a prompt's query blocks ``blk`` (``mixed_blocks``): for the denominators, and for the
+    values.  Splits are even, 16 at most, none under 256 keys.
+
+    A workgroup's time is its keys and some 64 more, and an XCD runs ``n_cu`` / 8 at a time.  The denominators' splits are
+    those whose rounds on the XCD with the most workgroups are shortest: a few past a round take as long as a round.  The
+    values' are a compromise of that and of the keys shared out evenly (whole splits come first and the rest fills the CUs,
+    which is what happens to the triangle of a long prompt), and every split of a block that has several costs 128 keys
+    more, since it is written and added; within 3 % the fewest.
+
+    us of attention, 16 heads; splits from the mean block over 256 CUs / from all keys over 1.5 workgroups a CU / these:
+    1800 tokens 160 / 126 / 120, 300 after 4000 118 / 134 / 92, 1000 after 4000 255 / 265 / 212, 1400 after 700 176 / 136 / 130,
+    4 x 100 after 3000 114 / 124 / 92; 4000 tokens of 32 heads 705 / 735 / 687.  It is not the best of all: 500 after 500 beside
+    100 after 2000 89 / 98 / 97."""
+    seqs = [(n, s) for n, s in zip(np.asarray(ntoks).tolist(), np.asarray(starts).tolist()) if n]
+    span, cus = max((n + s for n, s in seqs), default=1), max(1, n_cu // XCDS)
+    if span <= least:
+        return (KEYS * -(-span // KEYS), 1), (KEYS * -(-span // KEYS), 1)
+    ends = np.concatenate([np.arange(s + 1, s + n + 1, dtype=np.int32) for n, s in seqs])
+    keys = np.where(blk[1] > 0, ends[blk[0] + blk[1] - 1], 0).reshape(-1, XCDS, 1)
+    ps = KEYS * -(-span // (KEYS * np.arange(1, min(most, -(-span // least)) + 1, dtype=np.int32)))
+    pieces = keys // ps  # [rows of blocks, XCDS, choices]
+    rest = keys - pieces * ps
+    whole, rests, longest, share = pieces.sum(0), rest.sum(0), rest.max(0), int(keys.sum()) / n_cu
+    pieces += rest > 0
+    groups = pieces.sum(0)
+    added = groups - (pieces == 1).sum(0)
+    full = -(-groups // cus) * (ps + 64)
+    over = whole % cus  # whole splits of the last round; the rests fill the other CUs
+    tail = np.maximum(np.maximum(np.where(over > 0, ps, 0), longest), (over * ps + rests) / cus)
+    even = whole // cus * ps + tail + 64 * -(-groups // cus)
+
+    def first(cost, slack):
+        cost = np.maximum(cost.max(0), share)
+        best = int(ps[np.flatnonzero(cost <= slack * cost.min())[0]])
+        return best, -(-span // best)
+
+    return first(full, 1.0), first((full + even) / 2 + 128 / cus * added, 1.03)
 
 
 def mixed_parts(groups: int, span: int, n_cu: int = 256, least: int = 2 * KEYS):

@@ -505,9 +505,8 @@ class HybridStage:
         p["mixed"] = {}
         for tb in {t for t, _ in self.mixed_ok.values() if t}:
             blk = xops.mixed_blocks(ntoks, starts, tb)
-            cus = self.ex._n_cu  # (two of the denominators' workgroups share a CU, the values' have one to themselves)
-            p["mixed"][tb] = {"blocks": up(blk), "sums": xops.prompt_splits(ntoks, starts, tb, 2 * cus),
-                              "parts": xops.prompt_splits(ntoks, starts, tb, 3 * cus // 2)}
+            sums, parts = xops.prompt_splits(blk, ntoks, starts, self.ex._n_cu)
+            p["mixed"][tb] = {"blocks": up(blk), "sums": sums, "parts": parts}
         p["latent"] = {key: self._latent_plan(key, tb, ntoks, starts, rows, up)
                        for key, tb in self.latent_block.items() if tb}
         return p

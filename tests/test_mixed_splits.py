@@ -8,16 +8,43 @@ from src.ops import moe as eops
 from tests import nuvorax_utils as U
 
 
-@pytest.mark.parametrize("ntoks,starts", [([1], [0]), ([1800], [0]), ([100, 1801, 777], [0, 0, 0]), ([5, 8192], [4000, 0]),
-                                          ([40] * 200, [0] * 200), ([300], [30000])])
-@pytest.mark.parametrize("tokens,slots", [(16, 256), (8, 512), (16, 1)])
-def test_splits_follow_the_work(ntoks, starts, tokens, slots):
-    """Whole tiles, every key covered, 16 splits at most; none longer than a slot's share, 256 keys or the cap ask for."""
-    ps, n = xops.prompt_splits(ntoks, starts, tokens, slots)
-    span = max(a + b for a, b in zip(ntoks, starts))
-    keys = sum(s + min(k + tokens, t) for t, s in zip(ntoks, starts) for k in range(0, t, tokens))
-    assert ps % xops.KEYS == 0 and 1 <= n <= 16 and ps * n >= span > ps * (n - 1)
-    assert ps - xops.KEYS < max(256, -(-span // 16), keys // slots)
+PROMPTS = [([1], [0]), ([1800], [0]), ([100, 1801, 777], [0, 0, 0]), ([5, 8192], [4000, 0]), ([40] * 200, [0] * 200),
+           ([300], [30000]), ([300], [4000]), ([1000], [1000]), ([100] * 4, [3000] * 4), ([500, 100, 0], [500, 2000, 9])]
+
+
+@pytest.mark.parametrize("ntoks,starts", PROMPTS)
+@pytest.mark.parametrize("tokens,cus", [(16, 256), (8, 256), (16, 32), (16, 1)])
+def test_splits_take_the_fewest_rounds(ntoks, starts, tokens, cus):
+    """Whole tiles, every key covered, 16 splits at most, none under 256 keys.  The denominators': no other number is better
+    in rounds of the fullest XCD's workgroups, counted one by one; the values': at most twice that."""
+    blk = xops.mixed_blocks(ntoks, starts, tokens)
+    span = max(a + b for a, b in zip(ntoks, starts) if a)
+    most = min(16, -(-span // 256))
+    xcds = [[] for _ in range(8)]  # contexts of every XCD's blocks
+    for i, (t, k) in enumerate(blk.T.tolist()):
+        if k:
+            q, at = 0, 0
+            while t >= at + ntoks[q]:
+                at, q = at + ntoks[q], q + 1
+            xcds[i % 8].append(starts[q] + t + k - at)
+
+    def cost(size):
+        rounds = max(-(-sum(-(-c // size) for c in x) // max(1, cus // 8)) for x in xcds)
+        return max(rounds * (size + 64), sum(map(sum, xcds)) / cus)
+
+    least = min(cost(xops.KEYS * -(-span // (xops.KEYS * m))) for m in range(1, most + 1))
+    for (ps, n), slack in zip(xops.prompt_splits(blk, ntoks, starts, cus), (1.0, 2.0)):
+        assert ps % xops.KEYS == 0 and 1 <= n <= most and ps * n >= span > ps * (n - 1)
+        assert n == 1 or ps > 256 - xops.KEYS
+        assert cost(ps) <= slack * least + 1e-6
+
+
+def test_splits_of_portions_and_prompts():
+    """Contexts alike: as many as one round takes; a long prompt's triangle: the values keep few."""
+    for ntoks, starts, tokens, want in (([300], [4000], 16, (11, 11)), ([1000], [4000], 16, (4, 4)), ([1800], [0], 16, (8, 3)),
+                                        ([8192], [0], 8, (14, 3)), ([200], [0], 16, (1, 1)), ([], [], 16, (1, 1))):
+        got = xops.prompt_splits(xops.mixed_blocks(ntoks, starts, tokens), ntoks, starts)
+        assert (got[0][1], got[1][1]) == want, (ntoks, starts, got)
 
 
 @pytest.mark.parametrize("parts", [(256, 1), (256, 16), (288, 9), (32, 11)])
