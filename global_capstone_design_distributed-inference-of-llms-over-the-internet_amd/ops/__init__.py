@@ -990,9 +990,9 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
     ``ss_in`` (fused-norm consumer): ``x`` is the raw residual stream, ``w`` has the RMSNorm weight
     folded into its columns, and row r of the product is scaled by rsqrt(ss_in[r] / K + eps).
     ``tiles``: a prompt's product of row-major operands may run on this package's tile kernel (``prompt``), whose sums end
-    in another order than the library's.  The uniform decoders' executor does not ask for it: their logits feed the
-    sampler, and prompts with other last bits change 3 of 64 tokens drawn after them (logits 0.44 % apart, either as far
-    from the exact ones); 20 ragged prompts of Llama-2-7B through 2 blocks would take 4.72 ms instead of 5.05.
+    in another order than the library's, as far from 64-bit ones.  The hybrid decoders and fine-tuning ask for it.  The
+    uniform decoders' executor does not yet: 20 ragged prompts of Llama-2-7B through 2 blocks would take 4.72 ms instead of
+    5.05, and 0 to 7 of 64 tokens sampled after them would be others, as after any change of a sum's order.
     """
     if not _native(x):
         K = 32 * wp.shape[1] if wp is not None else w.shape[1]
