@@ -22,16 +22,18 @@ Here the same roles run as a chain of stage ranks, one process per GPU:
   stage forwards to its successor before computing; the payload (hidden states) follows on
   RCCL.  Stage k therefore never waits on a host round trip of stage k-1's compute.
 * The tail samples with per-session parameters and a device-resident repetition history
-  (reference semantics, ``ops.sample``), seeded by (session seed, position): the random draw
-  of a session never depends on which micro-batch, replica or batch mix it runs in.  The
-  LOGITS do, in their last bits, on the GPU: the decode GEMM form (and so its reduction order)
+  (reference semantics, ``ops.sample``), seeded by (session seed, position): on the CPU the
+  random draw of a session never depends on which micro-batch, replica or batch mix it runs in.
+  The GPU's kernel mixes in the row that a session has in its micro-batch, so a session placed
+  in another row draws other tokens.  The LOGITS depend on the mix, too, in their last bits, on the GPU: the decode GEMM form (and so its reduction order)
   is chosen per row bucket, and a failed-over session's KV is rebuilt by a prefill (hipBLASLt
   + FA2) where the original came from decode steps.  Exactness contract: on the CPU path
   (fp32 reference ops) a re-placed session's logits agree to fp32 rounding and its tokens equal
   the uninterrupted run's (``tests/test_channel_failover.py``, ``tests/test_failover_drill.py``);
-  on the GPU the tokens generated before a failure are identical and, after re-placement, the
-  teacher-forced logits agree within bf16 tolerance (``tests/test_failover_gpu.py``), so a
-  sampled token can differ only where two candidates are within that tolerance of each other.
+  on the GPU the tokens generated before a failure are identical as long as sessions keep their
+  rows and, after re-placement, the teacher-forced logits agree within bf16 tolerance (``tests/test_failover_gpu.py``), so a
+  sampled token in the same row can differ only where two candidates are within that tolerance of
+  each other.
 * Stop conditions are checked on the head from a pinned copy of each step's tokens one
   round later, so the decode loop never blocks the host on the device: the next step's
   inputs are gathered on the device from the previous step's sampled tokens.  A finished
