@@ -52,3 +52,29 @@ def test_products(rows, N, K, form):
     out = torch.full((R, N), float("nan"), device="cuda")
     torch.ops.mpamd.moe_gemm(form, rows_in, None, lists, wp, out, R, T, 0, 1, 0.0, 0)
     assert float((out.double().cpu() - z).norm() / z.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("form", [2, 3])
+def test_not_a_number_stays_in_its_rows(form):
+    """A row that holds something that is no number: its own outputs show it (with a limit the gate takes the limit for it, as
+    the pass over a product's rows does), no other row does."""
+    ops.require_native()
+    E, N, K, R = 2, 64, 128, 300
+    g = torch.Generator().manual_seed(form)
+    x = torch.randn(R, K, generator=g).to(torch.bfloat16)
+    x[70, 5], x[260, 9] = float("nan"), float("inf")
+    w = torch.randn(E, N, K, generator=g).div(K ** 0.5).to(torch.bfloat16)
+    wp, lists = torch.stack([ops.pack_weight(m) for m in w.cuda()]), _lists([180, 120])
+    tok, bad = torch.arange(R, dtype=torch.int32).cuda(), torch.zeros(R, dtype=torch.bool)
+    bad[70] = bad[260] = True
+    for glu, limit in ((0, 0.0), (1, 0.0), (1, 1.5)):
+        out = torch.empty(R, N // 2 if glu else N, dtype=torch.bfloat16, device="cuda")
+        torch.ops.mpamd.moe_gemm(form, x.cuda(), tok, lists, wp, out, R, R, glu, 16, limit, 0)
+        assert out[~bad].isfinite().all()
+        if limit:
+            z, want = torch.empty(R, N, dtype=torch.bfloat16, device="cuda"), torch.empty_like(out)
+            torch.ops.mpamd.moe_gemm(form, x.cuda(), tok, lists, wp, z, R, R, 0, 16, 0.0, 0)
+            ops.mixers.clamped_glu(z, want, 16, limit)
+            assert torch.equal(out.isfinite(), want.isfinite())
+        else:
+            assert out[70].isnan().all() and not (out[260].isfinite() & (out[260] != 0)).any()
