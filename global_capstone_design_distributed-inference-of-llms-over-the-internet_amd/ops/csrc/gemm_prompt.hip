@@ -13,7 +13,7 @@
 
 namespace mp {
 
-constexpr int GW_CUS = 256, GW_BAND = 8;
+constexpr int GW_CUS = WideTile::CUS, GW_BAND = 8;
 constexpr int64_t GW_SLAB = 256 * 256;  // fp32 elements of a part
 // stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
 // tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
@@ -37,8 +37,7 @@ __device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, in
   n0 = r / h * WideTile::BN;
 }
 template <int EPI>
-__device__ __forceinline__ void gw_store(const GemmPrompt& a, int m, int o, const f32x4& v, const f32x4& u, int g4) {
-  float y[4];
+__device__ __forceinline__ void gw_act(const GemmPrompt& a, const f32x4& v, const f32x4& u, float (&y)[4]) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (EPI == 1 && a.limit > 0.f) {
@@ -53,58 +52,69 @@ __device__ __forceinline__ void gw_store(const GemmPrompt& a, int m, int o, cons
       y[r] = v[r];
     }
   }
-  st_vec<4>(a.out + (int64_t)m * (EPI == 1 ? a.N / 2 : a.N) + (EPI == 1 ? o / 2 : o) + 4 * g4, y);
 }
+
+// A workgroup's tiles: every ``step``-th whole one of its XCD's run from ``first`` on, then a part of a left-over tile.
+template <int EPI>
+struct PromptWork {
+  static constexpr int STORES = WideTile::put_stores(EPI == 1);
+  typedef WideTile W;
+  const GemmPrompt& a;
+  int first, step, whole;  // (whole: how many whole ones)
+  int g;                   // the part
+  __device__ int id(int k) const { return k < whole ? first + k * step : a.full + g % a.rest; }
+  __device__ int begin(int k) const { return k < whole ? 0 : g / a.rest * (a.K / 64) / a.parts; }
+  __device__ int stages(int k) const {
+    return k < whole ? a.K / 64 : (g / a.rest + 1) * (a.K / 64) / a.parts - g / a.rest * (a.K / 64) / a.parts;
+  }
+  __device__ void rows(int k, W::Source& s) const {
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    s.from(a.x, ((uint32_t)(a.M - 1) * (uint32_t)a.xs + (uint32_t)a.K) * 2);
+    s.at = begin(k) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)  // (the launcher checks that they fit)
+      s.off[j] = (uint32_t)min(m0 + W::piece_row(j), a.M - 1) * (uint32_t)(a.xs * 2) + W::piece_byte();
+  }
+  __device__ void weights(int k, W::Source& s) const {
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    s.from(a.w, (uint32_t)a.N * (uint32_t)a.K * 2);
+    s.at = begin(k) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s.off[j] = (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
+  }
+  __device__ bool live(int k) const {
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    return m0 + 16 * W::MW * W::wm() < a.M;
+  }
+  __device__ bool store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
+    if (k == whole) {  // (nothing comes behind it)
+      float* s = a.slabs + (int64_t)g * GW_SLAB + (W::wave() * 32 * 64 + (threadIdx.x & 63)) * 4;
+#pragma unroll
+      for (int i = 0; i < W::NW; ++i)
+#pragma unroll
+        for (int j = 0; j < W::MW; ++j) *reinterpret_cast<f32x4*>(s + (i * 4 + j) * 256) = acc[i][j];
+      return false;
+    }
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    const int nw = n0 + 16 * W::NW * W::wn();
+    return W::put<EPI == 1>(a.out, EPI == 1 ? a.N / 2 : a.N, true, m0 + 16 * W::MW * W::wm(), a.M, EPI == 1 ? nw / 2 : nw, acc,
+                            [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI>(a, v, u, y); });
+  }
+};
 
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_prompt_kernel(GemmPrompt a) {
-  typedef WideTile W;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4, ks = a.K / 64, b = blockIdx.x;
-  const int blocks = (a.full + 7) / 8 * 8;  // of whole tiles
-  int id, s0 = 0, n = ks, part = 0;
-  if (b < blocks) {
-    id = (b & 7) * (blocks / 8) + (b >> 3);
-    if (id >= a.full) return;
-  } else {
-    const int all = a.rest * a.parts, g = ((b - blocks) & 7) * ((all + 7) / 8) + ((b - blocks) >> 3);
-    if (g >= all) return;
-    part = g / a.rest, id = a.full + g % a.rest;
-    s0 = part * ks / a.parts, n = (part + 1) * ks / a.parts - s0;
-  }
-  int m0, n0;
-  gw_tile(a, id, m0, n0);
-  uint32_t xo[4], wo[4];  // (the launcher checks that they fit)
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    xo[j] = (uint32_t)min(m0 + W::piece_row(j), a.M - 1) * (uint32_t)(a.xs * 2) + W::piece_byte();
-    wo[j] = (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
-  }
-  f32x4 acc[W::NW][W::MW];
-#pragma unroll
-  for (int i = 0; i < W::NW; ++i)
-#pragma unroll
-    for (int j = 0; j < W::MW; ++j) acc[i][j] = (f32x4)(0.f);
-  const int mw = m0 + 16 * W::MW * W::wm(), nw = n0 + 16 * W::NW * W::wn();
-  const char *x = (const char*)a.x + s0 * 128, *w = (const char*)a.w + s0 * 128;
-  W::run<false>(smem, x, w, xo, wo, n, mw < a.M, acc);
-  if (mw >= a.M) return;
-  if (n == ks) {
-#pragma unroll
-    for (int j = 0; j < W::MW; ++j) {
-      const int m = mw + 16 * j + c16;
-      if (m >= a.M) continue;
-#pragma unroll
-      for (int i = 0; i < W::NW; i += EPI == 1 ? 2 : 1)
-        if (nw + 16 * i < a.N) gw_store<EPI>(a, m, nw + 16 * i, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], g4);
-    }
-  } else {
-    float* s = a.slabs + (part * a.rest + id - a.full) * GW_SLAB + (W::wave() * 32 * 64 + lane) * 4;
-#pragma unroll
-    for (int i = 0; i < W::NW; ++i)
-#pragma unroll
-      for (int j = 0; j < W::MW; ++j) *reinterpret_cast<f32x4*>(s + (i * 4 + j) * 256) = acc[i][j];
-  }
+  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3, step = gridDim.x >> 3;
+  const int per = (a.full + 7) / 8, lo = xcd * per, run = min(per, a.full - lo);  // the XCD's run of whole tiles
+  const int all = a.rest * a.parts, each = (all + 7) / 8, g = xcd * each + at;
+  const int whole = at < run ? (run - at + step - 1) / step : 0, count = whole + (at < each && g < all);
+  if (count == 0) return;
+  WideTile::run<false>(smem, count, PromptWork<EPI>{a, lo + at, step, whole, g});
 }
 
 // a left-over tile's parts added and stored; blockIdx.y: two of the eight row groups of weights, two of the four of rows
@@ -134,7 +144,11 @@ __global__ __launch_bounds__(512) void gemm_prompt_close_kernel(GemmPrompt a) {
     if (m + 16 * j >= a.M) continue;
 #pragma unroll
     for (int i = 0; i < 2; i += EPI == 1 ? 2 : 1)
-      if (o + 16 * i < a.N) gw_store<EPI>(a, m + 16 * j, o + 16 * i, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], g4);
+      if (o + 16 * i < a.N) {
+        float y[4];
+        gw_act<EPI>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
+        st_vec<4>(a.out + (int64_t)(m + 16 * j) * (EPI == 1 ? a.N / 2 : a.N) + (EPI == 1 ? o / 2 + 8 * i : o + 16 * i) + 4 * g4, y);
+      }
   }
 }
 
@@ -169,7 +183,9 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
   a.rest = a.parts > 1 ? tiles % GW_CUS : 0;
   if (a.rest && ws == nullptr) return -3;
   a.full = tiles - a.rest;
-  const dim3 grid((a.full + 7) / 8 * 8 + (a.rest * a.parts + 7) / 8 * 8);
+  // as many workgroups to an XCD as it has tiles or parts, up to its CUs
+  const int per = (a.full + 7) / 8, each = (a.rest * a.parts + 7) / 8, most = per > each ? per : each;
+  const dim3 grid(8 * (most < GW_CUS / 8 ? most : GW_CUS / 8));
 #define MP_GW(E_)                                                                                                          \
   {                                                                                                                        \
     (void)hipFuncSetAttribute((const void*)gemm_prompt_kernel<E_>, hipFuncAttributeMaxDynamicSharedMemorySize, WideTile::LDS); \

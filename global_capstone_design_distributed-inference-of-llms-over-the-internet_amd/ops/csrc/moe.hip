@@ -588,55 +588,105 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
 // 8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s; the ring of 32-column stages took 687 us.  2700 tokens of two of
 // eight 14336-wide experts of width 4096: up 1502 -> 1253 us, down 803 -> 667 us; 4298 tokens of four of 32 1408-wide ones of
 // 2048: 260 -> 208 us, 151 -> 128 us.
+//
+// A workgroup makes every ``step``-th tile of its XCD's run.  Lane k of a wave knows tile k of up to 64 of them: the experts' tile
+// counts are summed over the lanes, then every lane looks for its own tile among them.
 template <bool GLU, typename TO>
-__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a) {
+struct MoeWork {
+  static constexpr int STORES = WideTile::put_stores(GLU);
   typedef WideTile W;
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  __shared__ int pick[4];
-  const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
-  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
-  if (W::wave() == 0) moe_pick(l, a.E, (a.N + W::BN - 1) / W::BN, W::BM, pick);
-  __syncthreads();
-  const int e = pick[0];
-  if (e < 0) return;
-  const int n0 = pick[1] * W::BN, m0 = pick[2] * W::BM, r0 = l.off[e], n = l.cnt[e], nt = a.N / 16;
-  const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * a.N * a.K;
-  uint32_t xo[4], wo[4];  // (the launcher checks that they fit)
+  const MoeGemm& a;
+  const MoeLists& l;
+  bool wide;
+  int en, mt;  // lane k: expert and weight tile (10 bits and the others), row tile of tile k
+  __device__ int expert(int k) const { return __builtin_amdgcn_readlane(en, k) & 1023; }
+  __device__ int n0(int k) const { return (__builtin_amdgcn_readlane(en, k) >> 10) * W::BN; }
+  __device__ int m0(int k) const { return __builtin_amdgcn_readlane(mt, k) * W::BM; }
+  __device__ int stages(int) const { return a.K / 64; }
+  __device__ void rows(int k, W::Source& s) const {
+    const int e = expert(k), m = m0(k), r0 = l.off[e], n = l.cnt[e];
+    s.from(a.x, 0xffffffffu);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int m = r0 + min(m0 + W::piece_row(j), n - 1), row = a.tok ? a.tok[m] : m;
-    xo[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + W::piece_byte();
-    wo[j] = (uint32_t)min(n0 / 16 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
-  }
-  f32x4 acc[W::NW][W::MW];
-#pragma unroll
-  for (int i = 0; i < W::NW; ++i)
-#pragma unroll
-    for (int j = 0; j < W::MW; ++j) acc[i][j] = (f32x4)(0.f);
-  const int mw = m0 + 16 * W::MW * W::wm(), nw = n0 + 16 * W::NW * W::wn();
-  W::run<true>(smem, (const char*)a.x, (const char*)w, xo, wo, a.K / 64, mw < n, acc);
-#pragma unroll
-  for (int j = 0; j < W::MW; ++j) {
-    const int m = mw + 16 * j + c16;
-    if (m >= n) continue;
-#pragma unroll
-    for (int i = 0; i < W::NW; i += GLU ? 2 : 1) {
-      const int o = nw + 16 * i;
-      if (o >= a.N) continue;
-      float y[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) y[r] = GLU ? moe_glu(acc[i][j][r], acc[GLU ? i + 1 : i][j][r], a.limit) : acc[i][j][r];
-      st_vec<4>((TO*)a.out + (int64_t)(r0 + m) * (GLU ? a.N / 2 : a.N) + (GLU ? o / 2 : o) + 4 * g4, y);
+    for (int j = 0; j < 4; ++j) {  // (the launcher checks that they fit)
+      const int q = r0 + min(m + W::piece_row(j), n - 1), row = a.tok ? a.tok[q] : q;
+      s.off[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + W::piece_byte();
     }
+  }
+  __device__ void weights(int k, W::Source& s) const {
+    const int t0 = n0(k) / 16, nt = a.N / 16;
+    s.from((const bf16_t*)a.w + (int64_t)expert(k) * a.N * a.K, (uint32_t)a.N * (uint32_t)a.K * 2);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s.off[j] = (uint32_t)min(t0 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
+  }
+  __device__ bool live(int k) const { return m0(k) + 16 * W::MW * W::wm() < l.cnt[expert(k)]; }
+  __device__ bool store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
+    const int e = expert(k), m = m0(k) + 16 * W::MW * W::wm(), o = n0(k) + 16 * W::NW * W::wn(), n = l.cnt[e];
+    const int cols = GLU ? a.N / 2 : a.N;
+    TO* out = (TO*)a.out + (int64_t)l.off[e] * cols;
+    if constexpr (sizeof(TO) == 2) {
+      return W::put<GLU>(out, cols, wide, m, n, GLU ? o / 2 : o, acc, [&](const f32x4& v, const f32x4& u, float(&y)[4]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = GLU ? moe_glu(v[r], u[r], a.limit) : v[r];
+      });
+    } else {
+      const int lane = threadIdx.x & 63;
+#pragma unroll
+      for (int j = 0; j < W::MW; ++j)
+#pragma unroll
+        for (int i = 0; i < W::NW; ++i)
+          if (m + 16 * j + (lane & 15) < n && o + 16 * i < a.N)
+            *reinterpret_cast<f32x4*>(out + (int64_t)(m + 16 * j + (lane & 15)) * cols + o + 16 * i + 4 * (lane >> 4)) = acc[i][j];
+      return false;
+    }
+  }
+};
+
+template <bool GLU, typename TO>
+__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
+  const int lane = threadIdx.x & 63, ntn = (a.N + WideTile::BN - 1) / WideTile::BN;
+  int total = 0;
+  for (int i = 0; i < a.E; i += 64) total += moe_tile_count(l, a.E, i, lane, WideTile::BM);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, 64);
+  const int all = __builtin_amdgcn_readfirstlane(total) * ntn, per = (all + 7) / 8, step = gridDim.x >> 3, at = blockIdx.x >> 3;
+  const int lo = (blockIdx.x & 7) * per + at, run = min(per, all - (int)(blockIdx.x & 7) * per);
+  const int tiles = at < run ? (run - at + step - 1) / step : 0;
+  for (int first = 0; first < tiles; first += 64) {
+    const int count = min(64, tiles - first), id = lo + min(first + lane, tiles - 1) * step;
+    int en = 0, mt = 0, base = 0;
+    for (int i = 0; i < a.E; i += 64) {
+      const int c = moe_tile_count(l, a.E, i, lane, WideTile::BM);
+      int sum = c;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(sum, d, 64);
+        if (lane >= d) sum += y;
+      }
+      for (int q = 0; q < min(64, a.E - i); ++q) {
+        const int ce = __builtin_amdgcn_readlane(c, q), b = (base + __builtin_amdgcn_readlane(sum, q) - ce) * ntn;
+        if (id >= b && id < b + ce * ntn) {
+          const int r = id - b, band = r / (MG_BAND * ntn), h = min(MG_BAND, ce - MG_BAND * band), s = r - band * MG_BAND * ntn;
+          en = i + q + (s / h << 10);
+          mt = MG_BAND * band + s % h;
+        }
+      }
+      base += __builtin_amdgcn_readlane(sum, 63);
+    }
+    if (first) __syncthreads();  // (the last tiles' operands have been read)
+    WideTile::run<true>(smem, count, MoeWork<GLU, TO>{a, l, wide, en, mt});
   }
 }
 
 template <bool GLU, typename TO>
 static int launch_moe_wide(const MoeGemm& a, int rows, int act, hipStream_t stream) {
-  const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN);
+  const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN), per = (tiles + 7) / 8;
   (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             WideTile::LDS);
-  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3((tiles + 7) / 8 * 8), dim3(512), WideTile::LDS, stream, a);
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3(8 * (per < WideTile::CUS / 8 ? per : WideTile::CUS / 8)), dim3(512),
+                     WideTile::LDS, stream, a, (uintptr_t)a.out % 16 == 0);
   return (int)hipGetLastError();
 }
 

@@ -1,30 +1,33 @@
 // Main loop of the 256 x 256 product tiles (moe.hip: experts, gemm_prompt.hip: prompts): eight waves of 64 rows x 128 weight
-// rows, 64 columns a stage in two LDS slots of 64 KiB.
+// rows, 64 columns a stage.  A workgroup stays on its CU for all its tiles, and its loads run ahead across them.
 //   * Rows arrive 128 bytes at a time (8 rows an instruction), whole cache lines: 32-column stages fetch every line twice,
 //     and 256 rows of lines are the whole L1, so the second half came from L2 again.  The 16-byte chunks of a row are
 //     permuted by its low bits on the way in, which leaves the operand reads free of bank conflicts (none counted).
 //     Weights come the same way, or packed in fragment order ([N / 16, K / 32, 64, 8]) as they lie.
-//   * The operands of a half stage are read from LDS while the MFMAs of the half before it run, across the one barrier a
-//     stage has: behind it the other slot has landed for all waves and this one is free.  The loads of the next stage but
-//     one are spread over the half stage behind the barrier: eight at once hold up the MFMAs that stand behind them.
+//   * All 160 KiB of LDS are a ring of five slots of one operand's stage.  Behind the one barrier of a stage its two slots are
+//     free: the rows of the stage after the next go to one, the weights of the stage after that to the other, so that
+//     weights, which come from HBM, have more than a stage and a half to arrive.  With two slots an operand and workgroups
+//     that end with their tile, weights that no cache held cost 4096 x 16384 x 4096 446 us (now 384, the library 353),
+//     4096 x 4096 x 14336 362 (322, 314), 6421 x 12288 x 4096 527 (474, 502); the early slot on the rows' side took 404,
+//     342 and 497 us.
+//   * The operands of a half stage are read from LDS while the MFMAs of the half before it run, across the barrier, one read
+//     to two MFMAs; the stage's loads are spread over the half stage behind the barrier: eight at once hold up the MFMAs that
+//     stand behind them.
 //   * A wave whose 64 rows are past the last only loads; the two waves of a SIMD have different rows, so a tile of up to 128
 //     rows takes half the time.
-// Bound by MFMA issue and, in part, by waits for the next stage.  Measured and left: four waves of 128 x 128 (the same time
-// where the tiles are full, 5-10 % more elsewhere; LDS is a quarter busy either way), a second barrier that frees the slot
-// sooner (6 % more), loads behind the reads (6 % more), lines of later
-// stages brought into L2 ahead (no change), 32 x 32 x 16 MFMAs (12 % more).
+// Bound by MFMA issue (three quarters of the time; the clock falls to 1.8 GHz under it) and by the issue of the loads, an eighth.
+// Measured and left: four waves of 128 x 128 (2 to 5 % more), a second barrier that frees the slot sooner (6 % more), 32 x 32
+// x 16 MFMAs (12 % more), loads over both halves of a stage (up to 8 % more).
 #pragma once
-#include <type_traits>
-
 #include "common.h"
 
 namespace mp {
 
 struct WideTile {
-  static constexpr int BM = 256, BN = 256, MW = 4, NW = 8, WM = 4, WN = 2, XB = BM * 128, SLOT = XB + BN * 128, LDS = 2 * SLOT;
+  static constexpr int BM = 256, BN = 256, MW = 4, NW = 8, WM = 4, WN = 2, SLOTS = 5, SLOT = 256 * 128, LDS = SLOTS * SLOT;
+  static constexpr int CUS = 256;  // workgroups of a launch at most: one to a CU
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
   typedef __attribute__((address_space(3))) void* lptr_t;
-  typedef __attribute__((address_space(1))) const void* gptr_t;
 
   static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
   static __device__ __forceinline__ int wm() { return wave() / WN; }  // (the waves of a SIMD, 4 apart, have different rows)
@@ -36,103 +39,200 @@ struct WideTile {
   static __device__ __forceinline__ int packed_tile(int j) { return 2 * wave() + (j >> 1); }
   static __device__ __forceinline__ int packed_byte(int j) { return 1024 * (j & 1) + (threadIdx.x & 63) * 16; }
 
-  // acc[i][j] += weight rows 16 (8 wn + i) .. x rows 16 (4 wm + j) .., over ``ks`` stages from ``x`` and ``w`` on; lane: row
-  // lane % 16, weight rows 4 (lane / 16) .. + 3.  xo, wo: byte offsets of the wave's pieces.  Starts and ends with LDS
-  // that other waves may still read.
-  template <bool PACKED>
-  static __device__ __forceinline__ void run(char* smem, const char* x, const char* w, const uint32_t (&xo)[4],
-                                             const uint32_t (&wo)[4], int ks, bool live, f32x4 (&acc)[NW][MW]) {
+  // Where an operand of a tile comes from: this lane's byte offsets of the wave's pieces from ``at`` bytes behind the base on.
+  struct Source {
+    __amdgpu_buffer_rsrc_t base;
+    uint32_t off[4], at;
+    __device__ __forceinline__ void from(const void* p, uint32_t bytes) {
+      base = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+      at = 0;
+    }
+  };
+
+  // The workgroup's tiles 0 .. count - 1 (at least one).  ``work``:
+  //   int stages(k)                  stages of tile k, at least one
+  //   void rows(k, Source&)          its rows
+  //   void weights(k, Source&)       its weight rows
+  //   bool live(k)                   has this wave rows in it?
+  //   bool store(k, acc)             acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (4 wm + j) ..; lane: row lane % 16, weight
+  //                                  rows 4 (lane / 16) .. + 3.  True: at least work.STORES stores were issued for sure.
+  // Ends with no load in flight.
+  template <bool PACKED, class Work>
+  static __device__ __forceinline__ void run(char* smem, int count, const Work& work) {
     constexpr int WSTEP = PACKED ? 2048 : 128;
-    const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4, wv = wave();
-    auto issue1 = [&](int st, int j) {  // one of this wave's pieces of stage st
-      char* b = smem + (st & 1) * SLOT + wv * 4096;
-      if (j < 4)
-        __builtin_amdgcn_global_load_lds((gptr_t)(x + (int64_t)st * 128 + xo[j]), (lptr_t)(b + j * 1024), 16, 0, 0);
-      else
-        __builtin_amdgcn_global_load_lds((gptr_t)(w + (int64_t)st * WSTEP + wo[j - 4]), (lptr_t)(b + XB + (j - 4) * 1024), 16, 0,
-                                         0);
+    const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+    char* mine = smem + wave() * 4096;
+    Source x, w;
+    int xk = 0, wk = 0, xleft = work.stages(0), wleft = xleft;  // the tile that is being loaded, its stages left
+    work.rows(0, x);
+    work.weights(0, w);
+    auto load_x = [&](int j, int slot) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x.base, (lptr_t)(mine + slot * SLOT + j * 1024), 16, x.off[j], x.at, 0, 0);
     };
-    auto issue = [&](int st) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) issue1(st, j);
+    auto load_w = [&](int j, int slot) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.base, (lptr_t)(mine + slot * SLOT + j * 1024), 16, w.off[j], w.at, 0, 0);
+    };
+    // (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
+    auto next_x = [&] {
+      if (--xleft > 0) x.at += 128;
+      else if (xk + 1 < count) xleft = work.stages(++xk), work.rows(xk, x);
+      else xleft = 1;
+    };
+    auto next_w = [&] {
+      if (--wleft > 0) w.at += WSTEP;
+      else if (wk + 1 < count) wleft = work.stages(++wk), work.weights(wk, w);
+      else wleft = 1;
     };
     // a row's chunk c lies at 16 (c ^ row % 8)
     const int s0 = 16 * (g4 ^ (c16 & 7)), s1 = 16 * ((4 + g4) ^ (c16 & 7));
-    const int xr0 = (16 * MW * wm() + c16) * 128, wr0 = XB + (PACKED ? 2 * NW * wn() * 1024 + lane * 16 : (16 * NW * wn() + c16) * 128);
+    const int xr = (16 * MW * wm() + c16) * 128, wr = PACKED ? 2048 * NW * wn() + lane * 16 : (16 * NW * wn() + c16) * 128;
     u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
-    auto take1 = [&](int st, int h, int r, u16x8(&xr)[MW], u16x8(&wr)[NW]) {  // one operand of a half stage
-      const char* b = smem + (st & 1) * SLOT;
-      if (r < MW) xr[r] = *reinterpret_cast<const u16x8*>(b + xr0 + (h ? s1 : s0) + r * 2048);
-      else if (PACKED) wr[r - MW] = *reinterpret_cast<const u16x8*>(b + wr0 + (2 * (r - MW) + h) * 1024);
-      else wr[r - MW] = *reinterpret_cast<const u16x8*>(b + wr0 + (h ? s1 : s0) + (r - MW) * 2048);
-    };
-    auto multiply = [&](const u16x8(&xr)[MW], const u16x8(&wr)[NW]) {
+    f32x4 acc[NW][MW];
+    auto multiply = [&](const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
 #pragma unroll
       for (int i = 0; i < NW; ++i)
 #pragma unroll
         for (int j = 0; j < MW; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[i]), __builtin_bit_cast(bf16x8, xr[j]),
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i]), __builtin_bit_cast(bf16x8, xf[j]),
                                                               acc[i][j], 0, 0, 0);
     };
-    // the order inside a half stage, in eighths: 4 MFMAs, 1 or 2 of the 12 reads, 1 load.  Without the fences the compiler
-    // moves the MFMAs behind the barrier and the reads stand alone.
-    auto half = [&](auto reads, auto loads) {
-      constexpr bool R = decltype(reads)::value, L = decltype(loads)::value;
+    int px = 1, pw = 0;  // slots of the stage's rows and weights
+    auto take1 = [&](int h, int r, u16x8(&xf)[MW], u16x8(&wf)[NW]) {  // one operand of a half stage
+      if (r < MW) xf[r] = *reinterpret_cast<const u16x8*>(smem + px * SLOT + xr + (h ? s1 : s0) + r * 2048);
+      else wf[r - MW] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (PACKED ? h * 1024 : h ? s1 : s0) + (r - MW) * 2048);
+    };
+    auto take = [&](int h, u16x8(&xf)[MW], u16x8(&wf)[NW]) {
 #pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        if constexpr (L) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-        if constexpr (R) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (i & 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        } else {
-          __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        }
+      for (int r = 0; r < MW + NW; ++r) take1(h, r, xf, wf);
+    };
+    auto fill = [&](int m, int freed_x, int freed_w) {  // load m of the eight behind a barrier: rows of the next stage but one
+      if (m < 4) load_x(m, freed_w);                    // where the stage's weights were, then weights of the one behind it
+      else load_w(m - 4, freed_x);
+    };
+    // the order inside a half stage: 32 MFMAs, a read behind each second, a load behind each fourth.  Without the fences the
+    // compiler moves the MFMAs behind the barrier and the reads stand alone.
+    auto order = [&](bool loads) {
+#pragma unroll
+      for (int m = 0; m < NW * MW; ++m) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (m < 24 && m % 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (loads && m % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    auto stage = [&](int st, auto next, auto load) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < MW + NW; ++r) take1(st, 1, r, xb, wb);
-      multiply(xa, wa);
-      half(std::true_type{}, std::false_type{});
-      if constexpr (decltype(next)::value) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_wait_barrier();  // stage st + 1 has landed for all waves, and all have read stage st
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < NW; ++i) {  // (loads write LDS: the compiler keeps the order of loads and reads)
-          if constexpr (decltype(load)::value) issue1(st + 2, i);
-#pragma unroll
-          for (int r = i * 12 / NW; r < (i + 1) * 12 / NW; ++r) take1(st + 1, 0, r, xa, wa);
-        }
-      }
-      multiply(xb, wb);
-      half(next, load);
+    auto turn = [&] {  // to the next stage's slots
+      px = px >= SLOTS - 2 ? px + 2 - SLOTS : px + 2;
+      pw = pw >= SLOTS - 2 ? pw + 2 - SLOTS : pw + 2;
     };
-    __syncthreads();
-    issue(0);
-    if (ks > 1) issue(1);
-    if (ks > 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_wait_barrier();
-    if (!live) {
-      for (int st = 0; st + 1 < ks; ++st) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_wait_barrier();
-        if (st + 2 < ks) issue(st + 2);
-      }
-      return;
+    // the next stage has landed for all waves, and all have read this one.  In flight: the weights of the stage after it and
+    // the stores of the tile before
+    auto meet = [&](int stored) {
+      if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + Work::STORES) : "memory");
+      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      lds_wait_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll 1
+    for (int s = 0; s < SLOTS; s += 2) {  // w 0, x 0, w 1, x 1, w 2
+#pragma unroll
+      for (int j = 0; j < 4; ++j) load_w(j, s);
+      next_w();
+      if (s + 1 == SLOTS) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) load_x(j, s + 1);
+      next_x();
     }
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    lds_wait_barrier();
+    take(0, xa, wa);
+    int stored = 0;
+    for (int k = 0; k < count; ++k) {
+      const int n = work.stages(k);
+      if (!work.live(k)) {
+        for (int st = 0; st < n; ++st) {
+          meet(stored);
+          stored = 0;
+          const int fx = px, fw = pw;
+          turn();
 #pragma unroll
-    for (int r = 0; r < MW + NW; ++r) take1(0, 0, r, xa, wa);
-    int st = 0;
-    for (; st + 2 < ks; ++st) stage(st, std::true_type{}, std::true_type{});
-    if (st + 1 < ks) stage(st++, std::true_type{}, std::false_type{});
-    stage(st, std::false_type{}, std::false_type{});
+          for (int m = 0; m < 8; ++m) fill(m, fx, fw);
+          next_x();
+          next_w();
+        }
+        take(0, xa, wa);
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int j = 0; j < MW; ++j) acc[i][j] = (f32x4)(0.f);
+      for (int st = 0; st < n; ++st) {
+        __builtin_amdgcn_sched_barrier(0);
+        take(1, xb, wb);
+        multiply(xa, wa);
+        order(false);
+        meet(stored);
+        stored = 0;
+        const int fx = px, fw = pw;
+        turn();
+#pragma unroll
+        for (int m = 0; m < NW * MW; ++m) {  // (loads write LDS: the compiler keeps the order of loads and reads)
+          if (m < 24 && m % 2) take1(0, m / 2, xa, wa);
+          if (m % 4 == 3) fill(m / 4, fx, fw);
+        }
+        multiply(xb, wb);
+        order(true);
+        next_x();
+        next_w();
+      }
+      stored = work.store(k, acc);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  }
+
+  // Rows of ``acc`` from m on (those below ``end``) to out[row][cols], columns from ``col`` on.  GLU: ``act`` makes one of each
+  // two fragments (gate, up), else of each one.  A lane holds 4 columns of a row in a fragment; neighbouring fragments trade
+  // halves between the lane's rows of 16, so that a lane stores 16 bytes and an instruction 64 bytes of each of 16 rows (8
+  // bytes a lane: 6421 x 12288 x 4096 506 -> 480 us).  ``wide``: out is 16-byte aligned.  True: all of them were stored.
+  static constexpr int put_stores(bool glu) { return MW * NW / (glu ? 4 : 2); }
+  template <bool GLU, class Act>
+  static __device__ __forceinline__ bool put(bf16_t* out, int cols, bool wide, int m, int end, int col, const f32x4 (&acc)[NW][MW],
+                                             Act act) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+    typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+    constexpr int S = GLU ? 2 : 1;
+    const int c16 = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4, lc = col + 16 * (g4 & 1) + 8 * (g4 >> 1);
+    const bool whole = wide && m + 16 * MW <= end && col + 16 * NW / S <= cols;
+    bf16_t* at = out + (int64_t)(m + c16) * cols + lc;
+    auto each = [&](auto store) {
+#pragma unroll
+      for (int j = 0; j < MW; ++j) {
+#pragma unroll
+        for (int i = 0; i < NW; i += 2 * S) {
+          uint32_t d[2][2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float y[4];
+            act(acc[i + h * S][j], acc[i + h * S + S - 1][j], y);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) d[h][r] = (uint32_t)f2bf(y[2 * r]) | (uint32_t)f2bf(y[2 * r + 1]) << 16;
+          }
+          const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false));
+          const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false));
+          store(j, 16 * i / S, at + (int64_t)16 * j * cols + 16 * i / S, (u32x4){a[0], b[0], a[1], b[1]});
+        }
+      }
+    };
+    if (whole) {
+      each([](int, int, bf16_t* p, const u32x4& v) { *reinterpret_cast<u32x4*>(p) = v; });
+    } else {
+      each([&](int j, int c, bf16_t* p, const u32x4& v) {
+        if (m + 16 * j + c16 >= end || lc + c >= cols) return;  // (columns come in sixteens)
+        *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
+        *reinterpret_cast<u32x2*>(p + 4) = (u32x2){v[2], v[3]};
+      });
+    }
+    return whole;
   }
 };
 

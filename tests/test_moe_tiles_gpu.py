@@ -54,6 +54,30 @@ def test_products(rows, N, K, form):
     assert float((out.double().cpu() - z).norm() / z.norm()) < 1e-5
 
 
+@pytest.mark.parametrize("E,N,K,each", [(70, 64, 64, 130), (3, 256, 128, 22400)])
+def test_many_experts_and_many_tiles(E, N, K, each):
+    """Experts past a wave's 64 lanes, and more than 64 tiles to a workgroup (which takes them 64 at a time); rows that begin
+    at 8 bytes.  The tolerance as above."""
+    ops.require_native()
+    if E == 3:
+        N = 16640  # 65 weight tiles of 264 row tiles: 17160 tiles on 256 workgroups
+    counts = [each + e % 2 for e in range(E)]
+    R = sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(R, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(E, N, K, generator=g, device="cuda").div(K ** 0.5).to(torch.bfloat16)
+    wp, lists = torch.stack([ops.pack_weight(m) for m in w]), _lists(counts)
+    room = torch.full((R * N + 4,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for out in (room[:R * N].view(R, N), room[4:].view(R, N)):
+        out.fill_(float("nan"))
+        torch.ops.mpamd.moe_gemm(3, x, None, lists, wp, out, R, R, 0, 1, 0.0, 0)
+        at = 0
+        for e, n in enumerate(counts):
+            want = x[at:at + n].float() @ w[e].float().t()
+            assert float((out[at:at + n].float() - want).norm() / want.norm()) < 2.0 ** -8
+            at += n
+
+
 @pytest.mark.parametrize("form", [2, 3])
 def test_not_a_number_stays_in_its_rows(form):
     """A row that holds something that is no number: its own outputs show it (with a limit the gate takes the limit for it, as
