@@ -14,15 +14,15 @@ namespace {
 
 int64_t gemm_prompt_ws(int64_t M, int64_t N, int64_t K) { return mp_gemm_prompt_ws((int)M, (int)N, (int)K); }
 
-// out[M, N'] = epilogue(x[M, K] w[N, K]^T)
+// out[M, N'] = epilogue(x[M, K] w[N, K]^T); epi 8: x[M, K] w[K, N]
 void gemm_prompt(const at::Tensor& x, const at::Tensor& w, at::Tensor& out, const c10::optional<at::Tensor>& ws, int64_t epi,
                double limit) {
   MP_CHECK(x.is_cuda() && w.is_cuda() && out.is_cuda() && x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "2-d GPU tensors");
   MP_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16, "bf16");
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  MP_CHECK(M >= 1 && K >= 64 && K % 64 == 0 && N >= 16 && N % 16 == 0 && w.size(1) == K, "K in steps of 64, N in steps of 16");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(epi == 8 ? 1 : 0);
+  MP_CHECK(M >= 1 && K >= 64 && K % 64 == 0 && N >= 16 && N % 16 == 0 && w.size(epi == 8 ? 0 : 1) == K, "K in steps of 64, N in steps of 16");
   check_rows(x, M, K, "x");
-  check_rows(w, N, K, "w");
+  check_rows(w, w.size(0), w.size(1), "w");
   check_rows(out, M, epi == 1 ? N / 2 : N, "out");
   MP_CHECK(w.is_contiguous() && out.is_contiguous() && out.size(0) == M && x.stride(0) % 8 == 0 && x.stride(0) >= K, "strides");
   MP_CHECK(M * x.stride(0) < (1ll << 31) && N * K < (1ll << 31), "operands of at most 4 GiB");

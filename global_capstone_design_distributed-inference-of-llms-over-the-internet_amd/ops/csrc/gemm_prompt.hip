@@ -1,5 +1,5 @@
-// Products of prompt-sized steps: y[M, N'] = epilogue(x[M, K] w[N, K]^T), both operands row-major, 256 x 256 tiles of
-// wide_tile.h.  Epilogues: none; the gated forms over gate / up rows in blocks of 16 (silu(g) u, or with a limit
+// Products of prompt-sized steps: y[M, N'] = epilogue(x[M, K] w[N, K]^T), both operands row-major, or x[M, K] w[K, N] for
+// gradients; 256 x 256 tiles of wide_tile.h.  Epilogues: none; the gated forms over gate / up rows in blocks of 16 (silu(g) u, or with a limit
 // g sigmoid(1.702 g) (u + 1) on clamped inputs), N' = N / 2; max(y, 0)^2.  Everything up to the one store is 32 bits: next to
 // a library product and an activation kernel, the product's rows are neither written, read back nor rounded.
 //
@@ -14,6 +14,7 @@
 namespace mp {
 
 constexpr int GW_CUS = WideTile::CUS, GW_BAND = 8;
+constexpr int GW_COLUMNS = 8;  // in place of an epilogue: w is [K, N], no epilogue
 constexpr int64_t GW_SLAB = 256 * 256;  // fp32 elements of a part
 // stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
 // tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
@@ -70,7 +71,7 @@ struct PromptWork {
   __device__ void rows(int k, W::Source& s) const {
     int m0, n0;
     gw_tile(a, id(k), m0, n0);
-    s.from(a.x, ((uint32_t)(a.M - 1) * (uint32_t)a.xs + (uint32_t)a.K) * 2);
+    s.from(a.x, ((uint32_t)(a.M - 1) * (uint32_t)a.xs + (uint32_t)a.K) * 2, 128);
     s.at = begin(k) * 128;
 #pragma unroll
     for (int j = 0; j < 4; ++j)  // (the launcher checks that they fit)
@@ -79,10 +80,13 @@ struct PromptWork {
   __device__ void weights(int k, W::Source& s) const {
     int m0, n0;
     gw_tile(a, id(k), m0, n0);
-    s.from(a.w, (uint32_t)a.N * (uint32_t)a.K * 2);
-    s.at = begin(k) * 128;
+    s.from(a.w, (uint32_t)a.N * (uint32_t)a.K * 2, EPI == GW_COLUMNS ? (uint32_t)a.N * 128 : 128);
+    s.at = begin(k) * s.step;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s.off[j] = (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
+    for (int j = 0; j < 4; ++j)
+      s.off[j] = EPI == GW_COLUMNS
+                     ? ((uint32_t)W::column_row(j) * (uint32_t)a.N + (uint32_t)min(n0 + W::column_first(j), a.N - 8)) * 2
+                     : (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
   }
   __device__ bool live(int k) const {
     int m0, n0;
@@ -114,7 +118,7 @@ __global__ __launch_bounds__(512) void gemm_prompt_kernel(GemmPrompt a) {
   const int all = a.rest * a.parts, each = (all + 7) / 8, g = xcd * each + at;
   const int whole = at < run ? (run - at + step - 1) / step : 0, count = whole + (at < each && g < all);
   if (count == 0) return;
-  WideTile::run<false>(smem, count, PromptWork<EPI>{a, lo + at, step, whole, g});
+  WideTile::run<EPI == GW_COLUMNS ? WideTile::COLUMNS : WideTile::ROWS>(smem, count, PromptWork<EPI>{a, lo + at, step, whole, g});
 }
 
 // a left-over tile's parts added and stored; blockIdx.y: two of the eight row groups of weights, two of the four of rows
@@ -195,6 +199,7 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
   if (epi == 0) MP_GW(0)
   else if (epi == 1) MP_GW(1)
   else if (epi == 4) MP_GW(4)
+  else if (epi == GW_COLUMNS) MP_GW(GW_COLUMNS)
   else return -4;
 #undef MP_GW
   return (int)hipGetLastError();

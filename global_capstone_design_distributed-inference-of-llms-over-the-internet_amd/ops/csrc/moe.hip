@@ -605,7 +605,7 @@ struct MoeWork {
   __device__ int stages(int) const { return a.K / 64; }
   __device__ void rows(int k, W::Source& s) const {
     const int e = expert(k), m = m0(k), r0 = l.off[e], n = l.cnt[e];
-    s.from(a.x, 0xffffffffu);
+    s.from(a.x, 0xffffffffu, 128);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // (the launcher checks that they fit)
       const int q = r0 + min(m + W::piece_row(j), n - 1), row = a.tok ? a.tok[q] : q;
@@ -614,7 +614,7 @@ struct MoeWork {
   }
   __device__ void weights(int k, W::Source& s) const {
     const int t0 = n0(k) / 16, nt = a.N / 16;
-    s.from((const bf16_t*)a.w + (int64_t)expert(k) * a.N * a.K, (uint32_t)a.N * (uint32_t)a.K * 2);
+    s.from((const bf16_t*)a.w + (int64_t)expert(k) * a.N * a.K, (uint32_t)a.N * (uint32_t)a.K * 2, 2048);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       s.off[j] = (uint32_t)min(t0 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide
       base += __builtin_amdgcn_readlane(sum, 63);
     }
     if (first) __syncthreads();  // (the last tiles' operands have been read)
-    WideTile::run<true>(smem, count, MoeWork<GLU, TO>{a, l, wide, en, mt});
+    WideTile::run<WideTile::PACKED>(smem, count, MoeWork<GLU, TO>{a, l, wide, en, mt});
   }
 }
 

@@ -3,7 +3,10 @@
 //   * Rows arrive 128 bytes at a time (8 rows an instruction), whole cache lines: 32-column stages fetch every line twice,
 //     and 256 rows of lines are the whole L1, so the second half came from L2 again.  The 16-byte chunks of a row are
 //     permuted by its low bits on the way in, which leaves the operand reads free of bank conflicts (none counted).
-//     Weights come the same way, or packed in fragment order ([N / 16, K / 32, 64, 8]) as they lie.
+//     Weights come the same way, packed in fragment order ([N / 16, K / 32, 64, 8]) as they lie, or as columns of a [K, N]
+//     matrix: 64 rows of 512 bytes a stage.  Their 32-byte chunks are permuted by the row, and the transposing LDS read
+//     turns them into operands (8 rows' 32 bytes in 8 different groups of banks).  The compiler lets that read wait for all
+//     loads into LDS that it knows of, so this form issues its own; they have no registers to write.
 //   * All 160 KiB of LDS are a ring of five slots of one operand's stage.  Behind the one barrier of a stage its two slots are
 //     free: the rows of the stage after the next go to one, the weights of the stage after that to the other, so that
 //     weights, which come from HBM, have more than a stage and a half to arrive.  With two slots an operand and workgroups
@@ -26,7 +29,11 @@ namespace mp {
 struct WideTile {
   static constexpr int BM = 256, BN = 256, MW = 4, NW = 8, WM = 4, WN = 2, SLOTS = 5, SLOT = 256 * 128, LDS = SLOTS * SLOT;
   static constexpr int CUS = 256;  // workgroups of a launch at most: one to a CU
+  enum Weights { ROWS, PACKED, COLUMNS };
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+  typedef __attribute__((ext_vector_type(4))) short s16x4;
+  typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   typedef __attribute__((address_space(3))) void* lptr_t;
 
   static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
@@ -39,13 +46,23 @@ struct WideTile {
   static __device__ __forceinline__ int packed_tile(int j) { return 2 * wave() + (j >> 1); }
   static __device__ __forceinline__ int packed_byte(int j) { return 1024 * (j & 1) + (threadIdx.x & 63) * 16; }
 
-  // Where an operand of a tile comes from: this lane's byte offsets of the wave's pieces from ``at`` bytes behind the base on.
+  // the same of columns: row of a stage, and first of 8 columns
+  static __device__ __forceinline__ int column_row(int j) { return 2 * (4 * wave() + j) + ((threadIdx.x & 63) >> 5); }
+  static __device__ __forceinline__ int column_first(int j) {
+    const int row = column_row(j), chunk = (threadIdx.x & 31) >> 1;
+    return 16 * (chunk ^ ((row & 3) | (row >> 3 & 1) << 2)) + 8 * (threadIdx.x & 1);
+  }
+
+  // Where an operand of a tile comes from: this lane's byte offsets of the wave's pieces from ``at`` bytes behind the base on,
+  // ``step`` bytes a stage.
   struct Source {
     __amdgpu_buffer_rsrc_t base;
-    uint32_t off[4], at;
-    __device__ __forceinline__ void from(const void* p, uint32_t bytes) {
+    u32x4 words;  // of ``base``
+    uint32_t off[4], at, step;
+    __device__ __forceinline__ void from(const void* p, uint32_t bytes, uint32_t stage) {
       base = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-      at = 0;
+      words = (u32x4){(uint32_t)(uintptr_t)p, (uint32_t)((uintptr_t)p >> 32) & 0xffff, bytes, 0x00020000};
+      at = 0, step = stage;
     }
   };
 
@@ -57,49 +74,66 @@ struct WideTile {
   //   bool store(k, acc)             acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (4 wm + j) ..; lane: row lane % 16, weight
   //                                  rows 4 (lane / 16) .. + 3.  True: at least work.STORES stores were issued for sure.
   // Ends with no load in flight.
-  template <bool PACKED, class Work>
+  template <Weights FORM, class Work>
   static __device__ __forceinline__ void run(char* smem, int count, const Work& work) {
-    constexpr int WSTEP = PACKED ? 2048 : 128;
     const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
     char* mine = smem + wave() * 4096;
     Source x, w;
     int xk = 0, wk = 0, xleft = work.stages(0), wleft = xleft;  // the tile that is being loaded, its stages left
     work.rows(0, x);
     work.weights(0, w);
-    auto load_x = [&](int j, int slot) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(x.base, (lptr_t)(mine + slot * SLOT + j * 1024), 16, x.off[j], x.at, 0, 0);
+    auto load = [&](const Source& s, int j, int slot) {
+      const lptr_t to = (lptr_t)(mine + slot * SLOT + j * 1024);
+      if constexpr (FORM == COLUMNS)  // (m0: nothing else of this form uses it; 5 cycles from a scalar that a vector instruction wrote to its use)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"((uint32_t)(uintptr_t)to),
+                     "v"(s.off[j]), "s"(s.words), "s"(s.at)
+                     : "memory");
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, to, 16, s.off[j], s.at, 0, 0);
     };
-    auto load_w = [&](int j, int slot) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.base, (lptr_t)(mine + slot * SLOT + j * 1024), 16, w.off[j], w.at, 0, 0);
-    };
+    auto load_x = [&](int j, int slot) { load(x, j, slot); };
+    auto load_w = [&](int j, int slot) { load(w, j, slot); };
     // (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
     auto next_x = [&] {
-      if (--xleft > 0) x.at += 128;
+      if (--xleft > 0) x.at += x.step;
       else if (xk + 1 < count) xleft = work.stages(++xk), work.rows(xk, x);
       else xleft = 1;
     };
     auto next_w = [&] {
-      if (--wleft > 0) w.at += WSTEP;
+      if (--wleft > 0) w.at += w.step;
       else if (wk + 1 < count) wleft = work.stages(++wk), work.weights(wk, w);
       else wleft = 1;
     };
     // a row's chunk c lies at 16 (c ^ row % 8)
     const int s0 = 16 * (g4 ^ (c16 & 7)), s1 = 16 * ((4 + g4) ^ (c16 & 7));
-    const int xr = (16 * MW * wm() + c16) * 128, wr = PACKED ? 2048 * NW * wn() + lane * 16 : (16 * NW * wn() + c16) * 128;
+    const int xr = (16 * MW * wm() + c16) * 128;
+    const int wr = FORM == PACKED    ? 2048 * NW * wn() + lane * 16
+                   : FORM == COLUMNS ? (8 * g4 + (c16 >> 2)) * 512 + 256 * wn() + 32 * (c16 >> 2 | (g4 & 1) << 2) + 8 * (c16 & 3)
+                                     : (16 * NW * wn() + c16) * 128;
     u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
     f32x4 acc[NW][MW];
+    auto multiply1 = [&](int i, const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
+#pragma unroll
+      for (int j = 0; j < MW; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i]), __builtin_bit_cast(bf16x8, xf[j]),
+                                                            acc[i][j], 0, 0, 0);
+    };
     auto multiply = [&](const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
 #pragma unroll
-      for (int i = 0; i < NW; ++i)
-#pragma unroll
-        for (int j = 0; j < MW; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i]), __builtin_bit_cast(bf16x8, xf[j]),
-                                                              acc[i][j], 0, 0, 0);
+      for (int i = 0; i < NW; ++i) multiply1(i, xf, wf);
     };
     int px = 1, pw = 0;  // slots of the stage's rows and weights
     auto take1 = [&](int h, int r, u16x8(&xf)[MW], u16x8(&wf)[NW]) {  // one operand of a half stage
-      if (r < MW) xf[r] = *reinterpret_cast<const u16x8*>(smem + px * SLOT + xr + (h ? s1 : s0) + r * 2048);
-      else wf[r - MW] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (PACKED ? h * 1024 : h ? s1 : s0) + (r - MW) * 2048);
+      if (r < MW) {
+        xf[r] = *reinterpret_cast<const u16x8*>(smem + px * SLOT + xr + (h ? s1 : s0) + r * 2048);
+      } else if constexpr (FORM == COLUMNS) {
+        const char* p = smem + ((pw * SLOT + wr) ^ (32 * (r - MW))) + h * 16384;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 2048));
+        wf[r - MW] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        wf[r - MW] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (FORM == PACKED ? h * 1024 : h ? s1 : s0) + (r - MW) * 2048);
+      }
     };
     auto take = [&](int h, u16x8(&xf)[MW], u16x8(&wf)[NW]) {
 #pragma unroll
@@ -116,6 +150,7 @@ struct WideTile {
       for (int m = 0; m < NW * MW; ++m) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         if (m < 24 && m % 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (FORM == COLUMNS && m < 24 && m % 2 && m / 2 >= MW) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         if (loads && m % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -175,6 +210,18 @@ struct WideTile {
         stored = 0;
         const int fx = px, fw = pw;
         turn();
+        if constexpr (FORM == COLUMNS) {  // (its loads are of no kind that ``order`` knows)
+#pragma unroll
+          for (int i = 0; i < NW; ++i) {
+            if (i < 6) take1(0, 2 * i, xa, wa), take1(0, 2 * i + 1, xa, wa);
+            multiply1(i, xb, wb);
+            fill(i, fx, fw);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          next_x();
+          next_w();
+          continue;
+        }
 #pragma unroll
         for (int m = 0; m < NW * MW; ++m) {  // (loads write LDS: the compiler keeps the order of loads and reads)
           if (m < 24 && m % 2) take1(0, m / 2, xa, wa);
@@ -198,8 +245,6 @@ struct WideTile {
   template <bool GLU, class Act>
   static __device__ __forceinline__ bool put(bf16_t* out, int cols, bool wide, int m, int end, int col, const f32x4 (&acc)[NW][MW],
                                              Act act) {
-    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-    typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
     constexpr int S = GLU ? 2 : 1;
     const int c16 = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4, lc = col + 16 * (g4 & 1) + 8 * (g4 >> 1);
     const bool whole = wide && m + 16 * MW <= end && col + 16 * NW / S <= cols;

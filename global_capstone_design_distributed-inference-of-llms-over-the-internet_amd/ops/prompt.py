@@ -1,10 +1,12 @@
 """Products of prompt-sized steps (csrc/gemm_prompt.hip) and when they run in place of the library's.
 
-``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel.
+``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel;
+``gemm_columns``: y = x w, a gradient's way back through a projection.
 The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
-on how its 256 x 256 tiles fill 256 CUs, 1.05 to 1.45.  So the choice is measured, as it is for the decode GEMMs, for
+on how its 256 x 256 tiles fill 256 CUs, 1.1 to 1.5.  So the choice is measured, as it is for the decode GEMMs, for
 the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning): shapes in the committed table
-(``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows) run here at the row-tile
+(``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows, weights that no cache holds,
+as a model's do not stay there from one step to the next) run here at the row-tile
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
 both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
 
@@ -13,6 +15,7 @@ tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at
 """
 from __future__ import annotations
 
+import itertools
 import json
 import os
 import threading
@@ -21,7 +24,8 @@ from typing import Dict, FrozenSet, Iterable, Optional, Tuple
 import torch
 
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "prompt_gemm_gfx950.json")
-EPILOGUES = (0, 1, 4)
+COLUMNS = 8  # in an epilogue's place: x w
+EPILOGUES = (0, 1, 4, COLUMNS)
 TILE, MAX_ROWS = 256, 8192
 Shape = Tuple[int, int, int]  # N, K, epilogue
 
@@ -64,29 +68,47 @@ def chosen(M: int, N: int, K: int, epilogue: int) -> bool:
     return TILE < M <= MAX_ROWS and shape_ok(M, N, K, epilogue) and -(-M // TILE) in table().get((N, K, epilogue), ())
 
 
-def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
-    """Is this product of rows [M, K] with weights [N, K] one that runs here?  Callers that differentiate it, and operands
-    the kernel does not read (other types, strides, alignments), keep the library's."""
-    if w is None or x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+def _reads(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Are these operands that the kernel reads (types, strides, alignments), in a call that is not differentiated?"""
+    if x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
-    if not (chosen(x.shape[0], w.shape[0], w.shape[1], epilogue) and x.shape[1] == w.shape[1] and x.is_cuda and
-            w.device == x.device and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0 and
+    if not (x.is_cuda and w.device == x.device and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0 and
             x.stride(0) >= x.shape[1] and x.shape[0] * x.stride(0) < 1 << 31):
         return False
     return x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not (
         torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
 
 
+def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
+    """Is this product of rows [M, K] with weights [N, K] one that runs here?  Callers that differentiate it, and operands
+    the kernel does not read, keep the library's."""
+    return w is not None and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and \
+        chosen(x.shape[0], w.shape[0], w.shape[1], epilogue) and _reads(x, w)
+
+
+def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0):
+    need = torch.ops.mpamd.gemm_prompt_ws(x.shape[0], N, x.shape[1])
+    ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+    torch.ops.mpamd.gemm_prompt(x, w, y, ws, epilogue, limit)
+    return y
+
+
 def gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, epilogue: int = 0, limit: float = 0.0):
     """epilogue 0: x w^T; 1: the gated forms over gate / up rows in blocks of 16 (``limit`` 0: silu); 4: max(., 0)^2."""
-    M, (N, K) = x.shape[0], w.shape
+    M, N = x.shape[0], w.shape[0]
     cols = N // 2 if epilogue == 1 else N
     y = out if out is not None and out.is_contiguous() and out.dtype == x.dtype and out.data_ptr() % 16 == 0 else \
         torch.empty(M, cols, dtype=x.dtype, device=x.device)
-    need = torch.ops.mpamd.gemm_prompt_ws(M, N, K)
-    ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
-    torch.ops.mpamd.gemm_prompt(x, w, y, ws, epilogue, limit)
+    _run(x, w, y, N, epilogue, limit)
     return y if out is None or y is out else out.copy_(y)
+
+
+def gemm_columns(x: torch.Tensor, w: torch.Tensor, always: bool = False) -> torch.Tensor:
+    """x w of rows [M, K] and weights [K, N]: on the kernel where the table says so (or ``always``), else the library's."""
+    if always or (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[0] and
+                  chosen(x.shape[0], w.shape[1], w.shape[0], COLUMNS) and _reads(x, w)):
+        return _run(x, w, torch.empty(x.shape[0], w.shape[1], dtype=x.dtype, device=x.device), w.shape[1], COLUMNS)
+    return torch.mm(x, w)
 
 
 # ------------------------------------------------------------------ the table
@@ -107,6 +129,15 @@ def shapes(cfg) -> Iterable[Shape]:
         out = {(cfg.q_dim + 2 * cfg.kv_dim, H, 0), (H, cfg.q_dim, 0)}
         if not cfg.is_moe:
             out |= {(2 * cfg.intermediate_size, H, 1), (H, cfg.intermediate_size, 0)}
+    return sorted(s for s in out if shape_ok(MAX_ROWS, *s) and s[0] * s[1] >= 1 << 22)
+
+
+def train_shapes(cfg) -> Iterable[Shape]:
+    """What fine-tuning adds: gate / up rows as they are, and every projection's way back."""
+    from . import train
+
+    H, F, Q, A = cfg.hidden_size, cfg.intermediate_size, cfg.q_dim, cfg.q_dim + 2 * cfg.kv_dim
+    out = {(2 * F, H, 0), (F, H, COLUMNS), (H, 2 * F, COLUMNS), (Q, H, COLUMNS), (H, A, COLUMNS)} if train.shape_ok(cfg) else set()
     return sorted(s for s in out if shape_ok(MAX_ROWS, *s) and s[0] * s[1] >= 1 << 22)
 
 
@@ -141,7 +172,11 @@ def sweep(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
 
     got = {}
     for N, K, epi in todo:
-        w = torch.empty(N, K, device=device).normal_(0, 0.02).to(torch.bfloat16)
+        # (as many weights as push each other out of the 256 MB of cache; what a step's rows are was just written)
+        many = max(1, min(8, -(-(600 << 20) // (2 * N * K))))
+        ws = [torch.empty(*((K, N) if epi == COLUMNS else (N, K)), device=device).normal_(0, 0.02).to(torch.bfloat16)
+              for _ in range(many)]
+        turn = itertools.cycle(ws)
         tiles = []
         for m in range(2, MAX_ROWS // TILE + 1):
             ratios = []
@@ -151,13 +186,18 @@ def sweep(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
                 y = torch.empty(M, N // 2 if epi == 1 else N, dtype=x.dtype, device=device)
 
                 def lib():
-                    torch.mm(x, w.t(), out=z)
+                    if epi == COLUMNS:
+                        return torch.mm(x, next(turn), out=z)
+                    torch.mm(x, next(turn).t(), out=z)
                     if epi == 1:
                         swiglu(z, out=y)
                     elif epi == 4:
                         hybrid.relu2(z, y)
 
-                t = [min(v) for v in zip(*[(ms(lib), ms(lambda: gemm(x, w, y, epi))) for _ in range(3)])]
+                def tile():
+                    _run(x, next(turn), y, N, epi)
+
+                t = [min(v) for v in zip(*[(ms(lib), ms(tile)) for _ in range(3)])]
                 ratios.append(t[0] / t[1])
             if min(ratios) >= 1.0 and sum(ratios) / 3 >= 1.03:
                 tiles.append(m)

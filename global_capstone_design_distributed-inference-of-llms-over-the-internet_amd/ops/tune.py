@@ -32,7 +32,7 @@ def tune_prompt(out=None) -> int:
     if not torch.cuda.is_available():
         print("tune: needs an MI355X", file=sys.stderr)
         return 2
-    todo = sorted({s for cfg in PRESETS.values() for s in prompt.shapes(cfg)})
+    todo = sorted({s for cfg in PRESETS.values() for f in (prompt.shapes, prompt.train_shapes) for s in f(cfg)})
     prompt.save(out or prompt.TABLE, prompt.tune(todo, log=lambda m: print(f"tune: {m}", file=sys.stderr, flush=True)))
     return 0
 

@@ -33,7 +33,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..models.weights import split_gate_up
-from ..ops import train
+from ..ops import prompt, train
 from ..ops.moe import moe_mlp_torch
 from ..ops.reference import rope_cos_sin
 
@@ -174,10 +174,10 @@ class AutogradStage:
         gp = None if prompts is None else torch.empty_like(prompts)
         for i in reversed(range(len(kept))):
             lay, (x, qkv, a32, lse, x2, gu) = self.w.layers[i], kept.pop()
-            dgu = train.glu_grad_(gu, torch.mm(g, lay.down))
-            g = train.norm_grad(x2, torch.mm(dgu, lay.gate_up), lay.post_norm, eps, g)
-            dqkv = train.attention_grad(qkv, B, nh, nkv, D, a32, lse, torch.mm(g, lay.o), table)
-            g = train.norm_grad(x, torch.mm(dqkv, lay.qkv), lay.input_norm, eps, g)
+            dgu = train.glu_grad_(gu, prompt.gemm_columns(g, lay.down))
+            g = train.norm_grad(x2, prompt.gemm_columns(dgu, lay.gate_up), lay.post_norm, eps, g)
+            dqkv = train.attention_grad(qkv, B, nh, nkv, D, a32, lse, prompt.gemm_columns(g, lay.o), table)
+            g = train.norm_grad(x, prompt.gemm_columns(dqkv, lay.qkv), lay.input_norm, eps, g)
             if gp is not None:
                 d = g.view(B, T, -1)[:, :gp.shape[2]]
                 gp[i] = d.sum(0, keepdim=True) if gp.shape[1] == 1 else d

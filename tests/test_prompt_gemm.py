@@ -58,6 +58,20 @@ def test_left_over_tiles_in_parts(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
+def test_products_with_columns(M, N, K):
+    """x w, as a gradient goes back through a projection: ends of tiles and of a wave's columns, tiles in parts."""
+    ops.require_native()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = torch.randn(K, N, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    want = x.double() @ w.double()
+    got = prompt.gemm_columns(x, w, always=True)
+    assert float((got.double() - want).norm() / want.norm()) < BF16
+    assert torch.equal(got, prompt.gemm_columns(x, w, always=True))
+
+
+@pytest.mark.gpu
 def test_not_a_number_and_infinity_pass():
     ops.require_native()
     x = torch.ones(260, 64, dtype=torch.bfloat16, device="cuda")
@@ -90,6 +104,18 @@ def test_table_and_rule(monkeypatch):
     assert not prompt.ok(x, w, 0)  # the CPU
     assert prompt.shapes(__import__("src.models.config", fromlist=["PRESETS"]).PRESETS["llama2-7b"]) == \
         [(4096, 4096, 0), (4096, 11008, 0), (12288, 4096, 0), (22016, 4096, 1)]
+
+
+def test_products_with_columns_elsewhere(monkeypatch):
+    """What the kernel does not read, and shapes outside the table, keep the library's product."""
+    monkeypatch.setitem(prompt._STATE, "table", {(64, 128, prompt.COLUMNS): frozenset({2})})
+    monkeypatch.setattr(prompt, "_run", lambda *a: pytest.fail("not on the CPU"))
+    x, w = torch.randn(300, 128), torch.randn(128, 64)
+    assert prompt.chosen(300, 64, 128, prompt.COLUMNS) and not prompt.chosen(300, 128, 64, prompt.COLUMNS)
+    for a, b in ((x, w), (x.bfloat16(), w.bfloat16()), (x.bfloat16(), w.t().contiguous().t().bfloat16())):
+        assert torch.equal(prompt.gemm_columns(a, b), a @ b)
+    with pytest.raises(RuntimeError):
+        prompt.gemm_columns(x, w[:64])
 
 
 def test_table_switched_off(monkeypatch):
