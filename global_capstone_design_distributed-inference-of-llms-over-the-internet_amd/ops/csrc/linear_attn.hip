@@ -198,7 +198,10 @@ static int launch_scan(const LinArgs& a, const int32_t* seg, int nseg, int n, hi
 }
 
 // ---------------------------------------------------------------------------------------
-// Prompts.  A segment's tokens are taken 32 at a time by one workgroup per (segment, head); wave w holds VT 16-column
+// Prompts.  A segment's tokens are taken 32 at a time by one workgroup per (segment, head) of NW waves: four, or eight where a
+// state has more than 128 columns (in four, a wave's 64 columns of 256 rows are 256 registers and the rest was spilled, 968
+// bytes a lane: 16 heads of 256 x 256 over 4300 tokens took 523 + 181 us in two passes, in eight 221 + 74).  Bound by the
+// chain of a block: gates, scores, products with the state, the heads' norm, a barrier between each.  Wave w holds VT 16-column
 // tiles of S for all of D in fp32 accumulators.  With G_t the log2 decays summed from the block's start and i_t the log2
 // input weights (retention: 0), every weight of a block is exp2 of a difference that is never positive:
 //
@@ -241,27 +244,27 @@ constexpr float L2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
 // LDS position of columns d .. d + 3 (d a multiple of 4) of a 32-column slice
 __device__ __forceinline__ int kpos(int d) { return (d & ~31) + 8 * ((d & 15) >> 2) + 4 * ((d >> 4) & 1); }
 
-template <int KIND, int DF, int VT, bool STATE>
+template <int KIND, int DF, int VT, int NW, bool STATE>
 struct ChunkLds {
-  static constexpr int QS = 32 * DF + 8, VS = 64 * VT + 8;
+  static constexpr int QS = 32 * DF + 8, VS = 16 * VT * NW + 8;
   static constexpr int NQK = (STATE ? 1 : 2) * (KIND == RETENTION ? 2 : 1);  // q, k as hi (+ lo)
   static constexpr int K = 0, KL = LC_TOK * QS, Q = (KIND == RETENTION ? 2 : 1) * LC_TOK * QS, QL = Q + LC_TOK * QS;
   static constexpr int VV = NQK * LC_TOK * QS, AH = VV + LC_TOK * VS, AL = AH + LC_TOK * LC_AS;
   static constexpr int FL = (STATE ? AH : AL + LC_TOK * LC_AS);  // floats from here (in bf16 elements, a multiple of 8)
-  static constexpr int NFL = 32 * 5 + 64 + 32 + 128 + 8 + (KIND == MLSTM ? 32 * DF : 0);
+  static constexpr int NFL = 32 * 5 + 64 + 32 + 32 * NW + 8 + (KIND == MLSTM ? 32 * DF : 0);
   static constexpr size_t BYTES = FL * 2 + NFL * 4;
 };
 
-template <int KIND, int DF, int VT, bool STATE>
-__global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) void linear_chunk_kernel(LinArgs a, const int32_t* __restrict__ seg,
+template <int KIND, int DF, int VT, int NW, bool STATE>
+__global__ __launch_bounds__(64 * NW, NW == 8 || DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) void linear_chunk_kernel(LinArgs a, const int32_t* __restrict__ seg,
                                                                                  int nseg, float* __restrict__ ws) {
-  typedef ChunkLds<KIND, DF, VT, STATE> L;
-  constexpr int NI = DF > 4 ? DF / 4 : 1;  // pair items of a thread
+  typedef ChunkLds<KIND, DF, VT, NW, STATE> L;
+  constexpr int NT = 64 * NW, NI = DF > NW ? DF / NW : 1;  // pair items of a thread
   constexpr int DT = 2 * DF;
   extern __shared__ __attribute__((aligned(16))) bf16_t lc[];
   float* fl = reinterpret_cast<float*>(lc + L::FL);
   float *xs = fl, *ys = fl + 32, *inter = fl + 64, *upd = fl + 96, *flo = fl + 128, *asum = fl + 160, *qnv = fl + 224,
-        *rss = fl + 256, *scal = fl + 384, *nrm = fl + 392;
+        *rss = fl + 256, *scal = rss + 32 * NW, *nrm = scal + 8;
 
   const int h = blockIdx.x, sg = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -276,7 +279,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
   const bf16_t* zb = (const bf16_t*)a.z + (int64_t)tok0 * a.zs;
   const float ld = KIND == RETENTION ? a.decay[h] : 0.f, qks = a.qs * a.ks;
 
-  for (int x = tid; x < L::FL / 8; x += 256) *reinterpret_cast<u16x8*>(lc + 8 * x) = (u16x8)(0);  // pads stay 0
+  for (int x = tid; x < L::FL / 8; x += NT) *reinterpret_cast<u16x8*>(lc + 8 * x) = (u16x8)(0);  // pads stay 0
   f32x4 S[DT][VT];
   {
     const float* sp = src < 0 ? a.state + row * blk : ws + ((int64_t)src * H + h) * wst;
@@ -295,7 +298,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
   if constexpr (KIND == MLSTM) {
     const float* np = src < 0 ? a.aux + row * (D + 1) : ws + ((int64_t)src * H + h) * wst + blk;
     if (!STATE && !fresh) m_in = src < 0 ? np[D] * L2E : np[D + 2];
-    for (int d = tid; d < 32 * DF; d += 256)
+    for (int d = tid; d < 32 * DF; d += NT)
       nrm[kpos(d & ~3) + (d & 3)] = !STATE && !fresh && d < D ? np[d] : 0.f;
   }
 
@@ -303,7 +306,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
   int it_row[NI], it_c0[NI], it_c1[NI], it_cs[NI];
 #pragma unroll
   for (int n = 0; n < NI; ++n) {
-    const int x = tid + 256 * n, per = D >> 4, r = x / per, it = x - r * per;
+    const int x = tid + NT * n, per = D >> 4, r = x / per, it = x - r * per;
     it_row[n] = r < LC_TOK ? r : -1;
     const int nr = KIND == RETENTION ? a.rot >> 4 : 0;
     it_cs[n] = it < nr ? 8 * it : -1;
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
     }
 #pragma unroll
     for (int n = 0; n < VT; ++n) {
-      const int x = tid + 256 * n, r = x / vper;
+      const int x = tid + NT * n, r = x / vper;
       rv[n] = *reinterpret_cast<const u16x8*>(zb + (int64_t)(b + min(r, last)) * a.zs + 2 * H * D + h * V +
                                               (x - r * vper) * 8);
     }
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
     }
 #pragma unroll
     for (int n = 0; n < VT; ++n) {
-      const int x = tid + 256 * n, r = x / vper;
+      const int x = tid + NT * n, r = x / vper;
       if (r < LC_TOK)
         *reinterpret_cast<u16x8*>(lc + L::VV + r * L::VS + (x - r * vper) * 8) = r < nb ? rv[n] : (u16x8)(0);
     }
@@ -441,47 +444,53 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
   for (int b = 0; b < ntok; b += LC_TOK) {
     const int nb = min(LC_TOK, ntok - b);
     stash(nb);
-    if (b + LC_TOK < ntok) fetch(b + LC_TOK);
+    // (where a wave's share of the state is 128 registers, the next block's rows would be spilled ahead of it)
+    constexpr bool LATE = !STATE && DF * VT >= 16;
+    if (!LATE && b + LC_TOK < ntok) fetch(b + LC_TOK);
     __syncthreads();
     const float dec = scal[0];
     f32x4 O[2][VT];
     if constexpr (!STATE) {
-      // scores of tile (query half w >> 1, key half w & 1); a lane owns query c16, keys 4 g4 ..
-      const int it = w >> 1, jt = w & 1;
-      f32x4 sc = (f32x4)(0.f);
-      if (jt <= it) {
+      if (w < 4) {
+        // scores of tile (query half w >> 1, key half w & 1); a lane owns query c16, keys 4 g4 ..
+        const int it = w >> 1, jt = w & 1;
+        f32x4 sc = (f32x4)(0.f);
+        if (jt <= it) {
 #pragma unroll
-        for (int f = 0; f < DF; ++f) {
-          const u16x8 kh = *reinterpret_cast<const u16x8*>(kf + 16 * jt * L::QS + 32 * f);
-          const u16x8 qh = *reinterpret_cast<const u16x8*>(qf + 16 * it * L::QS + 32 * f);
-          sc = mfma_c(kh, qh, sc);
-          if constexpr (KIND == RETENTION) {
-            const u16x8 kl = *reinterpret_cast<const u16x8*>(kf + LO + 16 * jt * L::QS + 32 * f);
-            const u16x8 ql = *reinterpret_cast<const u16x8*>(qf + LO + 16 * it * L::QS + 32 * f);
-            sc = mfma_c(kh, ql, sc);
-            sc = mfma_c(kl, qh, sc);
+          for (int f = 0; f < DF; ++f) {
+            const u16x8 kh = *reinterpret_cast<const u16x8*>(kf + 16 * jt * L::QS + 32 * f);
+            const u16x8 qh = *reinterpret_cast<const u16x8*>(qf + 16 * it * L::QS + 32 * f);
+            sc = mfma_c(kh, qh, sc);
+            if constexpr (KIND == RETENTION) {
+              const u16x8 kl = *reinterpret_cast<const u16x8*>(kf + LO + 16 * jt * L::QS + 32 * f);
+              const u16x8 ql = *reinterpret_cast<const u16x8*>(qf + LO + 16 * it * L::QS + 32 * f);
+              sc = mfma_c(kh, ql, sc);
+              sc = mfma_c(kl, qh, sc);
+            }
           }
         }
-      }
-      const int i = 16 * it + c16;
-      const float xi = xs[i];
-      u16x4 ah, al;
-      float sum = 0.f;
+        const int i = 16 * it + c16;
+        const float xi = xs[i];
+        u16x4 ah, al;
+        float sum = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = 16 * jt + 4 * g4 + r;
-        const float x = j <= i ? sc[r] * __builtin_amdgcn_exp2f(ys[j] - xi) * qks : 0.f;
-        ah[r] = f2bf(x);
-        al[r] = f2bf(x - bf2f(ah[r]));
-        sum += x;
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * jt + 4 * g4 + r;
+          const float x = j <= i ? sc[r] * __builtin_amdgcn_exp2f(ys[j] - xi) * qks : 0.f;
+          ah[r] = f2bf(x);
+          al[r] = f2bf(x - bf2f(ah[r]));
+          sum += x;
+        }
+        *reinterpret_cast<u16x4*>(lc + L::AH + i * LC_AS + 8 * g4 + 4 * jt) = ah;
+        *reinterpret_cast<u16x4*>(lc + L::AL + i * LC_AS + 8 * g4 + 4 * jt) = al;
+        if constexpr (KIND == MLSTM) {
+          sum += __shfl_xor(sum, 16, 64);
+          sum += __shfl_xor(sum, 32, 64);
+          if (g4 == 0) asum[32 * jt + i] = sum;
+        }
       }
-      *reinterpret_cast<u16x4*>(lc + L::AH + i * LC_AS + 8 * g4 + 4 * jt) = ah;
-      *reinterpret_cast<u16x4*>(lc + L::AL + i * LC_AS + 8 * g4 + 4 * jt) = al;
-      if constexpr (KIND == MLSTM) {
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        if (g4 == 0) asum[32 * jt + i] = sum;
-        const int t = tid >> 3, p0 = (tid & 7) * 4 * DF;  // n . q of token t, an eighth of the columns each
+      if (KIND == MLSTM && w >= NW - 4) {
+        const int t = (tid - (NT - 256)) >> 3, p0 = (tid & 7) * 4 * DF;  // n . q of token t, an eighth of the columns each
         float s = 0.f;
 #pragma unroll
         for (int p = 0; p < 4 * DF; p += 4) {
@@ -552,6 +561,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
           if constexpr (KIND == RETENTION) s = mfma_c(kl, wh[v], s);
         }
       }
+      if (LATE) __builtin_amdgcn_sched_barrier(0);  // (operands of all steps at once would be spilled)
     }
     if constexpr (!STATE) {
 #pragma unroll
@@ -559,6 +569,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
 #pragma unroll
         for (int v = 0; v < VT; ++v) O[i2][v] *= inter[16 * i2 + c16];
     }
+    if (LATE && b + LC_TOK < ntok) fetch(b + LC_TOK);
     u16x4 gz[2][VT];
     if constexpr (!STATE) {
 #pragma unroll
@@ -570,7 +581,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
     }
     __syncthreads();
     if constexpr (KIND == MLSTM) {
-      for (int p = tid; p < 32 * DF; p += 256) {
+      for (int p = tid; p < 32 * DF; p += NT) {
         float n = nrm[p] * dec;
 #pragma unroll 8
         for (int j = 0; j < LC_TOK; ++j) n += upd[j] * bf2f(lc[L::K + j * L::QS + p]);
@@ -588,6 +599,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
           den = 1.f / (fmaxf(fabsf(qnv[i] * inter[i] + asum[i] + asum[32 + i]), flo[i]) + 1e-6f);
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
+          if (LATE) vf[v] = lds_tr8(vt + 16 * v, 16 * L::VS);  // (not kept across the state's products)
           O[i2][v] = mfma_c(vf[v], ah, O[i2][v]);
           O[i2][v] = mfma_c(vf[v], al, O[i2][v]);
           O[i2][v] *= den;
@@ -605,7 +617,10 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
 #pragma unroll
       for (int i2 = 0; i2 < 2; ++i2) {
         const int i = 16 * i2 + c16;
-        const float sc = 1.f / sqrtf((rss[i] + rss[32 + i] + rss[64 + i] + rss[96 + i]) * inv_v + a.eps);
+        float sq = 0.f;
+#pragma unroll
+        for (int u = 0; u < NW; ++u) sq += rss[32 * u + i];
+        const float sc = 1.f / sqrtf(sq * inv_v + a.eps);
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
           const int col = (w * VT + v) * 16 + 4 * g4;
@@ -637,7 +652,7 @@ __global__ __launch_bounds__(256, DF * VT <= 4 || (DF == 4 && VT == 2) ? 2 : 1) 
       }
   if constexpr (KIND == MLSTM) {
     float* np = dst < 0 ? a.aux + row * (D + 1) : sp + blk;
-    for (int d = tid; d < D; d += 256) np[d] = nrm[kpos(d & ~3) + (d & 3)];
+    for (int d = tid; d < D; d += NT) np[d] = nrm[kpos(d & ~3) + (d & 3)];
     if (tid == 0) {
       np[D] = dst < 0 ? m_in * LN2 : m_in;
       if (dst >= 0) np[D + 1] = gsum;
@@ -691,19 +706,19 @@ __global__ __launch_bounds__(256) void linear_prefix_kernel(LinArgs a, const int
 
 template <int KIND, bool STATE>
 static int launch_linear_chunk(const LinArgs& a, const int32_t* seg, int nseg, float* ws, hipStream_t stream) {
-#define MP_LC(DF_, VT_)                                                                                              \
-  {                                                                                                                  \
-    constexpr size_t lds = ChunkLds<KIND, DF_, VT_, STATE>::BYTES;                                                   \
-    if (lds > 65536)                                                                                                 \
-      (void)hipFuncSetAttribute((const void*)linear_chunk_kernel<KIND, DF_, VT_, STATE>,                             \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                               \
-    hipLaunchKernelGGL((linear_chunk_kernel<KIND, DF_, VT_, STATE>), dim3(a.H, nseg), dim3(256), lds, stream, a, seg, \
-                       nseg, ws);                                                                                    \
+#define MP_LC(DF_, VT_, NW_)                                                                                            \
+  {                                                                                                                     \
+    constexpr size_t lds = ChunkLds<KIND, DF_, VT_, NW_, STATE>::BYTES;                                                 \
+    if (lds > 65536)                                                                                                    \
+      (void)hipFuncSetAttribute((const void*)linear_chunk_kernel<KIND, DF_, VT_, NW_, STATE>,                           \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                                  \
+    hipLaunchKernelGGL((linear_chunk_kernel<KIND, DF_, VT_, NW_, STATE>), dim3(a.H, nseg), dim3(64 * NW_), lds, stream, \
+                       a, seg, nseg, ws);                                                                               \
   }
-#define MP_LCV(DF_)                 \
-  if (a.V <= 64) MP_LC(DF_, 1)      \
-  else if (a.V <= 128) MP_LC(DF_, 2) \
-  else MP_LC(DF_, 4)
+#define MP_LCV(DF_)                     \
+  if (a.V <= 64) MP_LC(DF_, 1, 4)       \
+  else if (a.V <= 128) MP_LC(DF_, 2, 4) \
+  else MP_LC(DF_, 2, 8)
   if (a.D <= 64) { MP_LCV(2) } else if (a.D <= 128) { MP_LCV(4) } else { MP_LCV(8) }
 #undef MP_LCV
 #undef MP_LC

@@ -93,20 +93,46 @@ def hgrn2(z, bias, lower, norm, state, q_seq, q_ctx, out, eps, plan=None, packed
 CHUNK_MAX = 256
 
 
-def hgrn2_plan(ntoks, heads: int, n_cu: int = 256, seg_tokens: int = None):
+# tokens that a segment's start (its state arrives) and a segment's slot (read and written between the two passes) cost, and
+# what the pass over the segments' own contributions adds to a step that has any
+SEG_START, SEG_SLOT, SEG_CUT = 32, 3, 0.35
+
+
+def segment_tokens(n, room: int) -> int:
+    """Tokens of a segment, whole 16-token blocks, for sequences of ``n`` tokens and ``room`` segments that run at once
+    (all heads of each): the length whose rounds are shortest.  Segments that overflow ``room`` by a few cost a whole round:
+    1801, 750, 1400 and 349 tokens where 16 run at once: in 18 segments hgrn2_chunk took 285 us, in 16 179; in 35 segments
+    linear_chunk of 256 columns 221 us and its prefix 64, in 16 172 and 38."""
+    n = np.asarray(n, dtype=np.int64)
+    T = [128]
+    while T[-1] < n.max():
+        T.append(16 * -(-int(T[-1] * 1.09) // 16))
+    T = np.asarray(T)
+    k = -(-n[None] // T[:, None])
+    per = 16 * -(-n[None] // (16 * k))
+    segs = k.sum(1)
+    rounds = -(-segs // max(1, room))
+    est = np.maximum(per.max(1), rounds * (n.sum() / segs)) + rounds * SEG_START
+    cut = (k > 1).any(1)
+    return int(T[np.argmin(est * (1 + SEG_CUT * cut) + SEG_SLOT * np.where(k > 1, k, 0).sum(1))])
+
+
+def hgrn2_plan(ntoks, heads: int, n_cu: int = 256, seg_tokens: int = None, per_cu: int = 2):
     """Segments of a ragged step for the chunk form: int32 ``seqs`` [2, n] (first flat token, tokens of every
     sequence that brings any), ``seg`` [4, nseg], ``multi`` [4, nm] and the number of workspace slots
-    (csrc/hgrn2.hip).  Sequences are cut so that about two workgroups per CU exist, at whole 16-token blocks."""
+    (csrc/hgrn2.hip).  Sequences are cut at whole 16-token blocks, so that the step's rounds of ``per_cu`` workgroups a CU are
+    short (``segment_tokens``), or into segments of about ``seg_tokens``."""
     n = np.asarray(ntoks, dtype=np.int64)
     off = np.concatenate([[0], np.cumsum(n)[:-1]])
     keep = n > 0
     off, n = off[keep], n[keep]
     if seg_tokens is None:
-        want = max(1, -(-2 * n_cu // max(heads, 1)))  # segments over the whole step
-        seg_tokens = max(128, 16 * (-(-int(n.sum()) // want) // 16))
+        seg_tokens = whole = segment_tokens(n, per_cu * n_cu // max(heads, 1)) if len(n) else 128
+    else:
+        whole = seg_tokens * 3 // 2  # (tokens up to which a sequence is not cut)
     seg, multi, slots = [], [], 0
     for o, c in zip(off.tolist(), n.tolist()):
-        k = max(1, -(-c // seg_tokens)) if c > seg_tokens * 3 // 2 else 1
+        k = max(1, -(-c // seg_tokens)) if c > whole else 1
         per = 16 * -(-c // (16 * k))
         k = -(-c // per)
         if k == 1:

@@ -128,11 +128,11 @@ def softcap(x, cap):
 
 
 # ------------------------------------------------------------------ scalar-decay linear attention
-def linear_plan(ntoks, heads: int, n_cu: int = 256, seg_tokens: int = None):
+def linear_plan(ntoks, heads: int, n_cu: int = 256, seg_tokens: int = None, per_cu: int = 2):
     """Segments of a ragged step, shared with the gated recurrence (``hybrid.hgrn2_plan``)."""
     from .hybrid import hgrn2_plan
 
-    return hgrn2_plan(ntoks, heads, n_cu, seg_tokens)
+    return hgrn2_plan(ntoks, heads, n_cu, seg_tokens, per_cu)
 
 
 def retention(z, rope, log_decay, state, q_seq, q_ctx, out, eps, plan=None, packed=False):

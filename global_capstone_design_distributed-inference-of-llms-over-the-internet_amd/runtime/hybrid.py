@@ -92,8 +92,11 @@ class HybridStage:
         self.windows = sorted({(self._window_key(sp), sp.reach) for sp in specs if sp.mixer == "window_attention"})
         self.side = torch.cuda.Stream(ex.device) if ex.device.type == "cuda" and PARALLEL_EXPERTS and \
             any(sp.parallel and sp.moe for sp in specs) else None
-        self.rec_heads = min([sp.heads for sp in specs if sp.mixer == "hgrn2"], default=0)
-        self.lin_heads = min([sp.heads for sp in specs if sp.mixer in ("retention", "mlstm")], default=0)
+        # heads of the layer whose prompts fill the CUs with the fewest segments, and workgroups of it that share a CU (one,
+        # where a state is past 128 x 128)
+        most = lambda *kinds: max([(sp.heads, 1 if max(sp.dim, sp.vdim) > 128 else 2) for sp in specs if sp.mixer in kinds],  # noqa: E731
+                                  key=lambda x: x[0] / x[1], default=None)
+        self.rec_fill, self.lin_fill = most("hgrn2"), most("retention", "mlstm")
         self.gated = any(sp.mixer in ("gated_delta", "mamba2", "gla") for sp in specs)
         self.gated_waves = min([sp.heads * -(-sp.vdim // 16) for sp in specs if sp.mixer in ("mamba2", "gla")], default=0)
         self.max_chunk = max([sp.reach for sp in specs if sp.reach], default=1)
@@ -485,12 +488,12 @@ class HybridStage:
             return {}
         up = lambda a: torch.from_numpy(a).to(self.ex.device, non_blocking=True)  # noqa: E731
         p = {"blocks": {tb: up(hops.talk_blocks(ntoks, tb)) for tb in set(self.talk_block.values()) if tb}}
-        if self.rec_heads:
-            h = hops.hgrn2_plan(ntoks, self.rec_heads, self.ex._n_cu)
+        if self.rec_fill:
+            h = hops.hgrn2_plan(ntoks, self.rec_fill[0], self.ex._n_cu, per_cu=self.rec_fill[1])
             p.update(seqs=up(h["seqs"]), seg=up(h["seg"]), multi=up(h["multi"]) if h["slots"] else None,
                      slots=h["slots"])
-        if self.lin_heads:
-            h = mops.linear_plan(ntoks, self.lin_heads, self.ex._n_cu)
+        if self.lin_fill:
+            h = mops.linear_plan(ntoks, self.lin_fill[0], self.ex._n_cu, per_cu=self.lin_fill[1])
             p["linear"] = {"seqs": up(h["seqs"]), "seg": up(h["seg"]), "slots": h["slots"],
                            "multi": up(h["multi"]) if h["slots"] else None}
         p["window"] = {}

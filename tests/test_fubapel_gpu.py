@@ -185,6 +185,16 @@ def test_linear_attention_prompts(kind, dt, H, D, V, rot, form):
 
 
 @pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("H,D,V,rot", [(2, 48, 136, 16), (1, 128, 144, 64), (1, 160, 248, 0), (2, 256, 136, 256)])
+def test_linear_attention_prompts_of_wide_states(kind, H, D, V, rot):
+    """Eight waves from 129 columns on: columns that end inside a wave's, whole and in segments."""
+    ntoks, starts = [33, 1, 150, 64], [0, 5, 9, 64]
+    for seg in (None, 32):
+        c = lin_case(kind, ntoks, H, D, V, "bf16", starts, rot)
+        check_lin(c, "bf16", run_lin(c, "bf16", lin_plan(ntoks, H, seg)))
+
+
+@pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("dt", sorted(DTYPES))
 @pytest.mark.parametrize("H,D,V,rot", LIN_SHAPES + [(1, 300, 64, 300)])
 def test_linear_attention_decode(kind, dt, H, D, V, rot):

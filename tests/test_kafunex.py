@@ -229,6 +229,23 @@ def test_recurrent_plan_covers_every_token():
                 assert all(c[1] % 16 == 0 for c in chain[:-1])
 
 
+def test_recurrent_plan_fits_its_rounds():
+    """Without a length given: every token once, whole blocks, and never more rounds than the same step in segments of twice
+    the length would take."""
+    for ntoks in ([1], [5, 0, 1000, 1, 17], [128] * 9, [4000], [1801, 750, 1400, 349], [0, 0], [8192], [40] * 100):
+        for heads, per_cu in ((1, 2), (16, 1), (32, 2), (600, 1)):
+            p = hops.hgrn2_plan(ntoks, heads, per_cu=per_cu)
+            seg = p["seg"].T.tolist()
+            assert sorted(t for o, n, _, _ in seg for t in range(o, o + n)) == list(range(sum(ntoks)))
+            if not seg:
+                continue
+            T = max(n for _, n, _, _ in seg)
+            room = max(1, per_cu * 256 // heads)
+            twice = sum(-(-n // (2 * T)) for n in ntoks)
+            assert all(n % 16 == 0 for _, n, _, d in seg if d >= 0)
+            assert -(-len(seg) // room) * T <= -(-twice // room) * 2 * T + 200 * -(-len(seg) // room)
+
+
 # ------------------------------------------------------------------ executor
 def test_whole_prompts(model):
     cfg, w, d = model
