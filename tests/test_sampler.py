@@ -1,4 +1,5 @@
 """Sampler semantics (reference src/rpc_handler.py:327-403) on the CPU path."""
+import pytest
 import torch
 
 from src import ops
@@ -36,3 +37,50 @@ def test_batch_sampler_cpu():
     assert torch.equal(out, torch.argmax(lg, -1))
     out = s(lg, [SamplingParams(1.0, 0.9, 5, 1.5)] * 3, [[1], [2, 2], []], [session_seed("a", 1)] * 3)
     assert out.shape == (3,) and int(out.max()) < 50
+
+
+def _batch(n, V, seed):
+    g = torch.Generator().manual_seed(seed)
+    hist = [torch.randint(0, V, (k % 70,), generator=g).tolist() for k in range(n)]
+    par = [SamplingParams(0.5 + 0.1 * (k % 9), 0.8 + 0.01 * (k % 20), (0, 50, 7)[k % 3], 1.0 + 0.1 * (k % 5)) for k in range(n)]
+    return (3 * torch.randn(n, V, generator=g)).bfloat16(), par, hist, torch.randint(0, 1 << 62, (n,), generator=g).tolist()
+
+
+def _one_by_one(lg, par, hist, seeds):
+    """What a row gets when its parameters come as tensors of their own."""
+    from src import ops
+
+    rec = torch.zeros(len(par), 50, dtype=torch.int32)
+    for r, h in enumerate(hist):
+        h = h[-50:]
+        rec[r, :len(h)] = torch.tensor(h, dtype=torch.int32)
+    t = lambda v, dt: torch.tensor(v, dtype=dt, device=lg.device)  # noqa: E731
+    return ops.sample(lg, t([p.temperature for p in par], torch.float32), t([p.top_p for p in par], torch.float32),
+                      t([p.top_k for p in par], torch.int32), t([p.repetition_penalty for p in par], torch.float32),
+                      rec.to(lg.device), t([min(len(h), 50) for h in hist], torch.int32), t(seeds, torch.int64))
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_batch_sampler_calls_in_flight(dev):
+    """Calls that are not waited for keep their own rows' parameters, histories and seeds, of any number of rows."""
+    s = BatchSampler(dev, max_rows=24)
+    steps = [_batch(n, 700, k) for k, n in enumerate((24, 1, 7, 24, 60, 3, 24, 2))]
+    lgs = [lg.to(dev) for lg, *_ in steps]
+    got = [s(lg, *rest) for lg, (_, *rest) in zip(lgs, steps)]
+    for lg, g, (_, *rest) in zip(lgs, got, steps):
+        assert torch.equal(g.cpu(), torch.cat([_one_by_one(lg[i:i + 24], *[r[i:i + 24] for r in rest])
+                                               for i in range(0, len(g), 24)]).cpu())
+
+
+@pytest.mark.gpu
+def test_batch_sampler_on_several_streams():
+    s, (lg, *rest) = BatchSampler("cuda"), _batch(64, 32000, 1)
+    lg = lg.cuda()
+    want = s(lg, *rest)
+    torch.cuda.synchronize()
+    got = []
+    for st in [torch.cuda.Stream() for _ in range(3)] * 2:
+        with torch.cuda.stream(st):
+            got.append(s(lg, *rest))
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, want) for g in got)
