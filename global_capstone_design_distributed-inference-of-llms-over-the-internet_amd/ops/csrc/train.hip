@@ -58,13 +58,21 @@ struct Tile {
   static_assert(ROWS * CH % 256 == 0, "whole chunks per thread");
   u16x8 v[N];
   __device__ __forceinline__ void fetch(const bf16_t* p, int64_t ld, int r0, int T) {
+    const char* base = reinterpret_cast<const char*>(p + (int64_t)r0 * ld);
+    const int last = min(ROWS, T - r0) - 1;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const int c = threadIdx.x + 256 * j, r = r0 + c / CH;
-      v[j] = r < T ? *reinterpret_cast<const u16x8*>(p + (int64_t)r * ld + (c % CH) * 8) : (u16x8)(0);
+      const int c = threadIdx.x + 256 * j;
+      v[j] = *reinterpret_cast<const u16x8*>(base + (uint32_t)min(c / CH, last) * (uint32_t)(ld * 2) + (c % CH) * 16);
     }
   }
-  __device__ __forceinline__ void stash(unsigned char* lds) const {
+  // ``rows`` of them are the matrix's, the others zeros
+  __device__ __forceinline__ void stash(unsigned char* lds, int rows) {
+    if (rows < ROWS) {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if ((int)(threadIdx.x + 256 * j) / CH >= rows) v[j] = (u16x8)(0);
+    }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const int c = threadIdx.x + 256 * j;
@@ -102,14 +110,15 @@ __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u16x8 (&t
 }
 
 // Forward and dQ: a workgroup has 64 queries of one head, 16 a wave, and walks the keys 64 at a time.
-// 2 x 777 tokens, 32 heads of 128 (8 kv heads): forward 59 us, dQ 74 us.  Bound by the chain of a tile's steps and by LDS
-// reads (24 KiB a wave and tile), not by MFMA, which is 10 and 12 us of it.  The fp32 batched products, softmax passes and
-// copies that it replaced were most of 12.3 ms for two blocks' forward and backward requests, 5.1 ms with these kernels.
+// Bound by the chain of a tile's steps, so three workgroups share a CU: one LDS buffer, the next tile's rows in registers
+// (two buffers of 70 KB let two workgroups in).  2 x 777 tokens, 32 heads of 128 (8 kv heads): forward 59 -> 46 us, dQ, dK and dV
+// together 179 -> 144.  The fp32 batched products, softmax passes and copies that it replaced were most of 12.3 ms for two
+// blocks' forward and backward requests.
 template <int D, bool GRAD>
-__global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
+__global__ __launch_bounds__(256, 3) void train_attn_q_kernel(TrainAttn a) {
   constexpr int KS = D / 32, DT = D / 16;
   typedef Tile<D, 64> KTile;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][KTile::BYTES];  // [buffer][K | V]
+  __shared__ __attribute__((aligned(16))) unsigned char smem[2][KTile::BYTES];  // [K | V]
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4;
   const int h = blockIdx.y, b = blockIdx.z, kvh = h / (a.nh / a.nkv);
   const int q0 = (gridDim.x - 1 - blockIdx.x) * 64;  // longest context first
@@ -148,12 +157,11 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
   KTile kt, vt;
   const int end = min(q0 + 64, a.T);
   kt.fetch(kp, a.ld, 0, a.T), vt.fetch(vp, a.ld, 0, a.T);
-  kt.stash(smem[0][0]), vt.stash(smem[0][1]);
-  __syncthreads();
-  for (int k0 = 0, cur = 0; k0 < end; k0 += 64, cur ^= 1) {
-    const bool more = k0 + 64 < end;
-    if (more) kt.fetch(kp, a.ld, k0 + 64, a.T), vt.fetch(vp, a.ld, k0 + 64, a.T);
-    const unsigned char *K = smem[cur][0], *V = smem[cur][1];
+  for (int k0 = 0; k0 < end; k0 += 64) {
+    kt.stash(smem[0], a.T - k0), vt.stash(smem[1], a.T - k0);
+    __syncthreads();
+    if (k0 + 64 < end) kt.fetch(kp, a.ld, k0 + 64, a.T), vt.fetch(vp, a.ld, k0 + 64, a.T);
+    const unsigned char *K = smem[0], *V = smem[1];
     if (k0 <= q0 + 16 * w + 15) {
       f32x4 s[4], dp[4];
 #pragma unroll
@@ -190,9 +198,12 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
         top = fmaxf(top, __shfl_xor(top, 32, 64)) * c2;
         const float mn = fmaxf(m, top), mu = mn == -INFINITY ? 0.f : mn;
         const float alpha = __builtin_amdgcn_exp2f(m - mu);
-        m = mn, l *= alpha;
+        m = mn;
+        if (__any(alpha != 1.f)) {  // (most tiles leave every maximum where it was)
+          l *= alpha;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+          for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+        }
 #pragma unroll
         for (int st = 0; st < 4; ++st)
 #pragma unroll
@@ -214,7 +225,6 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
         }
       }
     }
-    if (more) kt.stash(smem[cur ^ 1][0]), vt.stash(smem[cur ^ 1][1]);
     __syncthreads();
   }
   if (!live) return;
@@ -255,9 +265,10 @@ __global__ __launch_bounds__(256) void train_attn_q_kernel(TrainAttn a) {
 // dK and dV: a workgroup has 64 keys of one query head, 16 a wave, and walks the queries from the diagonal on, 32 at a
 // time.  A query head's part goes out in fp32; the heads of a group are added by train_kv_close_kernel: a workgroup per
 // kv head would leave most CUs idle (13 x 8 blocks a sequence of 777 tokens) and atomics would make the sum's order,
-// and so its bits, change from run to run.  114 us for the tokens above, bound as the kernel above, and 11 us to close.
+// and so its bits, change from run to run.  Two workgroups to a CU: with the registers of three it spills (142 us where two
+// take 81, both gradients of 700 tokens).
 template <int D>
-__global__ __launch_bounds__(256) void train_attn_kv_kernel(TrainAttn a) {
+__global__ __launch_bounds__(256, 2) void train_attn_kv_kernel(TrainAttn a) {
   constexpr int KS = D / 32, DT = D / 16;
   typedef Tile<D, 32> QTile;
   __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][QTile::BYTES];  // [buffer][Q | dO]
@@ -291,12 +302,12 @@ __global__ __launch_bounds__(256) void train_attn_kv_kernel(TrainAttn a) {
       st_ = threadIdx.x < 32 ? (r < a.T ? lp[r] : INFINITY) : (r < a.T ? dp_[r] : 0.f);
     }
   };
-  auto stash = [&](int buf) {
-    qt.stash(smem[buf][0]), gt.stash(smem[buf][1]);
+  auto stash = [&](int buf, int r0) {
+    qt.stash(smem[buf][0], a.T - r0), gt.stash(smem[buf][1], a.T - r0);
     if (threadIdx.x < 64) stats[buf][threadIdx.x >> 5][threadIdx.x & 31] = st_;
   };
   fetch(k0);
-  stash(0);
+  stash(0, k0);
   __syncthreads();
   for (int r0 = k0, cur = 0; r0 < a.T; r0 += 32, cur ^= 1) {
     const bool more = r0 + 32 < a.T;
@@ -334,7 +345,7 @@ __global__ __launch_bounds__(256) void train_attn_kv_kernel(TrainAttn a) {
         }
       }
     }
-    if (more) stash(cur ^ 1);
+    if (more) stash(cur ^ 1, r0 + 32);
     __syncthreads();
   }
   if (key >= a.T) return;
