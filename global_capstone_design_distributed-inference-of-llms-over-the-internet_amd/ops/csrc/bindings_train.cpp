@@ -10,6 +10,7 @@ int mp_train_attn(const void* qkv, int64_t ld, int B, int T, int nh, int nkv, in
 int mp_train_attn_grad(const void* qkv, int64_t ld, int B, int T, int nh, int nkv, int D, float scale, const float* out32,
                        const float* lse, const void* dout, float* delta, const float* cs, float* part, void* dqkv,
                        hipStream_t stream);
+int mp_train_angles(const double* inv, float* out, int n, int64_t T, hipStream_t stream);
 int mp_train_rope(void* x, int64_t ld, const float* cs, int64_t rows, int T, int heads, int D, hipStream_t stream);
 int mp_train_norm(const void* x, const void* y, const void* w, void* sum, void* out, int64_t rows, int H, float eps, int grad,
                   hipStream_t stream);
@@ -69,6 +70,17 @@ void train_attn_grad(const at::Tensor& qkv, int64_t B, int64_t nh, int64_t nkv, 
                "train_attn_grad");
 }
 
+// out[T, 2 n]: cos, then sin of t inv[d]
+void train_angles(const at::Tensor& inv, at::Tensor& out) {
+  MP_CHECK(inv.is_cuda() && inv.scalar_type() == at::kDouble && inv.dim() == 1 && inv.is_contiguous() && inv.numel() >= 1, "inv");
+  MP_CHECK(out.is_cuda() && out.device() == inv.device() && out.scalar_type() == at::kFloat && out.dim() == 2 && out.is_contiguous() &&
+               out.size(0) >= 1 && out.size(1) == 2 * inv.numel() && out.numel() < (1ll << 38),
+           "out fp32 [T, 2 n]");
+  const c10::hip::HIPGuard guard(inv.device().index());
+  check_launch(mp_train_angles(inv.data_ptr<double>(), out.data_ptr<float>(), inv.numel(), out.size(0), cur_stream()),
+               "train_angles");
+}
+
 void train_rope(at::Tensor& x, const at::Tensor& cs, int64_t heads, int64_t D) {
   MP_CHECK(x.dim() == 2 && heads >= 1 && D >= 16 && D % 16 == 0 && heads * D <= x.size(1) && x.size(1) % 8 == 0, "rope shape");
   const int64_t T = cs.numel() / D;
@@ -112,6 +124,7 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def(
       "train_attn_grad(Tensor qkv, int B, int nh, int nkv, float scale, Tensor out32, Tensor lse, Tensor dout, Tensor(a!) "
       "delta, Tensor cs, Tensor(b!) part, Tensor(c!) dqkv) -> ()");
+  m.def("train_angles(Tensor inv, Tensor(a!) out) -> ()");
   m.def("train_rope(Tensor(a!) x, Tensor cs, int heads, int D) -> ()");
   m.def(
       "train_norm(Tensor x, Tensor? y, Tensor w, Tensor(a!)? sum, Tensor(b!) out, float eps, bool grad=False) -> ()");
@@ -121,6 +134,7 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
 TORCH_LIBRARY_IMPL(mpamd, CUDA, m) {
   m.impl("train_attn", &train_attn);
   m.impl("train_attn_grad", &train_attn_grad);
+  m.impl("train_angles", &train_angles);
   m.impl("train_rope", &train_rope);
   m.impl("train_norm", &train_norm);
   m.impl("train_glu_grad", &train_glu_grad);

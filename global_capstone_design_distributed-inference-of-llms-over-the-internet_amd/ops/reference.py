@@ -74,8 +74,8 @@ def rmsnorm(x, w, eps, out=None, residual=None, mode=0, rows=None, ss=None):
     return y
 
 
-def rope_cos_sin(head_dim: int, max_pos: int, theta: float, device=None, scaling: Optional[dict] = None):
-    """fp32 cos/sin tables [max_pos, head_dim/2] (HF LlamaRotaryEmbedding, incl. llama3 scaling)."""
+def rope_inv(head_dim: int, theta: float, scaling: Optional[dict] = None) -> torch.Tensor:
+    """fp64 [head_dim/2] angles of a step of one position (HF LlamaRotaryEmbedding, incl. llama3 scaling)."""
     inv = 1.0 / (theta ** (torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim))
     if scaling and scaling.get("rope_type", scaling.get("type")) == "llama3":
         factor = scaling.get("factor", 8.0)
@@ -88,8 +88,13 @@ def rope_cos_sin(head_dim: int, max_pos: int, theta: float, device=None, scaling
         mid = (1 - smooth) * scaled / factor + smooth * scaled
         is_mid = (wl <= lo_wl) & (wl >= hi_wl)
         inv = torch.where(is_mid, mid, scaled)
+    return inv
+
+
+def rope_cos_sin(head_dim: int, max_pos: int, theta: float, device=None, scaling: Optional[dict] = None):
+    """fp32 cos/sin tables [max_pos, head_dim/2] of ``rope_inv``'s angles."""
     t = torch.arange(max_pos, dtype=torch.float64)
-    f = torch.outer(t, inv)
+    f = torch.outer(t, rope_inv(head_dim, theta, scaling))
     return f.cos().float().to(device), f.sin().float().to(device)
 
 

@@ -29,6 +29,13 @@ def angle_table(cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
     return torch.cat([cos, sin], 1).contiguous()
 
 
+def angles(inv: torch.Tensor, T: int) -> torch.Tensor:
+    """``angle_table`` of T positions from the angles ``inv`` [D / 2] (fp64, on the device) of one step."""
+    out = torch.empty(T, 2 * inv.numel(), dtype=torch.float32, device=inv.device)
+    torch.ops.mpamd.train_angles(inv, out)
+    return out
+
+
 def norm(x, w, eps, add=None):
     """(x + add, its norm times w); without ``add`` the first is ``x`` itself."""
     out = torch.empty_like(x)

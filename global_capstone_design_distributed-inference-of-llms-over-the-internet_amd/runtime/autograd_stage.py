@@ -35,7 +35,7 @@ from .. import ops
 from ..models.weights import split_gate_up
 from ..ops import prompt, train
 from ..ops.moe import moe_mlp_torch
-from ..ops.reference import rope_cos_sin
+from ..ops.reference import rope_cos_sin, rope_inv
 
 
 def _rms(x, w, eps):
@@ -72,6 +72,7 @@ class AutogradStage:
         self.dtype = dtype or (weights.layers[0].input_norm.dtype if cfg.model_type != "gpt2"
                                else weights.layers[0].ln1_w.dtype)
         self._cache = {}  # per-layer (gate, up) views, made once
+        self._inv = None  # the kernel form's rotary angles of one position, on the device (made once)
 
     @property
     def n_blocks(self) -> int:
@@ -184,8 +185,9 @@ class AutogradStage:
         return g, gp
 
     def _angles(self, T: int):
-        cfg = self.cfg
-        return train.angle_table(*rope_cos_sin(cfg.head_dim, T, cfg.rope_theta, self.device, cfg.rope_scaling))
+        if self._inv is None:
+            self._inv = rope_inv(self.cfg.head_dim, self.cfg.rope_theta, self.cfg.rope_scaling).to(self.device)
+        return train.angles(self._inv, T)
 
     # ------------------------------------------------------------------ public API
     def forward(self, hidden: torch.Tensor, prompts: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -36,6 +36,21 @@ def _attend(q, k, v):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,D", [(1, 64), (2, 128), (777, 128), (100003, 64)])
+def test_angles(T, D):
+    """64-bit cosines and sines rounded once: the host's, but for values on the edge of a rounding."""
+    from src import ops
+    from src.ops import train
+    from src.ops.reference import rope_cos_sin, rope_inv
+
+    ops.require_native()
+    scaling = {"rope_type": "llama3", "factor": 8.0, "original_max_position_embeddings": 8192} if T == 2 else None
+    got = train.angles(rope_inv(D, 500000.0, scaling).cuda(), T).cpu()
+    want = train.angle_table(*rope_cos_sin(D, T, 500000.0, None, scaling))
+    assert float((got != want).float().mean()) < 1e-4 and float((got - want).abs().max()) <= 2.0 ** -24
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nh,nkv,D", [(4, 4, 128), (4, 1, 128), (6, 3, 64)])
 @pytest.mark.parametrize("T", EDGES)
 def test_attention_and_its_gradient(T, nh, nkv, D):
