@@ -865,6 +865,15 @@ def add(a, b, out=None):
     return out
 
 
+def step_input(host, meta, x, dst):
+    """A decode step's inputs in one launch: ``meta`` from pinned ``host`` bytes, ``dst`` from ``x`` (or None: it is there)."""
+    if x is not None and not (x.shape == dst.shape and x.dtype == dst.dtype and x.is_contiguous() and
+                              (x.data_ptr() | x.numel() * x.element_size()) % 8 == 0):
+        dst.copy_(x)  # another type, strided rows, an odd width
+        x = None
+    torch.ops.mpamd.step_input(host, meta, x, dst)
+
+
 def _aligned_rows(x):
     """``x`` [R, V] with the 16-byte row pitch the logits kernels read (a copy only for other pitches)."""
     if x.stride(0) % 8 == 0 and x.stride(1) == 1:

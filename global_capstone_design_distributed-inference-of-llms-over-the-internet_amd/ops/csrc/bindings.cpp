@@ -3,6 +3,7 @@
 // Every op writes into caller-provided outputs and launches on the current HIP
 // stream, so a whole stage step can be captured into one hipGraph.  Shape and
 // dtype checks happen here, on the host, before any kernel sees a pointer.
+#include <c10/hip/HIPGuard.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
 #include <torch/library.h>
@@ -27,6 +28,7 @@ int mp_paged_attention(const void* q, int64_t q_stride, const void* kc, const vo
 int mp_embedding(const int64_t* ids, const void* table, void* out, int T, int H, int64_t vocab, hipStream_t stream);
 int mp_swiglu(const void* gu, void* out, int64_t T, int F, hipStream_t stream);
 int mp_add(const void* a, const void* b, void* y, int64_t n, hipStream_t stream);
+int mp_step_input(const uint64_t* host, uint64_t* meta, int nb, const uint64_t* x, uint64_t* dst, int64_t nx, hipStream_t stream);
 int mp_argmax(const void* logits, int64_t stride, int R, int V, int64_t* out, int f32, hipStream_t stream);
 int mp_sample(const void* logits, int64_t stride, int R, int V, const float* temps, const float* top_ps,
               const int32_t* top_ks, const float* rep_pens, int32_t* recent, int recent_stride, int32_t* recent_len,
@@ -474,6 +476,25 @@ void add(const at::Tensor& a, const at::Tensor& b, at::Tensor& y) {
   check_launch(mp_add(a.data_ptr(), b.data_ptr(), y.data_ptr(), a.numel(), cur_stream()), "add");
 }
 
+// meta <- host (pinned bytes); the front of dst <- x, where there is one
+void step_input(const at::Tensor& host, at::Tensor& meta, const c10::optional<at::Tensor>& x, at::Tensor& dst) {
+  auto word = [](const at::Tensor& t) { return t.is_contiguous() && (t.nbytes() | reinterpret_cast<uintptr_t>(t.data_ptr())) % 8 == 0; };
+  MP_CHECK(host.device().is_cpu() && host.is_pinned() && word(host), "host: pinned, words of 8 bytes");
+  MP_CHECK(meta.is_cuda() && word(meta) && meta.nbytes() == host.nbytes() && meta.nbytes() < (1u << 30), "meta");
+  int64_t nx = 0;
+  if (x.has_value()) {
+    MP_CHECK(x->is_cuda() && dst.is_cuda() && x->device() == meta.device() && dst.device() == meta.device(), "one device");
+    MP_CHECK(x->scalar_type() == dst.scalar_type() && word(*x) && dst.is_contiguous() &&
+                 reinterpret_cast<uintptr_t>(dst.data_ptr()) % 8 == 0 && x->nbytes() <= dst.nbytes(),
+             "x, dst: one type, words of 8 bytes");
+    nx = x->nbytes() / 8;
+  }
+  const c10::hip::HIPGuard guard(meta.device().index());
+  check_launch(mp_step_input((const uint64_t*)host.data_ptr(), (uint64_t*)meta.data_ptr(), meta.nbytes() / 8,
+                             nx ? (const uint64_t*)x->data_ptr() : nullptr, (uint64_t*)dst.data_ptr(), nx, cur_stream()),
+               "step_input");
+}
+
 void argmax(const at::Tensor& logits, at::Tensor& out) {
   const bool f32 = logits.scalar_type() == at::kFloat;
   if (!f32) check_bf16_cuda(logits, "logits");
@@ -842,6 +863,7 @@ TORCH_LIBRARY(mpamd, m) {
   m.def("embedding(Tensor ids, Tensor table, Tensor(a!) out) -> ()");
   m.def("swiglu(Tensor gu, Tensor(a!) out) -> ()");
   m.def("add(Tensor a, Tensor b, Tensor(a!) y) -> ()");
+  m.def("step_input(Tensor host, Tensor(a!) meta, Tensor? x, Tensor(b!) dst) -> ()");
   m.def("argmax(Tensor logits, Tensor(a!) out) -> ()");
   m.def(
       "sample(Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks, Tensor rep_pens, Tensor(c!) recent, "
@@ -880,6 +902,7 @@ TORCH_LIBRARY_IMPL(mpamd, CUDA, m) {
   m.impl("embedding", &embedding);
   m.impl("swiglu", &swiglu);
   m.impl("add", &add);
+  m.impl("step_input", &step_input);
   m.impl("argmax", &argmax);
   m.impl("sample", &sample);
   m.impl("gemm", &gemm);

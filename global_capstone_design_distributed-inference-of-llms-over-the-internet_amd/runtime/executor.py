@@ -1192,7 +1192,8 @@ class StageExecutor:
                 read = pg
         g = self._graph(key)
         out = g.replay(plan, x)
-        g.mark_replayed()
+        if key[6] or read is not None:  # only receives wait for a replay's end
+            g.mark_replayed()
         if read is not None:  # the next receive into that buffer must wait for this replay's copy
             read.done_ev = g.done_ev
         return out
@@ -1302,9 +1303,12 @@ class _DecodeGraph:
     """A captured decode step for a fixed (batch bucket, attention partition).
 
     Its metadata lives in ONE device blob (positions, slots | q_seq, q_ctx, last_rows) that a
-    replay refills with a single host-to-device copy from a double-buffered pinned staging
-    blob, padded for the bucket (padding rows: slot -1, context 0): six small copies / fills per
-    step otherwise (profiles/r2_decode_step_*.txt)."""
+    replay refills from a ring of pinned staging blobs, padded for the bucket (padding rows: slot
+    -1, context 0): six small copies / fills per step otherwise (profiles/r2_decode_step_*.txt).
+    One launch does it together with the copy of the rows.  An event costs the stream 6 us, so
+    that the ring has one for each half of its turns, not one a turn."""
+
+    TURNS = 16
 
     def __init__(self, ex: StageExecutor, B: int, part: Tuple[int, int], pool, hook=None):
         self.ex, self.B, self.part = ex, B, part
@@ -1313,22 +1317,22 @@ class _DecodeGraph:
             self.x = torch.zeros(B, dtype=torch.long, device=dev)
         else:
             self.x = torch.zeros(B, H, dtype=ex.hidden_dtype, device=dev)
-        nbytes = 16 * B + 12 * B  # int64 [2, B] + int32 [3 B]
+        nbytes = -(-28 * B // 8) * 8  # int64 [2, B] + int32 [3 B], in whole words of 8 bytes
         self.blob = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
         self.meta64 = self.blob[: 16 * B].view(torch.int64).view(2, B)
-        self.meta32 = self.blob[16 * B:].view(torch.int32)
-        self._stage = [torch.zeros(nbytes, dtype=torch.uint8, pin_memory=True) for _ in range(2)]
-        self._stage_ev = [None, None]
+        self.meta32 = self.blob[16 * B:28 * B].view(torch.int32)
+        self._stage = torch.zeros(self.TURNS, nbytes, dtype=torch.uint8, pin_memory=True)
+        self._half_ev = [None, None]
         self._k = 0
         host = self._stage[0].numpy()
         h64 = host[: 16 * B].view(np.int64).reshape(2, B)
-        h32 = host[16 * B:].view(np.int32)
+        h32 = host[16 * B:28 * B].view(np.int32)
         h64[0] = 0
         h64[1] = -1
         h32[:] = 0
         h32[2 * B:] = np.arange(B, dtype=np.int32)
         self.blob.copy_(self._stage[0])
-        self._stage[1].copy_(self._stage[0])
+        self._stage[1:].copy_(self._stage[0])
         if ex.gqa_decode_mfma:
             ex.decode_qblocks(B)  # allocated outside the capture
         self.bufs: dict = {}
@@ -1350,13 +1354,12 @@ class _DecodeGraph:
 
     def replay(self, plan: Plan, x: torch.Tensor) -> torch.Tensor:
         b, B = plan.T, self.B
-        self._k ^= 1
-        k = self._k
-        if self._stage_ev[k] is not None:
-            self._stage_ev[k].synchronize()  # the copy issued two replays ago
+        k, half = self._k, self.TURNS // 2
+        if k % half == 0 and self._half_ev[k // half] is not None:
+            self._half_ev[k // half].synchronize()  # this half's last reads: a whole half ago
         host = self._stage[k].numpy()
         h64 = host[: 16 * B].view(np.int64).reshape(2, B)
-        h32 = host[16 * B:].view(np.int32)
+        h32 = host[16 * B:28 * B].view(np.int32)
         h64[:, :b] = plan.h64
         h64[0, b:] = 0
         h64[1, b:] = -1
@@ -1364,14 +1367,16 @@ class _DecodeGraph:
         h32[b:B] = 0
         h32[B:B + b] = plan.h32[b:2 * b]
         h32[B + b:2 * B] = 0
-        self.blob.copy_(self._stage[k], non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record()
-        self._stage_ev[k] = ev
         if self.ex.is_first:
-            self.x[:b].copy_(x.view(-1))
-        elif x.data_ptr() != self.x.data_ptr():  # (a hop received into the static input: no copy)
-            self.x[:b].copy_(x)
+            x = x.view(-1)
+        elif x.data_ptr() == self.x.data_ptr():  # (a hop received into the static input: no copy)
+            x = None
+        ops.step_input(self._stage[k], self.blob, x, self.x[:b])
+        self._k = (k + 1) % self.TURNS
+        if k % half == half - 1:
+            ev = torch.cuda.Event()
+            ev.record()
+            self._half_ev[k // half] = ev
         self.graph.replay()
         return self.out[:b]
 

@@ -72,3 +72,39 @@ def test_pipeline_split_equals_single_stage_on_gpu():
         b = e1.forward([("x", 1)], e0.forward([("x", 1)], t))
         assert torch.equal(a, b)
         t = torch.argmax(a.float(), -1)
+
+
+@pytest.mark.parametrize("rows,width,dtype", [(1, 1, torch.long), (5, 1, torch.long), (256, 1, torch.long), (3, 4, torch.bfloat16),
+                                              (64, 4096, torch.bfloat16), (70, 4100, torch.float32), (3, 5, torch.bfloat16)])
+def test_step_input(rows, width, dtype):
+    """Metadata and rows arrive whole, and rows past the step's own stay; an odd width goes by a copy."""
+    from src import ops
+
+    ops.require_native()
+    n = -(-28 * rows // 8) * 8
+    host = torch.randint(0, 256, (n,), dtype=torch.uint8).pin_memory()
+    meta = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    x = torch.randint(-99, 99, (rows, width), device="cuda").to(dtype)
+    dst = torch.full((rows + 3, width), 7, dtype=dtype, device="cuda")
+    ops.step_input(host, meta, x, dst[:rows])
+    assert torch.equal(meta.cpu(), host) and torch.equal(dst[:rows], x) and bool((dst[rows:] == 7).all())
+    with pytest.raises(RuntimeError, match="pinned"):
+        ops.step_input(host.clone(), meta, None, dst)
+
+
+def test_steps_ahead_of_the_device():
+    """More steps than staging blobs, none waited for: the logits of steps that were."""
+    cfg = resolve_model("small-llama")
+    w = random_stage_weights(cfg, 0, cfg.num_hidden_layers, has_embed=True, has_head=True, device="cuda", seed=5)
+    outs = []
+    for wait in (True, False):
+        ex = StageExecutor(cfg, w, "cuda", kv_cache_bytes=128 << 20, max_sessions=4, max_seq_len=512)
+        ids = torch.arange(3 * 20, device="cuda").view(3, 20) % cfg.vocab_size
+        ex.forward([(f"s{i}", 20) for i in range(3)], ids.view(-1))
+        res = []
+        for k in range(41):
+            res.append(ex.forward([(f"s{i}", 1) for i in range(3)], torch.tensor([1, 2, 3], device="cuda") + k).clone())
+            if wait:
+                torch.cuda.synchronize()
+        outs.append(torch.stack(res))
+    assert torch.equal(*outs)
