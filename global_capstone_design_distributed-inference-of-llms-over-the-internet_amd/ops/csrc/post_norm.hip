@@ -13,30 +13,43 @@
 
 namespace mp {
 
-template <typename T>
+// Bound by latency with few rows, by arithmetic with many.  A thread has one pair of columns, or two where W is a multiple of
+// 4 (VEC = 4: one load, one store of each result), and a row as many workgroups as it takes, so that nothing is a loop.  The
+// angle is reduced in double, in turns: a long context's angle has few fraction bits left in fp32, and sine and cosine of
+// half turns need no reduction of their own.  4 rows of 4096: 10.5 -> 4.8 us, 3802 rows: 66 -> 28 us, against a workgroup a
+// row, with a division in double and the sine of radians.
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void embed_pos_kernel(const int64_t* __restrict__ ids, const T* __restrict__ table,
                                                         int64_t vocab, const int64_t* __restrict__ pos,
                                                         const double* __restrict__ inv, float* __restrict__ res,
-                                                        T* __restrict__ xb, int W, int packed_mt) {
-  const int t = blockIdx.x;
+                                                        T* __restrict__ xb, int W, int per_row, int packed_mt) {
+  const int t = blockIdx.x / per_row, c = ((blockIdx.x - t * per_row) * 256 + threadIdx.x) * VEC;
+  if (c >= W) return;
   int64_t id = ids[t];
   if (id < 0 || id >= vocab) id = 0;  // never read out of bounds; the host validates ids
-  const double p = (double)pos[t];
-  const T* src = table + id * W;
-  for (int i = threadIdx.x; 2 * i < W; i += blockDim.x) {
-    // the angle is reduced in double: a long context's angle has few fraction bits left in fp32
-    constexpr double TWO_PI = 6.283185307179586476925286766559;
-    double a = p * inv[i];
-    a -= TWO_PI * floor(a / TWO_PI);
-    float s, c;
-    sincosf((float)a, &s, &c);
-    const float x0 = ld_f(src, 2 * i) + s;
-    res[(int64_t)t * W + 2 * i] = x0;
-    st_act(xb, t, 2 * i, W, packed_mt, x0);
-    if (2 * i + 1 < W) {
-      const float x1 = ld_f(src, 2 * i + 1) + c;
-      res[(int64_t)t * W + 2 * i + 1] = x1;
-      st_act(xb, t, 2 * i + 1, W, packed_mt, x1);
+  constexpr double TURN = 0.15915494309189533576888376337251;  // 1 / (2 pi)
+  const double p = (double)pos[t] * TURN;
+  const T* src = table + id * W + c;
+  float v[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; j += 2) {
+    const double a = p * inv[c / 2 + j / 2];
+    sincospif((float)(2.0 * (a - rint(a))), &v[j], &v[j + 1]);
+  }
+  if constexpr (VEC == 4) {
+    float x[VEC];
+    ld_vec<VEC>(src, x);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) v[j] += x[j];
+    st_vec<VEC>(res + (int64_t)t * W + c, v);
+    st_act_vec<VEC>(xb, t, c, W, packed_mt, v);
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if (c + j >= W) break;
+      v[j] += ld_f(src, j);
+      res[(int64_t)t * W + c + j] = v[j];
+      st_act(xb, t, c + j, W, packed_mt, v[j]);
     }
   }
 }
@@ -149,12 +162,21 @@ extern "C" int mp_embed_pos(const int64_t* ids, const void* table, int64_t vocab
   using namespace mp;
   (void)hipGetLastError();
   if (T == 0) return 0;
-  if (f32)
-    hipLaunchKernelGGL(embed_pos_kernel<float>, dim3(T), dim3(256), 0, stream, ids, (const float*)table, vocab, pos,
-                       inv, res, (float*)xb, W, packed_mt);
-  else
-    hipLaunchKernelGGL(embed_pos_kernel<bf16_t>, dim3(T), dim3(256), 0, stream, ids, (const bf16_t*)table, vocab, pos,
-                       inv, res, (bf16_t*)xb, W, packed_mt);
+  // pairs of pairs need whole groups of 4 columns, on their natural alignment (a table may be a view of anything)
+  const bool quad = W % 4 == 0 && reinterpret_cast<uintptr_t>(table) % (f32 ? 16 : 8) == 0 &&
+                    reinterpret_cast<uintptr_t>(res) % 16 == 0;
+  const int per_row = (W + (quad ? 1023 : 511)) / (quad ? 1024 : 512);
+#define MP_EP(T_, VEC_)                                                                                                   \
+  hipLaunchKernelGGL((embed_pos_kernel<T_, VEC_>), dim3((unsigned)T * per_row), dim3(256), 0, stream, ids, (const T_*)table, \
+                     vocab, pos, inv, res, (T_*)xb, W, per_row, packed_mt)
+  if (f32) {
+    if (quad) MP_EP(float, 4);
+    else MP_EP(float, 2);
+  } else {
+    if (quad) MP_EP(bf16_t, 4);
+    else MP_EP(bf16_t, 2);
+  }
+#undef MP_EP
   return (int)hipGetLastError();
 }
 

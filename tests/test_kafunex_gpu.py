@@ -33,6 +33,20 @@ def test_embedding_and_positions(dt, W):
 
 
 @pytest.mark.parametrize("dt", sorted(DTYPES))
+@pytest.mark.parametrize("W,off", [(2, 0), (4, 0), (1020, 0), (1028, 0), (4096, 1), (511, 0)])
+def test_embedding_of_far_positions(dt, W, off):
+    """Tables at any address, rows of a group or less and of more than a workgroup's; position 10^6.  Values below 8 are rounded
+    by 2^-22, the half turns by 2^-25 (times pi), sine and cosine by two units of 2^-24."""
+    table = torch.rand(7 * W + off).to(DTYPES[dt]).to(DEV)[off:].view(7, W)
+    ids, pos = torch.tensor([6, 0, 3]), torch.tensor([0, 999999, 1000000])
+    res, xb = torch.empty(3, W, device=DEV), torch.empty(3, W, dtype=DTYPES[dt], device=DEV)
+    hops.embed_pos(ids.to(DEV), table, pos.to(DEV), hops.position_frequencies(W, DEV), res, xb)
+    want = torch.cat([O.sinusoid(1, W, start=int(p)) for p in pos]) + table.cpu()[ids].double()
+    assert float((res.cpu().double() - want).abs().max()) < 2.0 ** -22 + 3.15 * 2.0 ** -25 + 2.0 ** -23
+    assert torch.equal(xb, res.to(DTYPES[dt]))
+
+
+@pytest.mark.parametrize("dt", sorted(DTYPES))
 @pytest.mark.parametrize("n,W", [(1, 64), (300, 70), (5, 4096), (300, 4096), (3, 33), (2, 6144)])
 def test_residual_and_row_norms(dt, n, W):
     y, res, w = torch.randn(n, W).to(DTYPES[dt]), torch.randn(n, W), torch.randn(W)
