@@ -124,6 +124,11 @@ struct ChooseArgs {
   int32_t* lists;     // moe_lists
   int32_t* tok;       // [T top] token of every row
 };
+struct RouteIn {  // the router's own operands, where the choice makes the logits as well
+  const bf16_t *x, *w;
+  int64_t xs;
+  int mt, W, ks;
+};
 
 constexpr int CH_WAVES = 16;
 
@@ -160,8 +165,12 @@ __device__ __forceinline__ void moe_active(const int32_t* cnt, const MoeLists& l
 // time: all slices of the logits are asked for at once, the rows are placed from registers, and up to
 // 64 experts take code of an eighth the size, which is fetched cold in every launch: 12.9 -> 9.3 -> 5.2 us for 6 tokens.
 // (Above that a lane has 8 logits to ask for, and 8 slices of each are enough.)
-template <int CH_PER, bool ALONE>
-__global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a, int per) {
+// NT > 0: up to 16 tokens and 16 NT experts, and the logits are made here, a slice of K a wave, in the sums and the order that
+// the router's own launch and the choice after it have.  One CU reads the router's weights (64 to 256 KB) in 1 to 2 us,
+// less than the launch and the round trip of the slices that it saves.  Two launches took 11.2 us for 6 tokens of 8 experts
+// and, a branch beginning between them, 14.7 for 4 tokens of 32; this one takes 8.9 and 11.2.
+template <int CH_PER, bool ALONE, int NT>
+__global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a, int per, RouteIn in_) {
   constexpr int AHEAD = CH_PER == 1 ? 16 : 8;
   extern __shared__ float sm[];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, E = a.E, gs = E / a.groups;
@@ -172,6 +181,41 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
   float* gz = z + E;                           // and its groups' best
   const MoeLists l = moe_lists(a.lists, E);
   for (int e = tid; e < E; e += blockDim.x) hist[e] = 0;
+  float* logit = sm + 2 * E + 1 + nw * 2 * E;  // (NT) [S][16 NT][17]
+  if constexpr (NT > 0) {
+    constexpr int U = NT == 1 ? 8 : 4;
+    const int c16 = lane & 15, g4 = lane >> 4, row = min(c16, a.T - 1), k1 = min(in_.W, (wv + 1) * in_.ks);
+    if (wv < a.S) {  // (uniform)
+      f32x4 acc[4][NT];  // a quarter of the slice's 32-column steps each, as the router's four waves
+      const bf16_t* wp[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q][n] = (f32x4)(0.f);
+        wp[n] = in_.w + (int64_t)min(16 * n + c16, E - 1) * in_.W + 8 * g4;
+      }
+      for (int k = wv * in_.ks; k < k1; k += 32 * U) {
+        u16x8 b[U], w[U][NT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int kk = min(k + 32 * u, in_.W - 32);  // (past the slice: loaded, not used)
+          b[u] = *reinterpret_cast<const u16x8*>(in_.x + act_at(row, kk + 8 * g4, in_.xs, in_.mt));
+#pragma unroll
+          for (int n = 0; n < NT; ++n) w[u][n] = *reinterpret_cast<const u16x8*>(wp[n] + kk);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (k + 32 * u < k1)  // (uniform)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[u & 3][n] = mfma_bf(w[u][n], b[u], acc[u & 3][n]);
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          logit[(wv * 16 * NT + 16 * n + 4 * g4 + r) * 17 + c16] = acc[0][n][r] + acc[1][n][r] + acc[2][n][r] + acc[3][n][r];
+    }
+  }
   __syncthreads();
   const int t0 = (blockIdx.x * nw + wv) * per;
   // the next token's logits are on their way while this one's experts are ranked
@@ -181,7 +225,9 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
     for (int j = 0; j < CH_PER; ++j) {
       const int e = lane + 64 * j;
       nx[j] = 0.f;
-      if (64 * j < E) {  // (uniform)
+      if constexpr (NT > 0) {
+        for (int s = 0; s < a.S; ++s) nx[j] += logit[(s * 16 * NT + min(e, E - 1)) * 17 + min(t, 15)];
+      } else if (64 * j < E) {  // (uniform)
         for (int s = 0; s < a.S; s += AHEAD) {  // so many slices' loads in flight, added in order
           float p[AHEAD];
 #pragma unroll
@@ -754,7 +800,11 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
   const MoeLists l = moe_lists(lists, E);
   int ks = (W + S - 1) / S;
   ks = (ks + 31) / 32 * 32;
-  if (!f32 && W % 32 == 0 && (mt > 0 || xs % 8 == 0)) {
+  const bool mfma = !f32 && W % 32 == 0 && (mt > 0 || xs % 8 == 0);
+  // few tokens and experts: one launch (E > 32: a single CU would read 512 KB of weights and more)
+  const int fused = mfma && T <= CH_WAVES && S <= CH_WAVES && E <= 32 ? (E + 15) / 16 : 0;
+  if (fused) {
+  } else if (mfma) {
 #define MP_RT(NT_, U_)                                                                                                  \
   hipLaunchKernelGGL((moe_router_mfma_kernel<NT_, U_>), dim3((T + 15) / 16, (E + 16 * NT_ - 1) / (16 * NT_), S),        \
                      dim3(256), 0, stream, (const bf16_t*)x, xs, mt, (const bf16_t*)w, part, T, E, W, ks, l.cnt)
@@ -771,14 +821,16 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
       hipLaunchKernelGGL(moe_router_any_kernel<bf16_t>, grid, dim3(256), 0, stream, (const bf16_t*)x, xs, mt,
                          (const bf16_t*)w, part, T, E, W, ks, l.cnt);
   }
+  const RouteIn in{(const bf16_t*)x, (const bf16_t*)w, xs, mt, W, ks};
   const ChooseArgs a{part, ctx, S, T, E, top, groups, keep, scale, ew, idx, slot, lists, tok};
   const int nw = E <= 256 ? CH_WAVES : CH_WAVES / 2;  // (LDS: 8 E bytes a wave)
-  const size_t lds = (2 * E + 1 + nw * 2 * E) * sizeof(float);
+  const size_t lds = (2 * E + 1 + nw * 2 * E + fused * S * 16 * 17) * sizeof(float);
   // one token a wave as long as that fills no more than the chip; a single workgroup also places the rows
   const int per = (T + 256 * nw - 1) / (256 * nw), nb = (T + nw * per - 1) / (nw * per);
-  auto choose = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(nw * 64), lds, stream, a, per); };
-  if (E <= 64) nb > 1 ? choose(moe_choose_kernel<1, false>) : choose(moe_choose_kernel<1, true>);
-  else nb > 1 ? choose(moe_choose_kernel<MOE_EXPERTS / 64, false>) : choose(moe_choose_kernel<MOE_EXPERTS / 64, true>);
+  auto choose = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(nw * 64), lds, stream, a, per, in); };
+  if (fused) fused == 1 ? choose(moe_choose_kernel<1, true, 1>) : choose(moe_choose_kernel<1, true, 2>);
+  else if (E <= 64) nb > 1 ? choose(moe_choose_kernel<1, false, 0>) : choose(moe_choose_kernel<1, true, 0>);
+  else nb > 1 ? choose(moe_choose_kernel<MOE_EXPERTS / 64, false, 0>) : choose(moe_choose_kernel<MOE_EXPERTS / 64, true, 0>);
   if (nb > 1) hipLaunchKernelGGL(moe_place_kernel, dim3((T * top + 255) / 256), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }

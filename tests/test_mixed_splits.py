@@ -85,3 +85,25 @@ def test_one_workgroup_chooses_and_places(E, top, groups, keep, T):
     p, idx = eops._choose_cpu(x.float(), w.float(), torch.ones_like(ctx), spec)
     c = eops.choose(x.to(DEV), w.to(DEV), ctx.to(DEV), spec, scratch())
     check_choice(c, torch.zeros(T, E).scatter_(1, idx, p), ctx > 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,top", [(5, 2), (16, 4), (17, 4), (32, 4)])
+@pytest.mark.parametrize("W", [64, 256, 2048, 4096, 7168])
+@pytest.mark.parametrize("packed", [False, True])
+def test_choice_in_one_launch_has_the_same_sums(E, top, W, packed):
+    """Up to 16 tokens and 32 experts the choice makes the logits too: the very weights of the same tokens among 17."""
+    from src import ops
+    from tests.test_nuvorax_gpu import DEV, check_choice, scratch
+
+    ops.require_native()
+    g = torch.Generator().manual_seed(E + W)
+    x, w = torch.randn(17, W, generator=g).to(torch.bfloat16), (torch.randn(E, W, generator=g) * 3 / W ** 0.5).to(torch.bfloat16)
+    spec, xd, wd = MoESpec(E, top, 8, 1.0, 1, 1, 1.9), x.to(DEV), w.to(DEV)
+    many = eops.choose(xd, wd, torch.ones(17, dtype=torch.int32, device=DEV), spec, scratch())
+    p, idx = eops._choose_cpu(x.float(), w.float(), torch.ones(17, dtype=torch.int32), spec)
+    for T in (1, 6, 15, 16):
+        rows = ops.pack_act(xd[:T].contiguous()) if packed else xd[:T]
+        few = eops.choose(rows, wd, torch.ones(T, dtype=torch.int32, device=DEV), spec, scratch(), packed=packed)
+        assert torch.equal(few.weights, many.weights[:T])
+        check_choice(few, torch.zeros(T, E).scatter_(1, idx[:T], p[:T]), torch.ones(T, dtype=torch.bool))
