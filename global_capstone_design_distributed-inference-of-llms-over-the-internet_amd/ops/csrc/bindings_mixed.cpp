@@ -30,9 +30,10 @@ int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, const int32_t
                  int keep, float scale, int f32, hipStream_t stream);
 int mp_moe_combine(const void* y, int f32, const float* ew, const int32_t* slot, void* out, int64_t T, int top, int H,
                    hipStream_t stream);
+int64_t mp_moe_gemm_ws(int form, int K);
 int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt, const int32_t* tok, const int32_t* lists,
                 const void* w, void* out, int out_f32, int rows, int E, int N, int K, int block, float limit, int f32,
-                hipStream_t stream);
+                float* ws, hipStream_t stream);
 }
 
 namespace {
@@ -171,6 +172,7 @@ void mixed_attention(const at::Tensor& z, const at::Tensor& qn, const at::Tensor
                "mixed_attention");
 }
 
+int64_t moe_gemm_ws(int64_t form, int64_t K) { return mp_moe_gemm_ws((int)form, (int)K); }
 int64_t moe_lists(int64_t E) { return mp_moe_lists((int)E); }
 int64_t moe_router_splits(int64_t T, int64_t W, int64_t E, bool f32) {
   return mp_moe_router_splits((int)T, (int)W, (int)E, f32);
@@ -216,7 +218,8 @@ void moe_route(const at::Tensor& x, const at::Tensor& w, const at::Tensor& ctx, 
 
 // form 0: w [E, N, K]; 1, 2, 3: w in fragment order [E, N / 16, K / 32, 64, 8].  ``glu``: N gate / up rows, out [rows, N / 2]
 void moe_gemm(int64_t form, const at::Tensor& x, const opt_tensor& tok, const at::Tensor& lists, const at::Tensor& w,
-              at::Tensor& out, int64_t rows, int64_t tokens, int64_t glu, int64_t block, double limit, int64_t packed) {
+              at::Tensor& out, int64_t rows, int64_t tokens, int64_t glu, int64_t block, double limit, int64_t packed,
+              const opt_tensor& ws) {
   const int f32 = act_type(w, "w");
   MP_CHECK(w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "w contiguous, aligned");
   int64_t N, K;
@@ -235,9 +238,15 @@ void moe_gemm(int64_t form, const at::Tensor& x, const opt_tensor& tok, const at
   MP_CHECK(out.is_cuda() && out.dim() == 2 && out.is_contiguous() && out.size(0) >= rows && out.size(1) == O, "out [rows, O]");
   const int of = act_type(out, "out");
   MP_CHECK(glu ? of == f32 : (of || !f32), "out: the activations' type (down products: or fp32)");
+  const int64_t need = mp_moe_gemm_ws((int)form, (int)K);
+  float* parts = nullptr;
+  if (ws.has_value() && need > 0) {
+    parts = const_cast<float*>(f32_vec(*ws, need, "ws"));
+    MP_CHECK(reinterpret_cast<uintptr_t>(parts) % 16 == 0, "ws 16-B aligned");
+  }
   check_launch(mp_moe_gemm((int)form, (int)glu, x.data_ptr(), xs, mt, tok.has_value() ? i32_vec(*tok, rows, "tok") : nullptr,
                            i32_vec(lists, mp_moe_lists(E), "lists"), w.data_ptr(), out.data_ptr(), of, rows, E, N, K,
-                           block, (float)limit, f32, cur_stream()),
+                           block, (float)limit, f32, parts, cur_stream()),
                "moe_gemm");
 }
 
@@ -276,7 +285,8 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def("moe_combine(Tensor y, Tensor ew, Tensor slot, Tensor(a!) out) -> ()");
   m.def(
       "moe_gemm(int form, Tensor x, Tensor? tok, Tensor lists, Tensor w, Tensor(a!) out, int rows, int tokens, int glu, "
-      "int block, float limit, int packed) -> ()");
+      "int block, float limit, int packed, Tensor(b!)? ws=None) -> ()");
+  m.def("moe_gemm_ws(int form, int K) -> int", &moe_gemm_ws);
 }
 
 TORCH_LIBRARY_IMPL(mpamd, CUDA, m) {

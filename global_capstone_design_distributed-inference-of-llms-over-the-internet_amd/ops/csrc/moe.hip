@@ -632,11 +632,62 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
 
 // Many rows per expert, K in steps of 64: 256 x 256 tiles (wide_tile.h) of gathered rows and packed weights.
 // 8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s; the ring of 32-column stages took 687 us.  2700 tokens of two of
-// eight 14336-wide experts of width 4096: up 1502 -> 1253 us, down 803 -> 667 us; 4298 tokens of four of 32 1408-wide ones of
-// 2048: 260 -> 208 us, 151 -> 128 us.
+// eight 14336-wide experts of width 4096: up 1502 us on that ring, 1130 with every tile dealt alike, now 1103; down 803, 699, 616
+// and 20 to add the halves; 4298 tokens of four of 32 1408-wide ones of 2048: 260, 225, 216 and 151, 125, 123.
 //
-// A workgroup makes every ``step``-th tile of its XCD's run.  Lane k of a wave knows tile k of up to 64 of them: the experts' tile
-// counts are summed over the lanes, then every lane looks for its own tile among them.
+// A tile of up to 128 rows takes 0.5 to 0.8 of the time of one of more (``wide_tile.h``), so tiles are dealt by time.  Every XCD gets an
+// eighth of the whole tiles and an eighth of the half ones, each a run in order, whose CUs then share few rows and few weights.
+// Its G workgroups take whole tiles in turn; those that the r left over do not reach take two half ones first, and the
+// other half ones go round.  Where all that is left fits one half round, and a workspace is there, the r are cut at the
+// middle of K instead: a workgroup makes a half, and moe_gemm_close_kernel adds the two.  A workgroup's half tiles lie
+// between its whole ones, sooner in some than in others: their weights come from HBM a second time, and all at once that
+// bound them.
+// Lane k of a wave knows tile k of up to 64 of them: the experts' tile counts are summed over the lanes, then every lane
+// looks for its own tile among them.
+constexpr int MW_SPLIT = 16;  // whole tiles an XCD cuts at most (twice as many fill 32 workgroups)
+struct MoeDeal {
+  int f0, q, r, h0, halves;  // whole tiles from f0 on: q a workgroup, r left over; half ones from h0 on
+  bool split;
+  __device__ MoeDeal(const MoeLists& l, int E, int ntn, int xcd, int G, bool can_split) {
+    const int lane = threadIdx.x & 63;
+    int f = 0, h = 0;
+    for (int i = lane; i < E; i += 64) f += (l.cnt[i] + 127) >> 8, h += ((l.cnt[i] + 255) >> 8) - ((l.cnt[i] + 127) >> 8);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) f += __shfl_xor(f, d, 64), h += __shfl_xor(h, d, 64);
+    const int64_t F = (int64_t)__builtin_amdgcn_readfirstlane(f) * ntn, H = (int64_t)__builtin_amdgcn_readfirstlane(h) * ntn;
+    f0 = (int)(F * xcd >> 3), h0 = (int)(H * xcd >> 3);
+    const int run = (int)(F * (xcd + 1) >> 3) - f0;
+    halves = (int)(H * (xcd + 1) >> 3) - h0, q = run / G, r = run % G;
+    split = can_split && r > 0 && r <= MW_SPLIT && 2 * r + halves <= G;
+  }
+};
+// per lane: expert, weight tile and row tile of whole or half tile ``id``
+__device__ __forceinline__ void moe_find(const MoeLists& l, int E, int ntn, bool half, int id, int& e, int& nt, int& mt) {
+  const int lane = threadIdx.x & 63;
+  int fb = 0, hb = 0;
+  e = nt = mt = 0;
+  for (int i = 0; i < E; i += 64) {
+    const int c = i + lane < E ? l.cnt[i + lane] : 0, f = (c + 127) >> 8, h = ((c + 255) >> 8) - f;
+    int fs = f, hs = h;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(fs, d, 64), z = __shfl_up(hs, d, 64);
+      if (lane >= d) fs += y, hs += z;
+    }
+    for (int g = 0; g < min(64, E - i); ++g) {
+      const int fe = __builtin_amdgcn_readlane(f, g), he = __builtin_amdgcn_readlane(h, g);
+      const int ce = half ? he : fe;
+      const int first = (half ? hb + __builtin_amdgcn_readlane(hs, g) - he : fb + __builtin_amdgcn_readlane(fs, g) - fe) * ntn;
+      if (id >= first && id < first + ce * ntn) {
+        const int s = id - first, band = s / (MG_BAND * ntn), n = min(MG_BAND, ce - MG_BAND * band), u = s - band * MG_BAND * ntn;
+        e = i + g, nt = u / n;
+        mt = half ? fe : MG_BAND * band + u % n;
+      }
+    }
+    fb += __builtin_amdgcn_readlane(fs, 63), hb += __builtin_amdgcn_readlane(hs, 63);
+  }
+}
+
 template <bool GLU, typename TO>
 struct MoeWork {
   static constexpr int STORES = WideTile::put_stores(GLU);
@@ -644,14 +695,18 @@ struct MoeWork {
   const MoeGemm& a;
   const MoeLists& l;
   bool wide;
-  int en, mt;  // lane k: expert and weight tile (10 bits and the others), row tile of tile k
+  float* ws;
+  int en, mt, pt;  // lane k: expert and weight tile (10 bits and the others), row tile of tile k; 0, or its place in ws + 1
+  __device__ int part(int k) const { return __builtin_amdgcn_readlane(pt, k); }
+  __device__ int first(int k) const { return part(k) && !(part(k) & 1) ? (a.K / 64 + 1) / 2 : 0; }  // its first stage
   __device__ int expert(int k) const { return __builtin_amdgcn_readlane(en, k) & 1023; }
   __device__ int n0(int k) const { return (__builtin_amdgcn_readlane(en, k) >> 10) * W::BN; }
   __device__ int m0(int k) const { return __builtin_amdgcn_readlane(mt, k) * W::BM; }
-  __device__ int stages(int) const { return a.K / 64; }
+  __device__ int stages(int k) const { return !part(k) ? a.K / 64 : (a.K / 64 + (part(k) & 1)) / 2; }
   __device__ void rows(int k, W::Source& s) const {
     const int e = expert(k), m = m0(k), r0 = l.off[e], n = l.cnt[e];
     s.from(a.x, 0xffffffffu, 128);
+    s.at = 128 * first(k);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // (the launcher checks that they fit)
       const int q = r0 + min(m + W::piece_row(j), n - 1), row = a.tok ? a.tok[q] : q;
@@ -661,12 +716,25 @@ struct MoeWork {
   __device__ void weights(int k, W::Source& s) const {
     const int t0 = n0(k) / 16, nt = a.N / 16;
     s.from((const bf16_t*)a.w + (int64_t)expert(k) * a.N * a.K, (uint32_t)a.N * (uint32_t)a.K * 2, 2048);
+    s.at = 2048 * first(k);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       s.off[j] = (uint32_t)min(t0 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
   }
   __device__ bool live(int k) const { return m0(k) + 16 * W::MW * W::wm() < l.cnt[expert(k)]; }
+  // (a lane's sums as they lie, 16 bytes each: whoever adds the parts has the same lanes)
+  static __device__ __forceinline__ f32x4* kept(float* ws, int place) {
+    return reinterpret_cast<f32x4*>(ws) + ((int64_t)place * 8 + W::wave()) * W::NW * W::MW * 64 + (threadIdx.x & 63);
+  }
   __device__ bool store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
+    if (!GLU && part(k)) {
+      f32x4* to = kept(ws, part(k) - 1);
+#pragma unroll
+      for (int i = 0; i < W::NW; ++i)
+#pragma unroll
+        for (int j = 0; j < W::MW; ++j) to[(i * W::MW + j) * 64] = acc[i][j];
+      return true;
+    }
     const int e = expert(k), m = m0(k) + 16 * W::MW * W::wm(), o = n0(k) + 16 * W::NW * W::wn(), n = l.cnt[e];
     const int cols = GLU ? a.N / 2 : a.N;
     TO* out = (TO*)a.out + (int64_t)l.off[e] * cols;
@@ -689,50 +757,72 @@ struct MoeWork {
 };
 
 template <bool GLU, typename TO>
-__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide) {
+__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide, float* ws) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
   const int lane = threadIdx.x & 63, ntn = (a.N + WideTile::BN - 1) / WideTile::BN;
-  int total = 0;
-  for (int i = 0; i < a.E; i += 64) total += moe_tile_count(l, a.E, i, lane, WideTile::BM);
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, 64);
-  const int all = __builtin_amdgcn_readfirstlane(total) * ntn, per = (all + 7) / 8, step = gridDim.x >> 3, at = blockIdx.x >> 3;
-  const int lo = (blockIdx.x & 7) * per + at, run = min(per, all - (int)(blockIdx.x & 7) * per);
-  const int tiles = at < run ? (run - at + step - 1) / step : 0;
-  for (int first = 0; first < tiles; first += 64) {
-    const int count = min(64, tiles - first), id = lo + min(first + lane, tiles - 1) * step;
-    int en = 0, mt = 0, base = 0;
-    for (int i = 0; i < a.E; i += 64) {
-      const int c = moe_tile_count(l, a.E, i, lane, WideTile::BM);
-      int sum = c;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(sum, d, 64);
-        if (lane >= d) sum += y;
+  const int G = gridDim.x >> 3, at = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+  const MoeDeal d(l, a.E, ntn, xcd, G, !GLU && ws != nullptr);
+  const int free = d.r > 0 && !d.split ? G - d.r : 0, early = min(d.halves, 2 * free);  // half tiles of those the r do not reach
+  const int mine = at - d.r;
+  const int whole = d.q + (!d.split && at < d.r);
+  const int n1 = free > 0 && mine >= 0 && early > mine ? (early - mine + free - 1) / free : 0;
+  const int rest = (d.split ? 2 * d.r + d.halves : d.halves - early) - at;
+  const int halves = n1 + (rest > 0 ? (rest + G - 1) / G : 0), n = whole + halves;
+  const int shift = n * at / G;
+  for (int first = 0; first < n; first += 64) {
+    const int count = min(64, n - first), k = first + min(lane, count - 1);
+    const int before = (k * halves + shift) / n;  // half tiles ahead of tile k
+    bool half = ((k + 1) * halves + shift) / n > before;
+    int id = d.f0 + at + (k - before) * G, pt = 0;
+    if (half) {
+      id = before < n1 ? mine + before * free : early + at + (before - n1) * G;
+      if (d.split && id < 2 * d.r) {
+        pt = 1 + 2 * (xcd * MW_SPLIT + (id >> 1)) + (id & 1);
+        id = d.f0 + d.q * G + (id >> 1);
+        half = false;
+      } else {
+        id += d.h0 - (d.split ? 2 * d.r : 0);
       }
-      for (int q = 0; q < min(64, a.E - i); ++q) {
-        const int ce = __builtin_amdgcn_readlane(c, q), b = (base + __builtin_amdgcn_readlane(sum, q) - ce) * ntn;
-        if (id >= b && id < b + ce * ntn) {
-          const int r = id - b, band = r / (MG_BAND * ntn), h = min(MG_BAND, ce - MG_BAND * band), s = r - band * MG_BAND * ntn;
-          en = i + q + (s / h << 10);
-          mt = MG_BAND * band + s % h;
-        }
-      }
-      base += __builtin_amdgcn_readlane(sum, 63);
     }
+    int e, nt, mt;
+    moe_find(l, a.E, ntn, half, id, e, nt, mt);
     if (first) __syncthreads();  // (the last tiles' operands have been read)
-    WideTile::run<WideTile::PACKED>(smem, count, MoeWork<GLU, TO>{a, l, wide, en, mt});
+    WideTile::run<WideTile::PACKED>(smem, count, MoeWork<GLU, TO>{a, l, wide, ws, e + (nt << 10), mt, pt});
   }
 }
 
+// The cut tiles' two sums added, rounded and stored; workgroup (XCD, tile of it).  Bound by the 64 MB at most that they lie in.
+__global__ __launch_bounds__(512) void moe_gemm_close_kernel(MoeGemm a, bool wide, float* ws, int G) {
+  typedef MoeWork<false, bf16_t> Work;
+  const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
+  const int ntn = (a.N + WideTile::BN - 1) / WideTile::BN, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const MoeDeal d(l, a.E, ntn, xcd, G, true);
+  if (!d.split || at >= d.r) return;
+  int e, nt, mt;
+  moe_find(l, a.E, ntn, false, d.f0 + d.q * G + at, e, nt, mt);
+  const Work work{a, l, wide, nullptr, e + (nt << 10), mt, 0};
+  if (!work.live(0)) return;
+  const int place = 2 * (xcd * MW_SPLIT + at);
+  const f32x4 *p = Work::kept(ws, place), *q = Work::kept(ws, place + 1);
+  f32x4 acc[WideTile::NW][WideTile::MW];
+#pragma unroll
+  for (int i = 0; i < WideTile::NW; ++i)
+#pragma unroll
+    for (int j = 0; j < WideTile::MW; ++j) acc[i][j] = p[(i * WideTile::MW + j) * 64] + q[(i * WideTile::MW + j) * 64];
+  work.store(0, acc);
+}
+
 template <bool GLU, typename TO>
-static int launch_moe_wide(const MoeGemm& a, int rows, int act, hipStream_t stream) {
-  const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN), per = (tiles + 7) / 8;
+static int launch_moe_wide(const MoeGemm& a, int rows, int act, float* ws, hipStream_t stream) {
+  const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN), per = (tiles + 7) / 8 + 1;
+  const int G = per < WideTile::CUS / 8 ? per : WideTile::CUS / 8;  // (whole and half tiles are shared out apart: one more)
+  const bool wide = (uintptr_t)a.out % 16 == 0;
   (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             WideTile::LDS);
-  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3(8 * (per < WideTile::CUS / 8 ? per : WideTile::CUS / 8)), dim3(512),
-                     WideTile::LDS, stream, a, (uintptr_t)a.out % 16 == 0);
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3(8 * G), dim3(512), WideTile::LDS, stream, a, wide, ws);
+  if constexpr (!GLU && sizeof(TO) == 2)
+    if (ws) hipLaunchKernelGGL(moe_gemm_close_kernel, dim3(8 * MW_SPLIT), dim3(512), 0, stream, a, wide, ws, G);
   return (int)hipGetLastError();
 }
 
@@ -850,10 +940,16 @@ extern "C" int mp_moe_combine(const void* y, int f32, const float* ew, const int
   return (int)hipGetLastError();
 }
 
+// floats of the workspace that lets form 3 cut the tiles of its last round (bf16 down products): from K = 4096 on, half a
+// tile is 45 us and more, and adding the halves 15
+extern "C" int64_t mp_moe_gemm_ws(int form, int K) {
+  return form == 3 && K % 64 == 0 && K >= 4096 ? 8ll * mp::MW_SPLIT * 2 * mp::WideTile::BM * mp::WideTile::BN : 0;
+}
+
 // form 0: any shape, 1: few rows per expert, 2: many, 3: very many
 extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt, const int32_t* tok,
                            const int32_t* lists, const void* w, void* out, int out_f32, int rows, int E, int N, int K,
-                           int block, float limit, int f32, hipStream_t stream) {
+                           int block, float limit, int f32, float* ws, hipStream_t stream) {
   using namespace mp;
   (void)hipGetLastError();
   if (rows == 0) return 0;
@@ -875,7 +971,7 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
     const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31);
     const bool big = form == 3 && rows >= 384 * E;
 #define MP_MT(GLU_, TO_)                                                        \
-  return wide  ? launch_moe_wide<GLU_, TO_>(a, rows, act, stream) \
+  return wide  ? launch_moe_wide<GLU_, TO_>(a, rows, act, GLU_ || sizeof(TO_) != 2 ? nullptr : ws, stream) \
          : big ? launch_moe_tile<GLU_, TO_, 4, 8, 4, 2>(a, rows, act, stream) \
                : launch_moe_tile<GLU_, TO_, 4, 4, 2, 2>(a, rows, act, stream);
     if (glu) MP_MT(true, bf16_t)

@@ -17,7 +17,7 @@
 //     to two MFMAs; the stage's loads are spread over the half stage behind the barrier: eight at once hold up the MFMAs that
 //     stand behind them.
 //   * A wave whose 64 rows are past the last only loads; the two waves of a SIMD have different rows, so a tile of up to 128
-//     rows takes half the time.
+//     rows takes half the MFMA time (0.8 of a whole tile's where its weights come from HBM: the ring covers less of the wait).
 // Bound by MFMA issue (three quarters of the time; the clock falls to 1.8 GHz under it) and by the issue of the loads, an eighth.
 // Measured and left: four waves of 128 x 128 (2 to 5 % more), a second barrier that frees the slot sooner (6 % more), 32 x 32
 // x 16 MFMAs (12 % more), loads over both halves of a stage (up to 8 % more).

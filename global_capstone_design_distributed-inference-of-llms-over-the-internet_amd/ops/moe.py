@@ -165,7 +165,9 @@ def experts(x, c: Choice, up, down, up_p, down_p, block, e, packed=False):
     y = e("moe_y", (R, W), dt if form > 1 and R >= NARROW_ROWS * m.experts else torch.float32)
     torch.ops.mpamd.moe_gemm(form, x, c.tok, c.lists, up_p if form else up, act, R, c.tokens, 1, block, float(m.limit),
                              int(packed))
-    torch.ops.mpamd.moe_gemm(form, act, None, c.lists, down_p if form else down, y, R, c.tokens, 0, 1, 0.0, 0)
+    n = torch.ops.mpamd.moe_gemm_ws(form, m.ff) if y.dtype == torch.bfloat16 else 0
+    torch.ops.mpamd.moe_gemm(form, act, None, c.lists, down_p if form else down, y, R, c.tokens, 0, 1, 0.0, 0,
+                             e("moe_parts", (n,), torch.float32) if n else None)
     return y
 
 

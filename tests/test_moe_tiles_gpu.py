@@ -102,3 +102,27 @@ def test_not_a_number_stays_in_its_rows(form):
             assert torch.equal(out.isfinite(), want.isfinite())
         else:
             assert out[70].isnan().all() and not (out[260].isfinite() & (out[260] != 0)).any()
+
+
+@pytest.mark.parametrize("counts,N,K", [([300, 0, 129, 100], 800, 4096), ([1062, 898, 793, 730, 607, 544, 435, 331], 4096, 4160),
+                                        ([257] * 70, 304, 4096), ([2049], 768, 4160), ([40, 20], 512, 4096)])
+def test_tiles_of_the_last_round_in_halves(counts, N, K):
+    """With a workspace, whole tiles that some workgroups would make alone are cut at the middle of K (also of an odd number of
+    stages), half-full ones go round; every output is written, none of the workspace is read that was not.  Two sums of half
+    the products each, added in 32 bits: the tolerance as above."""
+    ops.require_native()
+    E, R = len(counts), sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(R, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(E, N, K, generator=g, device="cuda").div(K ** 0.5).to(torch.bfloat16)
+    wp, lists = torch.stack([ops.pack_weight(m) for m in w]), _lists(counts)
+    need = torch.ops.mpamd.moe_gemm_ws(3, K)
+    assert need > 0 == torch.ops.mpamd.moe_gemm_ws(3, 4032)
+    ws = torch.full((need,), float("nan"), device="cuda")
+    out = torch.full((R, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    torch.ops.mpamd.moe_gemm(3, x, None, lists, wp, out, R, R, 0, 1, 0.0, 0, ws)
+    at = 0
+    for e, n in enumerate(counts):
+        want = x[at:at + n].float() @ w[e].float().t()
+        assert n == 0 or float((out[at:at + n].float() - want).norm() / want.norm()) < 2.0 ** -8
+        at += n
