@@ -7,10 +7,18 @@
 // one sequence (row = token-major x the GQA group's HB heads: row r is token tok0 + r / HB,
 // head hbase + r % HB), and streams the causal context in 64-token steps:
 //
-//   * K and V tiles [64 tok][128 d] are staged once per step for all NW waves through a
-//     double-buffered LDS image (256-B rows, 16-B chunks XOR-swizzled by the row so both the
-//     row reads of K and the transposed reads of V are bank-conflict-free); the next step's
-//     tiles are fetched into registers while the current one computes (one barrier per step).
+//   * K and V tiles [64 tok][128 d] are staged once per step for all NW waves through two LDS slots
+//     each (256-B rows, 16-B chunks XOR-swizzled by the row so both the row reads of K and the
+//     transposed reads of V are bank-conflict-free).  Loads go straight to LDS, a step ahead, and
+//     the page of the step behind them is looked up a step before that (one barrier per step).
+//   * A step takes the softmax and O of its scores and makes the NEXT step's scores, so that the
+//     exponentials have the MFMAs of K . Q^T between them and the next maximum those of V^T . P^T.
+//     Bound by VALU and MFMA issue, which add up: a step of 32 rows is 1024 cycles of MFMA and about 1250
+//     of VALU (512 of them exponentials), two waves a SIMD.  7995 tokens of 32 / 8 heads: 686 us with the
+//     phases one after the other and tiles by way of registers, 670 with loads straight to LDS and the phases mixed,
+//     641 with pages looked up ahead and the maximum exchanged without LDS.  (Measured and left: a
+//     barrier for every second step 660; wave priorities 645; spills in the loop 1142, as their waits cover
+//     the tiles' loads.)
 //   * S^T = K . Q^T per wave: 2 x (D/16) v_mfma_f32_32x32x16_bf16 (A = K rows from LDS with
 //     ds_read_b128, B = Q^T fragments held in registers for the whole kernel).  The
 //     accumulator's COLUMN is the query row, so each lane owns one row and 16 of its
@@ -129,27 +137,36 @@ __global__ __launch_bounds__(NW * 64) void attn_fa_kernel(
   for (int dt = 0; dt < D / 32; ++dt) o[dt] = (f32x16)(0.f);
   float m = -INFINITY, l = 0.f;  // running max (log2 units, scale applied) and sum of row r
 
-  u16x8 kreg[CPT], vreg[CPT];
-  auto fetch = [&](int s0) {
-    const int64_t pg = bt[s0 >> page_log2];
-    const bf16_t* kp = kc + pg * page_stride + head_off + (int64_t)(s0 & (page_size - 1)) * D;
-    const bf16_t* vp = vc + pg * page_stride + head_off + (int64_t)(s0 & (page_size - 1)) * D;
+  // A tile goes straight to LDS, two KiB a wave: 1-KiB blocks of 8 rows x 64 columns, whose lanes' rows and chunks are the
+  // image's.  (Loads the compiler knows of make every transposed read wait for them; these are waited for by hand.)
+  const int fr = (lane >> 2) & 7;  // row of a block
+  uint32_t off[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; ++j) {
+    const int blk = CPT * w + j, row = 8 * (blk >> 1) + fr, ch = 8 * (blk & 1) + 4 * (lane >> 5) + ((lane & 3) ^ ((row >> 2) & 3));
+    off[j] = (uint32_t)(row * D + ch * 8) * 2;
+  }
+  auto page = [&](int s0) { return s0 < end ? bt[s0 >> page_log2] : 0; };
+  auto fetch = [&](const bf16_t* from, int s0, int64_t pg, int tile) {
+    const uint64_t at = (uint64_t)(uintptr_t)(from + pg * page_stride + head_off + (int64_t)(s0 & (page_size - 1)) * D);
+    const u32x4_fa words = {(uint32_t)__builtin_amdgcn_readfirstlane((int)at),
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) & 0xffff, (uint32_t)TILE, 0x00020000u};
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      const int c = tid + NT * j, row = c >> 4, ch = c & 15;
-      kreg[j] = *reinterpret_cast<const u16x8*>(kp + row * D + ch * 8);
-      vreg[j] = *reinterpret_cast<const u16x8*>(vp + row * D + ch * 8);
+      const uint32_t to = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(smem + tile * TILE + (CPT * w + j) * 1024);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(to), "v"(off[j]), "s"(words)
+                   : "memory");
     }
   };
-  auto stash = [&](int buf, int s0) {
-    unsigned char* kb = smem + buf * 2 * TILE;
+  // the wave's loads have landed; rows of V past the context are cleared (stale cache bytes never meet a p = 0; stale scores
+  // are masked)
+  auto landed = [&](int s0, int tile) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (s0 + STEP > end)
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const int c = tid + NT * j, row = c >> 4, ch = c & 15;
-      const bool past = s0 + row >= end;  // past the context: stale cache bytes never meet a p = 0
-      *reinterpret_cast<u16x8*>(kb + fa_off(row, ch)) = past ? (u16x8)(0) : kreg[j];
-      *reinterpret_cast<u16x8*>(kb + TILE + fa_off(row, ch)) = past ? (u16x8)(0) : vreg[j];
-    }
+      for (int j = 0; j < CPT; ++j)
+        if (s0 + 8 * ((CPT * w + j) >> 1) + fr >= end)
+          *reinterpret_cast<u16x8*>(smem + tile * TILE + (CPT * w + j) * 1024 + lane * 16) = (u16x8)(0);
   };
 
   // per-lane LDS bases (every read of a step is one of them + an immediate):
@@ -160,99 +177,142 @@ __global__ __launch_bounds__(NW * 64) void attn_fa_kernel(
   const int grp = lane >> 4, gi = lane & 15, tq = gi >> 2, tp = gi & 3;
   const int kbase0 = fa_off(r, hh), kbase1 = fa_off(r, 2 + hh);
   const int trc = 2 * (grp & 1) + (tp >> 1);
-  const int vbase0 = TILE + fa_off(4 * hh + tq, trc) + 8 * (tp & 1);
-  const int vbase1 = TILE + fa_off(8 + 4 * hh + tq, trc) + 8 * (tp & 1);
+  const int vbase0 = fa_off(4 * hh + tq, trc) + 8 * (tp & 1);
+  const int vbase1 = fa_off(8 + 4 * hh + tq, trc) + 8 * (tp & 1);
 
+  // A step takes the softmax of its scores and its part of O, and makes the scores of the next one, S^T = K . Q^T (two
+  // accumulation chains, halves of d, summed afterwards).  In groups of one MFMA, the VALU work of two scores and the LDS reads
+  // of the MFMA four on, which the fences keep as written: first the exponentials beside the next scores, then the next
+  // maximum beside O.
+  f32x16 st[2];
+  float lm;  // largest of st on this lane
+  u16x8 ka[4];
+  auto key = [&](const unsigned char* kt, int sub, int s) {
+    return *reinterpret_cast<const u16x8*>(kt + ((s & 1) ? kbase1 : kbase0) + 8192 * sub + 512 * (s >> 1));
+  };
+  auto value = [&](const unsigned char* vt, int i) {  // i: 8 sub + 4 s2 + dt
+    const u16x4 lo = tr16(vt + vbase0 + 4096 * (i >> 2) + 512 * (i & 3));
+    const u16x4 hi = tr16(vt + vbase1 + 4096 * (i >> 2) + 512 * (i & 3));
+    return (u16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto across = [](float x) {  // the larger of a row's two lanes
+    const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
+  };
+  auto largest = [&](int sub) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) lm = fmaxf(lm, st[sub][j]);
+  };
+  auto step = [&](int b0, const unsigned char* kt, const unsigned char* vt) {
+    // ---- online softmax of row r over this lane's 32 tokens (raw scores; the scale is
+    //      folded into the exponent's FMA) ----
+#pragma unroll
+    for (int s = 0; s < 4; ++s) ka[s] = key(kt, 0, s);
+    if (b0 + STEP > wave_lim0) {  // diagonal / last step: causal and context mask
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int tk = b0 + 32 * sub + 4 * hh + (j & 3) + 8 * (j >> 2);
+          st[sub][j] = tk < lim ? st[sub][j] : -INFINITY;
+        }
+      lm = -INFINITY;
+      largest(0), largest(1);
+    }
+    lm = across(lm) * scale_log2;
+    // rescale O and l only when some row's maximum grew by more than the threshold
+    if (!__all(lm <= m + FA_RESCALE_THR)) {
+      const float m_new = fmaxf(m, lm);
+      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) o[dt] *= alpha;
+      m = m_new;
+    }
+    const float mu = m == -INFINITY ? 0.f : m;  // fully masked row so far: every p is 0
+    float ps = 0.f;
+    unsigned pk[2][8];
+    auto weigh = [&](int sub, int i) {
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[sub][2 * i], scale_log2, -mu));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[sub][2 * i + 1], scale_log2, -mu));
+      ps += p0 + p1;
+      pk[sub][i] = pk_bf16(p0, p1);
+    };
+    auto pf = [&](int sub, int s2) {
+      return __builtin_bit_cast(u16x8, (u32x4_fa){pk[sub][4 * s2], pk[sub][4 * s2 + 1], pk[sub][4 * s2 + 2], pk[sub][4 * s2 + 3]});
+    };
+    f32x16 sa[2], sb[2];
+    sa[0] = sa[1] = sb[0] = sb[1] = (f32x16)(0.f);
+    u16x8 va[4];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      sa[s >> 2] = mfma32x16(ka[s & 3], qf[s], sa[s >> 2]);
+      ka[s & 3] = s < 4 ? key(kt, 0, s + 4) : key(kt, 1, s - 4);
+      weigh(0, s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      sb[s >> 2] = mfma32x16(ka[s & 3], qf[s], sb[s >> 2]);
+      if (s < 4) ka[s] = key(kt, 1, s + 4);
+      else va[s - 4] = value(vt, s - 4);
+      weigh(1, s);
+      if (s == 3) st[0] = sa[0] + sa[1];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- O^T += V^T . P^T: A = V^T by transposed LDS reads, B = P from registers ----
+    lm = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      o[s & 3] = mfma32x16(va[s & 3], pf(0, s >> 2), o[s & 3]);
+      va[s & 3] = value(vt, 4 + s);
+      if (s == 2) largest(0);
+      if (s == 5) st[1] = sb[0] + sb[1];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      o[s & 3] = mfma32x16(va[s & 3], pf(1, s >> 2), o[s & 3]);
+      if (s < 4) va[s] = value(vt, 12 + s);
+      if (s == 2) largest(1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    l += ps;
+  };
+
+  // tiles: K of even and odd steps, V of even and odd steps.  A step reads its V and the next one's K.
+  int pg0 = page(start), pg1 = page(start + STEP), pg2 = page(start + 2 * STEP);  // (a step's V is in the page of its K)
   if (start < end) {
-    fetch(start);
-    stash(0, start);
+    fetch(kc, start, pg0, 0);
+    fetch(vc, start, pg0, 2);
+    if (start + STEP < end) fetch(kc, start + STEP, pg1, 1);
+    landed(start, 2);
+  }
+  __syncthreads();
+  if (start < wave_ctx) {
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      f32x16 sa[2];
+      sa[0] = sa[1] = (f32x16)(0.f);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) sa[s >> 2] = mfma32x16(key(smem, sub, s), qf[s], sa[s >> 2]);
+      st[sub] = sa[0] + sa[1];
+    }
+    lm = -INFINITY;
+    largest(0), largest(1);
   }
   __syncthreads();
   int it = 0;
   for (int b0 = start; b0 < end; b0 += STEP, ++it) {
     const int cur = it & 1;
     const bool more = b0 + STEP < end;
-    if (more) fetch(b0 + STEP);
-    if (b0 < wave_ctx) {
-      const unsigned char* tb = smem + cur * 2 * TILE;
-      // ---- S^T = K . Q^T for the step's 64 tokens: 4 independent accumulation chains
-      //      (two 32-token subtiles x two halves of d), summed afterwards ----
-      f32x16 sa[2][2];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          sa[sub][half] = (f32x16)(0.f);
-#pragma unroll
-          for (int s = 4 * half; s < 4 * half + 4; ++s) {
-            const u16x8 a = *reinterpret_cast<const u16x8*>(tb + ((s & 1) ? kbase1 : kbase0) + 8192 * sub +
-                                                            512 * (s >> 1));
-            sa[sub][half] = mfma32x16(a, qf[s], sa[sub][half]);
-          }
-        }
-      f32x16 st[2];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) st[sub] = sa[sub][0] + sa[sub][1];
-      // ---- online softmax of row r over this lane's 32 tokens (raw scores; the scale is
-      //      folded into the exponent's FMA) ----
-      if (b0 + STEP > wave_lim0) {  // diagonal / last step: causal and context mask
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const int tk = b0 + 32 * sub + 4 * hh + (j & 3) + 8 * (j >> 2);
-            st[sub][j] = tk < lim ? st[sub][j] : -INFINITY;
-          }
-      }
-      float lm = -INFINITY;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) lm = fmaxf(lm, st[sub][j]);
-      lm = fmaxf(lm, __shfl_xor(lm, 32, 64)) * scale_log2;
-      // rescale O and l only when some row's maximum grew by more than the threshold
-      if (!__all(lm <= m + FA_RESCALE_THR)) {
-        const float m_new = fmaxf(m, lm);
-        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
-        l *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt) o[dt] *= alpha;
-        m = m_new;
-      }
-      const float mu = m == -INFINITY ? 0.f : m;  // fully masked row so far: every p is 0
-      u16x8 pf[2][2];
-      float ps = 0.f;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          unsigned pk[4];
-#pragma unroll
-          for (int j = 0; j < 8; j += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[sub][8 * s2 + j], scale_log2, -mu));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[sub][8 * s2 + j + 1], scale_log2, -mu));
-            ps += p0 + p1;
-            pk[j >> 1] = pk_bf16(p0, p1);
-          }
-          pf[sub][s2] = __builtin_bit_cast(u16x8, (u32x4_fa){pk[0], pk[1], pk[2], pk[3]});
-        }
-      l += ps;
-      // ---- O^T += V^T . P^T: A = V^T by transposed LDS reads, B = P from registers ----
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2) {
-            const int imm = 8192 * sub + 4096 * s2 + 512 * dt;
-            const u16x4 lo = tr16(tb + vbase0 + imm);
-            const u16x4 hi = tr16(tb + vbase1 + imm);
-            const u16x8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            o[dt] = mfma32x16(a, pf[sub][s2], o[dt]);
-          }
-      }
-    }
-    if (more) stash(cur ^ 1, b0 + STEP);
+    if (b0 + 2 * STEP < end) fetch(kc, b0 + 2 * STEP, pg2, cur);
+    if (more) fetch(vc, b0 + STEP, pg1, 2 + (cur ^ 1));
+    pg1 = pg2, pg2 = page(b0 + 3 * STEP);
+    const unsigned char *kt = smem + (cur ^ 1) * TILE, *vt = smem + (2 + cur) * TILE;
+    if (b0 < wave_ctx) step(b0, kt, vt);
+    if (more) landed(b0 + STEP, 2 + (cur ^ 1));
     __syncthreads();
   }
   // ---- epilogue: lane owns row r; O^T accumulator register j of d-tile dt holds
