@@ -35,7 +35,8 @@
 // with 160 registers and 35 KB (V in rows, transposed by the read; the queries turned once) 3 fit, so
 // the 640 slices of 12 sessions of 1.7k to 5.8k tokens (32 / 8 heads) run at once - 45 us for 184 MB
 // where 2 to a CU took 58 in a full round and a quarter one; 64 sessions up to 512: 25.0 -> 20.6 us,
-// one of 900: 12.3 -> 10.1.
+// one of 900: 12.3 -> 10.1.  A grid column was a session on one XCD, some XCDs with two of the 12: slices turned over
+// all XCDs take 43 us instead of 47 in a whole step; 1, 2, 20 and 64 sessions take as long as before.
 // (K/V loads keep the default cache policy here: non-temporal loads, a win for the MHA decode
 // kernel in attention.hip, measured 12-14 % SLOWER on this kernel at 64 / 256 sessions, cold
 // caches - profiles/r3_i/attn_nt.jsonl vs attn_def.jsonl.)
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256, 3) void attn_mfma_kernel(
     const int32_t* __restrict__ block_tables, int bt_stride, const int32_t* __restrict__ q_seq,
     const int32_t* __restrict__ q_ctx, const int32_t* __restrict__ qb_tok0, const int32_t* __restrict__ qb_ntok,
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int nkv, int nh,
-    int page_log2, int PS, int NP, float scale_log2, int packed_mt, RopeFuseM rf) {
+    int page_log2, int PS, int NP, int NB, float scale_log2, int packed_mt, RopeFuseM rf) {
   constexpr int TB = 16 / HB;
   constexpr int KD = D / 32;  // k-chunks of the QK^T product
   constexpr int DT = D / 16;  // 16-column tiles of O
@@ -92,9 +93,12 @@ __global__ __launch_bounds__(256, 3) void attn_mfma_kernel(
   __shared__ __attribute__((aligned(256))) unsigned char s_wave[4][WB];
   __shared__ float s_m[4][16], s_l[4][16];
 
-  const int b = blockIdx.x, p = blockIdx.z;
+  const int p = blockIdx.z;
   const int hbase = blockIdx.y * HB;
   const int g = hbase / (nh / nkv);
+  // (decode: a session's slices go over all XCDs; with its kv heads spread as well, whose rows share pages, 12 took 47 us;
+  // NB = gridDim.x, as an argument: read as gridDim.x it comes 0.3 us late)
+  const int b = ROPE ? xcd_turn(blockIdx.x, NB, p) : blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, qd = lane >> 4;
   // ROPE (decode): block b is token b (``decode_qblocks``: one token per block, in order), so the
@@ -603,7 +607,7 @@ static void launch_attn_mfma(const void* q, int64_t q_stride, const void* kc, co
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(NB, nh / HB, NP), dim3(256), 0, stream, (const bf16_t*)q, q_stride,
                        (const bf16_t*)kc, (const bf16_t*)vc, bt, bt_stride, q_seq, q_ctx, qb_tok0, qb_ntok,
-                       (bf16_t*)out, ws_o, ws_ml, nkv, nh, page_log2, PS, NP, scale_log2, packed_mt, rf);
+                       (bf16_t*)out, ws_o, ws_ml, nkv, nh, page_log2, PS, NP, NB, scale_log2, packed_mt, rf);
   };
   if (rf.pos && rf.qp.part) go(attn_mfma_kernel<D, HB, true, true>);
   else if (rf.pos) go(attn_mfma_kernel<D, HB, true, false>);

@@ -208,4 +208,14 @@ __device__ __forceinline__ u16x8 qkv_part_load8(const QkvPart& qp, int row, int 
   return qkv_part_finish8(qp, row, col, f, rs);
 }
 
+// Workgroups go to the 8 XCDs in turn, so that in a grid of rows of n, n even, a column meets the XCDs of one residue only:
+// one XCD with n = 8, 16, ...  Where columns are not of one length (sessions, or the slices of a context, the last of which
+// are often empty), some XCDs then read most of the bytes.  xcd_turn gives the work of column ``x`` of a row whose columns
+// are turned by ``by``: for any n and ``by`` an order of all n.
+__host__ __device__ __forceinline__ int xcd_residues(int n) { return (n & 7) == 0 ? 8 : n & -n; }  // n's power of two, up to 8
+__host__ __device__ __forceinline__ int xcd_turn(int x, int n, int by) {
+  const int at = x + (by & (xcd_residues(n) - 1));
+  return at < n ? at : at - n;
+}
+
 }  // namespace mp

@@ -52,6 +52,13 @@ def _attend(q, k, v, weight=None):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,nkv", [(4, 2), (8, 8), (12, 1), (16, 2), (24, 3)])
+def test_every_session_and_slice_is_met(T, nkv):
+    """Grids whose columns (sessions) are turned over the XCDs, with slices that shorter sessions do not have."""
+    test_edges(64, 4 * nkv, nkv, [1 + 37 * t * t % 401 for t in range(T)], 128, True)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("marked", [False, True])
 @pytest.mark.parametrize("D,nh,nkv", SHAPES)
 @pytest.mark.parametrize("ctxs,part", [([1, 31, 32, 33, 64, 65], 128), ([127, 128, 129, 159, 160, 161], 256),

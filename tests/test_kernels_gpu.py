@@ -114,6 +114,16 @@ def test_paged_attention_explicit_partitions(parts):
     torch.testing.assert_close(out.float(), o_ref.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("nh,nkv", [(8, 8), (6, 3)])
+@pytest.mark.parametrize("num_parts", [2, 3, 4, 6, 8, 12, 16])
+def test_paged_attention_every_slice_is_met(num_parts, nh, nkv):
+    """Grids whose columns (slices of a context) are turned over the XCDs; the last slices are empty."""
+    q, kc, vc, bt, q_seq, q_ctx = _attn_case(nh, nkv, 128, [64 * num_parts - 3, 64, 1])
+    out = ops.paged_attention(q, kc, vc, bt, q_seq, q_ctx, nh, nkv, 0.088, part_size=64, num_parts=num_parts)
+    o_ref = ref.paged_attention(q.float(), kc.float(), vc.float(), bt, q_seq, q_ctx, nh, nkv, 0.088)
+    torch.testing.assert_close(out.float(), o_ref.float(), atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("ctxs,parts", [([300, 17, 1, 0], (64, 5)), ([150], (64, 3)), ([4097, 2], (128, 33))])
 def test_paged_attention_inlaunch_combine_equals_reduce_kernel(ctxs, parts, packed, monkeypatch):
