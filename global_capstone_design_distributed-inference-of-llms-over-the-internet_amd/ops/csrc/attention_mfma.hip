@@ -36,10 +36,10 @@
 // the 640 slices of 12 sessions of 1.7k to 5.8k tokens (32 / 8 heads) run at once - 45 us for 184 MB
 // where 2 to a CU took 58 in a full round and a quarter one; 64 sessions up to 512: 25.0 -> 20.6 us,
 // one of 900: 12.3 -> 10.1.  A grid column was a session on one XCD, some XCDs with two of the 12: slices turned over
-// all XCDs take 43 us instead of 47 in a whole step; 1, 2, 20 and 64 sessions take as long as before.
-// (K/V loads keep the default cache policy here: non-temporal loads, a win for the MHA decode
-// kernel in attention.hip, measured 12-14 % SLOWER on this kernel at 64 / 256 sessions, cold
-// caches - profiles/r3_i/attn_nt.jsonl vs attn_def.jsonl.)
+// all XCDs take 43 us instead of 47 in a whole step (and 37.6 with FAR); 1, 2, 20 and 64 sessions as long as before.
+// FAR: values are loaded past the caches, so that they leave L2 to the keys, whose rows a wave reads as halves of lines, two
+// instructions a line.  Keys stay cached: with both past the caches 12 sessions take 43 us, as with neither, and 64 short ones
+// 22.7 instead of 18.4.
 #include "common.h"
 #include "mx_common.h"
 
@@ -78,7 +78,7 @@ constexpr int VT_PITCH = 36;  // bf16 per LDS row of the transposed V tile (32 t
 // compile-time choice: as a run-time one the LDS-or-global q / k / v loads compiled to flat
 // loads, which count against vmcnt, so the RoPE prologue waited for the K / V stream issued
 // before them.
-template <int D, int HB, bool ROPE, bool FOLD = false>
+template <int D, int HB, bool ROPE, bool FOLD = false, bool FAR = false>
 __global__ __launch_bounds__(256, 3) void attn_mfma_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int bt_stride, const int32_t* __restrict__ q_seq,
@@ -136,7 +136,10 @@ __global__ __launch_bounds__(256, 3) void attn_mfma_kernel(
     asm volatile("" : "+v"(vlane));  // (two offsets formed at each use instead of held)
     vlane *= 8;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) vr[i] = *reinterpret_cast<const u16x8*>(vpage + (i & 3) * 512 + (vlane + (i >> 2) * 2048));
+    for (int i = 0; i < NV; ++i) {
+      const u16x8* from = reinterpret_cast<const u16x8*>(vpage + (i & 3) * 512 + (vlane + (i >> 2) * 2048));
+      vr[i] = FAR ? __builtin_nontemporal_load(from) : *from;
+    }
   };
   f32x4 o[DT];
 #pragma unroll
@@ -609,8 +612,13 @@ static void launch_attn_mfma(const void* q, int64_t q_stride, const void* kc, co
                        (const bf16_t*)kc, (const bf16_t*)vc, bt, bt_stride, q_seq, q_ctx, qb_tok0, qb_ntok,
                        (bf16_t*)out, ws_o, ws_ml, nkv, nh, page_log2, PS, NP, NB, scale_log2, packed_mt, rf);
   };
-  if (rf.pos && rf.qp.part) go(attn_mfma_kernel<D, HB, true, true>);
-  else if (rf.pos) go(attn_mfma_kernel<D, HB, true, false>);
+  // Slices of 512 tokens on (4 steps a wave): values past the caches, see above.  Both forms, us: 12 sessions of 1500 to 6000
+  // tokens (slices of 1024) 43.5 -> 37.6, 32 of 700 to 2200 (1024) 41.3 -> 35.8, 64 of 500 to 1000 (512) 42.8 -> 35.7, 8 of
+  // 1500 to 6000 (512) 26.6 -> 26.2; shorter slices, few steps that wait for each load: 48 of 300 to 700 (384) 21.0 -> 21.9,
+  // 4 of 2000 to 6000 (256) 16.0 -> 16.8, 64 of 100 to 512 (256) 18.4 -> 19.4.
+  const bool far = PS >= 512;
+  if (rf.pos && rf.qp.part) far ? go(attn_mfma_kernel<D, HB, true, true, true>) : go(attn_mfma_kernel<D, HB, true, true>);
+  else if (rf.pos) far ? go(attn_mfma_kernel<D, HB, true, false, true>) : go(attn_mfma_kernel<D, HB, true, false>);
   else go(attn_mfma_kernel<D, HB, false, false>);
 }
 

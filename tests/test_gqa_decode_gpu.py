@@ -62,7 +62,8 @@ def test_every_session_and_slice_is_met(T, nkv):
 @pytest.mark.parametrize("marked", [False, True])
 @pytest.mark.parametrize("D,nh,nkv", SHAPES)
 @pytest.mark.parametrize("ctxs,part", [([1, 31, 32, 33, 64, 65], 128), ([127, 128, 129, 159, 160, 161], 256),
-                                       ([1, 96, 511, 640, 900], 128), ([1, 2300], 256), ([40, 8197], 128)])
+                                       ([1, 96, 511, 640, 900], 128), ([1, 2300], 256), ([40, 8197], 128),
+                                       ([1, 97, 511, 512, 513, 640, 1153, 2300], 512)])
 def test_edges(D, nh, nkv, ctxs, part, marked):
     """Slices past a context, waves without a step, tails of a step, 1 to 65 slices; the cache past each context is NaN."""
     ops.require_native()
