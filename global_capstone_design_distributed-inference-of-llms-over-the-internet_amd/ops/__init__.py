@@ -236,9 +236,12 @@ _TUNE_POOL_BYTES = 1 << 30
 # Committed decode-kernel table (ops/tuned/decode_kernels_gfx950.json, written by
 # ``python -m src.ops.tune`` on an MI355X): the autotuners' per-shape choices and the
 # executors' end-to-end qkv-fold decisions.  Loaded by default, so two boxes running the same
-# tree run the same kernel mix (a start-up timing race used to pick a different kernel for 4 of
-# 35 Llama-2-7B shapes from box to box).  ``MPAMD_GEMM_AUTOTUNE``: "1" (default) times only
-# shapes the table lacks, "0" never times (untabled shapes take the first kernel), "force"
+# tree run the same kernel mix.  It holds every product of every preset: a start-up timing race
+# picked other kernels for 58 of 197 of them in three processes, and the kernel is the order of
+# the sums (an fp8 Llama-3-8B batch: logits 0.0035 apart and an eighth of the sampled tokens
+# others from one process to the next).  ``MPAMD_GEMM_AUTOTUNE``: "1" (default) times only
+# shapes the table lacks (a model of one's own: its last bits may change with the process;
+# ``python -m src.ops.tune --missing`` adds a preset's), "0" never times (untabled shapes take the first kernel), "force"
 # re-times every shape an executor uses.  ``MPAMD_KERNEL_TABLE``: another table, or "0" for none.
 KERNEL_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "decode_kernels_gfx950.json")
 _QKV_FOLD_PIN = {}  # (graph batch bucket, N, K, fp8) -> bool: the decode-graph A/B's decision
@@ -309,6 +312,15 @@ def load_kernel_table(path: Optional[str] = None) -> Optional[str]:
     _TABLE["file_sha"] = kernel_table_sha(
         {k: t.get(k, {}) for k in ("gemm", "w8", "fp8", "qkv_fold_cand", "qkv_fold")} | {"arch": "gfx950"})
     return _TABLE["file_sha"]
+
+
+def set_kernel_table(t: dict) -> None:
+    """These choices and no others (what was timed so far in this process is forgotten)."""
+    for name, dst in (("gemm", _SK_CHOICE), ("w8", _W8_CHOICE), ("fp8", _FP8_CHOICE), ("qkv_fold_cand", _QKV_FOLD_CAND),
+                      ("qkv_fold", _QKV_FOLD_PIN)):
+        dst.clear()
+        dst.update({_parse_key(s): v for s, v in t.get(name, {}).items()})
+    _TABLE["runtime"].clear()
 
 
 def save_kernel_table(path: str) -> str:

@@ -11,16 +11,120 @@ per (row bucket, N, K, epilogue) and one fold decision per (graph batch bucket, 
 written as JSON.  Executors load that file by default, so every box running the tree runs the
 same kernel mix (``ops.load_kernel_table``) and bench records carry its sha.
 
+``--missing N`` adds what the table lacks, and changes nothing that it has: every decode product that some preset
+(of ``--models``, default all, fp8 forms among them) would time at start-up, in N processes, and the folds of the Llama presets'
+decode batches; the choice that won most often enters.  One such race is not enough: of 197 products, three processes
+agreed on 139.  With every choice in the table, two processes give the same bits.
+
 ``--prompt`` writes the table of prompt products (``ops.prompt.TABLE``) instead: every projection of every preset, both
 kernels timed over the row-tile counts of steps of 257 to 8192 rows, twice; a count enters where both sweeps agree.
 """
 from __future__ import annotations
 
 import argparse
+import collections
+import dataclasses
 import gc
 import os
+import subprocess
 import sys
+import tempfile
 import time
+
+
+def every_spec() -> list:
+    """Every preset that decodes with packed weights, and the fp8 form of those that have one."""
+    from ..models.config import PRESETS
+
+    names = [n for n, c in PRESETS.items() if c.model_type != "gpt2"]
+    return names + [n + ":fp8" for n in names if not PRESETS[n].hybrid and not PRESETS[n].is_moe]
+
+
+def stage(spec: str, whole: bool, batch: int = 4, device="cuda"):
+    """An executor over the whole preset, or over one block of each kind that it has with its embedding and head: all its
+    products."""
+    from ..models.config import resolve_model
+    from ..models.weights import random_stage_weights
+    from ..runtime.executor import StageExecutor
+
+    name, _, opt = spec.partition(":")
+    cfg = resolve_model(name)
+    n = cfg.num_hidden_layers
+    if not whole:
+        layers = tuple(dict.fromkeys(cfg.layers)) if cfg.hybrid else ()
+        n = len(layers) or 1
+        cfg = dataclasses.replace(cfg, layers=layers, num_hidden_layers=n) if cfg.hybrid else cfg
+    w = random_stage_weights(cfg, 0, n, has_embed=True, has_head=True, device=device, seed=0, fp8=opt == "fp8")
+    return StageExecutor(cfg, w, device, max_sessions=batch + 8, max_seq_len=512, kv_cache_bytes=8 << 30, graph_max_batch=64,
+                         max_tokens_per_step=max(8192, 128 * batch), warmup=False)
+
+
+def elect(sweeps) -> dict:
+    """One table of several: each entry's most frequent value (of equals, the one that came first)."""
+    out = {}
+    for part in {p: None for t in sweeps for p in t if isinstance(t[p], dict)}:
+        out[part] = {k: collections.Counter(t[part][k] for t in sweeps if k in t[part]).most_common(1)[0][0]
+                     for k in sorted({k for t in sweeps for k in t.get(part, {})})}
+    return out
+
+
+def tune_missing(specs, batches, out=None) -> int:
+    """This process' choices for the products that the table lacks, or (``batches``) for the folds of whole models."""
+    import torch
+
+    from .. import ops
+
+    if not torch.cuda.is_available():
+        print("tune: needs an MI355X", file=sys.stderr)
+        return 2
+    os.environ["MPAMD_GEMM_AUTOTUNE"] = "1"
+    ops.load_kernel_table()
+    for spec in specs:
+        ex = stage(spec, bool(batches), max(batches, default=4))
+        for b in batches:
+            ex.warmup_serving(b, 128)
+        del ex
+        gc.collect()
+        torch.cuda.empty_cache()
+    print(f"tune: {','.join(specs)}: {len(ops.kernel_table_report()['tuned_at_runtime'])} products timed", flush=True)
+    ops.save_kernel_table(out)
+    return 0
+
+
+def tune_missing_often(specs, sweeps: int, batches, out=None) -> int:
+    """``tune_missing`` in ``sweeps`` processes for each preset, as each start of a server is one: inside one process later races
+    are won by others (of 4-row products of 16512 x 4096, 'pk' won all of three processes' and 6 of 15 in one)."""
+    import json
+
+    from .. import ops
+
+    out = out or ops.KERNEL_TABLE
+    ops.load_kernel_table()
+    folds = [s for s in specs if s.split(":")[0] in ("llama2-7b", "llama3-8b", "llama3-70b")]
+    with tempfile.TemporaryDirectory() as tmp:
+        for todo, more in ((specs, []), (folds, ["--batches", ",".join(map(str, batches))])):
+            base, got = ops.kernel_table(), []
+            for spec in todo:
+                for _ in range(sweeps):
+                    path = os.path.join(tmp, "t.json")
+                    subprocess.run([sys.executable, "-m", __spec__.name, "--missing", "1", "--models", spec, "--out", path, *more],
+                                   check=True)
+                    with open(path) as f:
+                        t = json.load(f)
+                    if t == base:
+                        break  # nothing to time
+                    got.append(t)
+            t = elect([base] + got)
+            for p in t:
+                for k in t[p]:
+                    votes = collections.Counter(g[p][k] for g in got if k in g[p])
+                    if len(votes) > 1:
+                        print(f"tune: {p} {k}: {dict(votes)}", flush=True)
+            ops.set_kernel_table(t)
+            sha = ops.save_kernel_table(out)
+            os.environ["MPAMD_KERNEL_TABLE"] = out
+    print(f"tune: wrote {out} (sha {sha})", flush=True)
+    return 0
 
 
 def tune_prompt(out=None) -> int:
@@ -39,15 +143,21 @@ def tune_prompt(out=None) -> int:
 
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description=__doc__.split("\n\n")[0])
-    ap.add_argument("--models", default="small-llama,tiny-llama,llama2-7b,llama3-8b,llama3-70b:fp8",
-                    help="comma-separated presets; ':fp8' = fp8 (W8A16) projection weights")
-    ap.add_argument("--batches", default="64", help="decode batches whose qkv-fold A/B is pinned")
+    ap.add_argument("--models", default=None, help="comma-separated presets; ':fp8' = fp8 (W8A16) projection weights; "
+                    "default: small-llama,tiny-llama,llama2-7b,llama3-8b,llama3-70b:fp8, or all with --missing")
+    ap.add_argument("--batches", default=None, help="decode batches whose qkv-fold A/B is pinned (64; 24,32,48,64 with --missing)")
     ap.add_argument("--prompt-len", type=int, default=128)
     ap.add_argument("--out", default=None, help="default: the committed table path")
     ap.add_argument("--prompt", action="store_true", help="time the prompt products of every preset")
+    ap.add_argument("--missing", type=int, default=0, metavar="N", help="add what the table lacks, by N processes")
     a = ap.parse_args(argv)
     if a.prompt:
         return tune_prompt(a.out)
+    batches = [int(b) for b in (a.batches or "").split(",") if b]
+    if a.missing:
+        specs = [m for m in (a.models or "").split(",") if m] or every_spec()
+        return tune_missing(specs, batches, a.out) if a.missing == 1 else \
+            tune_missing_often(specs, a.missing, batches or [24, 32, 48, 64], a.out)
     os.environ["MPAMD_KERNEL_TABLE"] = "0"   # time everything: nothing pre-loaded
     os.environ.setdefault("MPAMD_GEMM_AUTOTUNE", "1")
     import torch
@@ -60,8 +170,8 @@ def main(argv=None) -> int:
     if not torch.cuda.is_available():
         print("tune: needs an MI355X", file=sys.stderr)
         return 2
-    batches = [int(b) for b in a.batches.split(",") if b]
-    for spec in [m for m in a.models.split(",") if m]:
+    batches = batches or [64]
+    for spec in [m for m in (a.models or "small-llama,tiny-llama,llama2-7b,llama3-8b,llama3-70b:fp8").split(",") if m]:
         name, _, opt = spec.partition(":")
         cfg = resolve_model(name)
         t0 = time.time()
