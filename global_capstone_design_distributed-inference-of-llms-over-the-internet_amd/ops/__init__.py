@@ -231,6 +231,7 @@ def _use_sk(M: int, N: int, K: int, epilogue: int) -> bool:
 
 
 _TUNE_POOL_BYTES = 1 << 30
+TUNE_ROUNDS = 3  # of an autotuner that is not told (``tune --missing``: more)
 
 # ---------------------------------------------------------------------------------------
 # Committed decode-kernel table (ops/tuned/decode_kernels_gfx950.json, written by
@@ -365,7 +366,7 @@ def pin_qkv_fold(bucket: int, N: int, K: int, fp8: bool, fold: bool) -> None:
     _QKV_FOLD_PIN[(int(bucket), int(N), int(K), bool(fp8))] = bool(fold)
 
 
-def autotune_gemm(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 24, rounds: int = 3) -> dict:
+def autotune_gemm(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 24, rounds: Optional[int] = None) -> dict:
     """Time every applicable decode-GEMM kernel (one-group, stream-K, shared-A variants) on each
     (N, K, epilogue) for each M bucket and record the fastest for ``linear``.  Returns the table.
 
@@ -414,7 +415,7 @@ def autotune_gemm(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 24, round
                                  ss_out=norm_stats_buffer(device)[0], ss_zero=norm_stats_buffer(device)[0])
                 out = y if epi in (1, 4) else (res if epi == 3 else y.view(M, ncols))
                 t = {k: float("inf") for k in cands}
-                for _ in range(rounds):
+                for _ in range(rounds or TUNE_ROUNDS):
                     for mode in cands:
                         _GEMM_SK = mode
                         for i in range(2):
@@ -433,7 +434,7 @@ def autotune_gemm(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 24, round
                 best = best if t[best] < 0.97 * t["pk"] else "pk"
                 # then the same kernel with the rotated k walk, kept if it wins by > 1 %
                 tr = {best: float("inf"), best + "+r": float("inf")}
-                for _ in range(rounds):
+                for _ in range(rounds or TUNE_ROUNDS):
                     for mode in tr:
                         _GEMM_SK = mode
                         for i in range(2):
@@ -1130,7 +1131,7 @@ def linear_partials(x, M: int, wp=None, w8=None, w_scale=None, out=None, rot: bo
 
 
 def autotune_qkv_fold(N: int, K: int, device, fp8: bool = False, ms=(16, 32, 48, 64), iters: int = 24,
-                      rounds: int = 3) -> dict:
+                      rounds: Optional[int] = None) -> dict:
     """Per M bucket: the qkv GEMM as partial slabs (no reduce launch) vs the kernel the GEMM
     autotuner chose for the full projection; the fold is kept where it wins by > 3 %.  Weights
     rotated over ~1 GiB of copies, as in ``autotune_gemm``."""
@@ -1169,7 +1170,7 @@ def autotune_qkv_fold(N: int, K: int, device, fp8: bool = False, ms=(16, 32, 48,
                 linear_partials(xp, M, wp=ws[i % copies], out=y)
 
         t = {"full": float("inf"), "part": float("inf")}
-        for _ in range(rounds):
+        for _ in range(rounds or TUNE_ROUNDS):
             for name, fn in (("full", full), ("part", part)):
                 for i in range(2):
                     fn(i)
@@ -1260,7 +1261,7 @@ def _fp8_kind(M: int, N: int, K: int, epilogue: int) -> int:
     return -1 if name is None else _FP8_KERNELS[name]
 
 
-def autotune_fp8(shapes, device, ms=(32, 48, 64), iters: int = 12, rounds: int = 3) -> dict:
+def autotune_fp8(shapes, device, ms=(32, 48, 64), iters: int = 12, rounds: Optional[int] = None) -> dict:
     """``autotune_gemm`` for the fp8 GEMM: time both forms on each (N, K, epilogue) per M bucket
     (M <= 16 always runs the one-group form) on weights rotated over ~1 GiB, keep the faster."""
     global _FP8_MODE
@@ -1285,7 +1286,7 @@ def autotune_fp8(shapes, device, ms=(32, 48, 64), iters: int = 12, rounds: int =
                 asc = torch.ones(((M + 15) // 16) * 16, dtype=torch.float32, device=device)
                 out = torch.empty(M, ncols, dtype=torch.bfloat16, device=device)
                 t = {k: float("inf") for k in _FP8_KERNELS}
-                for _ in range(rounds):
+                for _ in range(rounds or TUNE_ROUNDS):
                     for name in _FP8_KERNELS:
                         _FP8_MODE = name
                         for i in range(2):
@@ -1433,7 +1434,7 @@ def linear_mx(ax, as_, w8, w_scale, a_rows: int, out=None, epilogue: int = 0, re
     return out
 
 
-def autotune_w8(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 12, rounds: int = 3) -> dict:
+def autotune_w8(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 12, rounds: Optional[int] = None) -> dict:
     """``autotune_gemm`` for the W8A16 GEMM: ring vs split-K ring per (N, K, epilogue) and M
     bucket, on fp8 weights rotated over ~1 GiB (decode never finds them in the Infinity Cache)."""
     global _W8_MODE
@@ -1468,7 +1469,7 @@ def autotune_w8(shapes, device, ms=(4, 16, 32, 48, 64), iters: int = 12, rounds:
                     torch.empty(packed_numel(M, ncols), dtype=torch.bfloat16, device=device) if epi == 1
                     else torch.empty(M, N, dtype=torch.bfloat16, device=device))
                 t = {k: float("inf") for k in names}
-                for _ in range(rounds):
+                for _ in range(rounds or TUNE_ROUNDS):
                     for name in names:
                         _W8_MODE = name
                         for i in range(2):
