@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from src import ops
+from src.models.config import MoESpec
 from src.ops import moe
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +127,43 @@ def test_tiles_of_the_last_round_in_halves(counts, N, K):
         want = x[at:at + n].float() @ w[e].float().t()
         assert n == 0 or float((out[at:at + n].float() - want).norm() / want.norm()) < 2.0 ** -8
         at += n
+
+
+@pytest.mark.parametrize("T,W,ff", [(2700, 4096, 4096), (600, 256, 2048)])
+def test_the_same_prompt_has_the_same_bits(T, W, ff):
+    """Tiles that are cut in K hold the same rows in each pass: an expert's rows lie in the order of their tokens."""
+    ops.require_native()
+    E, g = 8, torch.Generator(device="cuda").manual_seed(T)
+    draw = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    x, router = draw(T, W).to(torch.bfloat16), draw(E, W).div(W ** 0.5).to(torch.bfloat16)
+    up, down = (torch.stack([ops.pack_weight(m) for m in draw(E, *s).div(s[1] ** 0.5).to(torch.bfloat16)])
+                for s in ((2 * ff, W), (W, ff)))
+    spec, ctx = MoESpec(E, 2, ff, 0.0), torch.ones(T, dtype=torch.int32, device="cuda")
+    assert moe.expert_form(2 * T, E, False) == 3
+
+    def mlp():
+        e = lambda name, shape, dtype=torch.bfloat16: torch.empty(shape, dtype=dtype, device="cuda")  # noqa: E731
+        return moe.mixtral_mlp(x, ctx, router, up, down, spec, torch.empty_like(x), e)
+
+    out = mlp()
+    for _ in range(5):
+        assert torch.equal(mlp(), out)
+
+
+@pytest.mark.parametrize("T,E,top", [(17, 5, 2), (300, 64, 64), (511, 8, 2), (512, 8, 2), (1024, 65, 8), (4100, 512, 4), (9000, 3, 1)])
+def test_rows_in_the_order_of_their_tokens(T, E, top):
+    """Choices up to the ends of a wave's 64, of its share that stays in registers (512) and past it; rows without a choice."""
+    ops.require_native()
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(T, 64, generator=g).to(torch.bfloat16), torch.randn(E, 64, generator=g).to(torch.bfloat16)
+    ctx = (torch.rand(T, generator=g) < 0.9).to(torch.int32)
+    e = lambda name, shape, dtype=torch.bfloat16: torch.full(shape, -7, dtype=dtype, device="cuda")  # noqa: E731
+    c = moe.choose(x.cuda(), w.cuda(), ctx.cuda(), MoESpec(E, top, 64, 1.0), e)
+    lists, slot, tok = c.lists.tolist(), c.slot.cpu(), c.tok.tolist()
+    counts, off = lists[:E], lists[E:2 * E + 1]
+    assert off == [sum(counts[:i]) for i in range(E + 1)] and off[E] == int(ctx.sum()) * top
+    assert lists[3 * E + 1] == sum(n > 0 for n in counts)
+    assert [tok[r] for r in slot[ctx > 0].flatten().tolist()] == [t for t in range(T) if ctx[t] for _ in range(top)]
+    assert bool((slot[ctx == 0] == -1).all())
+    for a, b in zip(off, off[1:]):
+        assert tok[a:b] == sorted(set(tok[a:b]))
