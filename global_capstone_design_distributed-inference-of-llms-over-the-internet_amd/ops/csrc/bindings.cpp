@@ -5,7 +5,9 @@
 // dtype checks happen here, on the host, before any kernel sees a pointer.
 #include <c10/hip/HIPGuard.h>
 #include <ATen/ATen.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/HIPContext.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
 
 #include <cmath>
@@ -476,10 +478,17 @@ void add(const at::Tensor& a, const at::Tensor& b, at::Tensor& y) {
   check_launch(mp_add(a.data_ptr(), b.data_ptr(), y.data_ptr(), a.numel(), cur_stream()), "add");
 }
 
+// Tells torch's allocator of pinned memory that work on the current stream reads ``host``, as a copy of torch's own does: a block
+// that is let go of is handed out again only when that work is done.  False: memory of another kind.
+bool reads_pinned(const at::Tensor& host) {
+  return at::getHostAllocator(at::kCUDA)->record_event(host.data_ptr(), host.storage().data_ptr().get_context(),
+                                                       c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+}
+
 // meta <- host (pinned bytes); the front of dst <- x, where there is one
 void step_input(const at::Tensor& host, at::Tensor& meta, const c10::optional<at::Tensor>& x, at::Tensor& dst) {
   auto word = [](const at::Tensor& t) { return t.is_contiguous() && (t.nbytes() | reinterpret_cast<uintptr_t>(t.data_ptr())) % 8 == 0; };
-  MP_CHECK(host.device().is_cpu() && host.is_pinned() && word(host), "host: pinned, words of 8 bytes");
+  MP_CHECK(host.device().is_cpu() && word(host), "host: words of 8 bytes");
   MP_CHECK(meta.is_cuda() && word(meta) && meta.nbytes() == host.nbytes() && meta.nbytes() < (1u << 30), "meta");
   int64_t nx = 0;
   if (x.has_value()) {
@@ -490,6 +499,7 @@ void step_input(const at::Tensor& host, at::Tensor& meta, const c10::optional<at
     nx = x->nbytes() / 8;
   }
   const c10::hip::HIPGuard guard(meta.device().index());
+  MP_CHECK(reads_pinned(host) || host.is_pinned(), "host: pinned");
   check_launch(mp_step_input((const uint64_t*)host.data_ptr(), (uint64_t*)meta.data_ptr(), meta.nbytes() / 8,
                              nx ? (const uint64_t*)x->data_ptr() : nullptr, (uint64_t*)dst.data_ptr(), nx, cur_stream()),
                "step_input");

@@ -92,6 +92,28 @@ def test_step_input(rows, width, dtype):
         ops.step_input(host.clone(), meta, None, dst)
 
 
+def test_step_input_keeps_its_memory():
+    """Pinned memory that is let go of while a queued step has still to read it is not handed out before the step has."""
+    from src import ops
+
+    ops.require_native()
+    n = 16 * 28 * 64
+    meta, dst = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.zeros(1, dtype=torch.long, device="cuda")
+    ring = torch.randint(0, 200, (2, n), dtype=torch.uint8).pin_memory()
+    want, at = ring[1].clone(), ring.data_ptr()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)
+    ops.step_input(ring[1], meta, None, dst)
+    read = torch.cuda.Event()
+    read.record()
+    del ring
+    other = [torch.full((2, n), 255, dtype=torch.uint8).pin_memory() for _ in range(3)]
+    assert not read.query()  # (10 ms and more of queued work)
+    assert all(t.data_ptr() != at for t in other)
+    torch.cuda.synchronize()
+    assert torch.equal(meta.cpu(), want)
+
+
 def test_steps_ahead_of_the_device():
     """More steps than staging blobs, none waited for: the logits of steps that were."""
     cfg = resolve_model("small-llama")
