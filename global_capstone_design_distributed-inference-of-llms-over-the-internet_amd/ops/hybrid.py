@@ -94,7 +94,9 @@ CHUNK_MAX = 256
 
 
 # tokens that a segment's start (its state arrives) and a segment's slot (read and written between the two passes) cost, and
-# what the pass over the segments' own contributions adds to a step that has any
+# what the pass over the segments' own contributions adds to a step that has any.  20 steps of 1 to 31 sequences, 270 to 8192
+# tokens, in retention (32 heads of 128 x 128), mLSTM (16 of 256 x 256) and HGRN2 (32 of 128 x 128): 1.03 of the time of the
+# best length on average, 1.12 at most; lengths of a 16th or a 32nd of the step 1.14 and 2.5
 SEG_START, SEG_SLOT, SEG_CUT = 32, 3, 0.35
 
 

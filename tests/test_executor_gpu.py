@@ -114,19 +114,41 @@ def test_step_input_keeps_its_memory():
     assert torch.equal(meta.cpu(), want)
 
 
+class _Waited:
+    """An event that notes whether it was waited for while it was still to come."""
+
+    def __init__(self, event, seen):
+        self.event, self.seen = event, seen
+
+    def synchronize(self):
+        self.seen.append(not self.event.query())
+        self.event.synchronize()
+
+
 def test_steps_ahead_of_the_device():
-    """More steps than staging blobs, none waited for: the logits of steps that were."""
+    """Many more steps than staging blobs, queued behind other work and none waited for, each of other sessions in another order:
+    the logits of steps that were.  A blob is filled again only when the half of the ring that it is in has been read."""
     cfg = resolve_model("small-llama")
     w = random_stage_weights(cfg, 0, cfg.num_hidden_layers, has_embed=True, has_head=True, device="cuda", seed=5)
-    outs = []
+    steps, lens = 240, [20, 3, 47, 31, 8]
+    who = [[(k * m + i) % 5 for i in range(3)] for k in range(steps) for m in (1 + k % 4,)]
+    toks = torch.randint(0, cfg.vocab_size, (steps, 3), device="cuda")
+    ids = torch.randint(0, cfg.vocab_size, (sum(lens),), device="cuda")
+    outs, seen = [], []
     for wait in (True, False):
-        ex = StageExecutor(cfg, w, "cuda", kv_cache_bytes=128 << 20, max_sessions=4, max_seq_len=512)
-        ids = torch.arange(3 * 20, device="cuda").view(3, 20) % cfg.vocab_size
-        ex.forward([(f"s{i}", 20) for i in range(3)], ids.view(-1))
-        res = []
-        for k in range(41):
-            res.append(ex.forward([(f"s{i}", 1) for i in range(3)], torch.tensor([1, 2, 3], device="cuda") + k).clone())
+        ex = StageExecutor(cfg, w, "cuda", kv_cache_bytes=128 << 20, max_sessions=8, max_seq_len=512, warmup=False)
+        ex.forward([(f"s{i}", n) for i, n in enumerate(lens)], ids)
+        res = torch.empty(steps, 3, cfg.vocab_size, dtype=torch.bfloat16, device="cuda")
+        torch.cuda.synchronize()
+        for k in range(steps):
+            if not wait and k % 40 == 1:
+                torch.cuda._sleep(10_000_000)
+            res[k].copy_(ex.forward([(f"s{i}", 1) for i in who[k]], toks[k]))
             if wait:
                 torch.cuda.synchronize()
-        outs.append(torch.stack(res))
+                continue
+            for g in ex._graphs.values():
+                g._half_ev = [_Waited(e, seen) if isinstance(e, torch.cuda.Event) else e for e in g._half_ev]
+        outs.append(res)
     assert torch.equal(*outs)
+    assert len(ex._graphs) == 1 and len(seen) == steps // 8 - 2 and sum(seen) >= 6

@@ -57,6 +57,31 @@ def test_left_over_tiles_in_parts(M, N, K):
         assert float((prompt.gemm(x, w, None, epi).double() - r).norm() / r.norm()) < BF16
 
 
+# more tiles than workgroups (256): a ring of five slots runs on into the next tile, of 1, 3 and 32 stages; last tiles of 18 rows
+# or of 3, whose other waves have none; whole tiles alone, and one with a part behind it
+MANY = [(1554, 14352, 64), (1554, 14336, 192), (1554, 14336, 2048), (4100, 4096, 2048), (4099, 4112, 2048), (8195, 4096, 128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", MANY)
+def test_several_tiles_to_a_workgroup(M, N, K):
+    ops.require_native()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    for epi in (0, 1, 4, prompt.COLUMNS):
+        if epi == 1 and N % 32:
+            continue
+        out = torch.full((M, N // 2 if epi == 1 else N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        v = w.t().contiguous() if epi == prompt.COLUMNS else w
+        prompt._run(x, v, out, N, epi)
+        want = z if epi == prompt.COLUMNS else _want(z, epi, 0.0)
+        assert float((out.double() - want).norm() / want.norm()) < BF16
+        again = torch.empty_like(out)
+        assert torch.equal(out, prompt._run(x, v, again, N, epi))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
 def test_products_with_columns(M, N, K):

@@ -66,6 +66,9 @@ def test_batch_sampler_calls_in_flight(dev):
     s = BatchSampler(dev, max_rows=24)
     steps = [_batch(n, 700, k) for k, n in enumerate((24, 1, 7, 24, 60, 3, 24, 2))]
     lgs = [lg.to(dev) for lg, *_ in steps]
+    if dev == "cuda":  # (the device has not begun with the first call when the second buffer is filled)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)
     got = [s(lg, *rest) for lg, (_, *rest) in zip(lgs, steps)]
     for lg, g, (_, *rest) in zip(lgs, got, steps):
         assert torch.equal(g.cpu(), torch.cat([_one_by_one(lg[i:i + 24], *[r[i:i + 24] for r in rest])
@@ -73,14 +76,22 @@ def test_batch_sampler_calls_in_flight(dev):
 
 
 @pytest.mark.gpu
-def test_batch_sampler_on_several_streams():
-    s, (lg, *rest) = BatchSampler("cuda"), _batch(64, 32000, 1)
-    lg = lg.cuda()
-    want = s(lg, *rest)
+@pytest.mark.parametrize("V", [32000, 50000, 70000])
+def test_batch_sampler_on_several_streams(V, monkeypatch):
+    """Rows in LDS, in the workspace and in its records: the workspace is one for all streams, so that a call waits for the one
+    before it.  Each call has its own logits, parameters, histories and seeds."""
+    s = BatchSampler("cuda", max_rows=48)
+    steps = [_batch(n, V, k) for k, n in enumerate((48, 31, 48, 48, 7, 48))]
+    lgs = [lg.cuda() for lg, *_ in steps]
+    want = [_one_by_one(lg, *rest) for lg, (_, *rest) in zip(lgs, steps)]
     torch.cuda.synchronize()
+    waited, wait = [], torch.cuda.Stream.wait_event
+    monkeypatch.setattr(torch.cuda.Stream, "wait_event", lambda st, ev: (waited.append(not ev.query()), wait(st, ev))[1])
     got = []
-    for st in [torch.cuda.Stream() for _ in range(3)] * 2:
+    for st, lg, (_, *rest) in zip([torch.cuda.Stream() for _ in range(3)] * 2, lgs, steps):
         with torch.cuda.stream(st):
+            torch.cuda._sleep(5_000_000)  # (two calls' streams are busy at once)
             got.append(s(lg, *rest))
     torch.cuda.synchronize()
-    assert all(torch.equal(g, want) for g in got)
+    assert len(waited) == 5 and any(waited)
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
