@@ -24,13 +24,8 @@ def rows_ok(B: int, T: int) -> bool:
     return 1 <= B <= 65535 and 1 <= T <= 1 << 24
 
 
-def angle_table(cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
-    """[T, D]: cos, then sin of every position's angles."""
-    return torch.cat([cos, sin], 1).contiguous()
-
-
 def angles(inv: torch.Tensor, T: int) -> torch.Tensor:
-    """``angle_table`` of T positions from the angles ``inv`` [D / 2] (fp64, on the device) of one step."""
+    """[T, D]: cos, then sin of every position's angles, from those of one step, ``inv`` [D / 2] (fp64, on the device)."""
     out = torch.empty(T, 2 * inv.numel(), dtype=torch.float32, device=inv.device)
     torch.ops.mpamd.train_angles(inv, out)
     return out

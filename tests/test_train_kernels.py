@@ -46,7 +46,7 @@ def test_angles(T, D):
     ops.require_native()
     scaling = {"rope_type": "llama3", "factor": 8.0, "original_max_position_embeddings": 8192} if T == 2 else None
     got = train.angles(rope_inv(D, 500000.0, scaling).cuda(), T).cpu()
-    want = train.angle_table(*rope_cos_sin(D, T, 500000.0, None, scaling))
+    want = torch.cat(rope_cos_sin(D, T, 500000.0, None, scaling), 1)
     assert float((got != want).float().mean()) < 1e-4 and float((got - want).abs().max()) <= 2.0 ** -24
 
 
@@ -65,7 +65,7 @@ def test_attention_and_its_gradient(T, nh, nkv, D):
     do = torch.randn(B * T, nh * D, generator=gen).to(torch.bfloat16)
     f = 10000.0 ** (-torch.arange(0, D, 2, dtype=torch.float64) / D)
     a = torch.arange(T, dtype=torch.float64)[:, None] * f
-    table = train.angle_table(a.cos().float(), a.sin().float()).cuda()
+    table = torch.cat([a.cos(), a.sin()], 1).float().cuda()
     qkv = train.rope_(x.cuda(), table, nh + nkv, D)
     w = x.double().view(B, T, -1, D)
     turned = torch.cat([_turn(w[:, :, :nh + nkv], T, D), w[:, :, nh + nkv:]], 2).reshape(B * T, -1)
