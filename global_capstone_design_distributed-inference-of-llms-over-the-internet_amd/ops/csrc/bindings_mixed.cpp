@@ -27,7 +27,7 @@ int64_t mp_moe_lists(int E);
 int mp_moe_router_splits(int T, int W, int E, int f32);
 int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, const int32_t* ctx, float* part, int S, float* ew,
                  int32_t* idx, int32_t* slot, int32_t* lists, int32_t* tok, int T, int E, int W, int top, int groups,
-                 int keep, float scale, int f32, hipStream_t stream);
+                 int keep, float scale, int f32, int ordered, hipStream_t stream);
 int mp_moe_combine(const void* y, int f32, const float* ew, const int32_t* slot, void* out, int64_t T, int top, int H,
                    hipStream_t stream);
 int64_t mp_moe_gemm_ws(int form, int K);
@@ -195,7 +195,7 @@ int act_rows(const at::Tensor& x, int64_t T, int64_t W, int64_t packed, int f32,
 
 void moe_route(const at::Tensor& x, const at::Tensor& w, const at::Tensor& ctx, at::Tensor& part, at::Tensor& ew,
                at::Tensor& idx, at::Tensor& slot, at::Tensor& lists, at::Tensor& tok, int64_t groups, int64_t keep,
-               double scale, int64_t packed) {
+               double scale, int64_t packed, bool ordered) {
   const int f32 = act_type(w, "router");
   MP_CHECK(w.dim() == 2 && w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "router [E, W]");
   MP_CHECK(ew.dim() == 2, "ew [T, top]");
@@ -212,7 +212,7 @@ void moe_route(const at::Tensor& x, const at::Tensor& w, const at::Tensor& ctx, 
                             const_cast<int32_t*>(i32_vec(slot, T * top, "slot")),
                             const_cast<int32_t*>(i32_vec(lists, mp_moe_lists(E), "lists")),
                             const_cast<int32_t*>(i32_vec(tok, T * top, "tok")), T, E, W, top, groups, keep,
-                            (float)scale, f32, cur_stream()),
+                            (float)scale, f32, ordered, cur_stream()),
                "moe_route");
 }
 
@@ -281,7 +281,7 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def("moe_router_splits(int T, int W, int E, bool f32) -> int", &moe_router_splits);
   m.def(
       "moe_route(Tensor x, Tensor w, Tensor ctx, Tensor(a!) part, Tensor(b!) ew, Tensor(c!) idx, Tensor(d!) slot, "
-      "Tensor(e!) lists, Tensor(f!) tok, int groups, int keep, float scale, int packed) -> ()");
+      "Tensor(e!) lists, Tensor(f!) tok, int groups, int keep, float scale, int packed, bool ordered=False) -> ()");
   m.def("moe_combine(Tensor y, Tensor ew, Tensor slot, Tensor(a!) out) -> ()");
   m.def(
       "moe_gemm(int form, Tensor x, Tensor? tok, Tensor lists, Tensor w, Tensor(a!) out, int rows, int tokens, int glu, "

@@ -3,9 +3,9 @@
 //   moe_router       logits[t, e] = x[t] . router[e] in 32-bit, over K slices
 //   moe_choose       softmax over all experts; a group of neighbouring experts counts as its best one; the ``top``
 //                    experts with the largest scores among the ``keep`` best groups; weights = scores / (sum + 1e-20)
-//                    * scale; rows of every expert
-//   moe_place        rows sorted by expert, then by token: first row of every expert, the token of every row, the row of
-//                    every choice
+//                    * scale.  Every choice also gets its place among its expert's rows
+//   moe_place        rows sorted by expert: first row of every expert, the token of every row, the row of every choice
+//   moe_order        the same, an expert's rows in the order of their tokens
 //   moe_combine      every token's rows, weighed and added
 //   moe_gemm_any     any shape and both element types
 //   moe_gemm_rows    bf16, few rows per expert: weights stream once through registers in fragment order
@@ -118,10 +118,11 @@ struct ChooseArgs {
   const float* part;  // [S][T][E]
   const int32_t* ctx;  // [T]; <= 0: a padding row, no choice
   int S, T, E, top, groups, keep;
+  bool ordered;  // (more than one workgroup) moe_order follows: rows are only counted
   float scale;
   float* ew;          // [T, top]
   int32_t* idx;       // [T, top] expert, -1: none
-  int32_t* slot;      // [T, top] row, -1: none
+  int32_t* slot;      // [T, top] place among its expert's rows, then (moe_place) the row
   int32_t* lists;     // moe_lists
   int32_t* tok;       // [T top] token of every row
 };
@@ -322,13 +323,19 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
           a.idx[at] = e;
           const int n = atomicAdd(&hist[e], 1);
           if (ALONE) pick[j] = rank[j], place[j] = n;
+          else a.slot[at] = n;
         }
     }
   }
   __syncthreads();
-  if constexpr (!ALONE) {
-    for (int e = tid; e < E; e += blockDim.x)
-      if (hist[e] > 0) atomicAdd(&l.cnt[e], hist[e]);
+  if constexpr (!ALONE) {  // places become places among all workgroups' rows
+    for (int e = tid; e < E; e += blockDim.x) base[e] = hist[e] > 0 ? atomicAdd(&l.cnt[e], hist[e]) : 0;
+    if (a.ordered) return;
+    __syncthreads();
+    for (int i = lane; i < per * a.top; i += 64) {
+      const int t = t0 + i / a.top, at = t0 * a.top + i;
+      if (t < a.T && a.idx[at] >= 0) a.slot[at] += base[a.idx[at]];
+    }
     return;
   }
   if (wv == 0) {
@@ -347,24 +354,42 @@ __global__ __launch_bounds__(CH_WAVES * 64) void moe_choose_kernel(ChooseArgs a,
     }
 }
 
-// A workgroup has an expert, its waves the choices in order, 64 at a time: once to count, once to place.  The order of an
-// expert's rows is that of its tokens: it decides which rows lie in a tile that moe_gemm_wide cuts in K, so that with places
-// by atomics the same prompt of 2700 tokens had other last bits (0.002 of its size) in each pass.
-// The choice and this together, against places by atomics: 2700 tokens of two of 8 experts 14.9 -> 13.3 us, 4298 of four of 32
-// 18.4 -> 20.7.
-__global__ __launch_bounds__(1024) void moe_place_kernel(ChooseArgs a) {
+__global__ __launch_bounds__(256) void moe_place_kernel(ChooseArgs a) {
+  __shared__ int32_t off[MOE_EXPERTS + 1];
+  const MoeLists l = moe_lists(a.lists, a.E);
+  if (threadIdx.x < 64) {
+    moe_prefix(l.cnt, off, a.E, threadIdx.x);
+    if (blockIdx.x == 0) moe_active(l.cnt, l, a.E, threadIdx.x);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0)
+    for (int e = threadIdx.x; e <= a.E; e += 256) l.off[e] = off[e];
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < a.T * a.top && a.idx[i] >= 0) {
+    const int r = off[a.idx[i]] + a.slot[i];
+    a.slot[i] = r;
+    a.tok[r] = i / a.top;
+  }
+}
+
+// A workgroup has an expert, its waves the choices in order, 64 at a time: once to count, once to place.  Rows in the order of
+// their tokens are for experts whose last tiles moe_gemm_wide cuts in K: a row's place then decides whether it is one sum or
+// two, and with places by atomics the same prompt of 2700 tokens had other last bits (0.002 of its size) in each pass.  Router,
+// choice and places of 2700 tokens of two of 8 experts: 19.6 us by atomics, 20.0 in order; 8192 tokens of four of 32, whose
+// products are not cut: 31 and 39.
+__global__ __launch_bounds__(1024) void moe_order_kernel(ChooseArgs a) {
   constexpr int U = 8;
   __shared__ int32_t off[MOE_EXPERTS + 1], part[16];
   const MoeLists l = moe_lists(a.lists, a.E);
   const int e = blockIdx.x, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = a.T * a.top, per = (n + 1023) / 1024 * 64, i0 = wv * per, i1 = min(n, i0 + per);
-  auto fetch = [&](int i, int (&v)[U]) {
+  int v[U], count = 0;
+  auto fetch = [&](int i) {
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = i + 64 * u + lane < i1 ? a.idx[i + 64 * u + lane] : -1;
   };
-  int v[U], count = 0;
   for (int i = i0; i < i1; i += 64 * U) {
-    fetch(i, v);
+    fetch(i);
 #pragma unroll
     for (int u = 0; u < U; ++u) count += __popcll(__ballot(v[u] == e));
   }
@@ -379,7 +404,7 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(ChooseArgs a) {
   int row = off[e];
   for (int w = 0; w < wv; ++w) row += part[w];
   for (int i = i0; i < i1; i += 64 * U) {
-    if (per > 64 * U) fetch(i, v);  // (else they are there)
+    if (per > 64 * U) fetch(i);  // (else they are there)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const unsigned long long m = __ballot(v[u] == e);
@@ -906,7 +931,7 @@ extern "C" int mp_moe_router_splits(int T, int W, int E, int f32) {
 
 extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, const int32_t* ctx, float* part, int S,
                             float* ew, int32_t* idx, int32_t* slot, int32_t* lists, int32_t* tok, int T, int E, int W,
-                            int top, int groups, int keep, float scale, int f32, hipStream_t stream) {
+                            int top, int groups, int keep, float scale, int f32, int ordered, hipStream_t stream) {
   using namespace mp;
   (void)hipGetLastError();
   if (T == 0) return 0;
@@ -936,7 +961,7 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
                          (const bf16_t*)w, part, T, E, W, ks, l.cnt);
   }
   const RouteIn in{(const bf16_t*)x, (const bf16_t*)w, xs, mt, W, ks};
-  const ChooseArgs a{part, ctx, S, T, E, top, groups, keep, scale, ew, idx, slot, lists, tok};
+  const ChooseArgs a{part, ctx, S, T, E, top, groups, keep, ordered != 0, scale, ew, idx, slot, lists, tok};
   const int nw = E <= 256 ? CH_WAVES : CH_WAVES / 2;  // (LDS: 8 E bytes a wave)
   const size_t lds = (2 * E + 1 + nw * 2 * E + fused * S * 16 * 17) * sizeof(float);
   // one token a wave as long as that fills no more than the chip; a single workgroup also places the rows
@@ -945,7 +970,8 @@ extern "C" int mp_moe_route(const void* x, int64_t xs, int mt, const void* w, co
   if (fused) fused == 1 ? choose(moe_choose_kernel<1, true, 1>) : choose(moe_choose_kernel<1, true, 2>);
   else if (E <= 64) nb > 1 ? choose(moe_choose_kernel<1, false, 0>) : choose(moe_choose_kernel<1, true, 0>);
   else nb > 1 ? choose(moe_choose_kernel<MOE_EXPERTS / 64, false, 0>) : choose(moe_choose_kernel<MOE_EXPERTS / 64, true, 0>);
-  if (nb > 1) hipLaunchKernelGGL(moe_place_kernel, dim3(E), dim3(1024), 0, stream, a);
+  if (nb > 1 && ordered) hipLaunchKernelGGL(moe_order_kernel, dim3(E), dim3(1024), 0, stream, a);
+  else if (nb > 1) hipLaunchKernelGGL(moe_place_kernel, dim3((T * top + 255) / 256), dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 

@@ -110,6 +110,12 @@ def _choose_cpu(x, w, ctx, m):
     return torch.where(live, p, torch.zeros_like(p)), torch.where(live, idx, torch.full_like(idx, -1))
 
 
+def _parts(m, tokens: int, packed: bool) -> int:
+    """fp32 workspace elements of a down product whose last tiles may be cut in K (0: none is).  Where they are, the rows of an
+    expert keep the order of their tokens, so that the same step always has the same rows in those tiles."""
+    return torch.ops.mpamd.moe_gemm_ws(expert_form(tokens * m.top, m.experts, packed), m.ff)
+
+
 def choose(x, w, ctx, spec, e, packed=False) -> Choice:
     """Router and choice of a step: ``x`` [T, W] (or packed), ``w`` [experts, W], ``ctx`` [T] (0: a padding row, which
     chooses nothing); ``e(name, shape, dtype)`` gives scratch."""
@@ -134,7 +140,7 @@ def choose(x, w, ctx, spec, e, packed=False) -> Choice:
     S = torch.ops.mpamd.moe_router_splits(T, W, E, w.dtype == torch.float32)
     part = e(f"moe_z{E}", (S, T, E), torch.float32)
     torch.ops.mpamd.moe_route(x, w, ctx, part, weights, idx, slot, lists, tok, spec.groups, spec.keep, float(spec.scale),
-                              int(packed))
+                              int(packed), _parts(spec, T, packed) > 0)
     return Choice(spec, weights, slot, tok, lists, T)
 
 
@@ -165,7 +171,7 @@ def experts(x, c: Choice, up, down, up_p, down_p, block, e, packed=False):
     y = e("moe_y", (R, W), dt if form > 1 and R >= NARROW_ROWS * m.experts else torch.float32)
     torch.ops.mpamd.moe_gemm(form, x, c.tok, c.lists, up_p if form else up, act, R, c.tokens, 1, block, float(m.limit),
                              int(packed))
-    n = torch.ops.mpamd.moe_gemm_ws(form, m.ff) if y.dtype == torch.bfloat16 else 0
+    n = _parts(m, c.tokens, packed) if form and y.dtype == torch.bfloat16 else 0
     torch.ops.mpamd.moe_gemm(form, act, None, c.lists, down_p if form else down, y, R, c.tokens, 0, 1, 0.0, 0,
                              e("moe_parts", (n,), torch.float32) if n else None)
     return y

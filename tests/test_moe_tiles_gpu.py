@@ -151,14 +151,18 @@ def test_the_same_prompt_has_the_same_bits(T, W, ff):
 
 
 @pytest.mark.parametrize("T,E,top", [(17, 5, 2), (300, 64, 64), (511, 8, 2), (512, 8, 2), (1024, 65, 8), (4100, 512, 4), (9000, 3, 1)])
-def test_rows_in_the_order_of_their_tokens(T, E, top):
-    """Choices up to the ends of a wave's 64, of its share that stays in registers (512) and past it; rows without a choice."""
+@pytest.mark.parametrize("ordered", [False, True])
+def test_places_of_rows(T, E, top, ordered, monkeypatch):
+    """Choices up to the ends of a wave's 64, of its share that stays in registers (512) and past it; tokens without a choice.
+    Every row has its token and its expert; in the order of the tokens where the down product is cut."""
     ops.require_native()
+    monkeypatch.setattr(moe, "_parts", lambda *a: int(ordered))
     g = torch.Generator().manual_seed(T)
     x, w = torch.randn(T, 64, generator=g).to(torch.bfloat16), torch.randn(E, 64, generator=g).to(torch.bfloat16)
     ctx = (torch.rand(T, generator=g) < 0.9).to(torch.int32)
     e = lambda name, shape, dtype=torch.bfloat16: torch.full(shape, -7, dtype=dtype, device="cuda")  # noqa: E731
-    c = moe.choose(x.cuda(), w.cuda(), ctx.cuda(), MoESpec(E, top, 64, 1.0), e)
+    spec = MoESpec(E, top, 64, 1.0)
+    c = moe.choose(x.cuda(), w.cuda(), ctx.cuda(), spec, e)
     lists, slot, tok = c.lists.tolist(), c.slot.cpu(), c.tok.tolist()
     counts, off = lists[:E], lists[E:2 * E + 1]
     assert off == [sum(counts[:i]) for i in range(E + 1)] and off[E] == int(ctx.sum()) * top
@@ -166,4 +170,12 @@ def test_rows_in_the_order_of_their_tokens(T, E, top):
     assert [tok[r] for r in slot[ctx > 0].flatten().tolist()] == [t for t in range(T) if ctx[t] for _ in range(top)]
     assert bool((slot[ctx == 0] == -1).all())
     for a, b in zip(off, off[1:]):
-        assert tok[a:b] == sorted(set(tok[a:b]))
+        assert len(set(tok[a:b])) == b - a and (not ordered or T <= 16 or tok[a:b] == sorted(tok[a:b]))
+
+
+def test_which_rows_are_ordered():
+    """Where the tiles of the last round are cut: wide experts with many rows each."""
+    ops.require_native()
+    for ff, tokens, packed, want in ((14336, 2700, False, True), (4096, 512, False, True), (4096, 511, False, False),
+                                     (4032, 2700, False, False), (1408, 4298, False, False), (14336, 2700, True, False)):
+        assert (moe._parts(MoESpec(8, 2, ff, 1.0), tokens, packed) > 0) == want
