@@ -29,7 +29,7 @@ struct GemmPrompt {
   float limit;
   int mt, nt;      // row and weight tiles
   int full, rest, parts;  // tiles made whole; tiles cut into parts
-  float* slabs;           // [parts][rest][8 waves][8][4][64 lanes][4]
+  float* slabs;           // [parts][rest][4 waves][8][8][64 lanes][4]
 };
 
 __device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, int& n0) {
@@ -37,11 +37,11 @@ __device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, in
   m0 = (GW_BAND * band + r % h) * WideTile::BM;
   n0 = r / h * WideTile::BN;
 }
-template <int EPI>
+template <int EPI, bool LIMIT>
 __device__ __forceinline__ void gw_act(const GemmPrompt& a, const f32x4& v, const f32x4& u, float (&y)[4]) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    if (EPI == 1 && a.limit > 0.f) {
+    if (EPI == 1 && LIMIT) {
       const float g = fminf(v[r], a.limit), w = fminf(fmaxf(u[r], -a.limit), a.limit);
       y[r] = g / (1.f + __expf(-1.702f * g)) * (w + 1.f);
     } else if (EPI == 1) {
@@ -68,50 +68,60 @@ struct PromptWork {
   __device__ int stages(int k) const {
     return k < whole ? a.K / 64 : (g / a.rest + 1) * (a.K / 64) / a.parts - g / a.rest * (a.K / 64) / a.parts;
   }
-  __device__ void rows(int k, W::Source& s) const {
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    s.from(a.x, ((uint32_t)(a.M - 1) * (uint32_t)a.xs + (uint32_t)a.K) * 2, 128);
-    s.at = begin(k) * 128;
+  __device__ void row_offsets(W::Source& s) const {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)  // (the launcher checks that they fit)
-      s.off[j] = (uint32_t)min(m0 + W::piece_row(j), a.M - 1) * (uint32_t)(a.xs * 2) + W::piece_byte();
+    for (int j = 0; j < W::PIECES; ++j) s.off[j] = (uint32_t)W::piece_row(j) * (uint32_t)(a.xs * 2) + W::piece_byte();
   }
-  __device__ void weights(int k, W::Source& s) const {
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    s.from(a.w, (uint32_t)a.N * (uint32_t)a.K * 2, EPI == GW_COLUMNS ? (uint32_t)a.N * 128 : 128);
-    s.at = begin(k) * s.step;
+  __device__ void weight_offsets(W::Source& s) const {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      s.off[j] = EPI == GW_COLUMNS
-                     ? ((uint32_t)W::column_row(j) * (uint32_t)a.N + (uint32_t)min(n0 + W::column_first(j), a.N - 8)) * 2
-                     : (uint32_t)min(n0 + W::piece_row(j), a.N - 1) * (uint32_t)(a.K * 2) + W::piece_byte();
+    for (int j = 0; j < W::PIECES; ++j)
+      s.off[j] = EPI == GW_COLUMNS ? ((uint32_t)W::column_row(j) * (uint32_t)a.N + W::column_first(j)) * 2
+                                   : (uint32_t)W::piece_row(j) * (uint32_t)(a.K * 2) + W::piece_byte();
   }
-  __device__ bool live(int k) const {
+  __device__ void rows(int k, W::Source& s) const {  // (the launcher checks that the bytes fit 32 bits)
     int m0, n0;
     gw_tile(a, id(k), m0, n0);
-    return m0 + 16 * W::MW * W::wm() < a.M;
+    s.from(a.x + m0 * a.xs, ((uint32_t)(a.M - 1 - m0) * (uint32_t)a.xs + (uint32_t)a.K) * 2, begin(k) * 128, 128);
   }
-  __device__ bool store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
+  __device__ void weights(int k, W::Source& s) const {  // (columns past the last of a row are the next row's first: not stored)
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    if (EPI == GW_COLUMNS)
+      s.from(a.w + n0, ((uint32_t)a.N * (uint32_t)a.K - n0) * 2, begin(k) * (uint32_t)a.N * 128, (uint32_t)a.N * 128);
+    else
+      s.from(a.w + (int64_t)n0 * a.K, (uint32_t)(a.N - n0) * (uint32_t)a.K * 2, begin(k) * 128, 128);
+  }
+  __device__ bool half(int k) const {
+    int m0, n0;
+    gw_tile(a, id(k), m0, n0);
+    return a.M - m0 <= W::BM / 2;
+  }
+  template <int M>
+  __device__ int store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
     if (k == whole) {  // (nothing comes behind it)
-      float* s = a.slabs + (int64_t)g * GW_SLAB + (W::wave() * 32 * 64 + (threadIdx.x & 63)) * 4;
+      float* s = a.slabs + (int64_t)g * GW_SLAB + (W::wave() * W::NW * W::MW * 64 + (threadIdx.x & 63)) * 4;
 #pragma unroll
       for (int i = 0; i < W::NW; ++i)
 #pragma unroll
-        for (int j = 0; j < W::MW; ++j) *reinterpret_cast<f32x4*>(s + (i * 4 + j) * 256) = acc[i][j];
-      return false;
+        for (int j = 0; j < M; ++j) {
+          *reinterpret_cast<f32x4*>(s + (i * W::MW + j) * 256) = W::taken(acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      return 0;
     }
     int m0, n0;
     gw_tile(a, id(k), m0, n0);
-    const int nw = n0 + 16 * W::NW * W::wn();
-    return W::put<EPI == 1>(a.out, EPI == 1 ? a.N / 2 : a.N, true, m0 + 16 * W::MW * W::wm(), a.M, EPI == 1 ? nw / 2 : nw, acc,
-                            [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI>(a, v, u, y); });
+    const int nw = n0 + 16 * W::NW * W::wn(), cols = EPI == 1 ? a.N / 2 : a.N;
+    auto go = [&](auto limit) {
+      return W::put<EPI == 1, M>(a.out + (int64_t)m0 * cols, cols, a.M - m0, EPI == 1 ? nw / 2 : nw, acc,
+                                 [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI, limit.value>(a, v, u, y); });
+    };
+    return EPI == 1 && a.limit > 0.f ? go(W::Int<1>()) : go(W::Int<0>());
   }
 };
 
 template <int EPI>
-__global__ __launch_bounds__(512) void gemm_prompt_kernel(GemmPrompt a) {
+__global__ __launch_bounds__(WideTile::THREADS, 1) void gemm_prompt_kernel(GemmPrompt a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3, step = gridDim.x >> 3;
   const int per = (a.full + 7) / 8, lo = xcd * per, run = min(per, a.full - lo);  // the XCD's run of whole tiles
@@ -121,27 +131,28 @@ __global__ __launch_bounds__(512) void gemm_prompt_kernel(GemmPrompt a) {
   WideTile::run<EPI == GW_COLUMNS ? WideTile::COLUMNS : WideTile::ROWS>(smem, count, PromptWork<EPI>{a, lo + at, step, whole, g});
 }
 
-// a left-over tile's parts added and stored; blockIdx.y: two of the eight row groups of weights, two of the four of rows
+// a left-over tile's parts added and stored; blockIdx.y: two of a wave's eight fragments of weights, two of the eight of rows
 template <int EPI>
-__global__ __launch_bounds__(512) void gemm_prompt_close_kernel(GemmPrompt a) {
+__global__ __launch_bounds__(WideTile::THREADS) void gemm_prompt_close_kernel(GemmPrompt a) {
   typedef WideTile W;
   const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4, r = blockIdx.x;
-  const int i0 = 2 * (blockIdx.y >> 1), j0 = 2 * (blockIdx.y & 1);
+  const int i0 = 2 * (blockIdx.y / (W::MW / 2)), j0 = 2 * (blockIdx.y % (W::MW / 2));
   int m0, n0;
   gw_tile(a, a.full + r, m0, n0);
-  const int m = m0 + 16 * (W::MW * W::wm() + j0) + c16, o = n0 + 16 * (W::NW * W::wn() + i0);
-  if (m0 + 16 * W::MW * W::wm() >= a.M || o >= a.N) return;
+  const int frags = a.M - m0 <= W::BM / 2 ? W::MW / 2 : W::MW;
+  const int m = m0 + 16 * (frags * W::wm() + j0) + c16, o = n0 + 16 * (W::NW * W::wn() + i0);
+  if (j0 >= frags || m - c16 >= a.M || o >= a.N) return;
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4)(0.f);
   for (int p = 0; p < a.parts; ++p) {
-    const float* s = a.slabs + (p * a.rest + r) * GW_SLAB + ((W::wave() * 32 + i0 * 4 + j0) * 64 + lane) * 4;
+    const float* s = a.slabs + (p * a.rest + r) * GW_SLAB + ((W::wave() * W::NW * W::MW + i0 * W::MW + j0) * 64 + lane) * 4;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] += *reinterpret_cast<const f32x4*>(s + (i * 4 + j) * 256);
+      for (int j = 0; j < 2; ++j) acc[i][j] += *reinterpret_cast<const f32x4*>(s + (i * W::MW + j) * 256);
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -150,7 +161,8 @@ __global__ __launch_bounds__(512) void gemm_prompt_close_kernel(GemmPrompt a) {
     for (int i = 0; i < 2; i += EPI == 1 ? 2 : 1)
       if (o + 16 * i < a.N) {
         float y[4];
-        gw_act<EPI>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
+        if (EPI == 1 && a.limit > 0.f) gw_act<EPI, true>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
+        else gw_act<EPI, false>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
         st_vec<4>(a.out + (int64_t)(m + 16 * j) * (EPI == 1 ? a.N / 2 : a.N) + (EPI == 1 ? o / 2 + 8 * i : o + 16 * i) + 4 * g4, y);
       }
   }
@@ -178,7 +190,8 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
                             float* ws, hipStream_t stream) {
   (void)hipGetLastError();
   using namespace mp;
-  if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31))
+  if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31) ||
+      N >= 1 << 22)  // (a tile's rows of the output below 2^31 bytes)
     return -1;
   if (epi == 1 && N % 32) return -2;
   GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, (M + 255) / 256, (N + 255) / 256, 0, 0, 1, ws};
@@ -193,8 +206,9 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
 #define MP_GW(E_)                                                                                                          \
   {                                                                                                                        \
     (void)hipFuncSetAttribute((const void*)gemm_prompt_kernel<E_>, hipFuncAttributeMaxDynamicSharedMemorySize, WideTile::LDS); \
-    hipLaunchKernelGGL((gemm_prompt_kernel<E_>), grid, dim3(512), WideTile::LDS, stream, a);                                  \
-    if (a.rest) hipLaunchKernelGGL((gemm_prompt_close_kernel<E_>), dim3(a.rest, 8), dim3(512), 0, stream, a);                 \
+    hipLaunchKernelGGL((gemm_prompt_kernel<E_>), grid, dim3(WideTile::THREADS), WideTile::LDS, stream, a);                                  \
+    if (a.rest) hipLaunchKernelGGL((gemm_prompt_close_kernel<E_>), dim3(a.rest, WideTile::MW * WideTile::NW / 4),          \
+                                   dim3(WideTile::THREADS), 0, stream, a);                                               \
   }
   if (epi == 0) MP_GW(0)
   else if (epi == 1) MP_GW(1)

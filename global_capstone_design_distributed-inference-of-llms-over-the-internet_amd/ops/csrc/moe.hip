@@ -743,7 +743,6 @@ struct MoeWork {
   typedef WideTile W;
   const MoeGemm& a;
   const MoeLists& l;
-  bool wide;
   float* ws;
   int en, mt, pt;  // lane k: expert and weight tile (10 bits and the others), row tile of tile k; 0, or its place in ws + 1
   __device__ int part(int k) const { return __builtin_amdgcn_readlane(pt, k); }
@@ -752,61 +751,72 @@ struct MoeWork {
   __device__ int n0(int k) const { return (__builtin_amdgcn_readlane(en, k) >> 10) * W::BN; }
   __device__ int m0(int k) const { return __builtin_amdgcn_readlane(mt, k) * W::BM; }
   __device__ int stages(int k) const { return !part(k) ? a.K / 64 : (a.K / 64 + (part(k) & 1)) / 2; }
+  __device__ void row_offsets(W::Source&) const {}
+  __device__ void weight_offsets(W::Source& s) const {
+#pragma unroll
+    for (int j = 0; j < W::PIECES; ++j) s.off[j] = (uint32_t)W::packed_tile(j) * (uint32_t)(a.K * 32) + W::packed_byte(j);
+  }
   __device__ void rows(int k, W::Source& s) const {
     const int e = expert(k), m = m0(k), r0 = l.off[e], n = l.cnt[e];
-    s.from(a.x, 0xffffffffu, 128);
-    s.at = 128 * first(k);
+    s.from(a.x, 0xffffffffu, 128 * first(k), 128);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {  // (the launcher checks that they fit)
+    for (int j = 0; j < W::PIECES; ++j) {  // (the launcher checks that they fit)
       const int q = r0 + min(m + W::piece_row(j), n - 1), row = a.tok ? a.tok[q] : q;
       s.off[j] = (uint32_t)row * (uint32_t)(a.xs * 2) + W::piece_byte();
     }
   }
   __device__ void weights(int k, W::Source& s) const {
-    const int t0 = n0(k) / 16, nt = a.N / 16;
-    s.from((const bf16_t*)a.w + (int64_t)expert(k) * a.N * a.K, (uint32_t)a.N * (uint32_t)a.K * 2, 2048);
-    s.at = 2048 * first(k);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      s.off[j] = (uint32_t)min(t0 + W::packed_tile(j), nt - 1) * (uint32_t)(a.K * 32) + W::packed_byte(j);
+    s.from((const bf16_t*)a.w + ((int64_t)expert(k) * a.N + n0(k)) * a.K, (uint32_t)(a.N - n0(k)) * (uint32_t)a.K * 2,
+           2048 * first(k), 2048);
   }
-  __device__ bool live(int k) const { return m0(k) + 16 * W::MW * W::wm() < l.cnt[expert(k)]; }
+  __device__ bool half(int k) const { return l.cnt[expert(k)] - m0(k) <= W::BM / 2; }
   // (a lane's sums as they lie, 16 bytes each: whoever adds the parts has the same lanes)
   static __device__ __forceinline__ f32x4* kept(float* ws, int place) {
-    return reinterpret_cast<f32x4*>(ws) + ((int64_t)place * 8 + W::wave()) * W::NW * W::MW * 64 + (threadIdx.x & 63);
+    return reinterpret_cast<f32x4*>(ws) + ((int64_t)place * 4 + W::wave()) * W::NW * W::MW * 64 + (threadIdx.x & 63);
   }
-  __device__ bool store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
-    if (!GLU && part(k)) {
+  template <int M>
+  __device__ int store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
+    const int lane = threadIdx.x & 63;
+    if (!GLU && part(k)) {  // (of a whole tile)
       f32x4* to = kept(ws, part(k) - 1);
 #pragma unroll
       for (int i = 0; i < W::NW; ++i)
 #pragma unroll
-        for (int j = 0; j < W::MW; ++j) to[(i * W::MW + j) * 64] = acc[i][j];
-      return true;
+        for (int j = 0; j < M; ++j) {
+          to[(i * W::MW + j) * 64] = W::taken(acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      return STORES * M / W::MW;
     }
-    const int e = expert(k), m = m0(k) + 16 * W::MW * W::wm(), o = n0(k) + 16 * W::NW * W::wn(), n = l.cnt[e];
+    const int e = expert(k), m = m0(k), o = n0(k) + 16 * W::NW * W::wn(), n = l.cnt[e];
     const int cols = GLU ? a.N / 2 : a.N;
-    TO* out = (TO*)a.out + (int64_t)l.off[e] * cols;
+    TO* out = (TO*)a.out + (int64_t)(l.off[e] + m) * cols;
     if constexpr (sizeof(TO) == 2) {
-      return W::put<GLU>(out, cols, wide, m, n, GLU ? o / 2 : o, acc, [&](const f32x4& v, const f32x4& u, float(&y)[4]) {
+      auto go = [&](float limit) {
+        return W::put<GLU, M>(out, cols, n - m, GLU ? o / 2 : o, acc, [&](const f32x4& v, const f32x4& u, float(&y)[4]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) y[r] = GLU ? moe_glu(v[r], u[r], a.limit) : v[r];
-      });
+          for (int r = 0; r < 4; ++r) y[r] = GLU ? moe_glu(v[r], u[r], limit) : v[r];
+        });
+      };
+      return GLU && a.limit > 0.f ? go(a.limit) : go(0.f);
     } else {
-      const int lane = threadIdx.x & 63;
+      const int r = 16 * M * W::wm() + (lane & 15);
 #pragma unroll
-      for (int j = 0; j < W::MW; ++j)
+      for (int j = 0; j < M; ++j)
 #pragma unroll
-        for (int i = 0; i < W::NW; ++i)
-          if (m + 16 * j + (lane & 15) < n && o + 16 * i < a.N)
-            *reinterpret_cast<f32x4*>(out + (int64_t)(m + 16 * j + (lane & 15)) * cols + o + 16 * i + 4 * (lane >> 4)) = acc[i][j];
-      return false;
+        for (int i = 0; i < W::NW; ++i) {
+          const f32x4 y = W::taken(acc[i][j]);
+          if (m + r + 16 * j < n && o + 16 * i < a.N)
+            *reinterpret_cast<f32x4*>(out + (int64_t)(r + 16 * j) * cols + o + 16 * i + 4 * (lane >> 4)) = y;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      return 0;
     }
   }
 };
 
 template <bool GLU, typename TO>
-__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide, float* ws) {
+__global__ __launch_bounds__(WideTile::THREADS, 1) void moe_gemm_wide_kernel(MoeGemm a, float* ws) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
   const int lane = threadIdx.x & 63, ntn = (a.N + WideTile::BN - 1) / WideTile::BN;
@@ -837,41 +847,49 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(MoeGemm a, bool wide
     int e, nt, mt;
     moe_find(l, a.E, ntn, half, id, e, nt, mt);
     if (first) __syncthreads();  // (the last tiles' operands have been read)
-    WideTile::run<WideTile::PACKED>(smem, count, MoeWork<GLU, TO>{a, l, wide, ws, e + (nt << 10), mt, pt});
+    WideTile::run<WideTile::PACKED>(smem, count, MoeWork<GLU, TO>{a, l, ws, e + (nt << 10), mt, pt});
   }
 }
 
-// The cut tiles' two sums added, rounded and stored; workgroup (XCD, tile of it).  Bound by the 64 MB at most that they lie in.
-__global__ __launch_bounds__(512) void moe_gemm_close_kernel(MoeGemm a, bool wide, float* ws, int G) {
+// The cut tiles' two sums added, rounded and stored; workgroup (XCD, tile of it), two of a wave's eight fragments of weights
+// and two of the eight of rows.  Bound by the 64 MB at most that they lie in.
+__global__ __launch_bounds__(WideTile::THREADS) void moe_gemm_close_kernel(MoeGemm a, float* ws, int G) {
+  typedef WideTile W;
   typedef MoeWork<false, bf16_t> Work;
   const MoeLists l = moe_lists(const_cast<int32_t*>(a.lists), a.E);
-  const int ntn = (a.N + WideTile::BN - 1) / WideTile::BN, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int lane = threadIdx.x & 63, ntn = (a.N + W::BN - 1) / W::BN, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int i0 = 2 * (blockIdx.y / (W::MW / 2)), j0 = 2 * (blockIdx.y % (W::MW / 2));
   const MoeDeal d(l, a.E, ntn, xcd, G, true);
   if (!d.split || at >= d.r) return;
   int e, nt, mt;
   moe_find(l, a.E, ntn, false, d.f0 + d.q * G + at, e, nt, mt);
-  const Work work{a, l, wide, nullptr, e + (nt << 10), mt, 0};
-  if (!work.live(0)) return;
+  e = __builtin_amdgcn_readfirstlane(e), nt = __builtin_amdgcn_readfirstlane(nt), mt = __builtin_amdgcn_readfirstlane(mt);
   const int place = 2 * (xcd * MW_SPLIT + at);
   const f32x4 *p = Work::kept(ws, place), *q = Work::kept(ws, place + 1);
-  f32x4 acc[WideTile::NW][WideTile::MW];
+  const int m = mt * W::BM + 16 * (W::MW * W::wm() + j0) + (lane & 15), o = nt * W::BN + 16 * (W::NW * W::wn() + i0);
+  bf16_t* out = (bf16_t*)a.out + ((int64_t)l.off[e] + m) * a.N + o + 4 * (lane >> 4);
 #pragma unroll
-  for (int i = 0; i < WideTile::NW; ++i)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < WideTile::MW; ++j) acc[i][j] = p[(i * WideTile::MW + j) * 64] + q[(i * WideTile::MW + j) * 64];
-  work.store(0, acc);
+    for (int i = 0; i < 2; ++i) {
+      if (m + 16 * j >= l.cnt[e] || o + 16 * i >= a.N) continue;
+      const int f = ((i0 + i) * W::MW + j0 + j) * 64;
+      const f32x4 s = p[f] + q[f];
+      const float y[4] = {s[0], s[1], s[2], s[3]};
+      st_vec<4>(out + (int64_t)16 * j * a.N + 16 * i, y);
+    }
 }
 
 template <bool GLU, typename TO>
 static int launch_moe_wide(const MoeGemm& a, int rows, int act, float* ws, hipStream_t stream) {
   const int tiles = (rows / WideTile::BM + act) * ((a.N + WideTile::BN - 1) / WideTile::BN), per = (tiles + 7) / 8 + 1;
   const int G = per < WideTile::CUS / 8 ? per : WideTile::CUS / 8;  // (whole and half tiles are shared out apart: one more)
-  const bool wide = (uintptr_t)a.out % 16 == 0;
   (void)hipFuncSetAttribute((const void*)moe_gemm_wide_kernel<GLU, TO>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             WideTile::LDS);
-  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3(8 * G), dim3(512), WideTile::LDS, stream, a, wide, ws);
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GLU, TO>), dim3(8 * G), dim3(WideTile::THREADS), WideTile::LDS, stream, a, ws);
   if constexpr (!GLU && sizeof(TO) == 2)
-    if (ws) hipLaunchKernelGGL(moe_gemm_close_kernel, dim3(8 * MW_SPLIT), dim3(512), 0, stream, a, wide, ws, G);
+    if (ws) hipLaunchKernelGGL(moe_gemm_close_kernel, dim3(8 * MW_SPLIT, WideTile::MW * WideTile::NW / 4),
+                               dim3(WideTile::THREADS), 0, stream, a, ws, G);
   return (int)hipGetLastError();
 }
 
@@ -1018,7 +1036,8 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
     if (mt > 0) return -1;
     // 256 x 256 tiles from 128 rows an expert on (ops/moe.py expert_form); where K is not in steps of 64, or a piece's
     // byte offset does not fit 32 bits, the ring of 32-column stages: its 256 x 256 form from 384 rows on, else 128 x 128
-    const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31);
+    const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31) &&
+                      N < 1 << 22 && (uintptr_t)out % 4 == 0;
     const bool big = form == 3 && rows >= 384 * E;
 #define MP_MT(GLU_, TO_)                                                        \
   return wide  ? launch_moe_wide<GLU_, TO_>(a, rows, act, GLU_ || sizeof(TO_) != 2 ? nullptr : ws, stream) \

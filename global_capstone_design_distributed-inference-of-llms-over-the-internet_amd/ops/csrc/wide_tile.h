@@ -1,4 +1,4 @@
-// Main loop of the 256 x 256 product tiles (moe.hip: experts, gemm_prompt.hip: prompts): eight waves of 64 rows x 128 weight
+// Main loop of the 256 x 256 product tiles (moe.hip: experts, gemm_prompt.hip: prompts): four waves of 128 rows x 128 weight
 // rows, 64 columns a stage.  A workgroup stays on its CU for all its tiles, and its loads run ahead across them.
 //   * Rows arrive 128 bytes at a time (8 rows an instruction), whole cache lines: 32-column stages fetch every line twice,
 //     and 256 rows of lines are the whole L1, so the second half came from L2 again.  The 16-byte chunks of a row are
@@ -8,276 +8,273 @@
 //     turns them into operands (8 rows' 32 bytes in 8 different groups of banks).  The compiler lets that read wait for all
 //     loads into LDS that it knows of, so this form issues its own; they have no registers to write.
 //   * All 160 KiB of LDS are a ring of five slots of one operand's stage.  Behind the one barrier of a stage its two slots are
-//     free: the rows of the stage after the next go to one, the weights of the stage after that to the other, so that
-//     weights, which come from HBM, have more than a stage and a half to arrive.  With two slots an operand and workgroups
-//     that end with their tile, weights that no cache held cost 4096 x 16384 x 4096 446 us (now 384, the library 353),
-//     4096 x 4096 x 14336 362 (322, 314), 6421 x 12288 x 4096 527 (474, 502); the early slot on the rows' side took 404,
-//     342 and 497 us.
-//   * The operands of a half stage are read from LDS while the MFMAs of the half before it run, across the barrier, one read
-//     to two MFMAs; the stage's loads are spread over the half stage behind the barrier: eight at once hold up the MFMAs that
-//     stand behind them.
-//   * A wave whose 64 rows are past the last only loads; the two waves of a SIMD have different rows, so a tile of up to 128
-//     rows takes half the MFMA time (0.8 of a whole tile's where its weights come from HBM: the ring covers less of the wait).
-// Bound by MFMA issue (three quarters of the time; the clock falls to 1.8 GHz under it) and by the issue of the loads, an eighth.
-// Measured and left: four waves of 128 x 128 (2 to 5 % more), a second barrier that frees the slot sooner (6 % more), 32 x 32
-// x 16 MFMAs (12 % more), loads over both halves of a stage (up to 8 % more).
+//     free: the rows of the stage after the next go to one, and before the next barrier the weights of the stage after
+//     that to the other.  Rows and weights are thus always at the same stage, and a stage's loads, one to eight MFMAs, never
+//     wait for each other.
+//   * A wave has its SIMD for itself: 256 sums in accumulation registers, the operands of two half stages in the others.  It
+//     reads 128 KB of operands a stage and CU where eight waves of 64 x 128 read 192.  Operands of a half stage are read
+//     while the MFMAs of the half before it run, across the barrier, one read to three MFMAs.
+//   * The MFMAs stand in inline asm and in this order: left to the compiler, sums move from register to register.  From one
+//     to the next only one operand changes (blocks of 2 x 2, there and back), which costs less power and so lets the clock
+//     rise: 3 % of a loop of MFMAs alone, 1 to 2 % here.
+//   * Nothing in the loop but the loads' 8 instructions depends on the tile: a tile moves the base of what is loaded, not
+//     the lanes' offsets, and what is behind its rows and weights is behind the end of the buffer, which loads as zero.
+//   * A tile of up to 128 rows has 64 rows a wave and half the MFMAs.
+// A stage takes 2330 (rows and weights in L2) to 2450 cycles, 2050 of them MFMAs; a tile's end 8300.  Bound by MFMA issue and, at 1.75
+// of 2.4 GHz, by power.  Eight waves, whose loop decided anew at each stage what to load next, took 2680 to 2900 cycles a
+// stage: 4096 x 4096 x 16384 393 us (now 361), 6421 x 12288 x 4096 484 (450), 4298 x 16384 x 4096 449 (438),
+// columns of 4096 x 4096 x 16384 383 (354).  Eight waves with this loop: 378, 477, 448 us.
+// Measured and left: loads in the first half stage behind the barrier alone (2 to 6 % more), one load to 4 to 6 MFMAs, one read
+// to 2 or 4, 32 x 32 x 16 MFMAs (12 % more on eight waves).
 #pragma once
 #include "common.h"
 
 namespace mp {
 
 struct WideTile {
-  static constexpr int BM = 256, BN = 256, MW = 4, NW = 8, WM = 4, WN = 2, SLOTS = 5, SLOT = 256 * 128, LDS = SLOTS * SLOT;
+  static constexpr int BM = 256, BN = 256, MW = 8, NW = 8, WM = 2, WN = 2, THREADS = 64 * WM * WN;
+  static constexpr int PIECES = 8;  // loads of a wave and operand in a stage
+  static constexpr int SLOTS = 5, SLOT = 256 * 128, LDS = SLOTS * SLOT;
   static constexpr int CUS = 256;  // workgroups of a launch at most: one to a CU
   enum Weights { ROWS, PACKED, COLUMNS };
+  template <int V>
+  struct Int {
+    static constexpr int value = V;
+  };
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   typedef __attribute__((address_space(3))) void* lptr_t;
 
   static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
-  static __device__ __forceinline__ int wm() { return wave() / WN; }  // (the waves of a SIMD, 4 apart, have different rows)
+  static __device__ __forceinline__ int wm() { return wave() / WN; }
   static __device__ __forceinline__ int wn() { return wave() % WN; }
   // row of the tile that piece j of this wave reads on this lane, and the byte of it in a stage
-  static __device__ __forceinline__ int piece_row(int j) { return 8 * (4 * wave() + j) + ((threadIdx.x & 63) >> 3); }
+  static __device__ __forceinline__ int piece_row(int j) { return 8 * (PIECES * wave() + j) + ((threadIdx.x & 63) >> 3); }
   static __device__ __forceinline__ int piece_byte() { return 16 * ((threadIdx.x & 7) ^ ((threadIdx.x & 63) >> 3)); }
   // the same of packed weights: 16-row tile and byte
-  static __device__ __forceinline__ int packed_tile(int j) { return 2 * wave() + (j >> 1); }
+  static __device__ __forceinline__ int packed_tile(int j) { return PIECES / 2 * wave() + (j >> 1); }
   static __device__ __forceinline__ int packed_byte(int j) { return 1024 * (j & 1) + (threadIdx.x & 63) * 16; }
-
   // the same of columns: row of a stage, and first of 8 columns
-  static __device__ __forceinline__ int column_row(int j) { return 2 * (4 * wave() + j) + ((threadIdx.x & 63) >> 5); }
+  static __device__ __forceinline__ int column_row(int j) { return 2 * (PIECES * wave() + j) + ((threadIdx.x & 63) >> 5); }
   static __device__ __forceinline__ int column_first(int j) {
     const int row = column_row(j), chunk = (threadIdx.x & 31) >> 1;
     return 16 * (chunk ^ ((row & 3) | (row >> 3 & 1) << 2)) + 8 * (threadIdx.x & 1);
   }
 
   // Where an operand of a tile comes from: this lane's byte offsets of the wave's pieces from ``at`` bytes behind the base on,
-  // ``step`` bytes a stage.
+  // ``step`` bytes a stage.  An offset from ``bytes`` on loads as zero.
   struct Source {
     __amdgpu_buffer_rsrc_t base;
     u32x4 words;  // of ``base``
-    uint32_t off[4], at, step;
-    __device__ __forceinline__ void from(const void* p, uint32_t bytes, uint32_t stage) {
+    uint32_t off[PIECES], at, step;
+    __device__ __forceinline__ void from(const void* p, uint32_t bytes, uint32_t first, uint32_t stage) {
       base = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
       words = (u32x4){(uint32_t)(uintptr_t)p, (uint32_t)((uintptr_t)p >> 32) & 0xffff, bytes, 0x00020000};
-      at = 0, step = stage;
+      at = first, step = stage;
     }
   };
 
   // The workgroup's tiles 0 .. count - 1 (at least one).  ``work``:
   //   int stages(k)                  stages of tile k, at least one
-  //   void rows(k, Source&)          its rows
+  //   void row_offsets(Source&), weight_offsets(Source&)   the lane's offsets, once
+  //   void rows(k, Source&)          tile k's rows (may change the offsets)
   //   void weights(k, Source&)       its weight rows
-  //   bool live(k)                   has this wave rows in it?
-  //   bool store(k, acc)             acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (4 wm + j) ..; lane: row lane % 16, weight
-  //                                  rows 4 (lane / 16) .. + 3.  True: at least work.STORES stores were issued for sure.
+  //   bool half(k)                   has it at most 128 rows?
+  //   int store<M>(k, acc)           acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (M wm + j) .., j < M; lane: row lane % 16,
+  //                                  weight rows 4 (lane / 16) .. + 3.  At least how many stores were issued: 0 or
+  //                                  work.STORES of M = 8, half of them of M = 4.
   // Ends with no load in flight.
   template <Weights FORM, class Work>
   static __device__ __forceinline__ void run(char* smem, int count, const Work& work) {
     const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
-    char* mine = smem + wave() * 4096;
+    char* mine = smem + wave() * (PIECES * 1024);
     Source x, w;
-    int xk = 0, wk = 0, xleft = work.stages(0), wleft = xleft;  // the tile that is being loaded, its stages left
+    int lk = 0, left = work.stages(0);  // the tile that is being loaded, its stages left
+    work.row_offsets(x);
+    work.weight_offsets(w);
     work.rows(0, x);
     work.weights(0, w);
+    // A load in asm needs its place in m0 one instruction before, and scalars that a vector instruction wrote (the compiler
+    // may keep some in lanes) five before: ``aim`` fixes them all, and two MFMAs stand between it and ``load`` (five waits in
+    // front of each load cost 5 % at 1554 x 4096 x 28672: 347 us now).  Nothing else of this form uses m0.
+    auto place = [&](int j, int slot) { return (lptr_t)(mine + slot * SLOT + j * 1024); };
+    auto aim = [&](Source& s, int j, int slot) {
+      if constexpr (FORM == COLUMNS)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 1" : "+s"(s.words), "+s"(s.at) : "s"((uint32_t)(uintptr_t)place(j, slot)));
+    };
     auto load = [&](const Source& s, int j, int slot) {
-      const lptr_t to = (lptr_t)(mine + slot * SLOT + j * 1024);
-      if constexpr (FORM == COLUMNS)  // (m0: nothing else of this form uses it; 5 cycles from a scalar that a vector instruction wrote to its use)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"((uint32_t)(uintptr_t)to),
-                     "v"(s.off[j]), "s"(s.words), "s"(s.at)
-                     : "memory");
+      if constexpr (FORM == COLUMNS)
+        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(s.off[j]), "s"(s.words), "s"(s.at) : "memory");
       else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, to, 16, s.off[j], s.at, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, place(j, slot), 16, s.off[j], s.at, 0, 0);
     };
-    auto load_x = [&](int j, int slot) { load(x, j, slot); };
-    auto load_w = [&](int j, int slot) { load(w, j, slot); };
-    // (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
-    auto next_x = [&] {
-      if (--xleft > 0) x.at += x.step;
-      else if (xk + 1 < count) xleft = work.stages(++xk), work.rows(xk, x);
-      else xleft = 1;
+    auto load_now = [&](Source& s, int j, int slot) {
+      aim(s, j, slot);
+      if constexpr (FORM == COLUMNS) asm volatile("s_nop 2");
+      load(s, j, slot);
     };
-    auto next_w = [&] {
-      if (--wleft > 0) w.at += w.step;
-      else if (wk + 1 < count) wleft = work.stages(++wk), work.weights(wk, w);
-      else wleft = 1;
+    // to the next stage (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
+    auto step = [&] {
+      x.at += x.step, w.at += w.step;
+      if (__builtin_expect(--left == 0, 0)) {
+        x.at -= x.step, w.at -= w.step;
+        left = 1;
+        if (lk + 1 < count) left = work.stages(++lk), work.rows(lk, x), work.weights(lk, w);
+      }
     };
     // a row's chunk c lies at 16 (c ^ row % 8)
     const int s0 = 16 * (g4 ^ (c16 & 7)), s1 = 16 * ((4 + g4) ^ (c16 & 7));
-    const int xr = (16 * MW * wm() + c16) * 128;
     const int wr = FORM == PACKED    ? 2048 * NW * wn() + lane * 16
                    : FORM == COLUMNS ? (8 * g4 + (c16 >> 2)) * 512 + 256 * wn() + 32 * (c16 >> 2 | (g4 & 1) << 2) + 8 * (c16 & 3)
                                      : (16 * NW * wn() + c16) * 128;
     u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
     f32x4 acc[NW][MW];
-    auto multiply1 = [&](int i, const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
-#pragma unroll
-      for (int j = 0; j < MW; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i]), __builtin_bit_cast(bf16x8, xf[j]),
-                                                            acc[i][j], 0, 0, 0);
-    };
-    auto multiply = [&](const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
-#pragma unroll
-      for (int i = 0; i < NW; ++i) multiply1(i, xf, wf);
-    };
-    int px = 1, pw = 0;  // slots of the stage's rows and weights
-    auto take1 = [&](int h, int r, u16x8(&xf)[MW], u16x8(&wf)[NW]) {  // one operand of a half stage
-      if (r < MW) {
+    int px = 1, pw = 0;          // slots of the stage's rows and weights
+    int fx, fw = 0;              // slots that the last barrier freed
+    int stored = 0;              // stores in flight of the tile before: none, of 64 rows a wave, of 128
+    int mode = 0;                // the rows' fragments that xa holds
+    auto take1 = [&](int h, int r, int xr, u16x8(&xf)[MW], u16x8(&wf)[NW], int m) {  // one operand of a half stage
+      if (r < m) {
         xf[r] = *reinterpret_cast<const u16x8*>(smem + px * SLOT + xr + (h ? s1 : s0) + r * 2048);
       } else if constexpr (FORM == COLUMNS) {
-        const char* p = smem + ((pw * SLOT + wr) ^ (32 * (r - MW))) + h * 16384;
+        const char* p = smem + ((pw * SLOT + wr) ^ (32 * (r - m))) + h * 16384;
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 2048));
-        wf[r - MW] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        wf[r - m] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       } else {
-        wf[r - MW] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (FORM == PACKED ? h * 1024 : h ? s1 : s0) + (r - MW) * 2048);
+        wf[r - m] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (FORM == PACKED ? h * 1024 : h ? s1 : s0) + (r - m) * 2048);
       }
     };
-    auto take = [&](int h, u16x8(&xf)[MW], u16x8(&wf)[NW]) {
+    auto tile = [&](auto fragments, int k) __attribute__((always_inline)) {
+      constexpr int M = decltype(fragments)::value;  // fragments of a wave's rows
+      constexpr int R = M == MW ? 3 : 2;             // MFMAs to a read
+      const int xr = (16 * M * wm() + c16) * 128;
+      // MFMA q of a half stage: two fragments of rows at a time
+      auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
+        const int J = q / 16, b = q % 16 / 4, s = q % 4, down = J & 1;
+        const int i = 2 * (down ? 3 - b : b) + ((s == 1 || s == 2) != down), j = 2 * J + ((s >= 2) != (b & 1));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
+      };
+      // a half stage: the products of the operands read before, reads of the next half's, the loads of a stage of one operand
+      auto half_stage = [&](auto second) __attribute__((always_inline)) {
+        constexpr bool B = decltype(second)::value;
 #pragma unroll
-      for (int r = 0; r < MW + NW; ++r) take1(h, r, xf, wf);
-    };
-    auto fill = [&](int m, int freed_x, int freed_w) {  // load m of the eight behind a barrier: rows of the next stage but one
-      if (m < 4) load_x(m, freed_w);                    // where the stage's weights were, then weights of the one behind it
-      else load_w(m - 4, freed_x);
-    };
-    // the order inside a half stage: 32 MFMAs, a read behind each second, a load behind each fourth.  Without the fences the
-    // compiler moves the MFMAs behind the barrier and the reads stand alone.
-    auto order = [&](bool loads) {
-#pragma unroll
-      for (int m = 0; m < NW * MW; ++m) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (m < 24 && m % 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (FORM == COLUMNS && m < 24 && m % 2 && m / 2 >= MW) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (loads && m % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    auto turn = [&] {  // to the next stage's slots
-      px = px >= SLOTS - 2 ? px + 2 - SLOTS : px + 2;
-      pw = pw >= SLOTS - 2 ? pw + 2 - SLOTS : pw + 2;
-    };
-    // the next stage has landed for all waves, and all have read this one.  In flight: the weights of the stage after it and
-    // the stores of the tile before
-    auto meet = [&](int stored) {
-      if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + Work::STORES) : "memory");
-      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      lds_wait_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-#pragma unroll 1
-    for (int s = 0; s < SLOTS; s += 2) {  // w 0, x 0, w 1, x 1, w 2
-#pragma unroll
-      for (int j = 0; j < 4; ++j) load_w(j, s);
-      next_w();
-      if (s + 1 == SLOTS) break;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) load_x(j, s + 1);
-      next_x();
-    }
-    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-    lds_wait_barrier();
-    take(0, xa, wa);
-    int stored = 0;
-    for (int k = 0; k < count; ++k) {
-      const int n = work.stages(k);
-      if (!work.live(k)) {
-        for (int st = 0; st < n; ++st) {
-          meet(stored);
-          stored = 0;
-          const int fx = px, fw = pw;
-          turn();
-#pragma unroll
-          for (int m = 0; m < 8; ++m) fill(m, fx, fw);
-          next_x();
-          next_w();
+        for (int q = 0; q < NW * M; ++q) {
+          constexpr int AT = B ? 1 : M - 3;
+          if (q % M == AT - 1) aim(B ? x : w, q / M, B ? fw : fx);
+          multiply1(q, B ? xb : xa, B ? wb : wa);
+          if (q % R == R - 1 && q / R < M + NW) take1(!B, q / R, xr, B ? xa : xb, B ? wa : wb, M);
+          if (q % M == AT) load(B ? x : w, q / M, B ? fw : fx);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        take(0, xa, wa);
-        continue;
+      };
+      if (mode != M) {  // (read for the tile before, which had other rows)
+#pragma unroll
+        for (int r = 0; r < M; ++r) take1(0, r, xr, xa, wa, M);
+        mode = M;
       }
 #pragma unroll
       for (int i = 0; i < NW; ++i)
 #pragma unroll
-        for (int j = 0; j < MW; ++j) acc[i][j] = (f32x4)(0.f);
+        for (int j = 0; j < M; ++j) acc[i][j] = (f32x4)(0.f);
+      asm volatile("s_nop 7");
+      const int n = work.stages(k);
+#pragma unroll 1
       for (int st = 0; st < n; ++st) {
         __builtin_amdgcn_sched_barrier(0);
-        take(1, xb, wb);
-        multiply(xa, wa);
-        order(false);
-        meet(stored);
+        half_stage(Int<0>());
+        // the next stage has landed for all waves, and all have read this one.  In flight: the weights of the stage after the
+        // next and the stores of the tile before
+        if (stored == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+        else if (stored < Work::STORES) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES + Work::STORES / 2) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES + Work::STORES) : "memory");
         stored = 0;
-        const int fx = px, fw = pw;
-        turn();
-        if constexpr (FORM == COLUMNS) {  // (its loads are of no kind that ``order`` knows)
-#pragma unroll
-          for (int i = 0; i < NW; ++i) {
-            if (i < 6) take1(0, 2 * i, xa, wa), take1(0, 2 * i + 1, xa, wa);
-            multiply1(i, xb, wb);
-            fill(i, fx, fw);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          next_x();
-          next_w();
-          continue;
-        }
-#pragma unroll
-        for (int m = 0; m < NW * MW; ++m) {  // (loads write LDS: the compiler keeps the order of loads and reads)
-          if (m < 24 && m % 2) take1(0, m / 2, xa, wa);
-          if (m % 4 == 3) fill(m / 4, fx, fw);
-        }
-        multiply(xb, wb);
-        order(true);
-        next_x();
-        next_w();
+        asm volatile("" : "+s"(stored));  // (one loop: the compiler would make the first stage a second one)
+        lds_wait_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        fx = px, fw = pw;
+        px = px >= SLOTS - 2 ? px + 2 - SLOTS : px + 2;
+        pw = pw >= SLOTS - 2 ? pw + 2 - SLOTS : pw + 2;
+        half_stage(Int<1>());
+        step();
       }
-      stored = work.store(k, acc);
+      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // (the last sums, which asm reads)
+      stored = work.template store<M>(k, acc);
+    };
+#pragma unroll 1
+    for (int s = 0; s < 2; ++s) {  // w 0, x 0, w 1, x 1
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j) load_now(w, j, 2 * s);
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j) load_now(x, j, 2 * s + 1);
+      step();
+    }
+    fx = SLOTS - 1;  // (w 2)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PIECES) : "memory");
+    lds_wait_barrier();
+#pragma unroll
+    for (int r = 0; r < NW; ++r) take1(0, r, 0, xa, wa, 0);
+    for (int k = 0; k < count; ++k) {
+      if (work.half(k)) tile(Int<MW / 2>(), k);
+      else tile(Int<MW>(), k);
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   }
 
-  // Rows of ``acc`` from m on (those below ``end``) to out[row][cols], columns from ``col`` on.  GLU: ``act`` makes one of each
-  // two fragments (gate, up), else of each one.  A lane holds 4 columns of a row in a fragment; neighbouring fragments trade
-  // halves between the lane's rows of 16, so that a lane stores 16 bytes and an instruction 64 bytes of each of 16 rows (8
-  // bytes a lane: 6421 x 12288 x 4096 506 -> 480 us).  ``wide``: out is 16-byte aligned.  True: all of them were stored.
+  // A sum out of the accumulation registers, where and when it is asked for: left to the compiler all 256 are moved at once,
+  // more than there is room for.
+  static __device__ __forceinline__ f32x4 taken(const f32x4& a) {
+    f32x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float t;
+      asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(t) : "a"(a[r]));
+      y[r] = t;
+    }
+    return y;
+  }
+
+  // Rows of ``acc`` (``run``, fragments M) to out[row][cols], ``out`` the tile's first row of ``rows``, columns from ``col`` on.
+  // GLU: ``act`` makes one of each two fragments (gate, up), else of each one.  A lane holds 4 columns of a row in a fragment;
+  // neighbouring fragments trade halves between the lane's rows of 16, so that a lane stores 16 bytes and an instruction 64
+  // bytes of each of 16 rows (8 bytes a lane: 6421 x 12288 x 4096 506 -> 480 us with eight waves).  Rows and columns that are
+  // not there are stored behind the end of the buffer, which drops them: all stores are issued.
   static constexpr int put_stores(bool glu) { return MW * NW / (glu ? 4 : 2); }
-  template <bool GLU, class Act>
-  static __device__ __forceinline__ bool put(bf16_t* out, int cols, bool wide, int m, int end, int col, const f32x4 (&acc)[NW][MW],
-                                             Act act) {
+  template <bool GLU, int M, class Act>
+  static __device__ __forceinline__ int put(bf16_t* out, int cols, int rows, int col, const f32x4 (&acc)[NW][MW], Act act) {
     constexpr int S = GLU ? 2 : 1;
     const int c16 = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4, lc = col + 16 * (g4 & 1) + 8 * (g4 >> 1);
-    const bool whole = wide && m + 16 * MW <= end && col + 16 * NW / S <= cols;
-    bf16_t* at = out + (int64_t)(m + c16) * cols + lc;
-    auto each = [&](auto store) {
+    const int m = 16 * M * wm() + c16;
+    const bool whole = 16 * M * WM <= rows && col + 16 * NW / S <= cols;
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(out, (short)0, min(rows, BM) * cols * 2, 0x00020000);
+    const uint32_t at = (uint32_t)(m * cols + lc) * 2;  // (the launchers check that a tile's rows are below 2^31 bytes)
 #pragma unroll
-      for (int j = 0; j < MW; ++j) {
+    for (int j = 0; j < M; ++j) {
 #pragma unroll
-        for (int i = 0; i < NW; i += 2 * S) {
-          uint32_t d[2][2];
+      for (int i = 0; i < NW; i += 2 * S) {
+        uint32_t d[2][2];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            float y[4];
-            act(acc[i + h * S][j], acc[i + h * S + S - 1][j], y);
+        for (int h = 0; h < 2; ++h) {
+          float y[4];
+          const f32x4 v = taken(acc[i + h * S][j]);
+          act(v, GLU ? taken(acc[i + h * S + S - 1][j]) : v, y);
 #pragma unroll
-            for (int r = 0; r < 2; ++r) d[h][r] = (uint32_t)f2bf(y[2 * r]) | (uint32_t)f2bf(y[2 * r + 1]) << 16;
-          }
-          const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false));
-          const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false));
-          store(j, 16 * i / S, at + (int64_t)16 * j * cols + 16 * i / S, (u32x4){a[0], b[0], a[1], b[1]});
+          for (int r = 0; r < 2; ++r)
+            d[h][r] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){y[2 * r], y[2 * r + 1]}, bf16x2));
         }
+        const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false));
+        const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false));
+        const bool there = whole || (m + 16 * j < rows && lc + 16 * i / S < cols);  // (columns come in sixteens)
+        __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], b[0], a[1], b[1]}, to, there ? at : 1u << 31,
+                                               (16 * j * cols + 16 * i / S) * 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    };
-    if (whole) {
-      each([](int, int, bf16_t* p, const u32x4& v) { *reinterpret_cast<u32x4*>(p) = v; });
-    } else {
-      each([&](int j, int c, bf16_t* p, const u32x4& v) {
-        if (m + 16 * j + c16 >= end || lc + c >= cols) return;  // (columns come in sixteens)
-        *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
-        *reinterpret_cast<u32x2*>(p + 4) = (u32x2){v[2], v[3]};
-      });
     }
-    return whole;
+    return put_stores(GLU) * M / MW;
   }
 };
 

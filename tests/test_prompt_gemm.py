@@ -60,6 +60,8 @@ def test_left_over_tiles_in_parts(M, N, K):
 # more tiles than workgroups (256): a ring of five slots runs on into the next tile, of 1, 3 and 32 stages; last tiles of 18 rows
 # or of 3, whose other waves have none; whole tiles alone, and one with a part behind it
 MANY = [(1554, 14352, 64), (1554, 14336, 192), (1554, 14336, 2048), (4100, 4096, 2048), (4099, 4112, 2048), (8195, 4096, 128)]
+# last tiles of 64, 65, 128 rows, which workgroups make with half a wave's rows between whole ones, and of 129
+MANY += [(1600, 14336, 192), (1601, 14336, 64), (1664, 14336, 128), (1665, 14336, 192)]
 
 
 @pytest.mark.gpu
