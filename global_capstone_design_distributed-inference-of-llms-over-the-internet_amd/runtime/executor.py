@@ -783,11 +783,11 @@ class StageExecutor:
                     ops.rmsnorm(h, g_in, eps, out=xn, residual=res, mode=2)
                 else:
                     ops.rmsnorm(mlp, g_in, eps, out=xn, residual=res, mode=1)
-                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p)
+                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p, tiles=bool(L.moe))
                 kc, vc = self.cache.layer(li)
                 self._rope_attend(qkv, positions, slots, kc, vc, q_seq, q_ctx, attn, ws, ps, np_, False, qblocks,
                                   max_ctx, decode)
-                ops.linear(attn, L.dense("o"), out=o, wp=L.o_p)
+                ops.linear(attn, L.dense("o"), out=o, wp=L.o_p, tiles=bool(L.moe))
                 self._ar(o)
                 ops.rmsnorm(o, g_post, eps, out=xn, residual=res, mode=1)
                 if L.moe:
