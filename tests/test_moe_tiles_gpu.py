@@ -179,3 +179,30 @@ def test_which_rows_are_ordered():
     for ff, tokens, packed, want in ((14336, 2700, False, True), (4096, 512, False, True), (4096, 511, False, False),
                                      (4032, 2700, False, False), (1408, 4298, False, False), (14336, 2700, True, False)):
         assert (moe._parts(MoESpec(8, 2, ff, 1.0), tokens, packed) > 0) == want
+
+
+@pytest.mark.parametrize("counts", [[1, 0], [16, 17], [33, 64], [65, 3]])
+def test_few_rows_of_large_experts(counts):
+    """64 MB of experts and more come past the caches where an expert's rows are one pass (64), else from them; an odd number of
+    weight tiles.  One sum of K exact products in 32 bits: 1e-5, gated ones rounded to bf16."""
+    ops.require_native()
+    E, N, K, R = 2, 4128, 4096, sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(R, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(E, N, K, generator=g, device="cuda").div(K ** 0.5).to(torch.bfloat16)
+    owner = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).tolist()
+    tok = torch.arange(R, dtype=torch.int32, device="cuda")
+    for rows in (N, N - 16):  # the second: 257 tiles, 67 MB
+        v = w[:, :rows].contiguous()
+        assert v.numel() * 2 >= 64 << 20
+        wp, lists = torch.stack([ops.pack_weight(m) for m in v]), _lists(counts)
+        z = torch.stack([v[e].double() @ x[i].double() for i, e in enumerate(owner)])
+        out = torch.full((R, rows), float("nan"), device="cuda")
+        torch.ops.mpamd.moe_gemm(1, x, tok, lists, wp, out, R, R, 0, 1, 0.0, 0)
+        assert float((out.double() - z).norm() / z.norm()) < 1e-5
+        if rows % 32 == 0:
+            u = z.view(R, rows // 32, 2, 16)
+            want = torch.nn.functional.silu(u[:, :, 0].reshape(R, -1)) * u[:, :, 1].reshape(R, -1)
+            act = torch.full((R, rows // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
+            torch.ops.mpamd.moe_gemm(1, x, tok, lists, wp, act, R, R, 1, 16, 0.0, 0)
+            assert float((act.double() - want).norm() / want.norm()) < 2.0 ** -8
