@@ -10,6 +10,9 @@ as a model's do not stay there from one step to the next) run here at the row-ti
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
 both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
 
+A second table holds the same of 1 to 256 rows whose weights have no packed copy (a short fine-tuning request): there the
+library leaves most CUs idle at some shapes, 60 rows of 4096 columns of a 28672-row matrix took 163 us, 60 here.
+
 Everything else keeps the library.  (No rule on the shape alone holds at the shapes that were timed: "less than a wave of
 tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at 10 of 31 row-tile counts.)
 """
@@ -24,13 +27,15 @@ from typing import Dict, FrozenSet, Iterable, Optional, Tuple
 import torch
 
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "prompt_gemm_gfx950.json")
+FEW_TABLE = TABLE.replace("prompt_gemm", "prompt_few")  # the same of few rows: 1 to 4 for up to 32, 64, 128, 256
 COLUMNS = 8  # in an epilogue's place: x w
 EPILOGUES = (0, 1, 4, COLUMNS)
 TILE, MAX_ROWS = 256, 8192
+FEW = (32, 64, 128, TILE)  # (a tile of up to 128 rows takes half the products; the library's times jump at all four)
 Shape = Tuple[int, int, int]  # N, K, epilogue
 
 _LOCK = threading.Lock()
-_STATE: dict = {"table": None}
+_STATE: dict = {"table": None, "few": None}
 
 
 def _key(shape: Shape) -> str:
@@ -48,13 +53,15 @@ def _load(path: str) -> Dict[Shape, FrozenSet[int]]:
     return out
 
 
-def table() -> Dict[Shape, FrozenSet[int]]:
-    """(N, K, epilogue) -> row-tile counts at which the kernel runs (read once; MPAMD_KERNEL_TABLE=0: none)."""
+def table(name: str = "table") -> Dict[Shape, FrozenSet[int]]:
+    """(N, K, epilogue) -> row-tile counts at which the kernel runs (read once; MPAMD_KERNEL_TABLE=0: none); ``few``: the
+    same of ``FEW``'s ranges."""
     with _LOCK:
-        if _STATE["table"] is None:
-            on = os.environ.get("MPAMD_KERNEL_TABLE") != "0" and os.path.exists(TABLE)
-            _STATE["table"] = _load(TABLE) if on else {}
-        return _STATE["table"]
+        if _STATE[name] is None:
+            path = FEW_TABLE if name == "few" else TABLE
+            on = os.environ.get("MPAMD_KERNEL_TABLE") != "0" and os.path.exists(path)
+            _STATE[name] = _load(path) if on else {}
+        return _STATE[name]
 
 
 def shape_ok(M: int, N: int, K: int, epilogue: int) -> bool:
@@ -66,6 +73,12 @@ def shape_ok(M: int, N: int, K: int, epilogue: int) -> bool:
 def chosen(M: int, N: int, K: int, epilogue: int) -> bool:
     """Does a step of M rows run this product here?"""
     return TILE < M <= MAX_ROWS and shape_ok(M, N, K, epilogue) and -(-M // TILE) in table().get((N, K, epilogue), ())
+
+
+def few(M: int, N: int, K: int, epilogue: int) -> bool:
+    """The same of a step of few rows, whose weights have no packed copy."""
+    return M <= TILE and shape_ok(M, N, K, epilogue) and \
+        next(i for i, n in enumerate(FEW, 1) if M <= n) in table("few").get((N, K, epilogue), ())
 
 
 def _reads(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -82,8 +95,10 @@ def _reads(x: torch.Tensor, w: torch.Tensor) -> bool:
 def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
     """Is this product of rows [M, K] with weights [N, K] one that runs here?  Callers that differentiate it, and operands
     the kernel does not read, keep the library's."""
-    return w is not None and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and \
-        chosen(x.shape[0], w.shape[0], w.shape[1], epilogue) and _reads(x, w)
+    if w is None or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        return False
+    shape = x.shape[0], w.shape[0], w.shape[1], epilogue
+    return (chosen(*shape) or few(*shape)) and _reads(x, w)
 
 
 def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0):
@@ -105,8 +120,11 @@ def gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, e
 
 def gemm_columns(x: torch.Tensor, w: torch.Tensor, always: bool = False) -> torch.Tensor:
     """x w of rows [M, K] and weights [K, N]: on the kernel where the table says so (or ``always``), else the library's."""
-    if always or (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[0] and
-                  chosen(x.shape[0], w.shape[1], w.shape[0], COLUMNS) and _reads(x, w)):
+    here = always
+    if not always and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[0]:
+        shape = x.shape[0], w.shape[1], w.shape[0], COLUMNS
+        here = (chosen(*shape) or few(*shape)) and _reads(x, w)
+    if here:
         return _run(x, w, torch.empty(x.shape[0], w.shape[1], dtype=x.dtype, device=x.device), w.shape[1], COLUMNS)
     return torch.mm(x, w)
 
@@ -147,13 +165,18 @@ def agreed(sweeps: Iterable[Dict[Shape, list]]) -> Dict[Shape, list]:
     return {s: [m for m in v if all(m in r[s] for r in rest)] for s, v in first.items()}
 
 
-def tune(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
-    """The row-tile counts of every shape at which the kernel is faster, in both of two sweeps."""
+ROWS = {m: (TILE * m - 251, TILE * m - 124, TILE * m) for m in range(2, MAX_ROWS // TILE + 1)}
+FEW_ROWS = {1: (8, 16, 32), 2: (33, 48, 64), 3: (65, 96, 128), 4: (129, 192, 256)}
+
+
+def tune(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS) -> Dict[Shape, list]:
+    """The row-tile counts of every shape at which the kernel is faster, in both of two sweeps (``rows``: what is timed of
+    each)."""
     todo = list(todo)
-    return agreed([sweep(todo, device, log) for _ in range(2)])
+    return agreed([sweep(todo, device, log, rows) for _ in range(2)])
 
 
-def sweep(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
+def sweep(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS) -> Dict[Shape, list]:
     """Time both products over the row-tile counts of every shape, best of three rounds in turn."""
     from . import hybrid, require_native, swiglu, use_tuned_gemms
 
@@ -178,9 +201,9 @@ def sweep(todo: Iterable[Shape], device="cuda", log=None) -> Dict[Shape, list]:
               for _ in range(many)]
         turn = itertools.cycle(ws)
         tiles = []
-        for m in range(2, MAX_ROWS // TILE + 1):
+        for m, counts in rows.items():
             ratios = []
-            for M in (TILE * m - 251, TILE * m - 124, TILE * m):
+            for M in counts:
                 x = torch.randn(M, K, device=device).to(torch.bfloat16)
                 z = torch.empty(M, N, dtype=x.dtype, device=device)
                 y = torch.empty(M, N // 2 if epi == 1 else N, dtype=x.dtype, device=device)

@@ -138,7 +138,10 @@ def tune_prompt(out=None) -> int:
         print("tune: needs an MI355X", file=sys.stderr)
         return 2
     todo = sorted({s for cfg in PRESETS.values() for f in (prompt.shapes, prompt.train_shapes) for s in f(cfg)})
-    prompt.save(out or prompt.TABLE, prompt.tune(todo, log=lambda m: print(f"tune: {m}", file=sys.stderr, flush=True)))
+    log = lambda m: print(f"tune: {m}", file=sys.stderr, flush=True)  # noqa: E731
+    prompt.save(out or prompt.TABLE, prompt.tune(todo, log=log))
+    few = (out + ".few") if out else prompt.FEW_TABLE
+    prompt.save(few, prompt.tune(todo, log=log, rows=prompt.FEW_ROWS))
     return 0
 
 

@@ -166,3 +166,30 @@ def test_sweeps_have_to_agree():
 def test_committed_table_reads():
     t = prompt._load(prompt.TABLE)
     assert t and all(prompt.shape_ok(8192, *s) and all(2 <= m <= 32 for m in v) for s, v in t.items())
+
+
+def test_few_rows(monkeypatch):
+    """Up to 256 rows go by a table of their own, whose four ranges end at 32, 64, 128 and 256."""
+    assert all(prompt.shape_ok(256, *s) and all(1 <= m <= 4 for m in v) for s, v in prompt._load(prompt.FEW_TABLE).items())
+    for got, (lo, hi) in {1: (1, 32), 2: (33, 64), 3: (65, 128), 4: (129, 256)}.items():
+        monkeypatch.setitem(prompt._STATE, "few", {(4096, 4096, 0): frozenset({got})})
+        assert [M for M in range(1, 400) if prompt.few(M, 4096, 4096, 0)] == list(range(lo, hi + 1))
+        assert set(prompt.FEW_ROWS[got]) <= set(range(lo, hi + 1))
+    assert not prompt.few(200, 4096, 4096, 1) and not prompt.few(200, 4096, 8192, 0) and not prompt.chosen(200, 4096, 4096, 0)
+    monkeypatch.setenv("MPAMD_KERNEL_TABLE", "0")
+    monkeypatch.setitem(prompt._STATE, "few", None)
+    assert prompt.table("few") == {}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 33, 128, 129, 256])
+@pytest.mark.parametrize("N,K,epi", [(4096, 28672, 8), (4096, 14336, 0)])
+def test_products_of_few_rows(M, N, K, epi):
+    """One row tile whose K is cut into as many parts as fill the CUs."""
+    ops.require_native()
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(*((K, N) if epi == 8 else (N, K)), device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    want = x.double() @ (w.double() if epi == 8 else w.double().t())
+    got = prompt._run(x, w, torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda"), N, epi)
+    assert float((got.double() - want).norm() / want.norm()) < BF16
