@@ -192,8 +192,7 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
                             float* ws, hipStream_t stream) {
   (void)hipGetLastError();
   using namespace mp;
-  if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31) ||
-      N >= 1 << 22)  // (a tile's rows of the output below 2^31 bytes)
+  if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31))
     return -1;
   if (epi == 1 && N % 32) return -2;
   GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, (M + 255) / 256, (N + 255) / 256, 0, 0, 1, ws};

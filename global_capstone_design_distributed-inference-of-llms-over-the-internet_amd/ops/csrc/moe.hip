@@ -1052,7 +1052,7 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
     // 256 x 256 tiles from 128 rows an expert on (ops/moe.py expert_form); where K is not in steps of 64, or a piece's
     // byte offset does not fit 32 bits, the ring of 32-column stages: its 256 x 256 form from 384 rows on, else 128 x 128
     const bool wide = form == 3 && K % 64 == 0 && (int64_t)rows * xs < (1ll << 31) && (int64_t)N * K < (1ll << 31) &&
-                      N < 1 << 22 && (uintptr_t)out % 4 == 0;
+                      (uintptr_t)out % 4 == 0;
     const bool big = form == 3 && rows >= 384 * E;
 #define MP_MT(GLU_, TO_)                                                        \
   return wide  ? launch_moe_wide<GLU_, TO_>(a, rows, act, GLU_ || sizeof(TO_) != 2 ? nullptr : ws, stream) \

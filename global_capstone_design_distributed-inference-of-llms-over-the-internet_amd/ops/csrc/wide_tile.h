@@ -248,12 +248,14 @@ struct WideTile {
   static __device__ __forceinline__ int put(bf16_t* out, int cols, int rows, int col, const f32x4 (&acc)[NW][MW], Act act) {
     constexpr int S = GLU ? 2 : 1;
     const int c16 = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4, lc = col + 16 * (g4 & 1) + 8 * (g4 >> 1);
-    const int m = 16 * M * wm() + c16;
-    const bool whole = 16 * M * WM <= rows && col + 16 * NW / S <= cols;
-    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(out, (short)0, min(rows, BM) * cols * 2, 0x00020000);
-    const uint32_t at = (uint32_t)(m * cols + lc) * 2;  // (the launchers check that a tile's rows are below 2^31 bytes)
+    const uint32_t at = (uint32_t)(c16 * cols + lc) * 2;
+    // a buffer is 16 rows: their bytes fit 31 bits wherever a matrix of as many columns and 64 rows has fewer than 2^31 elements
+    int left = rows - 16 * M * wm();
+    bf16_t* p = out + (int64_t)(16 * M * wm()) * cols;
 #pragma unroll
-    for (int j = 0; j < M; ++j) {
+    for (int j = 0; j < M; ++j, left -= 16, p += 16 * cols) {
+      const int bytes = left >= 16 ? 32 * cols : left > 0 ? 2 * left * cols : 0;  // (min and max would be made in lanes)
+      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(p, (short)0, bytes, 0x00020000);
 #pragma unroll
       for (int i = 0; i < NW; i += 2 * S) {
         uint32_t d[2][2];
@@ -268,9 +270,8 @@ struct WideTile {
         }
         const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false));
         const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false));
-        const bool there = whole || (m + 16 * j < rows && lc + 16 * i / S < cols);  // (columns come in sixteens)
-        __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], b[0], a[1], b[1]}, to, there ? at : 1u << 31,
-                                               (16 * j * cols + 16 * i / S) * 2, 0);
+        const bool there = lc + 16 * i / S < cols;  // (columns come in sixteens)
+        __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], b[0], a[1], b[1]}, to, there ? at : 1u << 31, 32 * i / S, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }

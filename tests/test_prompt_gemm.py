@@ -85,6 +85,21 @@ def test_several_tiles_to_a_workgroup(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 40, 130])
+def test_output_rows_of_many_columns(M):
+    """A tile's 256 rows of the output are more than 2^31 bytes; K exact products in 32 bits, rounded once."""
+    ops.require_native()
+    N, K = (1 << 22) + 48, 64
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).to(torch.bfloat16)
+    out = prompt.gemm(x, w, torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda"), 0)
+    for n in range(0, N, 1 << 20):
+        want = x.double() @ w[n:n + (1 << 20)].double().t()
+        assert float((out[:, n:n + (1 << 20)].double() - want).norm() / want.norm()) < BF16
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
 def test_products_with_columns(M, N, K):
     """x w, as a gradient goes back through a projection: ends of tiles and of a wave's columns, tiles in parts."""
