@@ -497,24 +497,36 @@ __device__ __forceinline__ void moe_rows_pass(const MoeGemm& a, const bf16_t* __
   f32x4 acc[NR][2];
 #pragma unroll
   for (int i = 0; i < NR; ++i) acc[i][0] = acc[i][1] = (f32x4)(0.f);
-  for (int s0 = wv; s0 < ks; s0 += 4 * U) {
-    u16x8 wf[U][2], xf[U][NR];
+  u16x8 wf[U][2], xf[U][NR];
+  const int mine = (ks - wv + 3) >> 2;  // this wave's steps
+  auto load = [&](int u, int s) {
+    const int64_t st = wv + 4 * min(s, mine - 1);  // (past the end: loaded, not used)
+    const u16x8 *p0 = reinterpret_cast<const u16x8*>(w0 + st * 512 + lane * 8), *p1 = reinterpret_cast<const u16x8*>(w1 + st * 512 + lane * 8);
+    wf[u][0] = ONCE ? __builtin_nontemporal_load(p0) : *p0;
+    wf[u][1] = ONCE ? __builtin_nontemporal_load(p1) : *p1;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t st = min(s0 + 4 * u, ks - 1);
-      const u16x8 *p0 = reinterpret_cast<const u16x8*>(w0 + st * 512 + lane * 8), *p1 = reinterpret_cast<const u16x8*>(w1 + st * 512 + lane * 8);
-      wf[u][0] = ONCE ? __builtin_nontemporal_load(p0) : *p0;
-      wf[u][1] = ONCE ? __builtin_nontemporal_load(p1) : *p1;
+    for (int i = 0; i < NR; ++i) xf[u][i] = *reinterpret_cast<const u16x8*>(xp[i] + st * xstep);
+  };
+  auto sum = [&](int u) {
 #pragma unroll
-      for (int i = 0; i < NR; ++i) xf[u][i] = *reinterpret_cast<const u16x8*>(xp[i] + st * xstep);
-    }
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc[i][h] = mfma_bf(wf[u][h], xf[u][i], acc[i][h]);
+  };
+  if (mine > 0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, u);
+    int s = 0;
+    for (; s + U < mine; s += U)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        sum(u);
+        load(u, s + U + u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (s0 + 4 * u < ks)  // (uniform)
-#pragma unroll
-        for (int i = 0; i < NR; ++i)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) acc[i][h] = mfma_bf(wf[u][h], xf[u][i], acc[i][h]);
+      if (s + u < mine) sum(u);  // (uniform)
   }
   __syncthreads();  // (the previous pass has read its sums)
 #pragma unroll
@@ -553,7 +565,7 @@ __device__ __forceinline__ void moe_rows(const MoeGemm& a, const bf16_t* __restr
                                          int n, int o0, int nt1, float* red) {
   for (int m0 = 0; m0 < n; m0 += 64) {
     const int left = n - m0;
-    if (left <= 16) moe_rows_pass<GLU, 1, 8, ONCE>(a, w0, w1, r0, m0, n, o0, nt1, red);
+    if (left <= 16) moe_rows_pass<GLU, 1, 6, ONCE>(a, w0, w1, r0, m0, n, o0, nt1, red);
     else if (left <= 32) moe_rows_pass<GLU, 2, 4, ONCE>(a, w0, w1, r0, m0, n, o0, nt1, red);
     else moe_rows_pass<GLU, 4, 4, ONCE>(a, w0, w1, r0, m0, n, o0, nt1, red);
   }

@@ -206,3 +206,22 @@ def test_few_rows_of_large_experts(counts):
             act = torch.full((R, rows // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
             torch.ops.mpamd.moe_gemm(1, x, tok, lists, wp, act, R, R, 1, 16, 0.0, 0)
             assert float((act.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("K", [32, 96, 128, 672, 768, 800, 1408, 1568])
+@pytest.mark.parametrize("n", [1, 17, 40])
+def test_few_rows_of_any_depth(n, K):
+    """Waves without a 32-column step, with fewer than are in flight at once (6, or 4 from 17 rows on), as many, one more and
+    one less.  One sum of K exact products in 32 bits."""
+    ops.require_native()
+    counts = [n, 0, 3]
+    E, N, R = len(counts), 48, sum(counts)
+    g = torch.Generator().manual_seed(K + n)
+    x = torch.randn(R, K, generator=g).to(torch.bfloat16)
+    w = torch.randn(E, N, K, generator=g).div(K ** 0.5).to(torch.bfloat16)
+    owner = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).tolist()
+    z = torch.stack([w[e].double() @ x[i].double() for i, e in enumerate(owner)])
+    out = torch.full((R, N), float("nan"), device="cuda")
+    torch.ops.mpamd.moe_gemm(1, x.cuda(), torch.arange(R, dtype=torch.int32, device="cuda"), _lists(counts),
+                             torch.stack([ops.pack_weight(m) for m in w.cuda()]), out, R, R, 0, 1, 0.0, 0)
+    assert float((out.double().cpu() - z).norm() / z.norm()) < 1e-5
