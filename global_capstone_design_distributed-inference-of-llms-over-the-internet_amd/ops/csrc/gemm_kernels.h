@@ -258,26 +258,32 @@ __device__ __forceinline__ int rw_krot(int n, int on) {
 
 constexpr int GU_MAX = 4;  // k-slices (of 32) per wave group (x 16 B per lane per column tile)
 
-template <int MT, int NT, int EPI, bool APK, bool OPK>
-__global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
-                                                          const bf16_t* __restrict__ wp, bf16_t* __restrict__ y,
-                                                          int64_t y_stride, const bf16_t* __restrict__ res,
-                                                          int64_t res_stride, int M, int N, int K,
-                                                          const EpiArgs ep) {
-  clear_other(ep);
-  __shared__ u64 rs_part[SS_PG][SS_ROWS];
-  __shared__ float rs_lds[SS_ROWS];
+// One workgroup's NT column tiles from ``nt0`` on.
+//
+// Bound by the weights' bytes, and short of them by what is not in flight while a workgroup begins and ends.  Up to 16 rows, and
+// up to 32 with two column tiles, every slice's registers take the load of the slice GU later as soon as its products are made
+// (one group in flight: 70 and 102 registers, three and two workgroups a CU; the sums and their order are the same).  The ping-pong of
+// two groups, which the other forms keep, held 132 and 190, one workgroup a CU: at 4096 columns and 16 rows 16384 weight rows
+// took 23.5 us (now 21.3), 28672 gated 40.7 (37.7), 32000 43.3 (39.3); 32 rows, 22016 gated 36.9 (34.3).  At 48 and 64 rows the
+// ping-pong is up to 8 % faster, at 32 rows and one tile 2 %.
+template <int MT, int NT>
+constexpr bool pk_rolling() { return MT == 1 || (MT == 2 && NT == 2); }
+
+template <int MT, int NT, int EPI, bool APK, bool OPK, bool ROLLING>
+__device__ __forceinline__ void gemm_packed_body(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                 const bf16_t* __restrict__ wp, bf16_t* __restrict__ y,
+                                                 int64_t y_stride, const bf16_t* __restrict__ res, int64_t res_stride,
+                                                 int M, int N, int K, const EpiArgs& ep, int nt0, float (*red)[MT * NT * 4][64],
+                                                 u64 (*rs_part)[SS_ROWS], float* rs_lds) {
   RowScale<EPI < 2> rsc;
   // fewer k-slices per group for the widest tiles keeps A + 2 x B + acc inside 256 VGPRs
   constexpr int GU = (MT * NT >= 6) ? 2 : 4;
-  __shared__ __attribute__((aligned(16))) float red[8][MT * NT * 4][64];
   // wave id made provably uniform (readfirstlane): the group loop then compiles to scalar
   // branches instead of an exec-masked divergent loop around the MFMAs
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, q = lane >> 4;
   const int nks = K >> 5;
   const int ngroups = nks / GU;
-  const int nt0 = blockIdx.x * NT;
 
   const bf16_t* wbase[NT];
 #pragma unroll
@@ -314,11 +320,48 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[mt][t] = (f32x4)(0.f);
 
-  // Ping-pong weight buffers (no register copies, which would force a vmcnt(0)), and the
-  // A fragments of group g issued BEFORE the prefetch of group g+8: vmcnt retires loads in
-  // issue order, so waiting for A leaves the weight prefetch in flight across the MFMAs.
-  u16x8 b0[NT][GU], b1[NT][GU], a[MT][GU];
   const int grot = rw_krot(ngroups, ep.rot);
+  int g = wid;
+  if constexpr (ROLLING && APK) {
+    u16x8 a[MT][GU], b[NT][GU];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      if (mt * 16 + c >= M) xrow[mt] -= c * 8;  // (load_a_rows: a row that is not there reads its tile's first)
+    auto load = [&](int u, int grp) {
+      const int64_t s = rw_rot(grp, grot, ngroups) * GU + u;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) a[mt][u] = MP_LOAD_A_FRAG(xrow[mt] + s * MT * 512);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b[t][u] = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(wbase[t] + s * 512));
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[mt][t] = mfma16(a[mt][u], b[t][u], acc[mt][t]);
+    };
+    if (g < ngroups) {
+#pragma unroll
+      for (int u = 0; u < GU; ++u) load(u, g);
+    }
+    rsc.load(ep, wp);
+    for (; g + 8 < ngroups; g += 8) {
+#pragma unroll
+      for (int u = 0; u < GU; ++u) {
+        multiply(u);
+        load(u, g + 8);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (g < ngroups) {
+#pragma unroll
+      for (int u = 0; u < GU; ++u) multiply(u);
+    }
+  } else {
+    // Ping-pong weight buffers (no register copies, which would force a vmcnt(0)), and the
+    // A fragments of group g issued BEFORE the prefetch of group g+8: vmcnt retires loads in
+    // issue order, so waiting for A leaves the weight prefetch in flight across the MFMAs.
+    u16x8 b0[NT][GU], b1[NT][GU], a[MT][GU];
 #define MP_LOAD_B(dst, grp)                                                                                   \
   _Pragma("unroll") for (int t = 0; t < NT; ++t) _Pragma("unroll") for (int u = 0; u < GU; ++u) dst[t][u] =    \
       __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(wbase[t] + (int64_t)(rw_rot(grp, grot, ngroups) * GU + u) * 512));
@@ -329,34 +372,34 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
 #define MP_MMA(bb)                                                                                            \
   _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) _Pragma("unroll") for (int u = 0; u < GU; ++u)            \
       _Pragma("unroll") for (int t = 0; t < NT; ++t) acc[mt][t] = mfma16(a[mt][u], bb[t][u], acc[mt][t]);
-  int g = wid;
-  if (g < ngroups) {
-    MP_LOAD_B(b0, g)
-  }
-  rsc.load(ep, wp);
-  while (g < ngroups) {
-    MP_LOAD_A(g)
-    if (g + 8 < ngroups) {
-      MP_LOAD_B(b1, g + 8)
-      MP_MMA(b0)
-    } else {
-      MP_MMA(b0)
-      break;
+    if (g < ngroups) {
+      MP_LOAD_B(b0, g)
     }
-    g += 8;
-    MP_LOAD_A(g)
-    if (g + 8 < ngroups) {
-      MP_LOAD_B(b0, g + 8)
-      MP_MMA(b1)
-    } else {
-      MP_MMA(b1)
-      break;
+    rsc.load(ep, wp);
+    while (g < ngroups) {
+      MP_LOAD_A(g)
+      if (g + 8 < ngroups) {
+        MP_LOAD_B(b1, g + 8)
+        MP_MMA(b0)
+      } else {
+        MP_MMA(b0)
+        break;
+      }
+      g += 8;
+      MP_LOAD_A(g)
+      if (g + 8 < ngroups) {
+        MP_LOAD_B(b0, g + 8)
+        MP_MMA(b1)
+      } else {
+        MP_MMA(b1)
+        break;
+      }
+      g += 8;
     }
-    g += 8;
-  }
 #undef MP_LOAD_B
 #undef MP_LOAD_A
 #undef MP_MMA
+  }
 
   // ---- combine the 8 waves' partial tiles through LDS ----
   rsc.finish(ep, rs_part, rs_lds);
@@ -406,6 +449,29 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
   }
 }
 
+// Workgroups of NT tiles up to ``wide`` of them; from there on one tile each (launch_gemm; NT = 2).
+template <int MT, int NT, int EPI, bool APK, bool OPK>
+__global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                          const bf16_t* __restrict__ wp, bf16_t* __restrict__ y,
+                                                          int64_t y_stride, const bf16_t* __restrict__ res,
+                                                          int64_t res_stride, int M, int N, int K,
+                                                          const EpiArgs ep, int wide) {
+  clear_other(ep);
+  __shared__ u64 rs_part[SS_PG][SS_ROWS];
+  __shared__ float rs_lds[SS_ROWS];
+  __shared__ __attribute__((aligned(16))) float red[8][MT * NT * 4][64];
+  const int at = blockIdx.x;
+  if constexpr (NT == 2 && EPI != 1 && pk_rolling<MT, NT>()) {
+    if (at >= wide) {  // (uniform)
+      gemm_packed_body<MT, 1, EPI, APK, OPK, true>(x, x_stride, wp, y, y_stride, res, res_stride, M, N, K, ep, wide + at,
+                                             reinterpret_cast<float(*)[MT * 4][64]>(&red[0][0][0]), rs_part, rs_lds);
+      return;
+    }
+  }
+  gemm_packed_body<MT, NT, EPI, APK, OPK, pk_rolling<MT, NT>()>(x, x_stride, wp, y, y_stride, res, res_stride, M, N, K, ep, at * NT,
+                                                                red, rs_part, rs_lds);
+}
+
 template <int MT>
 static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_t ys, const void* res, int64_t rs,
                        int M, int N, int K, int epi, int flags, const EpiArgs& ep, hipStream_t stream) {
@@ -413,10 +479,13 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
   // two column tiles per wave when there are enough workgroups to fill the 256 CUs
   const bool two = epi == 1 || (ntiles % 2 == 0 && ntiles / 2 >= 256);
   const bool apk = flags & 1, opk = flags & 2;
+  // Pairs past a whole number on every CU go out as single tiles, where there are no more of those than CUs: a CU's own rate
+  // bounds its last workgroup (4096 columns, 4 rows: 512 pairs 21.7 us; 513 25.3, so 24.0; 585 26.8, so 25.2; 640 27.3, so 26.2)
+  const int over = ntiles / 2 % 256, wide = ntiles / 2 - (epi != 1 && over <= 128 && pk_rolling<MT, 2>() ? over : 0);
 #define MP_LAUNCH(NT_, EPI_, APK_, OPK_)                                                                       \
-  hipLaunchKernelGGL((gemm_packed_kernel<MT, NT_, EPI_, APK_, OPK_>), dim3(ntiles / NT_), dim3(512), 0, stream, \
-                     (const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)y, ys, (const bf16_t*)res, rs, M, N, K, \
-                     ep)
+  hipLaunchKernelGGL((gemm_packed_kernel<MT, NT_, EPI_, APK_, OPK_>), dim3(NT_ == 2 ? ntiles - wide : ntiles), dim3(512), 0, \
+                     stream, (const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)y, ys, (const bf16_t*)res, rs, M, N, K, \
+                     ep, wide)
   // Only the packed-activation form is instantiated: row-major callers pack x first
   // (mp_pack_act).  The row-major-A variant miscompiled at MT=1/NT=1 (ROCm 7.2, wrong
   // results with several k-groups per wave) and loses to the packed form anyway.

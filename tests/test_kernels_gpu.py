@@ -288,6 +288,30 @@ def test_gemm_shared_a(kern, M, N, K, epi):
         assert applies
 
 
+@pytest.mark.parametrize("kern", ["pk", "pk+r"])
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(8192, 128), (8224, 1024), (12288, 1152), (12320, 2176), (16416, 640)])
+def test_gemm_pairs_and_single_tiles(kern, M, N, K):
+    """Workgroups of two column tiles, then of one where a few pairs are left over (256, 256 + 1, 256 + 128, 256 + 129, 512 + 1
+    pairs); waves without a group of 128 columns, with one, with two, one of the eight with more.  A sum of K exact products in 32 bits,
+    rounded to bf16 once (epilogue 2: twice)."""
+    ops.require_native()
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    res = torch.randn(M, N, device="cuda", generator=g).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    xp, wp = ops.pack_act(x), ops.pack_weight(w)
+    ops.set_gemm_sk(kern)
+    try:
+        for epi, want in ((0, z), (2, z + res.double()), (4, z.clamp_min(0) ** 2)):
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+            ops.linear(xp, None, out=out, epilogue=epi, residual=res if epi == 2 else None, wp=wp, a_rows=M)
+            assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
+    finally:
+        ops.set_gemm_sk("off")
+
+
 @pytest.mark.parametrize("M", [5, 33, 64])
 def test_gemm_stream_k_swiglu_packed_out(M):
     K, F = 4096, 11008
