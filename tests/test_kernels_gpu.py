@@ -312,6 +312,26 @@ def test_gemm_pairs_and_single_tiles(kern, M, N, K):
         ops.set_gemm_sk("off")
 
 
+@pytest.mark.parametrize("kern", ["rw", "rwk", "rwk+r"])
+@pytest.mark.parametrize("M", [1, 17, 64])
+@pytest.mark.parametrize("N,K", [(2048, 128), (4096, 640), (4096, 1152), (2048, 2176), (6144, 1664)])
+def test_gemm_rings_of_few_steps(kern, M, N, K):
+    """Waves of a ring with one slice, with fewer than its slots, as many, one more, and a last turn that is not full.  A sum of K
+    exact products in 32 bits, rounded to bf16 once."""
+    ops.require_native()
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.set_gemm_sk(kern)
+    try:
+        ops.linear(ops.pack_act(x), None, out=out, epilogue=0, wp=ops.pack_weight(w), a_rows=M)
+    finally:
+        ops.set_gemm_sk("off")
+    want = x.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("M", [5, 33, 64])
 def test_gemm_stream_k_swiglu_packed_out(M):
     K, F = 4096, 11008
