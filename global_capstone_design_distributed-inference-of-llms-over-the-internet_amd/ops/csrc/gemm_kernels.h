@@ -1065,23 +1065,18 @@ static int launch_gemm_sk(const void* x, void* y, int64_t ys, const void* w, con
 // template bodies behind one uniform branch.
 // Inside a workgroup the waves take interleaved k-slices (k = wave + 4 i) through an R-deep
 // register ring holding BOTH operands of a slice, loads issued R slices ahead in consumption
-// order (in-order vmcnt never drains the ring; loads past the end are clamped to a valid slice
-// and their MFMAs skipped), then the 4 partial tiles are summed through LDS and the shared
+// order (in-order vmcnt never drains the ring; the last turn that loads clamps what is past the
+// end to the last slice), then the 4 partial tiles are summed through LDS and the shared
 // epilogues run (row scale, SwiGLU, residual, the fused-norm producer).
 #ifndef MP_RW_WAVES
 #define MP_RW_WAVES 4
 #endif
 constexpr int RW_WAVES = MP_RW_WAVES;  // waves per ring workgroup (an ablation build sets 8)
-// Ring tail: the loads a wave issues R steps ahead run past its last k-step; they are clamped to a
-// valid step and their MFMAs skipped (in-order vmcnt needs every slot loaded).  Pointing those dead
-// weight loads at the L2-resident activation helps the 128-deep MX steps (profiles/r6mx) but not
-// these rings: 7B 64 / 1 sessions and 70B fp8 unchanged or 0.1-0.5 % slower (profiles/r6tail).
 constexpr int RW_QC = 128 / RW_WAVES;  // quads per LDS combine pass (waves x RW_QC x 1 KiB = 128 KiB)
 
-// Ring slots: a power of two (K / 32 / 4 waves is a multiple of it at K = 4096, 11008: no
-// clamped tail turn); 4 (MT + NT) VGPRs each (one wave per SIMD: the accumulators go to AGPRs).
-// Measured at M = 64 (lab, us): qkv depth 2 / 4 / 6 = 21.2 / 21.7 / 22.7, gate/up 35.1 / 35.3 /
-// 35.4, o 14.3 / 13.7 / 14.1: two slots of 4 waves already cover the latency where tiles are wide.
+// Ring slots; 4 (MT + NT) VGPRs each (one wave per SIMD: the accumulators go to AGPRs).  Two slots of 4 waves cover
+// the latency where tiles are wide: with 4 instead, and with 8 or 4 where they fit, no shape of 4 to 64 rows is 2 % faster, some
+// split ones are 4 % slower.
 // MP_RW_DEEP1 (default on): 8 slots for the narrowest forms (one row tile, one column tile: the
 // batch-1 o projection, 256 workgroups of 128 KB of weights each), whose 4 waves x 4 slots keep
 // only ~32 KB per CU in flight (batch 1: 2.809 -> 2.789 ms, profiles/r3_u).
@@ -1093,7 +1088,9 @@ constexpr int rw_depth() {
   if (MP_RW_DEEP1 && MT + NT <= 2) return 8;
   return 190 / (4 * (MT + NT)) >= 8 ? 4 : 2;
 }
-// fp8 weights: a slot is 4 MT + 2 NT VGPRs.  (4 slots for the 14-tile Llama-3-70B gate/up group
+// fp8 weights: a slot is 4 MT + 2 NT VGPRs, half the bytes.  With one row tile and up to 6 column tiles, all of K a wave, 8
+// slots: 4096 x 4096 8.1 -> 7.0 us, 6144 x 4096 8.5 -> 7.9, 4096 x 14336 21.2 -> 16.3, 22016 x 4096 gated 18.9 -> 18.1 (16 rows; 8 tiles:
+// 22.6 -> 22.8, split in K 9.0 -> 10.0).  (4 slots for the 14-tile Llama-3-70B gate/up group
 // measured 17.30-17.34 vs 17.23-17.25 ms with 2: profiles/r4ab2.)
 template <int MT, int NT, bool F8>
 constexpr int rw_depth2() {
@@ -1118,7 +1115,7 @@ __device__ __forceinline__ void rw_body(const bf16_t* __restrict__ x, const bf16
                                         bf16_t* __restrict__ y, int64_t ys, const bf16_t* __restrict__ res, int64_t rs,
                                         int M, int K, int tile0, const EpiArgs& ep, f32x4* red, u64 (*rs_part)[SS_ROWS],
                                         float* rs_lds, int mt0 = 0, int mta = MT) {
-  constexpr int R = rw_depth2<MT, NT, F8>();
+  constexpr int R = F8 && MT == 1 && NT <= 6 ? 8 : rw_depth2<MT, NT, F8>();
   constexpr int Q = MT * NT;
   constexpr int NQ = (Q + RW_WAVES - 1) / RW_WAVES;  // epilogue quads per wave
   RowScale<EPI < 2, RW_WAVES> rsc;
