@@ -1295,7 +1295,7 @@ class StageExecutor:
 def _decode_step(ex: StageExecutor, x, positions, slots, q_seq, q_ctx, last_rows, T, part):
     """The step a decode graph records: every row one token, ``part`` the attention partition of the graph key."""
     if ex._hybrid is not None:
-        return ex._hybrid.forward(x, positions, slots, q_seq, q_ctx, last_rows, T, span=part[0])
+        return ex._hybrid.forward(x, positions, slots, q_seq, q_ctx, last_rows, T, span=part[0], every=True)
     return ex._forward_llama(x, positions, slots, q_seq, q_ctx, last_rows, T, 0, part, decode=True)
 
 
