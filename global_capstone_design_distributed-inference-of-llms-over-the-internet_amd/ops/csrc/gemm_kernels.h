@@ -260,14 +260,13 @@ constexpr int GU_MAX = 4;  // k-slices (of 32) per wave group (x 16 B per lane p
 
 // One workgroup's NT column tiles from ``nt0`` on.
 //
-// Bound by the weights' bytes, and short of them by what is not in flight while a workgroup begins and ends.  Up to 16 rows, and
-// up to 32 with two column tiles, every slice's registers take the load of the slice GU later as soon as its products are made
+// Bound by the weights' bytes, and short of them by what is not in flight while a workgroup begins and ends.  ROLLING (up to 16 rows,
+// and up to 32 with two column tiles): every slice's registers take the load of the slice GU later as soon as its products are made
 // (one group in flight: 70 and 102 registers, three and two workgroups a CU; the sums and their order are the same).  The ping-pong of
 // two groups, which the other forms keep, held 132 and 190, one workgroup a CU: at 4096 columns and 16 rows 16384 weight rows
 // took 23.5 us (now 21.3), 28672 gated 40.7 (37.7), 32000 43.3 (39.3); 32 rows, 22016 gated 36.9 (34.3).  At 48 and 64 rows the
-// ping-pong is up to 8 % faster, at 32 rows and one tile 2 %.
-template <int MT, int NT>
-constexpr bool pk_rolling() { return MT == 1 || (MT == 2 && NT == 2); }
+// ping-pong is up to 8 % faster, at 32 rows and one tile 2 %, and with no more workgroups than CUs (one tile; 4096 x 11008
+// 18.0, 18.4 us; 865 tiles of 2048 columns 13.5, 12.9).
 
 template <int MT, int NT, int EPI, bool APK, bool OPK, bool ROLLING>
 __device__ __forceinline__ void gemm_packed_body(const bf16_t* __restrict__ x, int64_t x_stride,
@@ -450,7 +449,7 @@ __device__ __forceinline__ void gemm_packed_body(const bf16_t* __restrict__ x, i
 }
 
 // Workgroups of NT tiles up to ``wide`` of them; from there on one tile each (launch_gemm; NT = 2).
-template <int MT, int NT, int EPI, bool APK, bool OPK>
+template <int MT, int NT, int EPI, bool APK, bool OPK, bool ROLLING>
 __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
                                                           const bf16_t* __restrict__ wp, bf16_t* __restrict__ y,
                                                           int64_t y_stride, const bf16_t* __restrict__ res,
@@ -461,15 +460,15 @@ __global__ __launch_bounds__(512) void gemm_packed_kernel(const bf16_t* __restri
   __shared__ float rs_lds[SS_ROWS];
   __shared__ __attribute__((aligned(16))) float red[8][MT * NT * 4][64];
   const int at = blockIdx.x;
-  if constexpr (NT == 2 && EPI != 1 && pk_rolling<MT, NT>()) {
+  if constexpr (NT == 2 && EPI != 1 && ROLLING) {
     if (at >= wide) {  // (uniform)
       gemm_packed_body<MT, 1, EPI, APK, OPK, true>(x, x_stride, wp, y, y_stride, res, res_stride, M, N, K, ep, wide + at,
                                              reinterpret_cast<float(*)[MT * 4][64]>(&red[0][0][0]), rs_part, rs_lds);
       return;
     }
   }
-  gemm_packed_body<MT, NT, EPI, APK, OPK, pk_rolling<MT, NT>()>(x, x_stride, wp, y, y_stride, res, res_stride, M, N, K, ep, at * NT,
-                                                                red, rs_part, rs_lds);
+  gemm_packed_body<MT, NT, EPI, APK, OPK, ROLLING>(x, x_stride, wp, y, y_stride, res, res_stride, M, N, K, ep, at * NT, red, rs_part,
+                                                   rs_lds);
 }
 
 template <int MT>
@@ -481,11 +480,18 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
   const bool apk = flags & 1, opk = flags & 2;
   // Pairs past a whole number on every CU go out as single tiles, where there are no more of those than CUs: a CU's own rate
   // bounds its last workgroup (4096 columns, 4 rows: 512 pairs 21.7 us; 513 25.3, so 24.0; 585 26.8, so 25.2; 640 27.3, so 26.2)
-  const int over = ntiles / 2 % 256, wide = ntiles / 2 - (epi != 1 && over <= 128 && pk_rolling<MT, 2>() ? over : 0);
-#define MP_LAUNCH(NT_, EPI_, APK_, OPK_)                                                                       \
-  hipLaunchKernelGGL((gemm_packed_kernel<MT, NT_, EPI_, APK_, OPK_>), dim3(NT_ == 2 ? ntiles - wide : ntiles), dim3(512), 0, \
+  // (turned walks of 8192 columns and more: the ping-pong is 2 to 6 % faster, 8192 x 28672 69.4, 71.0 us)
+  const bool rolls = MT <= 2 && !(ep.rot && K >= 8192);
+  const int over = ntiles / 2 % 256, wide = ntiles / 2 - (epi != 1 && over <= 128 && rolls ? over : 0);
+#define MP_PACKED(NT_, EPI_, APK_, OPK_, ROLL_)                                                                \
+  hipLaunchKernelGGL((gemm_packed_kernel<MT, NT_, EPI_, APK_, OPK_, ROLL_>), dim3(NT_ == 2 ? ntiles - wide : ntiles), dim3(512), 0, \
                      stream, (const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)y, ys, (const bf16_t*)res, rs, M, N, K, \
                      ep, wide)
+#define MP_LAUNCH(NT_, EPI_, APK_, OPK_)                                    \
+  if constexpr (MT + 2 - NT_ <= 2) {                                        \
+    if (rolls && (NT_ == 2 || ntiles > 256)) MP_PACKED(NT_, EPI_, APK_, OPK_, true);  \
+    else MP_PACKED(NT_, EPI_, APK_, OPK_, false);                           \
+  } else MP_PACKED(NT_, EPI_, APK_, OPK_, false)
   // Only the packed-activation form is instantiated: row-major callers pack x first
   // (mp_pack_act).  The row-major-A variant miscompiled at MT=1/NT=1 (ROCm 7.2, wrong
   // results with several k-groups per wave) and loses to the packed form anyway.
@@ -508,6 +514,7 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
   }
 #undef MP_APK
 #undef MP_LAUNCH
+#undef MP_PACKED
   return 0;
 }
 
