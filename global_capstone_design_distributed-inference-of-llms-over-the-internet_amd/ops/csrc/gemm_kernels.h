@@ -265,8 +265,8 @@ constexpr int GU_MAX = 4;  // k-slices (of 32) per wave group (x 16 B per lane p
 // (one group in flight: 70 and 102 registers, three and two workgroups a CU; the sums and their order are the same).  The ping-pong of
 // two groups, which the other forms keep, held 132 and 190, one workgroup a CU: at 4096 columns and 16 rows 16384 weight rows
 // took 23.5 us (now 21.3), 28672 gated 40.7 (37.7), 32000 43.3 (39.3); 32 rows, 22016 gated 36.9 (34.3).  At 48 and 64 rows the
-// ping-pong is up to 8 % faster, at 32 rows and one tile 2 %, and with no more workgroups than CUs (one tile; 4096 x 11008
-// 18.0, 18.4 us; 865 tiles of 2048 columns 13.5, 12.9).
+// ping-pong is up to 8 % faster, at 32 rows and one tile 2 %.  (One tile and no more workgroups than CUs are as fast alone, but
+// begin sooner in a step: a small model's 178 -> 175 us, a chat of an 8B model 511 -> 506.)
 
 template <int MT, int NT, int EPI, bool APK, bool OPK, bool ROLLING>
 __device__ __forceinline__ void gemm_packed_body(const bf16_t* __restrict__ x, int64_t x_stride,
@@ -480,7 +480,7 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
   const bool apk = flags & 1, opk = flags & 2;
   // Pairs past a whole number on every CU go out as single tiles, where there are no more of those than CUs: a CU's own rate
   // bounds its last workgroup (4096 columns, 4 rows: 512 pairs 21.7 us; 513 25.3, so 24.0; 585 26.8, so 25.2; 640 27.3, so 26.2)
-  // (turned walks of 8192 columns and more: the ping-pong is 2 to 6 % faster, 8192 x 28672 69.4, 71.0 us)
+  // (pairs in turned walks of 8192 columns and more: the ping-pong is 2 to 6 % faster, 8192 x 28672 69.4, 71.0 us)
   const bool rolls = MT <= 2 && !(ep.rot && K >= 8192);
   const int over = ntiles / 2 % 256, wide = ntiles / 2 - (epi != 1 && over <= 128 && rolls ? over : 0);
 #define MP_PACKED(NT_, EPI_, APK_, OPK_, ROLL_)                                                                \
@@ -488,10 +488,10 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
                      stream, (const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)y, ys, (const bf16_t*)res, rs, M, N, K, \
                      ep, wide)
 #define MP_LAUNCH(NT_, EPI_, APK_, OPK_)                                    \
-  if constexpr (MT + 2 - NT_ <= 2) {                                        \
-    if (rolls && (NT_ == 2 || ntiles > 256)) MP_PACKED(NT_, EPI_, APK_, OPK_, true);  \
+  if constexpr (MT <= 2 && NT_ == 2) {                                      \
+    if (rolls) MP_PACKED(NT_, EPI_, APK_, OPK_, true);                      \
     else MP_PACKED(NT_, EPI_, APK_, OPK_, false);                           \
-  } else MP_PACKED(NT_, EPI_, APK_, OPK_, false)
+  } else MP_PACKED(NT_, EPI_, APK_, OPK_, (MT == 1))
   // Only the packed-activation form is instantiated: row-major callers pack x first
   // (mp_pack_act).  The row-major-A variant miscompiled at MT=1/NT=1 (ROCm 7.2, wrong
   // results with several k-groups per wave) and loses to the packed form anyway.
