@@ -1108,11 +1108,12 @@ constexpr int rw_depth2() {
   }
 }
 
-// Does a ring's last turn load nothing?  Above 64 rows and with wide fp8 groups of 33 rows and more the loop that loads to its end
-// is 1 to 3 % faster (128 rows: 4096 x 4096 15.9, 16.4 us; fp8, 64: 4096 x 14336 20.4, 20.9; 48: 22016 gated 24.1, 24.4).
+// Does a ring's last turn load nothing?  Above 48 rows, and with wide fp8 groups of 33 rows and more, the loop that loads to its end
+// is as fast or 1 to 3 % faster (a step of 64 chats 621.0, 621.9 us; 128 rows: 4096 x 4096 15.9, 16.4; fp8, 64: 4096 x 14336 20.4,
+// 20.9; 48: 22016 gated 24.1, 24.4).
 template <int MT, int NT, bool F8>
 constexpr bool ring_drains() {
-  return MT <= 4 && (!F8 || MT < 3 || NT < 4);
+  return F8 ? MT < 3 || (MT <= 4 && NT < 4) : MT <= 3;
 }
 
 // MX ring step (128 k): 8 MT + 8 NT + 1 VGPRs per slot (rsa: the step's block-scale word)
