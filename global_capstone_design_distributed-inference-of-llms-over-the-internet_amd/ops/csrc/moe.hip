@@ -703,9 +703,9 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
 }
 
 // Many rows per expert, K in steps of 64: 256 x 256 tiles (wide_tile.h) of gathered rows and packed weights.
-// 8192 x 4096 x 11008 (one expert): 511 us, 1445 TFLOP/s; the ring of 32-column stages took 687 us.  2700 tokens of two of
-// eight 14336-wide experts of width 4096: up 1502 us on that ring, 1130 with every tile dealt alike, now 1103; down 803, 699, 616
-// and 20 to add the halves; 4298 tokens of four of 32 1408-wide ones of 2048: 260, 225, 216 and 151, 125, 123.
+// 8192 x 4096 x 11008 (one expert): 511 us with eight waves; the ring of 32-column stages took 687 us.  2700 tokens of two of
+// eight 14336-wide experts of width 4096: up 1502 us on that ring, 1130 with every tile dealt alike, 1103 so, now (four waves) 1064;
+// down 803, 699, 616, 585 and 19 to add the halves; eight waves, 4298 tokens of four of 32 1408-wide ones of 2048: 260, 225, 216 and 151, 125, 123.
 //
 // A tile of up to 128 rows takes 0.5 to 0.8 of the time of one of more (``wide_tile.h``), so tiles are dealt by time.  Every XCD gets an
 // eighth of the whole tiles and an eighth of the half ones, each a run in order, whose CUs then share few rows and few weights.
