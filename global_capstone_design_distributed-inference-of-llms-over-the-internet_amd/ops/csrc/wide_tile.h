@@ -153,11 +153,15 @@ struct WideTile {
       constexpr int M = decltype(fragments)::value;  // fragments of a wave's rows
       constexpr int R = M == MW ? 3 : 2;             // MFMAs to a read
       const int xr = (16 * M * wm() + c16) * 128;
-      // MFMA q of a half stage: two fragments of rows at a time
-      auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW]) {
+      // MFMA q of a half stage: two fragments of rows at a time.  An operand that a vector instruction wrote (a cleared sum, a
+      // copy at the loop's head) has to be two wait states old, which nobody counts for asm: a stage's first MFMA has four with it.
+      auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], bool first) {
         const int J = q / 16, b = q % 16 / 4, s = q % 4, down = J & 1;
         const int i = 2 * (down ? 3 - b : b) + ((s == 1 || s == 2) != down), j = 2 * J + ((s >= 2) != (b & 1));
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
+        if (first)
+          asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
+        else
+          asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
       };
       // a half stage: the products of the operands read before, reads of the next half's, the loads of a stage of one operand
       auto half_stage = [&](auto second) __attribute__((always_inline)) {
@@ -166,7 +170,7 @@ struct WideTile {
         for (int q = 0; q < NW * M; ++q) {
           constexpr int AT = B ? 1 : M - 3;
           if (q % M == AT - 1) aim(B ? x : w, q / M, B ? fw : fx);
-          multiply1(q, B ? xb : xa, B ? wb : wa);
+          multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
           if (q % R == R - 1 && q / R < M + NW) take1(!B, q / R, xr, B ? xa : xb, B ? wa : wb, M);
           if (q % M == AT) load(B ? x : w, q / M, B ? fw : fx);
           __builtin_amdgcn_sched_barrier(0);
@@ -181,7 +185,6 @@ struct WideTile {
       for (int i = 0; i < NW; ++i)
 #pragma unroll
         for (int j = 0; j < M; ++j) acc[i][j] = (f32x4)(0.f);
-      asm volatile("s_nop 7");
       const int n = work.stages(k);
 #pragma unroll 1
       for (int st = 0; st < n; ++st) {
