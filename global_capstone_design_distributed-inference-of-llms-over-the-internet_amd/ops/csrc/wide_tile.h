@@ -98,24 +98,16 @@ struct WideTile {
     work.weight_offsets(w);
     work.rows(0, x);
     work.weights(0, w);
-    // A load in asm needs its place in m0 one instruction before, and scalars that a vector instruction wrote (the compiler
-    // may keep some in lanes) five before: ``aim`` fixes them all, and two MFMAs stand between it and ``load`` (five waits in
-    // front of each load cost 5 % at 1554 x 4096 x 28672: 347 us now).  Nothing else of this form uses m0.
+    // A load in asm has its place in m0, an operand of it that the compiler sets, and waits five states for scalars that a vector
+    // instruction wrote (the compiler may keep some in lanes).  In the loop two MFMAs stand in the place of waits (five waits in
+    // front of each load cost 5 % at 1554 x 4096 x 28672: 347 us now).
     auto place = [&](int j, int slot) { return (lptr_t)(mine + slot * SLOT + j * 1024); };
-    auto aim = [&](Source& s, int j, int slot) {
-      if constexpr (FORM == COLUMNS)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 1" : "+s"(s.words), "+s"(s.at) : "s"((uint32_t)(uintptr_t)place(j, slot)));
-    };
     auto load = [&](const Source& s, int j, int slot) {
       if constexpr (FORM == COLUMNS)
-        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(s.off[j]), "s"(s.words), "s"(s.at) : "memory");
+        asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                     :: "v"(s.off[j]), "s"(s.words), "s"(s.at), "{m0}"((uint32_t)(uintptr_t)place(j, slot)) : "memory");
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, place(j, slot), 16, s.off[j], s.at, 0, 0);
-    };
-    auto load_now = [&](Source& s, int j, int slot) {
-      aim(s, j, slot);
-      if constexpr (FORM == COLUMNS) asm volatile("s_nop 2");
-      load(s, j, slot);
     };
     // to the next stage (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
     auto step = [&] {
@@ -154,14 +146,28 @@ struct WideTile {
       constexpr int R = M == MW ? 3 : 2;             // MFMAs to a read
       const int xr = (16 * M * wm() + c16) * 128;
       // MFMA q of a half stage: two fragments of rows at a time.  An operand that a vector instruction wrote (a cleared sum, a
-      // copy at the loop's head) has to be two wait states old, which nobody counts for asm: a stage's first MFMA has four with it.
+      // copy at the loop's head) has to be two wait states old, which nobody counts for asm: a stage's first MFMA has them with it.
+      auto weight_of = [](int q) {
+        const int b = q % 16 / 4, s = q % 4, down = q / 16 & 1;
+        return 2 * (down ? 3 - b : b) + ((s == 1 || s == 2) != down);
+      };
+      auto row_of = [](int q) { return 2 * (q / 16) + ((q % 4 >= 2) != (q % 16 / 4 & 1)); };
       auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], bool first) {
-        const int J = q / 16, b = q % 16 / 4, s = q % 4, down = J & 1;
-        const int i = 2 * (down ? 3 - b : b) + ((s == 1 || s == 2) != down), j = 2 * J + ((s >= 2) != (b & 1));
+        const int i = weight_of(q), j = row_of(q);
         if (first)
-          asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
+          asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
         else
           asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
+      };
+      // MFMAs q - 1 and q and a load in asm behind them (more wait states than a first MFMA needs)
+      auto multiply2 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], const Source& s, int l, int slot) {
+        const int i = weight_of(q - 1), j = row_of(q - 1), i1 = weight_of(q), j1 = row_of(q);
+        const uint32_t to = (uint32_t)(uintptr_t)place(l, slot);
+        asm volatile("s_nop 2\n\tv_mfma_f32_16x16x32_bf16 %0, %2, %3, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %4, %5, %1\n\t"
+                     "buffer_load_dwordx4 %6, %7, %8 offen lds"
+                     : "+a"(acc[i][j]), "+a"(acc[i1][j1])
+                     : "v"(wf[i]), "v"(xf[j]), "v"(wf[i1]), "v"(xf[j1]), "v"(s.off[l]), "s"(s.words), "s"(s.at), "{m0}"(to)
+                     : "memory");
       };
       // a half stage: the products of the operands read before, reads of the next half's, the loads of a stage of one operand
       auto half_stage = [&](auto second) __attribute__((always_inline)) {
@@ -169,10 +175,10 @@ struct WideTile {
 #pragma unroll
         for (int q = 0; q < NW * M; ++q) {
           constexpr int AT = B ? 1 : M - 3;
-          if (q % M == AT - 1) aim(B ? x : w, q / M, B ? fw : fx);
-          multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
+          if (FORM == COLUMNS && q % M == AT) multiply2(q, B ? xb : xa, B ? wb : wa, B ? x : w, q / M, B ? fw : fx);
+          else if (FORM != COLUMNS || q % M != AT - 1) multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
           if (q % R == R - 1 && q / R < M + NW) take1(!B, q / R, xr, B ? xa : xb, B ? wa : wb, M);
-          if (q % M == AT) load(B ? x : w, q / M, B ? fw : fx);
+          if (FORM != COLUMNS && q % M == AT) load(B ? x : w, q / M, B ? fw : fx);
           __builtin_amdgcn_sched_barrier(0);
         }
       };
@@ -211,9 +217,9 @@ struct WideTile {
 #pragma unroll 1
     for (int s = 0; s < 2; ++s) {  // w 0, x 0, w 1, x 1
 #pragma unroll
-      for (int j = 0; j < PIECES; ++j) load_now(w, j, 2 * s);
+      for (int j = 0; j < PIECES; ++j) load(w, j, 2 * s);
 #pragma unroll
-      for (int j = 0; j < PIECES; ++j) load_now(x, j, 2 * s + 1);
+      for (int j = 0; j < PIECES; ++j) load(x, j, 2 * s + 1);
       step();
     }
     fx = SLOTS - 1;  // (w 2)

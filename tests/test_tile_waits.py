@@ -110,3 +110,19 @@ def test_sums_are_made_before_they_are_read(assembly):
             sums = {r for r in o.reads | o.writes if r[0] == "a"} if not o.mfma else None
             if sums:
                 assert _since(ops, before, i, lambda p: p.mfma and p.writes & sums, 16) >= 16, (name, o.text)
+
+
+def test_column_loads_know_their_place(assembly):
+    """A load into LDS in asm takes m0 (where it goes) as an operand that the compiler sets, and waits five states in its own
+    statement: the compiler may bring its other scalars back from lanes just ahead of it."""
+    loads = 0
+    for name, ops, before in assembly:
+        assert not any("m0" in o.writes for o in ops if o.block), name
+        for i, o in enumerate(ops):
+            if o.block and o.name.startswith("buffer_load"):
+                loads += 1
+                first = next(k for k in range(i, -1, -1) if k == 0 or ops[k - 1].block != o.block)
+                assert sum(p.waits for p in ops[first:i]) >= 5, name
+                put = next(k for k in range(first - 1, -1, -1) if "m0" in ops[k].writes)
+                assert not any(p.name.startswith("buffer_load") for p in ops[put:first]), name  # (set for this one)
+    assert loads == 48  # two operands of a stage, of whole and of half tiles; of a loop's turn ahead of the first
