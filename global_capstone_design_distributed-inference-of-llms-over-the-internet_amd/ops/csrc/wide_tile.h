@@ -280,7 +280,8 @@ struct WideTile {
         const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false));
         const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false));
         const bool there = lc + 16 * i / S < cols;  // (columns come in sixteens)
-        __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], b[0], a[1], b[1]}, to, there ? at : 1u << 31, 32 * i / S, 0);
+        // (all of the offset in the lane's part: the buffer's end is compared with that, less the scalar part, and may be 0)
+        __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], b[0], a[1], b[1]}, to, (there ? at : 1u << 31) + 32 * i / S, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }

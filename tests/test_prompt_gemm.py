@@ -100,6 +100,26 @@ def test_output_rows_of_many_columns(M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 17, 100, 129, 250, 300])
+@pytest.mark.parametrize("N", [32, 144, 288])
+def test_nothing_behind_the_output(M, N):
+    """What lies behind the output, up to where a whole tile would end, stays as it was: rows and columns that are not there."""
+    ops.require_native()
+    K = 128
+    g = torch.Generator().manual_seed(M + N)
+    x, w = (torch.randn(n, K, generator=g).to(torch.bfloat16).cuda() for n in (M, N))
+    for epi in (0, 1, 4, 8):
+        cols = N // 2 if epi == 1 else N
+        if epi == 1 and N % 32:
+            continue
+        room = torch.full((2 * prompt.TILE + M, cols), -3.0, dtype=torch.bfloat16, device="cuda")
+        prompt._run(x, w.t().contiguous() if epi == 8 else w, room[:M], N, epi)
+        assert bool((room[M:] == -3.0).all())
+        want = _want(x.double() @ w.double().t(), 0 if epi == 8 else epi, 0.0)
+        assert float((room[:M].double() - want).norm() / want.norm()) < BF16
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
 def test_products_with_columns(M, N, K):
     """x w, as a gradient goes back through a projection: ends of tiles and of a wave's columns, tiles in parts."""

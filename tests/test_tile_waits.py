@@ -126,3 +126,15 @@ def test_column_loads_know_their_place(assembly):
                 put = next(k for k in range(first - 1, -1, -1) if "m0" in ops[k].writes)
                 assert not any(p.name.startswith("buffer_load") for p in ops[put:first]), name  # (set for this one)
     assert loads == 48  # two operands of a stage, of whole and of half tiles; of a loop's turn ahead of the first
+
+
+def test_stores_end_with_the_buffer(assembly):
+    """An output's stores have no scalar offset: those of rows that are not there go to a buffer of 0 bytes, whose end less such
+    an offset is no number of bytes."""
+    stores = 0
+    for name, ops, _ in assembly:
+        for o in ops:
+            if o.name.startswith("buffer_store"):
+                stores += 1
+                assert re.search(r"s\[\d+:\d+\], 0 offen", o.text), (name, o.text)
+    assert stores
