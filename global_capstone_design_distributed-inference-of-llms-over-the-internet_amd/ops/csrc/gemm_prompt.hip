@@ -37,17 +37,17 @@ __device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, in
   m0 = (GW_BAND * band + r % h) * WideTile::BM;
   n0 = r / h * WideTile::BN;
 }
-// (the sigmoid's reciprocal by v_rcp_f32, off by 1 unit in 24 bits where a division, ten instructions, is off by a half: the
-// outputs, of 8 bits, are as far from 64 bits as before; 2700 x 28672 x 4096 457 -> 447 us)
+// (divisions, ten instructions each: v_rcp_f32 in their place takes 2 % off 2700 x 28672 x 4096, but is off by 1 unit in 24 bits
+// instead of a half, and 0 where 1 + exp(-v) is 2^126 and more)
 template <int EPI, bool LIMIT>
 __device__ __forceinline__ void gw_act(const GemmPrompt& a, const f32x4& v, const f32x4& u, float (&y)[4]) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (EPI == 1 && LIMIT) {
       const float g = fminf(v[r], a.limit), w = fminf(fmaxf(u[r], -a.limit), a.limit);
-      y[r] = g * __builtin_amdgcn_rcpf(1.f + __expf(-1.702f * g)) * (w + 1.f);
+      y[r] = g / (1.f + __expf(-1.702f * g)) * (w + 1.f);
     } else if (EPI == 1) {
-      y[r] = v[r] * __builtin_amdgcn_rcpf(1.f + __expf(-v[r])) * u[r];
+      y[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
     } else if (EPI == 4) {
       const float p = v[r] < 0.f ? 0.f : v[r];  // (not a number stays one)
       y[r] = p * p;

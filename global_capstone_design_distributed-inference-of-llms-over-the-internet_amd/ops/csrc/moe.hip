@@ -42,11 +42,10 @@ __device__ __forceinline__ int64_t act_at(int row, int col, int64_t xs, int mt) 
   return mt > 0 ? apk_off(row, col, mt) : (int64_t)row * xs + col;
 }
 
-// (v_rcp_f32 in place of a division: 1 unit in 24 bits, of outputs that have 8)
 __device__ __forceinline__ float moe_glu(float g, float u, float limit) {
-  if (limit <= 0.f) return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * u;  // (uniform)
+  if (limit <= 0.f) return g / (1.f + __expf(-g)) * u;  // (uniform)
   const float a = fminf(g, limit), b = fminf(fmaxf(u, -limit), limit);
-  return a * __builtin_amdgcn_rcpf(1.f + __expf(-MOE_ALPHA * a)) * (b + 1.f);
+  return a / (1.f + __expf(-MOE_ALPHA * a)) * (b + 1.f);
 }
 __device__ __forceinline__ float moe_glu_exact(float g, float u, float limit) {
   if (limit <= 0.f) return g / (1.f + expf(-g)) * u;

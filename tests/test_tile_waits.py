@@ -1,4 +1,4 @@
-"""Wait states in the 256 x 256 product tiles (csrc/wide_tile.h), whose MFMAs and column loads stand in inline asm: the
+"""Wait states and divisions in the 256 x 256 product tiles (csrc/wide_tile.h), whose MFMAs and column loads stand in inline asm: the
 compiler counts none for them, so the assembly that it makes of the kernels is read here."""
 import concurrent.futures as cf
 import os
@@ -74,7 +74,7 @@ def _since(ops, before, at, hit, far):
 
 
 @pytest.fixture(scope="module")
-def assembly(tmp_path_factory):
+def texts(tmp_path_factory):
     if not os.path.exists(build.HIPCC):
         pytest.skip("no hipcc")
     at = tmp_path_factory.mktemp("asm")
@@ -85,9 +85,14 @@ def assembly(tmp_path_factory):
                         *build.DEVICE_FLAGS, "-S", "--cuda-device-only", os.path.join(build.CSRC, src), "-o", out],
                        check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
         with open(out) as f:
-            return [k for k in _functions(f.read(), KERNELS[src])]
+            return f.read()
     with cf.ThreadPoolExecutor(2) as ex:
-        return [k for ks in ex.map(make, KERNELS) for k in ks]
+        return dict(zip(KERNELS, ex.map(make, KERNELS)))
+
+
+@pytest.fixture(scope="module")
+def assembly(texts):
+    return [k for src, text in texts.items() for k in _functions(text, KERNELS[src])]
 
 
 def test_operands_of_products_are_old_enough(assembly):
@@ -138,3 +143,15 @@ def test_stores_end_with_the_buffer(assembly):
                 stores += 1
                 assert re.search(r"s\[\d+:\d+\], 0 offen", o.text), (name, o.text)
     assert stores
+
+
+def test_gates_are_divided(texts):
+    """The gates' 1 / (1 + exp(-g)) is a division, correct to half a unit in 24 bits, and not the reciprocal instruction that a
+    division begins with, which is a whole one off."""
+    divided = 0
+    for src, text in texts.items():
+        for name, body in re.findall(r"^(_Z\w*gemm\w*):.*?\n(.*?)^\.Lfunc_end", text, re.S | re.M):
+            n = len(re.findall(r"\bv_div_fixup_f32", body))
+            assert len(re.findall(r"\bv_rcp_f32", body)) == n, name
+            divided += n > 0
+    assert divided == 2 + 7  # prompt products and their close; expert products of all forms
