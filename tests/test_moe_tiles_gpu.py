@@ -5,6 +5,7 @@ import torch
 from src import ops
 from src.models.config import MoESpec
 from src.ops import moe
+from tests.test_prompt_gemm import gates_far_below_zero
 
 pytestmark = pytest.mark.gpu
 
@@ -225,3 +226,15 @@ def test_few_rows_of_any_depth(n, K):
     torch.ops.mpamd.moe_gemm(1, x.cuda(), torch.arange(R, dtype=torch.int32, device="cuda"), _lists(counts),
                              torch.stack([ops.pack_weight(m) for m in w.cuda()]), out, R, R, 0, 1, 0.0, 0)
     assert float((out.double().cpu() - z).norm() / z.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("form", [1, 2, 3])
+def test_gates_far_below_zero(form):
+    """g / (1 + exp(-g)) u, rounded to bf16 once; the exponential of 88 is 1e-5 of itself off."""
+    ops.require_native()
+    x, w, z = gates_far_below_zero("cuda")
+    want = torch.nn.functional.silu(z[:, :16]) * z[:, 16:]
+    out = torch.full((3, 16), float("nan"), dtype=torch.bfloat16, device="cuda")
+    torch.ops.mpamd.moe_gemm(form, x, torch.arange(3, dtype=torch.int32, device="cuda"), _lists([3]), ops.pack_weight(w)[None].contiguous(),
+                             out, 3, 3, 1, 16, 0.0, 0)
+    assert float(((out.double() - want) / want).abs().max()) < 2.0 ** -8 + 2e-5

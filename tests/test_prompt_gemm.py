@@ -119,6 +119,26 @@ def test_nothing_behind_the_output(M, N):
         assert float((room[:M].double() - want).norm() / want.norm()) < BF16
 
 
+def gates_far_below_zero(device):
+    """(x [3, 64], w [32, 64], z): gates of -87 to -88.5, whose 1 + exp(88) lies above 2^126 (its reciprocal is no normal number of
+    32 bits), beside up rows of 2^100, which bring the product back to 1e-6.  Every sum is one product."""
+    x = torch.zeros(3, 64, dtype=torch.bfloat16, device=device)
+    x[0, 0] = x[1, 1] = x[2, 2] = 1
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=device)
+    w[:16, 0], w[:16, 1], w[:16, 2], w[16:, :3] = -87.0, -88.0, -88.5, 2.0 ** 100
+    return x, w, x.double() @ w.double().t()
+
+
+@pytest.mark.gpu
+def test_gates_far_below_zero():
+    """g / (1 + exp(-g)) u, rounded to bf16 once; the exponential of 88 is 1e-5 of itself off."""
+    ops.require_native()
+    x, w, z = gates_far_below_zero("cuda")
+    want = _want(z, 1, 0.0)
+    got = prompt.gemm(x, w, None, 1).double()
+    assert float(want.abs().min()) > 1e-7 and float(((got - want) / want).abs().max()) < BF16 + 2e-5
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
 def test_products_with_columns(M, N, K):

@@ -147,7 +147,7 @@ def test_stores_end_with_the_buffer(assembly):
 
 def test_gates_are_divided(texts):
     """The gates' 1 / (1 + exp(-g)) is a division, correct to half a unit in 24 bits, and not the reciprocal instruction that a
-    division begins with, which is a whole one off."""
+    division begins with, which is a whole one off, and 0 where its result is below the normal numbers."""
     divided = 0
     for src, text in texts.items():
         for name, body in re.findall(r"^(_Z\w*gemm\w*):.*?\n(.*?)^\.Lfunc_end", text, re.S | re.M):
