@@ -1109,6 +1109,16 @@ def _slab_view(device, S: int, M: int, N: int) -> torch.Tensor:
     return ws[off:off + S * M * N * 4].view(torch.float32).view(S, M, N)
 
 
+def partials_turned(N: int, K: int) -> bool:
+    """Do the workgroups of partial slabs of [N, K] bf16 weights begin at different columns (``rot``)?
+
+    Column tiles (32 K bytes each) lie on the same memory channels where that is a multiple of 512 KB.  Timed at 1 to 64
+    rows, turned over straight: 4096 x 16384 0.84 to 0.91, 4096 x 32768 0.95 to 0.99, 8192 x 16384 0.91 to 0.94 (from 48
+    rows on 1.00), 8192 x 32768 0.98 (from 32 rows on 1.01); 2048 x 16384, whose tiles are cut more often, 1.02 to 1.07.  Of
+    other K, 4096 x 8192 1.01 to 1.06, x 14336 1.00 and 8192 x 4096 1.02 to 1.06; only 8192 x 8192 would gain (0.91 to 0.99)."""
+    return K % 16384 == 0 and N >= 4096
+
+
 def linear_partials(x, M: int, wp=None, w8=None, w_scale=None, out=None, rot: bool = False):
     """The decode GEMM of a PACKED activation as fp32 split-K partial slabs [S, M, N] (a view into
     the GEMM workspace, valid until the next split-K GEMM on this device's stream): no epilogue,

@@ -156,9 +156,7 @@ class HybridStage:
         if y_in is None:
             y = None
         elif packed and ops.rwk_split(T, w.shape[0], w.shape[1]) > 0:
-            # column tiles 512 KB apart lie on the same memory channels: workgroups begin at different columns (4096 rows of 16384
-            # columns, 4 tokens: 26.6 -> 24.4 us with the sum; of 8192 columns 15.2 -> 16.0, so not there)
-            y = ops.linear_partials(y_in, T, wp=wp, out=e("y", (T, self.W)), rot=w.shape[1] % 16384 == 0)
+            y = ops.linear_partials(y_in, T, wp=wp, out=e("y", (T, self.W)), rot=ops.partials_turned(*w.shape))
         else:
             y = self._mm(y_in, w, wp, T, packed, e("y", (T, self.W)))
         if join is not None:

@@ -38,3 +38,9 @@ def test_table_is_set_and_saved_as_it_is(tmp_path):
     finally:
         ops.set_kernel_table(saved[0])
         ops._TABLE["runtime"].update(saved[1])
+
+
+def test_which_partial_slabs_are_turned():
+    """Where the measured turn is the faster one or makes no difference: not at 2048 rows of 16384 columns."""
+    assert [ops.partials_turned(N, K) for N, K in ((4096, 16384), (8192, 32768), (2048, 16384), (4096, 8192), (4096, 14336))] == \
+        [True, True, False, False, False]

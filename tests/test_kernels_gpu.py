@@ -332,6 +332,23 @@ def test_gemm_rings_of_few_steps(kern, M, N, K):
     assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("M", [1, 17, 48, 64])
+@pytest.mark.parametrize("N,K", [(4096, 16384), (2048, 16384), (4096, 1152), (2048, 2176)])
+def test_partial_slabs_straight_and_turned(M, N, K):
+    """Slabs of a product split in K, whose workgroups begin at the same columns or at different ones; their sum is one of K exact
+    products in 32 bits."""
+    ops.require_native()
+    if ops.rwk_split(M, N, K) <= 0:
+        pytest.skip("no split form")
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
+    want, xp, wp = x.double() @ w.double().t(), ops.pack_act(x), ops.pack_weight(w)
+    for rot in (False, True):
+        got = ops.linear_partials(xp, M, wp=wp, rot=rot).double().sum(0)
+        assert float((got - want).norm() / want.norm()) < 1e-5
+
+
 @pytest.mark.parametrize("M", [5, 33, 64])
 def test_gemm_stream_k_swiglu_packed_out(M):
     K, F = 4096, 11008
