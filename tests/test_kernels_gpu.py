@@ -313,7 +313,7 @@ def test_gemm_pairs_and_single_tiles(kern, M, N, K):
 
 
 @pytest.mark.parametrize("kern", ["rw", "rwk", "rwk+r"])
-@pytest.mark.parametrize("M", [1, 17, 64])
+@pytest.mark.parametrize("M", [1, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(2048, 128), (4096, 640), (4096, 1152), (2048, 2176), (6144, 1664)])
 def test_gemm_rings_of_few_steps(kern, M, N, K):
     """Waves of a ring with one slice, with fewer than its slots, as many, one more, and a last turn that is not full.  A sum of K
@@ -329,6 +329,24 @@ def test_gemm_rings_of_few_steps(kern, M, N, K):
     finally:
         ops.set_gemm_sk("off")
     want = x.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("kern", ["rw", "rwk", "rwk+r"])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(2048, 128), (4096, 640), (4096, 1152), (6144, 1664), (4096, 11008), (24576, 1152)])
+def test_w8a16_rings_of_few_steps(kern, M, N, K, monkeypatch):
+    """The same of fp8 weights, whose rings have 8 slots (up to 16 rows and 6 tiles) or fewer: waves of 1, 5, 9, 13 and 86 slices; groups
+    of 1 to 6 tiles.  A sum of K exact products in 32 bits, times a scale, rounded to bf16 once."""
+    monkeypatch.setattr(ops, "_W8_MODE", kern)
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    wq, ws = ops.pack_weight_fp8(torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5))
+    w8 = ops.w8_from_fp8(wq)
+    codes = ops.unpack_weight_w8(w8, torch.ones_like(ws), torch.float32)
+    want = x.double() @ codes.double().t() * ws.double()
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.linear_w8(ops.pack_act(x), w8, ws, M, out=out)
     assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
 
 
