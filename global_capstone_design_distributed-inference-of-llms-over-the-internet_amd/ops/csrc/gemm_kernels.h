@@ -480,7 +480,9 @@ static int launch_gemm(const void* x, int64_t xs, const void* w, void* y, int64_
   const bool apk = flags & 1, opk = flags & 2;
   // Pairs past a whole number on every CU go out as single tiles, where there are no more of those than CUs: a CU's own rate
   // bounds its last workgroup (4096 columns, 4 rows: 512 pairs 21.7 us; 513 25.3, so 24.0; 585 26.8, so 25.2; 640 27.3, so 26.2)
-  // (pairs in turned walks of 8192 columns and more: the ping-pong is 2 to 6 % faster, 8192 x 28672 69.4, 71.0 us)
+  // Turned walks of 8192 columns and more keep the ping-pong (1 to 32 rows; us, ping-pong and rolling): 8192 x 28672 69.3, 71.1; x 12288
+  // 31.8, 32.7; x 8192 22.9, 23.8; 16384 x 16384 80, 90; 57344 gated x 8192 138, 144, at 32 rows 169, 169; against it only 10240 x
+  // 8192 34.7, 32.2, whose left-over pairs go out alone.  Of 6144 columns both 18, of 4096 rolling is 5 to 18 % faster.
   const bool rolls = MT <= 2 && !(ep.rot && K >= 8192);
   const int over = ntiles / 2 % 256, wide = ntiles / 2 - (epi != 1 && over <= 128 && rolls ? over : 0);
 #define MP_PACKED(NT_, EPI_, APK_, OPK_, ROLL_)                                                                \
@@ -1108,9 +1110,11 @@ constexpr int rw_depth2() {
   }
 }
 
-// Does a ring's last turn load nothing?  Above 48 rows, and with wide fp8 groups of 33 rows and more, the loop that loads to its end
-// is as fast or 1 to 3 % faster (a step of 64 chats 621.0, 621.9 us; 128 rows: 4096 x 4096 15.9, 16.4; fp8, 64: 4096 x 14336 20.4,
-// 20.9; 48: 22016 gated 24.1, 24.4).
+// Does a ring's last turn load nothing?  (The turn before it loads the last step again where a wave's steps are no multiple of the
+// slots.)  Of bf16, up to 48 rows: no shape loses, split ones gain up to 2 % here.  At 64 and 96 rows both loops are alike (0.99 to
+// 1.01), at 128 the one that loads to its end is 1 to 2 % faster (4096 x 4096 16.2, 16.5 us; 4096 x 11008 28.0, 28.3).  fp8 from 33 rows
+// on: groups of up to 3 tiles gain 3 to 6 % (6144 x 4096, 64 rows: 14.6 -> 13.7), wider ones lose up to 2 % (22016 gated, 33 rows: 23.0,
+// 23.4; 4096 x 14336 split, 64 rows: 20.5, 20.9).
 template <int MT, int NT, bool F8>
 constexpr bool ring_drains() {
   return F8 ? MT < 3 || (MT <= 4 && NT < 4) : MT <= 3;

@@ -702,14 +702,15 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
 }
 
 // Many rows per expert, K in steps of 64: 256 x 256 tiles (wide_tile.h) of gathered rows and packed weights.
-// 8192 x 4096 x 11008 (one expert): 511 us with eight waves; the ring of 32-column stages took 687 us.  2700 tokens of two of
-// eight 14336-wide experts of width 4096: up 1502 us on that ring, 1130 with every tile dealt alike, 1103 so, now (four waves) 1064;
-// down 803, 699, 616, 585 and 19 to add the halves; eight waves, 4298 tokens of four of 32 1408-wide ones of 2048: 260, 225, 216 and 151, 125, 123.
+// On the ring of 32-column stages, with tiles of eight waves, and so: 2700 tokens of two of eight 14336-wide experts of width 4096 up
+// 1502, 1106, 1048 us, down (with the halves added) 803, 651, 568; 4298 tokens of four of 32 1408-wide ones of 2048 up 260, 209,
+// 197, down 151, 121, 112 (the last two in turn, means of five draws).
 //
-// A tile of up to 128 rows takes 0.5 to 0.8 of the time of one of more (``wide_tile.h``), so tiles are dealt by time.  Every XCD gets an
+// A tile of up to 128 rows makes half the products but loads as much: 0.78 to 0.86 of the time of one of more, 256 of either at once
+// (8 experts of 8192 x 1024, weights in the 256 MB cache: 28.2, 36.0 us; of 8192 x 4096, from HBM: 105, 125).  Every XCD gets an
 // eighth of the whole tiles and an eighth of the half ones, each a run in order, whose CUs then share few rows and few weights.
-// Its G workgroups take whole tiles in turn; those that the r left over do not reach take two half ones first, and the
-// other half ones go round.  Where all that is left fits one half round, and a workspace is there, the r are cut at the
+// Its G workgroups take whole tiles in turn; those that the r left over do not reach take two half ones first (one
+// first: within 1 %, but for down products of 1500 tokens, 4 % more), and the other half ones go round.  Where all that is left fits one half round, and a workspace is there, the r are cut at the
 // middle of K instead: a workgroup makes a half, and moe_gemm_close_kernel adds the two.  A workgroup's half tiles lie
 // between its whole ones, sooner in some than in others: their weights come from HBM a second time, and all at once that
 // bound them.
@@ -1051,8 +1052,10 @@ extern "C" int mp_moe_gemm(int form, int glu, const void* x, int64_t xs, int mt,
     if (form == 1) {
       if (!glu && !out_f32) return -1;
       const dim3 g((N / 16 + 1) / 2, act);
-      // past the caches from 64 MB of experts on: four such layers fill the 256 MB of cache, so that no weight is there in
-      // the next step (184 MB: 1 to 4 % faster, 369 MB 8 %; 4 and 8 MB, read from cache step after step, 4.8 -> 5.8 and 5.2 -> 6.7 us)
+      // past the caches from 64 MB of experts on (each of a layer's two products for itself).  Both products of a layer, past the caches
+      // over from them, 6 and 64 rows: up products of 64 MB and more 0.90 to 0.94 wherever the model's experts are more than the 256
+      // MB of cache, 0.90 to 1.07 where they are fewer (2 layers); 32 and 48 MB 0.93 to 0.97 from 8 layers on, up to 1.09 with
+      // fewer; 16 MB 0.98 to 1.02 with 16 layers, 1.02 to 1.12 with fewer, whose weights are still there in the next step
       const bool once = (int64_t)E * N * K * 2 >= 64ll << 20;
       auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(256), 0, stream, a); };
       if (glu) once ? launch(moe_gemm_rows_kernel<true, true>) : launch(moe_gemm_rows_kernel<true, false>);

@@ -20,10 +20,11 @@
 //   * Nothing in the loop but the loads' 8 instructions depends on the tile: a tile moves the base of what is loaded, not
 //     the lanes' offsets, and what is behind its rows and weights is behind the end of the buffer, which loads as zero.
 //   * A tile of up to 128 rows has 64 rows a wave and half the MFMAs.
-// A stage takes 2330 (rows and weights in L2) to 2450 cycles, 2050 of them MFMAs; a tile's end 8300.  Bound by MFMA issue and, at 1.75
-// of 2.4 GHz, by power.  Eight waves, whose loop decided anew at each stage what to load next, took 2680 to 2900 cycles a
-// stage: 4096 x 4096 x 16384 393 us (now 361), 6421 x 12288 x 4096 484 (450), 4298 x 16384 x 4096 449 (438),
-// columns of 4096 x 4096 x 16384 383 (354).  Eight waves with this loop: 378, 477, 448 us.
+// Counters of 4096 x 8192 x 8192, two tiles of 128 stages a workgroup, their ends counted in: 2480 cycles a stage, 2048 of them MFMAs
+// (82 % busy), no bank conflicts; columns 2720 (75 %).  Bound by MFMA issue and, at 1.7 to 2.0 of 2.4 GHz, by power.  Eight waves,
+// whose loop decided anew at each stage what to load next, and now, in turn: 4096 x 4096 x 16384 384, 355 us; 6421 x
+// 12288 x 4096 469, 440; 2700 x 28672 x 4096 gated 480, 454; columns of 4096 x 4096 x 16384 400, 381, 1554 x 4096 x 28672
+// 349, 332, but of 60 x 4096 x 28672 (a tile of half the rows, K in parts) 55, 60.
 // Measured and left: loads in the first half stage behind the barrier alone (2 to 6 % more), one load to 4 to 6 MFMAs, one read
 // to 2 or 4, 32 x 32 x 16 MFMAs (12 % more on eight waves).
 #pragma once
@@ -100,7 +101,7 @@ struct WideTile {
     work.weights(0, w);
     // A load in asm has its place in m0, an operand of it that the compiler sets, and waits five states for scalars that a vector
     // instruction wrote (the compiler may keep some in lanes).  In the loop two MFMAs stand in the place of waits (five waits in
-    // front of each load cost 5 % at 1554 x 4096 x 28672: 347 us now).
+    // front of each load cost 5 % at 1554 x 4096 x 28672).
     auto place = [&](int j, int slot) { return (lptr_t)(mine + slot * SLOT + j * 1024); };
     auto load = [&](const Source& s, int j, int slot) {
       if constexpr (FORM == COLUMNS)

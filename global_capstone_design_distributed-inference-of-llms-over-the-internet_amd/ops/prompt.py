@@ -11,7 +11,8 @@ counts where this kernel was at least as fast at all three row counts timed insi
 both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
 
 A second table holds the same of 1 to 256 rows whose weights have no packed copy (a short fine-tuning request): there the
-library leaves most CUs idle at some shapes, 60 rows of 4096 columns of a 28672-row matrix took 163 us, 60 here.
+library leaves most CUs idle at some shapes, 60 rows of 4096 columns of a 28672-row matrix took 163 us, 60 here.  (Its first
+range, timed at 8, 16 and 32 rows, holds at 1 to 7 too: this kernel is the faster one at all nine shapes.)
 
 Everything else keeps the library.  (No rule on the shape alone holds at the shapes that were timed: "less than a wave of
 tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at 10 of 31 row-tile counts.)
