@@ -238,3 +238,23 @@ def test_gates_far_below_zero(form):
     torch.ops.mpamd.moe_gemm(form, x, torch.arange(3, dtype=torch.int32, device="cuda"), _lists([3]), ops.pack_weight(w)[None].contiguous(),
                              out, 3, 3, 1, 16, 0.0, 0)
     assert float(((out.double() - want) / want).abs().max()) < 2.0 ** -8 + 2e-5
+
+
+@pytest.mark.parametrize("counts", [[1, 0, 16], [300, 130, 20], [128, 257, 100]])
+@pytest.mark.parametrize("N", [32, 160])
+def test_nothing_behind_the_output(counts, N):
+    """What lies behind the last expert's rows, up to where a whole tile would end, stays as it was."""
+    ops.require_native()
+    K, R = 128, sum(counts)
+    g = torch.Generator().manual_seed(N + R)
+    x = torch.randn(R, K, generator=g).to(torch.bfloat16)
+    w = torch.randn(len(counts), N, K, generator=g).div(K ** 0.5).to(torch.bfloat16)
+    wp, tok = torch.stack([ops.pack_weight(m) for m in w.cuda()]), torch.arange(R, dtype=torch.int32, device="cuda")
+    z = torch.cat([r.double() @ w[e].double().t() for e, r in enumerate(x.split(counts))])
+    for glu in (0, 1):
+        room = torch.full((R + 512, N // (1 + glu)), -3.0, dtype=torch.bfloat16, device="cuda")
+        torch.ops.mpamd.moe_gemm(3, x.cuda(), tok, _lists(counts), wp, room[:R], R, R, glu, 16, 0.0, 0)
+        v = z.view(R, N // 32, 2, 16)
+        want = torch.nn.functional.silu(v[:, :, 0].reshape(R, -1)) * v[:, :, 1].reshape(R, -1) if glu else z
+        assert bool((room[R:] == -3.0).all())
+        assert float((room[:R].double().cpu() - want).norm() / want.norm()) < 2.0 ** -8
