@@ -710,10 +710,10 @@ __global__ __launch_bounds__(WM * WN * 64) void moe_gemm_tile_kernel(MoeGemm a) 
 // (8 experts of 8192 x 1024, weights in the 256 MB cache: 28.2, 36.0 us; of 8192 x 4096, from HBM: 105, 125).  Every XCD gets an
 // eighth of the whole tiles and an eighth of the half ones, each a run in order, whose CUs then share few rows and few weights.
 // Its G workgroups take whole tiles in turn; those that the r left over do not reach take two half ones first (one
-// first: within 1 %, but for down products of 1500 tokens, 4 % more), and the other half ones go round.  Where all that is left fits one half round, and a workspace is there, the r are cut at the
-// middle of K instead: a workgroup makes a half, and moe_gemm_close_kernel adds the two.  A workgroup's half tiles lie
-// between its whole ones, sooner in some than in others: their weights come from HBM a second time, and all at once that
-// bound them.
+// first: within 1 %, but for down products of 1500 tokens, 4 % more), and the other half ones go round.  Where all that
+// is left fits one half round, and a workspace is there, the r are cut at the middle of K instead: a workgroup makes a
+// half, and moe_gemm_close_kernel adds the two.  A workgroup's half tiles lie between its whole ones, sooner in some than
+// in others: their weights come from HBM a second time, and all at once that bound them.
 // Lane k of a wave knows tile k of up to 64 of them: the experts' tile counts are summed over the lanes, then every lane
 // looks for its own tile among them.
 constexpr int MW_SPLIT = 16;  // whole tiles an XCD cuts at most (twice as many fill 32 workgroups)
