@@ -4,7 +4,7 @@
 ``gemm_columns``: y = x w, a gradient's way back through a projection.
 The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
 on how its 256 x 256 tiles fill 256 CUs, 1.2 to 1.6.  So the choice is measured, as it is for the decode GEMMs, for
-the callers that ask (``tiles`` of ``ops.linear``: the hybrid decoders, fine-tuning, Mixtral): shapes in the committed table
+the callers that ask (``tiles`` of ``ops.linear``: stages and fine-tuning): shapes in the committed table
 (``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows, weights that no cache holds,
 as a model's do not stay there from one step to the next) run here at the row-tile
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in

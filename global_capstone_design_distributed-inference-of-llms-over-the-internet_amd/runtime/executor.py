@@ -783,18 +783,18 @@ class StageExecutor:
                     ops.rmsnorm(h, g_in, eps, out=xn, residual=res, mode=2)
                 else:
                     ops.rmsnorm(mlp, g_in, eps, out=xn, residual=res, mode=1)
-                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p, tiles=bool(L.moe))
+                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p, tiles=True)
                 kc, vc = self.cache.layer(li)
                 self._rope_attend(qkv, positions, slots, kc, vc, q_seq, q_ctx, attn, ws, ps, np_, False, qblocks,
                                   max_ctx, decode)
-                ops.linear(attn, L.dense("o"), out=o, wp=L.o_p, tiles=bool(L.moe))
+                ops.linear(attn, L.dense("o"), out=o, wp=L.o_p, tiles=True)
                 self._ar(o)
                 ops.rmsnorm(o, g_post, eps, out=xn, residual=res, mode=1)
                 if L.moe:
                     self._moe_mlp(L, xn, T, mlp, act, e, q_ctx, packed=False)
                     continue
-                ops.linear(xn, L.dense("gate_up"), out=act, epilogue=1, wp=gu_p)
-                ops.linear(act, L.dense("down"), out=mlp, wp=L.down_p)
+                ops.linear(xn, L.dense("gate_up"), out=act, epilogue=1, wp=gu_p, tiles=True)
+                ops.linear(act, L.dense("down"), out=mlp, wp=L.down_p, tiles=True)
                 self._ar(mlp)
         hout = res if mlp is None else ops.add(res, mlp, out=e("hout", (T, H)))
         if not self.is_last:
