@@ -1012,9 +1012,9 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
     ``ss_in`` (fused-norm consumer): ``x`` is the raw residual stream, ``w`` has the RMSNorm weight
     folded into its columns, and row r of the product is scaled by rsqrt(ss_in[r] / K + eps).
     ``tiles``: a prompt's product of row-major operands may run on this package's tile kernel (``prompt``), whose sums end
-    in another order than the library's, as far from 64-bit ones or less.  Every stage and fine-tuning ask for it: 20 ragged
-    prompts of Llama-2-7B through 2 blocks 5041 -> 4235 us (0.0082 and 0.0073 from 64 bits), one of 7995 tokens of an 8B
-    model, whose gate / up products alone it takes, 6563 -> 6342.
+    in another order than the library's, as far from 64-bit ones or less.  Fine-tuning, hybrid decoders, Mixtral's attention and
+    dense stages without a head ask for it: 20 ragged prompts of Llama-2-7B through 2 blocks 5041 -> 4235 us (0.0082 and 0.0073
+    from 64 bits).  With a head they do not: tokens sampled from its logits would be others.
     """
     if not _native(x):
         K = 32 * wp.shape[1] if wp is not None else w.shape[1]
