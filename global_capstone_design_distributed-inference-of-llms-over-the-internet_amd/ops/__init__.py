@@ -1031,6 +1031,9 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
         M, K = x.shape
     N = w.shape[0] if w is not None else 16 * wp.shape[0]
     policy = policy or _GEMM_POLICY
+    if tiles and a_rows is None and not out_packed and policy == "auto" and w is not None and \
+            prompt.mid(M, N, K, epilogue) and prompt.reads(x, w):  # (faster than packing the rows for the decode kernels, too)
+        return prompt.gemm(x, w, out, epilogue, glu_limit, mid=True)
     ok = wp is not None and native_gemm_ok(M, N, K, epilogue, out_packed) and (
         a_rows is not None or (x.stride(0) % 8 == 0 and x.stride(1) == 1))
     if ok and (policy in ("auto", "native") or a_rows is not None or out_packed):
@@ -1058,7 +1061,7 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
     if w is None:
         raise RuntimeError(f"no row-major weight for the hipBLASLt path (M={M}, N={N}, K={K})")
     if tiles and policy != "hipblaslt" and prompt.ok(x, w, epilogue):
-        return prompt.gemm(x, w, out, epilogue, glu_limit)
+        return prompt.gemm(x, w, out, epilogue, glu_limit, mid=prompt.mid(M, N, K, epilogue))
     if epilogue == 0 and out is not None and out.is_contiguous() and out.dtype == x.dtype and \
             out.shape == (M, N) and x.dim() == 2:
         return torch.mm(x, w.t(), out=out)  # hipBLASLt straight into the caller's buffer (no copy)

@@ -9,12 +9,12 @@
 // Workgroups of the same part are neighbours, so that an XCD's CUs still walk the same columns of shared rows (ranges that
 // begin anywhere, as many as CUs, lost that: 176 left-over tiles of K 11008 took 310 us, made whole 216 us).
 #include "act_io.h"
+#include "gemm_act.h"
 #include "wide_tile.h"
 
 namespace mp {
 
 constexpr int GW_CUS = WideTile::CUS, GW_BAND = 8;
-constexpr int GW_COLUMNS = 8;  // in place of an epilogue: w is [K, N], no epilogue
 constexpr int64_t GW_SLAB = 256 * 256;  // fp32 elements of a part
 // stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
 // tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
@@ -37,30 +37,11 @@ __device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, in
   m0 = (GW_BAND * band + r % h) * WideTile::BM;
   n0 = r / h * WideTile::BN;
 }
-// (divisions, ten instructions each: v_rcp_f32 in their place takes 2 % off 2700 x 28672 x 4096, but is off by 1 unit in 24 bits
-// instead of a half, and 0 where 1 + exp(-v) is 2^126 and more)
-template <int EPI, bool LIMIT>
-__device__ __forceinline__ void gw_act(const GemmPrompt& a, const f32x4& v, const f32x4& u, float (&y)[4]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (EPI == 1 && LIMIT) {
-      const float g = fminf(v[r], a.limit), w = fminf(fmaxf(u[r], -a.limit), a.limit);
-      y[r] = g / (1.f + __expf(-1.702f * g)) * (w + 1.f);
-    } else if (EPI == 1) {
-      y[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
-    } else if (EPI == 4) {
-      const float p = v[r] < 0.f ? 0.f : v[r];  // (not a number stays one)
-      y[r] = p * p;
-    } else {
-      y[r] = v[r];
-    }
-  }
-}
-
 // A workgroup's tiles: every ``step``-th whole one of its XCD's run from ``first`` on, then a part of a left-over tile.
 template <int EPI>
 struct PromptWork {
   static constexpr int STORES = WideTile::put_stores(EPI == 1);
+  static constexpr bool TURNS = false;
   typedef WideTile W;
   const GemmPrompt& a;
   int first, step, whole;  // (whole: how many whole ones)
@@ -116,7 +97,7 @@ struct PromptWork {
     const int nw = n0 + 16 * W::NW * W::wn(), cols = EPI == 1 ? a.N / 2 : a.N;
     auto go = [&](auto limit) {
       return W::put<EPI == 1, M>(a.out + (int64_t)m0 * cols, cols, a.M - m0, EPI == 1 ? nw / 2 : nw, acc,
-                                 [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI, limit.value>(a, v, u, y); });
+                                 [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI, limit.value>(a.limit, v, u, y); });
     };
     return EPI == 1 && a.limit > 0.f ? go(W::Int<1>()) : go(W::Int<0>());
   }
@@ -163,8 +144,8 @@ __global__ __launch_bounds__(WideTile::THREADS) void gemm_prompt_close_kernel(Ge
     for (int i = 0; i < 2; i += EPI == 1 ? 2 : 1)
       if (o + 16 * i < a.N) {
         float y[4];
-        if (EPI == 1 && a.limit > 0.f) gw_act<EPI, true>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
-        else gw_act<EPI, false>(a, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
+        if (EPI == 1 && a.limit > 0.f) gw_act<EPI, true>(a.limit, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
+        else gw_act<EPI, false>(a.limit, acc[i][j], acc[EPI == 1 ? i + 1 : i][j], y);
         st_vec<4>(a.out + (int64_t)(m + 16 * j) * (EPI == 1 ? a.N / 2 : a.N) + (EPI == 1 ? o / 2 + 8 * i : o + 16 * i) + 4 * g4, y);
       }
   }

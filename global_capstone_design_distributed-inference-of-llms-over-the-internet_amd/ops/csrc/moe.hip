@@ -763,6 +763,7 @@ __device__ __forceinline__ void moe_find(const MoeLists& l, int E, int ntn, bool
 template <bool GLU, typename TO>
 struct MoeWork {
   static constexpr int STORES = WideTile::put_stores(GLU);
+  static constexpr bool TURNS = false;
   typedef WideTile W;
   const MoeGemm& a;
   const MoeLists& l;

@@ -32,11 +32,17 @@
 
 namespace mp {
 
-struct WideTile {
-  static constexpr int BM = 256, BN = 256, MW = 8, NW = 8, WM = 2, WN = 2, THREADS = 64 * WM * WN;
-  static constexpr int PIECES = 8;  // loads of a wave and operand in a stage
-  static constexpr int SLOTS = 5, SLOT = 256 * 128, LDS = SLOTS * SLOT;
-  static constexpr int CUS = 256;  // workgroups of a launch at most: one to a CU
+// F: fragments of 16 rows that a wave has of either operand: 8, the form above, or 4, see gemm_mid.hip.
+template <int F, int SLOTS_>
+struct TileLoop {
+  static constexpr int BM = 32 * F, BN = 32 * F, MW = F, NW = F, WM = 2, WN = 2, THREADS = 64 * WM * WN;
+  static constexpr int PIECES = F;  // loads of a wave and operand in a stage
+  static constexpr int SLOTS = SLOTS_, SLOT = BM * 128, LDS = SLOTS * SLOT;
+  static constexpr int AHEAD = (SLOTS - 1) / 2;  // stages that loads are ahead
+  static_assert(SLOTS % 2 == 1 && SLOTS >= 5 && LDS <= 160 * 1024);
+  static constexpr int ON_CU = 160 * 1024 / LDS;  // workgroups on a CU
+  static constexpr int CUS = 256 * ON_CU;      // workgroups of a launch at most
+  static constexpr int LINE = 2 * BN;          // bytes of a row of columns
   enum Weights { ROWS, PACKED, COLUMNS };
   template <int V>
   struct Int {
@@ -60,9 +66,11 @@ struct WideTile {
   static __device__ __forceinline__ int packed_tile(int j) { return PIECES / 2 * wave() + (j >> 1); }
   static __device__ __forceinline__ int packed_byte(int j) { return 1024 * (j & 1) + (threadIdx.x & 63) * 16; }
   // the same of columns: row of a stage, and first of 8 columns
-  static __device__ __forceinline__ int column_row(int j) { return 2 * (PIECES * wave() + j) + ((threadIdx.x & 63) >> 5); }
+  static __device__ __forceinline__ int column_row(int j) {
+    return 1024 / LINE * (PIECES * wave() + j) + (threadIdx.x & 63) / (LINE / 16);
+  }
   static __device__ __forceinline__ int column_first(int j) {
-    const int row = column_row(j), chunk = (threadIdx.x & 31) >> 1;
+    const int row = column_row(j), chunk = threadIdx.x % (LINE / 16) >> 1;
     return 16 * (chunk ^ ((row & 3) | (row >> 3 & 1) << 2)) + 8 * (threadIdx.x & 1);
   }
 
@@ -79,12 +87,17 @@ struct WideTile {
     }
   };
 
+  template <bool LANES>  // (of a value that is the same in all lanes, which the compiler may not see)
+  static __device__ __forceinline__ uint32_t scalar(uint32_t v) { return LANES ? __builtin_amdgcn_readfirstlane(v) : v; }
+
   // The workgroup's tiles 0 .. count - 1 (at least one).  ``work``:
   //   int stages(k)                  stages of tile k, at least one
   //   void row_offsets(Source&), weight_offsets(Source&)   the lane's offsets, once
   //   void rows(k, Source&)          tile k's rows (may change the offsets)
   //   void weights(k, Source&)       its weight rows
-  //   bool half(k)                   has it at most 128 rows?
+  //   bool half(k)                   has it at most half of its rows?
+  //   TURNS, int turn(k)             does a tile begin with another stage than its first: rows and weights are there, turn(k) stages
+  //                                  stand ahead of it and come last
   //   int store<M>(k, acc)           acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (M wm + j) .., j < M; lane: row lane % 16,
   //                                  weight rows 4 (lane / 16) .. + 3.  At least how many stores were issued: 0 or
   //                                  work.STORES of M = 8, half of them of M = 4.
@@ -95,6 +108,8 @@ struct WideTile {
     char* mine = smem + wave() * (PIECES * 1024);
     Source x, w;
     int lk = 0, left = work.stages(0);  // the tile that is being loaded, its stages left
+    int turn = 0;  // how many of them stand ahead of the one it begins with
+    if constexpr (Work::TURNS) turn = work.turn(0);
     work.row_offsets(x);
     work.weight_offsets(w);
     work.rows(0, x);
@@ -106,7 +121,7 @@ struct WideTile {
     auto load = [&](const Source& s, int j, int slot) {
       if constexpr (FORM == COLUMNS)
         asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                     :: "v"(s.off[j]), "s"(s.words), "s"(s.at), "{m0}"((uint32_t)(uintptr_t)place(j, slot)) : "memory");
+                     :: "v"(s.off[j]), "s"(s.words), "s"(scalar<Work::TURNS>(s.at)), "{m0}"((uint32_t)(uintptr_t)place(j, slot)) : "memory");
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, place(j, slot), 16, s.off[j], s.at, 0, 0);
     };
@@ -116,13 +131,20 @@ struct WideTile {
       if (__builtin_expect(--left == 0, 0)) {
         x.at -= x.step, w.at -= w.step;
         left = 1;
-        if (lk + 1 < count) left = work.stages(++lk), work.rows(lk, x), work.weights(lk, w);
+        if (lk + 1 < count) {
+          left = work.stages(++lk), work.rows(lk, x), work.weights(lk, w);
+          if constexpr (Work::TURNS) turn = work.turn(lk);
+        }
+      } else if (Work::TURNS && left == turn) {
+        const uint32_t n = work.stages(lk);
+        x.at -= n * x.step, w.at -= n * w.step;
       }
     };
     // a row's chunk c lies at 16 (c ^ row % 8)
     const int s0 = 16 * (g4 ^ (c16 & 7)), s1 = 16 * ((4 + g4) ^ (c16 & 7));
     const int wr = FORM == PACKED    ? 2048 * NW * wn() + lane * 16
-                   : FORM == COLUMNS ? (8 * g4 + (c16 >> 2)) * 512 + 256 * wn() + 32 * (c16 >> 2 | (g4 & 1) << 2) + 8 * (c16 & 3)
+                   : FORM == COLUMNS
+                       ? (8 * g4 + (c16 >> 2)) * LINE + ((32 * NW * wn()) ^ (32 * (c16 >> 2 | (g4 & 1) << 2))) + 8 * (c16 & 3)
                                      : (16 * NW * wn() + c16) * 128;
     u16x8 xa[MW], wa[NW], xb[MW], wb[NW];
     f32x4 acc[NW][MW];
@@ -134,9 +156,9 @@ struct WideTile {
       if (r < m) {
         xf[r] = *reinterpret_cast<const u16x8*>(smem + px * SLOT + xr + (h ? s1 : s0) + r * 2048);
       } else if constexpr (FORM == COLUMNS) {
-        const char* p = smem + ((pw * SLOT + wr) ^ (32 * (r - m))) + h * 16384;
+        const char* p = smem + ((pw * SLOT + wr) ^ (32 * (r - m))) + h * 32 * LINE;
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 2048));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 4 * LINE));
         wf[r - m] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       } else {
         wf[r - m] = *reinterpret_cast<const u16x8*>(smem + pw * SLOT + wr + (FORM == PACKED ? h * 1024 : h ? s1 : s0) + (r - m) * 2048);
@@ -144,15 +166,16 @@ struct WideTile {
     };
     auto tile = [&](auto fragments, int k) __attribute__((always_inline)) {
       constexpr int M = decltype(fragments)::value;  // fragments of a wave's rows
-      constexpr int R = M == MW ? 3 : 2;             // MFMAs to a read
+      constexpr int R = F == 4 ? 1 : M == MW ? 3 : 2;  // MFMAs to a read
+      constexpr int TURN = 2 * NW;                     // MFMAs of two fragments of rows
       const int xr = (16 * M * wm() + c16) * 128;
       // MFMA q of a half stage: two fragments of rows at a time.  An operand that a vector instruction wrote (a cleared sum, a
       // copy at the loop's head) has to be two wait states old, which nobody counts for asm: a stage's first MFMA has them with it.
       auto weight_of = [](int q) {
-        const int b = q % 16 / 4, s = q % 4, down = q / 16 & 1;
-        return 2 * (down ? 3 - b : b) + ((s == 1 || s == 2) != down);
+        const int b = q % TURN / 4, s = q % 4, down = q / TURN & 1;
+        return 2 * (down ? NW / 2 - 1 - b : b) + ((s == 1 || s == 2) != down);
       };
-      auto row_of = [](int q) { return 2 * (q / 16) + ((q % 4 >= 2) != (q % 16 / 4 & 1)); };
+      auto row_of = [](int q) { return 2 * (q / TURN) + ((q % 4 >= 2) != (q % TURN / 4 & 1)); };
       auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], bool first) {
         const int i = weight_of(q), j = row_of(q);
         if (first)
@@ -167,7 +190,7 @@ struct WideTile {
         asm volatile("s_nop 2\n\tv_mfma_f32_16x16x32_bf16 %0, %2, %3, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %4, %5, %1\n\t"
                      "buffer_load_dwordx4 %6, %7, %8 offen lds"
                      : "+a"(acc[i][j]), "+a"(acc[i1][j1])
-                     : "v"(wf[i]), "v"(xf[j]), "v"(wf[i1]), "v"(xf[j1]), "v"(s.off[l]), "s"(s.words), "s"(s.at), "{m0}"(to)
+                     : "v"(wf[i]), "v"(xf[j]), "v"(wf[i1]), "v"(xf[j1]), "v"(s.off[l]), "s"(s.words), "s"(scalar<Work::TURNS>(s.at)), "{m0}"(to)
                      : "memory");
       };
       // a half stage: the products of the operands read before, reads of the next half's, the loads of a stage of one operand
@@ -175,7 +198,7 @@ struct WideTile {
         constexpr bool B = decltype(second)::value;
 #pragma unroll
         for (int q = 0; q < NW * M; ++q) {
-          constexpr int AT = B ? 1 : M - 3;
+          constexpr int AT = B || M < 4 ? 1 : M - 3;
           if (FORM == COLUMNS && q % M == AT) multiply2(q, B ? xb : xa, B ? wb : wa, B ? x : w, q / M, B ? fw : fx);
           else if (FORM != COLUMNS || q % M != AT - 1) multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
           if (q % R == R - 1 && q / R < M + NW) take1(!B, q / R, xr, B ? xa : xb, B ? wa : wb, M);
@@ -197,11 +220,12 @@ struct WideTile {
       for (int st = 0; st < n; ++st) {
         __builtin_amdgcn_sched_barrier(0);
         half_stage(Int<0>());
-        // the next stage has landed for all waves, and all have read this one.  In flight: the weights of the stage after the
-        // next and the stores of the tile before
-        if (stored == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
-        else if (stored < Work::STORES) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES + Work::STORES / 2) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES + Work::STORES) : "memory");
+        // the next stage has landed for all waves, and all have read this one.  In flight: what is loaded of later stages (of five
+        // slots the weights of the stage after the next) and the stores of the tile before
+        constexpr int FLY = (SLOTS - 4) * PIECES;
+        if (stored == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLY) : "memory");
+        else if (stored < Work::STORES) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLY + Work::STORES / 2) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLY + Work::STORES) : "memory");
         stored = 0;
         asm volatile("" : "+s"(stored));  // (one loop: the compiler would make the first stage a second one)
         lds_wait_barrier();
@@ -216,15 +240,15 @@ struct WideTile {
       stored = work.template store<M>(k, acc);
     };
 #pragma unroll 1
-    for (int s = 0; s < 2; ++s) {  // w 0, x 0, w 1, x 1
+    for (int s = 0; s < AHEAD; ++s) {  // w 0, x 0, w 1, x 1 ..
 #pragma unroll
       for (int j = 0; j < PIECES; ++j) load(w, j, 2 * s);
 #pragma unroll
       for (int j = 0; j < PIECES; ++j) load(x, j, 2 * s + 1);
       step();
     }
-    fx = SLOTS - 1;  // (w 2)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PIECES) : "memory");
+    fx = SLOTS - 1;  // (the next weights)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 * AHEAD - 2) * PIECES) : "memory");
     lds_wait_barrier();
 #pragma unroll
     for (int r = 0; r < NW; ++r) take1(0, r, 0, xa, wa, 0);
@@ -289,5 +313,6 @@ struct WideTile {
     return put_stores(GLU) * M / MW;
   }
 };
+typedef TileLoop<8, 5> WideTile;
 
 }  // namespace mp

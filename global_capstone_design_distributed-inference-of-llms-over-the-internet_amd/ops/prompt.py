@@ -10,9 +10,12 @@ as a model's do not stay there from one step to the next) run here at the row-ti
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
 both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
 
-A second table holds the same of 1 to 256 rows whose weights have no packed copy (a short fine-tuning request): there the
-library leaves most CUs idle at some shapes, 60 rows of 4096 columns of a 28672-row matrix took 163 us, 60 here.  (Its first
-range, timed at 8, 16 and 32 rows, holds at 1 to 7 too: this kernel is the faster one at all nine shapes.)
+Up to 384 rows there are tiles of 128 x 128 as well (csrc/gemm_mid.hip), by a table of theirs, timed against what runs without
+them: 66 rows of Mistral-7B, forward and backward, 1031 -> 832 us.  The library's call costs the host 25 us, theirs 7, so they stay
+where they are up to 3 % slower on the GPU; weights of less than 4M elements always go there: a prompt of 153 tokens of a
+512-wide model, 503 -> 381 us for two blocks.  (Ranges that were timed at 8, 16 and 32 rows hold at 1 to 7 too: 1.0 to 1.7 times as
+fast as the library's at 33 of 36 shapes, 0.93 at the worst.)
+A third table holds those few of 1 to 256 rows that are best on the large tiles.
 
 Everything else keeps the library.  (No rule on the shape alone holds at the shapes that were timed: "less than a wave of
 tiles, K from 10240 on, parts that fill 218 CUs or more" picks the slower one at 10 of 31 row-tile counts.)
@@ -29,14 +32,18 @@ import torch
 
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned", "prompt_gemm_gfx950.json")
 FEW_TABLE = TABLE.replace("prompt_gemm", "prompt_few")  # the same of few rows: 1 to 4 for up to 32, 64, 128, 256
+MID_TABLE = TABLE.replace("prompt_gemm", "prompt_mid")  # those that the 128 x 128 tiles make, in ``MID``'s ranges
 COLUMNS = 8  # in an epilogue's place: x w
 EPILOGUES = (0, 1, 4, COLUMNS)
 TILE, MAX_ROWS = 256, 8192
 FEW = (32, 64, 128, TILE)  # (a tile of up to 128 rows takes half the products; the library's times jump at all four)
+MID = (32, 64, 96, 128, 192, 256, 384)
+SMALL = 1 << 22  # elements of a weight below which a product is bound by its call
 Shape = Tuple[int, int, int]  # N, K, epilogue
 
 _LOCK = threading.Lock()
-_STATE: dict = {"table": None, "few": None}
+_STATE: dict = {"table": None, "few": None, "mid": None}
+_PATHS = {"table": TABLE, "few": FEW_TABLE, "mid": MID_TABLE}
 
 
 def _key(shape: Shape) -> str:
@@ -56,10 +63,10 @@ def _load(path: str) -> Dict[Shape, FrozenSet[int]]:
 
 def table(name: str = "table") -> Dict[Shape, FrozenSet[int]]:
     """(N, K, epilogue) -> row-tile counts at which the kernel runs (read once; MPAMD_KERNEL_TABLE=0: none); ``few``: the
-    same of ``FEW``'s ranges."""
+    same of ``FEW``'s ranges; ``mid``: of ``MID``'s, those at which ``gemm_mid`` does."""
     with _LOCK:
         if _STATE[name] is None:
-            path = FEW_TABLE if name == "few" else TABLE
+            path = _PATHS[name]
             on = os.environ.get("MPAMD_KERNEL_TABLE") != "0" and os.path.exists(path)
             _STATE[name] = _load(path) if on else {}
         return _STATE[name]
@@ -82,7 +89,16 @@ def few(M: int, N: int, K: int, epilogue: int) -> bool:
         next(i for i, n in enumerate(FEW, 1) if M <= n) in table("few").get((N, K, epilogue), ())
 
 
-def _reads(x: torch.Tensor, w: torch.Tensor) -> bool:
+def mid(M: int, N: int, K: int, epilogue: int) -> bool:
+    """Does a step of M rows run this product on the 128 x 128 tiles?"""
+    if not shape_ok(M, N, K, epilogue) or M > MAX_ROWS:
+        return False
+    if N * K < SMALL:
+        return os.environ.get("MPAMD_KERNEL_TABLE") != "0"
+    return M <= MID[-1] and next(i for i, n in enumerate(MID, 1) if M <= n) in table("mid").get((N, K, epilogue), ())
+
+
+def reads(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Are these operands that the kernel reads (types, strides, alignments), in a call that is not differentiated?"""
     if x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
@@ -99,7 +115,7 @@ def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
     if w is None or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         return False
     shape = x.shape[0], w.shape[0], w.shape[1], epilogue
-    return (chosen(*shape) or few(*shape)) and _reads(x, w)
+    return (mid(*shape) or chosen(*shape) or few(*shape)) and reads(x, w)
 
 
 def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0):
@@ -109,24 +125,32 @@ def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0):
     return y
 
 
-def gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, epilogue: int = 0, limit: float = 0.0):
+def _run_mid(x, w, y, N: int, epilogue: int, limit: float = 0.0):
+    need = torch.ops.mpamd.gemm_mid_ws(x.shape[0], N, x.shape[1])
+    ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+    torch.ops.mpamd.gemm_mid(x, w, y, ws, epilogue, limit)
+    return y
+
+
+def gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, epilogue: int = 0, limit: float = 0.0,
+         mid: bool = False):
     """epilogue 0: x w^T; 1: the gated forms over gate / up rows in blocks of 16 (``limit`` 0: silu); 4: max(., 0)^2."""
     M, N = x.shape[0], w.shape[0]
     cols = N // 2 if epilogue == 1 else N
     y = out if out is not None and out.is_contiguous() and out.dtype == x.dtype and out.data_ptr() % 16 == 0 else \
         torch.empty(M, cols, dtype=x.dtype, device=x.device)
-    _run(x, w, y, N, epilogue, limit)
+    (_run_mid if mid else _run)(x, w, y, N, epilogue, limit)
     return y if out is None or y is out else out.copy_(y)
 
 
 def gemm_columns(x: torch.Tensor, w: torch.Tensor, always: bool = False) -> torch.Tensor:
     """x w of rows [M, K] and weights [K, N]: on the kernel where the table says so (or ``always``), else the library's."""
-    here = always
+    run = _run if always else None
     if not always and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[0]:
         shape = x.shape[0], w.shape[1], w.shape[0], COLUMNS
-        here = (chosen(*shape) or few(*shape)) and _reads(x, w)
-    if here:
-        return _run(x, w, torch.empty(x.shape[0], w.shape[1], dtype=x.dtype, device=x.device), w.shape[1], COLUMNS)
+        run = _run_mid if mid(*shape) else _run if chosen(*shape) or few(*shape) else None
+    if run and (always or reads(x, w)):
+        return run(x, w, torch.empty(x.shape[0], w.shape[1], dtype=x.dtype, device=x.device), w.shape[1], COLUMNS)
     return torch.mm(x, w)
 
 
@@ -168,19 +192,24 @@ def agreed(sweeps: Iterable[Dict[Shape, list]]) -> Dict[Shape, list]:
 
 ROWS = {m: (TILE * m - 251, TILE * m - 124, TILE * m) for m in range(2, MAX_ROWS // TILE + 1)}
 FEW_ROWS = {1: (8, 16, 32), 2: (33, 48, 64), 3: (65, 96, 128), 4: (129, 192, 256)}
+MID_ROWS = {1: (8, 16, 32), 2: (33, 48, 64), 3: (65, 80, 96), 4: (97, 112, 128), 5: (129, 160, 192), 6: (193, 224, 256),
+            7: (257, 320, 384)}
 
 
-def tune(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS) -> Dict[Shape, list]:
+def tune(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS, kernel=None) -> Dict[Shape, list]:
     """The row-tile counts of every shape at which the kernel is faster, in both of two sweeps (``rows``: what is timed of
-    each)."""
+    each; ``kernel``: ``_run_mid``, else ``_run``)."""
     todo = list(todo)
-    return agreed([sweep(todo, device, log, rows) for _ in range(2)])
+    return agreed([sweep(todo, device, log, rows, kernel or _run) for _ in range(2)])
 
 
-def sweep(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS) -> Dict[Shape, list]:
-    """Time both products over the row-tile counts of every shape, best of three rounds in turn."""
+def sweep(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS, kernel=None) -> Dict[Shape, list]:
+    """Time both products over the row-tile counts of every shape, best of three rounds in turn: the kernel and the library's, or
+    ``_run_mid`` and what would run in its place, where the library's call costs the host 20 us more, which is what the 3 % are for
+    elsewhere."""
     from . import hybrid, require_native, swiglu, use_tuned_gemms
 
+    kernel = kernel or _run
     require_native()
     use_tuned_gemms()
 
@@ -219,11 +248,15 @@ def sweep(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS) -> Dict[Sha
                         hybrid.relu2(z, y)
 
                 def tile():
+                    kernel(x, next(turn), y, N, epi)
+
+                def old():
                     _run(x, next(turn), y, N, epi)
 
-                t = [min(v) for v in zip(*[(ms(lib), ms(tile)) for _ in range(3)])]
+                other = old if kernel is _run_mid and (few(M, N, K, epi) or chosen(M, N, K, epi)) else lib
+                t = [min(v) for v in zip(*[(ms(other), ms(tile)) for _ in range(3)])]
                 ratios.append(t[0] / t[1])
-            if min(ratios) >= 1.0 and sum(ratios) / 3 >= 1.03:
+            if min(ratios) >= (0.97 if kernel is _run_mid else 1.0) and sum(ratios) / 3 >= (1.0 if kernel is _run_mid else 1.03):
                 tiles.append(m)
         got[(N, K, epi)] = tiles
         if log:

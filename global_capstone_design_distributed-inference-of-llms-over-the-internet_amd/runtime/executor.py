@@ -787,7 +787,9 @@ class StageExecutor:
                     ops.rmsnorm(h, g_in, eps, out=xn, residual=res, mode=2)
                 else:
                     ops.rmsnorm(mlp, g_in, eps, out=xn, residual=res, mode=1)
-                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p, tiles=tiles or bool(L.moe))
+                # (the packed weights of a unit norm carry its weight, the row-major ones do not)
+                rows = not (folded_bf16 and fold_native)
+                ops.linear(xn, L.dense("qkv"), out=qkv, wp=qkv_p, tiles=rows and (tiles or bool(L.moe)))
                 kc, vc = self.cache.layer(li)
                 self._rope_attend(qkv, positions, slots, kc, vc, q_seq, q_ctx, attn, ws, ps, np_, False, qblocks,
                                   max_ctx, decode)
@@ -797,7 +799,7 @@ class StageExecutor:
                 if L.moe:
                     self._moe_mlp(L, xn, T, mlp, act, e, q_ctx, packed=False)
                     continue
-                ops.linear(xn, L.dense("gate_up"), out=act, epilogue=1, wp=gu_p, tiles=tiles)
+                ops.linear(xn, L.dense("gate_up"), out=act, epilogue=1, wp=gu_p, tiles=rows and tiles)
                 ops.linear(act, L.dense("down"), out=mlp, wp=L.down_p, tiles=tiles)
                 self._ar(mlp)
         hout = res if mlp is None else ops.add(res, mlp, out=e("hout", (T, H)))
