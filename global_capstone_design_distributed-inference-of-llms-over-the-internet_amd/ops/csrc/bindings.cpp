@@ -30,6 +30,7 @@ int mp_paged_attention(const void* q, int64_t q_stride, const void* kc, const vo
 int mp_embedding(const int64_t* ids, const void* table, void* out, int T, int H, int64_t vocab, hipStream_t stream);
 int mp_swiglu(const void* gu, void* out, int64_t T, int F, hipStream_t stream);
 int mp_add(const void* a, const void* b, void* y, int64_t n, hipStream_t stream);
+int mp_plan_input(const uint64_t* host, uint64_t* meta, int64_t nb, uint64_t* table, int64_t nt, hipStream_t stream);
 int mp_step_input(const uint64_t* host, uint64_t* meta, int nb, const uint64_t* x, uint64_t* dst, int64_t nx, hipStream_t stream);
 int mp_argmax(const void* logits, int64_t stride, int R, int V, int64_t* out, int f32, hipStream_t stream);
 int mp_sample(const void* logits, int64_t stride, int R, int V, const float* temps, const float* top_ps,
@@ -505,6 +506,20 @@ void step_input(const at::Tensor& host, at::Tensor& meta, const c10::optional<at
                "step_input");
 }
 
+// meta, then table (where there is one) <- host (pinned bytes, one behind the other)
+void plan_input(const at::Tensor& host, at::Tensor& meta, const c10::optional<at::Tensor>& table) {
+  auto word = [](const at::Tensor& t) { return t.is_contiguous() && (t.nbytes() | reinterpret_cast<uintptr_t>(t.data_ptr())) % 8 == 0; };
+  const int64_t nt = table.has_value() ? table->nbytes() : 0;
+  MP_CHECK(host.device().is_cpu() && word(host), "host: words of 8 bytes");
+  MP_CHECK(meta.is_cuda() && word(meta) && (int64_t)(meta.nbytes() + nt) == (int64_t)host.nbytes() && host.nbytes() < (1u << 30), "meta");
+  MP_CHECK(nt == 0 || (table->is_cuda() && table->device() == meta.device() && word(*table)), "table");
+  const c10::hip::HIPGuard guard(meta.device().index());
+  MP_CHECK(reads_pinned(host) || host.is_pinned(), "host: pinned");
+  check_launch(mp_plan_input((const uint64_t*)host.data_ptr(), (uint64_t*)meta.data_ptr(), meta.nbytes() / 8,
+                             nt ? (uint64_t*)table->data_ptr() : nullptr, nt / 8, cur_stream()),
+               "plan_input");
+}
+
 void argmax(const at::Tensor& logits, at::Tensor& out) {
   const bool f32 = logits.scalar_type() == at::kFloat;
   if (!f32) check_bf16_cuda(logits, "logits");
@@ -873,6 +888,7 @@ TORCH_LIBRARY(mpamd, m) {
   m.def("embedding(Tensor ids, Tensor table, Tensor(a!) out) -> ()");
   m.def("swiglu(Tensor gu, Tensor(a!) out) -> ()");
   m.def("add(Tensor a, Tensor b, Tensor(a!) y) -> ()");
+  m.def("plan_input(Tensor host, Tensor(a!) meta, Tensor(b!)? table) -> ()");
   m.def("step_input(Tensor host, Tensor(a!) meta, Tensor? x, Tensor(b!) dst) -> ()");
   m.def("argmax(Tensor logits, Tensor(a!) out) -> ()");
   m.def(
@@ -912,6 +928,7 @@ TORCH_LIBRARY_IMPL(mpamd, CUDA, m) {
   m.impl("embedding", &embedding);
   m.impl("swiglu", &swiglu);
   m.impl("add", &add);
+  m.impl("plan_input", &plan_input);
   m.impl("step_input", &step_input);
   m.impl("argmax", &argmax);
   m.impl("sample", &sample);

@@ -138,6 +138,74 @@ class _Pinned:
             self.events[self.k] = ev
 
 
+class _PlanInput:
+    """Staging of what a step of several tokens per session takes in (its plan and a changed block table): one pinned buffer, one
+    device buffer and one launch a step.  A ring, so that the host runs ahead; an event costs the stream 6 us, so each half
+    of the turns has one, and a half is written again when the steps that read it are done.  A buffer that grew is a new one:
+    the launches tell the allocator of pinned memory which work reads the old one."""
+
+    TURNS = 4
+
+    def __init__(self, device, size: int):
+        self.device, self.size = device, 0
+        self.want = 0  # bytes that did not fit a step's buffer, on top of it
+        self._grow(size)
+
+    def _grow(self, size: int) -> None:
+        self.size = -(-size // 4096) * 4096
+        self._host = torch.empty(self.TURNS, self.size, dtype=torch.uint8, pin_memory=True)
+        self._np = self._host.numpy()
+        self._ev, self._k = [None, None], 0
+
+    def open(self, size: int) -> None:
+        """``size`` bytes of arrays, up to 15 more for each, and of the table."""
+        if size + self.want > self.size:
+            self._grow(size + self.want)
+        half = self.TURNS // 2
+        if self._k % half == 0 and self._ev[self._k // half] is not None:
+            self._ev[self._k // half].synchronize()
+        self._at = 0
+        self._dev = torch.empty(self.size, dtype=torch.uint8, device=self.device)
+
+    def room(self, shape, dtype):
+        """(host array to fill, device tensor that will hold it), or None: the buffer is full."""
+        n = int(np.prod(shape)) * np.dtype(dtype).itemsize
+        a = self._at
+        if a + n > self.size:
+            self.want += a + n - self.size
+            return None
+        self._at = a + -(-n // 16) * 16
+        return (self._np[self._k, a:a + n].view(dtype).reshape(shape),
+                self._dev[a:a + n].view(_TORCH[np.dtype(dtype)]).view(shape))
+
+    def put(self, a: np.ndarray) -> torch.Tensor:
+        got = self.room(a.shape, a.dtype)
+        if got is None:
+            return torch.from_numpy(np.ascontiguousarray(a)).to(self.device, non_blocking=True)
+        got[0][...] = a
+        return got[1]
+
+    def close(self, sessions: SessionManager) -> None:
+        k, n = self._k, min(self._at, self.size)
+        t = sessions.table.nbytes
+        here = t % 8 == 0 and n + t <= self.size
+        if not here:
+            self.want += t
+        table = here and sessions.take_table(self._np[k, n:n + t].view(np.int32))
+        if not here:
+            sessions.sync_table()
+        if n or table:
+            torch.ops.mpamd.plan_input(self._host[k, :n + t if table else n], self._dev[:n], sessions.table_dev if table else None)
+        half = self.TURNS // 2
+        if k % half == half - 1:
+            self._ev[k // half] = torch.cuda.Event()
+            self._ev[k // half].record()
+        self._k = (k + 1) % self.TURNS
+
+
+_TORCH = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32}
+
+
 class StageExecutor:
     def __init__(self, cfg: ModelConfig, weights: StageWeights, device, *, dtype=torch.bfloat16,
                  page_size: int = 64, max_sessions: int = 256, max_seq_len: Optional[int] = None,
@@ -210,7 +278,10 @@ class StageExecutor:
         self._recv_pin: Dict[int, tuple] = {}
         # qkv fold per decode-graph batch bucket (_confirm_qkv_fold's end-to-end A/B on THIS executor)
         self.qkv_fold_by_bucket: Dict[int, bool] = {}
-        self._pinned = _Pinned(2 * max_tokens_per_step, 2 * max_tokens_per_step + max_sessions, self.device)
+        gpu = self.device.type == "cuda"
+        self._input = _PlanInput(self.device, self._input_bytes(max_tokens_per_step, max_sessions)) if gpu else None
+        most = max_sessions if gpu else max_tokens_per_step  # tokens of a step whose plan is not staged there
+        self._pinned = _Pinned(2 * most, 2 * most + max_sessions, self.device)
         self.last_step_ms: Optional[float] = None
         # graph_hook(out): recorded at the END of every decode graph capture (the static output
         # buffer), e.g. the stage hop's RCCL send (parallel/engine.py graph hop); last_graphed
@@ -352,6 +423,9 @@ class StageExecutor:
         return self.cfg.hidden_width
 
     # ================================================================== planning
+    def _input_bytes(self, T: int, S: int) -> int:
+        return 24 * T + 4 * S + self.sessions.table.nbytes + (1 << 14)
+
     def plan(self, seqs: Sequence[Tuple[str, int]], *, reset: Sequence[bool] = (), max_length: Optional[int] = None,
              starts: Optional[Sequence[int]] = None) -> Plan:
         """Open/extend sessions and build device metadata for a ragged step.
@@ -378,14 +452,22 @@ class StageExecutor:
         if T > self.max_tokens:
             raise ValueError(f"step has {T} tokens > max_tokens_per_step {self.max_tokens}")
         rows = np.fromiter((s.row for s in sess), dtype=np.int32, count=S)
-        h64, h32 = self._pinned.next()
-        n64 = h64[: 2 * T].numpy().reshape(2, T) if T else np.empty((2, 0), np.int64)
-        n32 = h32[: 2 * T + S].numpy()
+        is_decode = bool(S and (ntoks == 1).all())
+        inp = self._input if T and not is_decode else None
+        if inp is not None:
+            inp.open(self._input_bytes(T, S))
+            (n64, m64), (n32, m32) = inp.room((2, T), np.int64), inp.room((2 * T + S,), np.int32)
+            dev = m64, m32
+        else:
+            dev = None
+            h64, h32 = self._pinned.next()
+            n64 = h64[: 2 * T].numpy().reshape(2, T) if T else np.empty((2, 0), np.int64)
+            n32 = h32[: 2 * T + S].numpy()
         native.build_meta(rows, st, ntoks, self.sessions.table, self.cache.page_size, n64[0], n64[1], n32[:T],
                           n32[T:2 * T], n32[2 * T:])
-        self.sessions.sync_table()
+        if inp is None:
+            self.sessions.sync_table()
         max_ctx = int((st + ntoks).max()) if S else 0
-        is_decode = bool(S and (ntoks == 1).all())
         pinned = self._pinned
 
         def upload():
@@ -398,18 +480,20 @@ class StageExecutor:
                 d32 = h32[: 2 * T + S].clone()
             return d64, d32
 
-        hp = self._hybrid.plan(ntoks, st, rows) if self._hybrid is not None and not is_decode else None
-        qb = sb = fb = None
+        qb = sb = fb = hp = None
         fa_waves = 4
-        if self.device.type == "cuda" and not is_decode and self._attn_fa:
-            fbn, fa_waves = ops.fa_plan(ntoks, self.nh, self.nkv, self._n_cu)
-            fb = torch.from_numpy(fbn).to(self.device, non_blocking=True)
-        if self.device.type == "cuda" and not is_decode and self._attn_mfma_prefill:
-            qb = torch.from_numpy(ops.query_blocks(ntoks, self.nh // self.nkv)).to(self.device, non_blocking=True)
-            if self._attn_grouped:
-                sb = torch.from_numpy(ops.query_superblocks(ntoks, self.nh // self.nkv)).to(self.device,
-                                                                                              non_blocking=True)
-        return Plan(sess, ntoks, st, T, max_ctx, is_decode, n64, n32, qb, sb, fb, fa_waves, hp, _upload=upload)
+        if self._hybrid is not None and not is_decode:
+            hp = self._hybrid.plan(ntoks, st, rows, inp.put if inp is not None else None)
+        if inp is not None:
+            if self._attn_fa:
+                fbn, fa_waves = ops.fa_plan(ntoks, self.nh, self.nkv, self._n_cu)
+                fb = inp.put(fbn)
+            if self._attn_mfma_prefill and (fb is None or T <= ops.wide_rows()):  # (packed steps', which have no other kernel)
+                qb = inp.put(ops.query_blocks(ntoks, self.nh // self.nkv))
+                if self._attn_grouped:
+                    sb = inp.put(ops.query_superblocks(ntoks, self.nh // self.nkv))
+            inp.close(self.sessions)
+        return Plan(sess, ntoks, st, T, max_ctx, is_decode, n64, n32, qb, sb, fb, fa_waves, hp, _dev=dev, _upload=upload)
 
     def commit(self, plan: Plan) -> None:
         for s, n in zip(plan.sessions, plan.ntoks):
@@ -565,6 +649,10 @@ class StageExecutor:
         """Paged attention: MFMA flash attention for prefill blocks (``qblocks``) and GQA decode,
         else the flash-decoding kernel."""
         table = self.sessions.table_dev
+        fb = getattr(self, "_cur_fb", None)
+        if fb is not None and not packed:
+            return ops.attention_fa(qkv, kc, vc, table, q_seq, q_ctx, fb, self.nh, self.nkv, self.scale, out=out,
+                                    workspace=ws, max_ctx=max_ctx, waves=getattr(self, "_cur_fw", 4))
         if qblocks is None and self.gqa_decode_mfma and self.device.type == "cuda":
             T = qkv.shape[0]
             ps2 = 128 * math.ceil(ps / 128)
@@ -572,10 +660,6 @@ class StageExecutor:
             return ops.attention_mfma(qkv, kc, vc, table, q_seq, q_ctx, self.decode_qblocks(T), self.nh, self.nkv,
                                       self.scale, out=out, workspace=ws, part_size=ps2, num_parts=np2,
                                       packed=packed)
-        fb = getattr(self, "_cur_fb", None)
-        if qblocks is not None and fb is not None and not packed:
-            return ops.attention_fa(qkv, kc, vc, table, q_seq, q_ctx, fb, self.nh, self.nkv, self.scale, out=out,
-                                    workspace=ws, max_ctx=max_ctx, waves=getattr(self, "_cur_fw", 4))
         if qblocks is not None:
             return ops.attention_mfma(qkv, kc, vc, table, q_seq, q_ctx, qblocks, self.nh, self.nkv, self.scale,
                                       out=out, workspace=ws, max_ctx=max_ctx, packed=packed,

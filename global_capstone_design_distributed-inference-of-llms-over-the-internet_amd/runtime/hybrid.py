@@ -487,12 +487,13 @@ class HybridStage:
         return x[:, W:]
 
     # ------------------------------------------------------------------ plans
-    def plan(self, ntoks, starts, rows) -> dict:
+    def plan(self, ntoks, starts, rows, up=None) -> dict:
         """Device description of a ragged step (not one token per session): ``ntoks`` tokens per session after the
-        ``starts`` it already holds; ``rows``: the sessions' rows of the block table."""
+        ``starts`` it already holds; ``rows``: the sessions' rows of the block table; ``up``: host array -> device tensor, there
+        when the step runs."""
         if self.ex.device.type != "cuda":
             return {}
-        up = lambda a: torch.from_numpy(a).to(self.ex.device, non_blocking=True)  # noqa: E731
+        up = up or (lambda a: torch.from_numpy(a).to(self.ex.device, non_blocking=True))
         p = {"blocks": {tb: up(hops.talk_blocks(ntoks, tb)) for tb in set(self.talk_block.values()) if tb}}
         if self.rec_fill:
             h = hops.hgrn2_plan(ntoks, self.rec_fill[0], self.ex._n_cu, per_cu=self.rec_fill[1])

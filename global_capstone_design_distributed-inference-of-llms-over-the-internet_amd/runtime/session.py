@@ -186,6 +186,15 @@ class SessionManager:
                 self._dirty = True
         s.last_used = time.monotonic()
 
+    def take_table(self, out: np.ndarray) -> bool:
+        """The block table into ``out`` (int32, its size) if the device's is older; the caller brings it there."""
+        with self.lock:
+            if not self._dirty:
+                return False
+            out[...] = self.table.reshape(-1)
+            self._dirty = False
+            return True
+
     def sync_table(self, stream=None) -> torch.Tensor:
         if self._dirty:
             with self.lock:
