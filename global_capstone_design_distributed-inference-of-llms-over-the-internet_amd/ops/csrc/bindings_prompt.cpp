@@ -6,6 +6,7 @@
 
 extern "C" {
 int64_t mp_gemm_prompt_ws(int M, int N, int K);
+int mp_gemm_prompt_frags(int M, int N, int K);
 int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit, float* ws,
                  hipStream_t stream);
 int64_t mp_gemm_mid_ws(int M, int N, int K);
@@ -16,6 +17,7 @@ int mp_gemm_mid(const void* x, int64_t xs, const void* w, void* out, int M, int 
 namespace {
 
 int64_t gemm_prompt_ws(int64_t M, int64_t N, int64_t K) { return mp_gemm_prompt_ws((int)M, (int)N, (int)K); }
+int64_t gemm_prompt_frags(int64_t M, int64_t N, int64_t K) { return mp_gemm_prompt_frags((int)M, (int)N, (int)K); }
 int64_t gemm_mid_ws(int64_t M, int64_t N, int64_t K) { return mp_gemm_mid_ws((int)M, (int)N, (int)K); }
 
 // out[M, N'] = epilogue(x[M, K] w[N, K]^T); epi 8: x[M, K] w[K, N]
@@ -56,6 +58,7 @@ void gemm_mid(const at::Tensor& x, const at::Tensor& w, at::Tensor& out, const c
 
 TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def("gemm_prompt_ws(int M, int N, int K) -> int", &gemm_prompt_ws);
+  m.def("gemm_prompt_frags(int M, int N, int K) -> int", &gemm_prompt_frags);
   m.def("gemm_mid_ws(int M, int N, int K) -> int", &gemm_mid_ws);
   m.def("gemm_mid(Tensor x, Tensor w, Tensor(a!) out, Tensor(b!)? ws, int epi, float limit) -> ()");
   m.def("gemm_prompt(Tensor x, Tensor w, Tensor(a!) out, Tensor(b!)? ws, int epi, float limit) -> ()");

@@ -42,6 +42,7 @@ struct MidWork {
   typedef typename W::Source Source;
   static constexpr int STORES = W::put_stores(EPI == 1);
   static constexpr bool TURNS = true;
+  static constexpr int FRAGS = W::MW;
   const GemmMid& a;
   int m0, n0, part, first, count, begin;  // its first stage, how many, the one that it begins with (from its first)
   __device__ int stages(int) const { return count; }

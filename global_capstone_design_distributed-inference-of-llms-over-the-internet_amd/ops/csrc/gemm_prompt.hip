@@ -1,5 +1,5 @@
 // Products of prompt-sized steps: y[M, N'] = epilogue(x[M, K] w[N, K]^T), both operands row-major, or x[M, K] w[K, N] for
-// gradients; 256 x 256 tiles of wide_tile.h.  Epilogues: none; the gated forms over gate / up rows in blocks of 16 (silu(g) u, or with a limit
+// gradients; tiles of wide_tile.h, 256 weight rows wide and 128 to 256 rows high.  Epilogues: none; the gated forms over gate / up rows in blocks of 16 (silu(g) u, or with a limit
 // g sigmoid(1.702 g) (u + 1) on clamped inputs), N' = N / 2; max(y, 0)^2.  Everything up to the one store is 32 bits: next to
 // a library product and an activation kernel, the product's rows are neither written, read back nor rounded.
 //
@@ -8,111 +8,12 @@
 // equal parts, one per CU, fp32 parts go to a workspace and a second kernel adds a tile's parts in order and stores it.
 // Workgroups of the same part are neighbours, so that an XCD's CUs still walk the same columns of shared rows (ranges that
 // begin anywhere, as many as CUs, lost that: 176 left-over tiles of K 11008 took 310 us, made whole 216 us).
-#include "act_io.h"
-#include "gemm_act.h"
-#include "wide_tile.h"
+#include "gemm_prompt.h"
+#include <algorithm>
+
+extern "C" void mp_gemm_prompt_low(const mp::GemmPrompt* a, int epi, hipStream_t stream);
 
 namespace mp {
-
-constexpr int GW_CUS = WideTile::CUS, GW_BAND = 8;
-constexpr int64_t GW_SLAB = 256 * 256;  // fp32 elements of a part
-// stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
-// tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
-constexpr int GW_SPLIT_STAGES = 24;
-
-struct GemmPrompt {
-  const bf16_t* x;
-  int64_t xs;
-  const bf16_t* w;
-  bf16_t* out;
-  int M, N, K;
-  float limit;
-  int mt, nt;      // row and weight tiles
-  int full, rest, parts;  // tiles made whole; tiles cut into parts
-  float* slabs;           // [parts][rest][4 waves][8][8][64 lanes][4]
-};
-
-__device__ __forceinline__ void gw_tile(const GemmPrompt& a, int id, int& m0, int& n0) {
-  const int band = id / (GW_BAND * a.nt), h = min(GW_BAND, a.mt - GW_BAND * band), r = id - band * GW_BAND * a.nt;
-  m0 = (GW_BAND * band + r % h) * WideTile::BM;
-  n0 = r / h * WideTile::BN;
-}
-// A workgroup's tiles: every ``step``-th whole one of its XCD's run from ``first`` on, then a part of a left-over tile.
-template <int EPI>
-struct PromptWork {
-  static constexpr int STORES = WideTile::put_stores(EPI == 1);
-  static constexpr bool TURNS = false;
-  typedef WideTile W;
-  const GemmPrompt& a;
-  int first, step, whole;  // (whole: how many whole ones)
-  int g;                   // the part
-  __device__ int id(int k) const { return k < whole ? first + k * step : a.full + g % a.rest; }
-  __device__ int begin(int k) const { return k < whole ? 0 : g / a.rest * (a.K / 64) / a.parts; }
-  __device__ int stages(int k) const {
-    return k < whole ? a.K / 64 : (g / a.rest + 1) * (a.K / 64) / a.parts - g / a.rest * (a.K / 64) / a.parts;
-  }
-  __device__ void row_offsets(W::Source& s) const {
-#pragma unroll
-    for (int j = 0; j < W::PIECES; ++j) s.off[j] = (uint32_t)W::piece_row(j) * (uint32_t)(a.xs * 2) + W::piece_byte();
-  }
-  __device__ void weight_offsets(W::Source& s) const {
-#pragma unroll
-    for (int j = 0; j < W::PIECES; ++j)
-      s.off[j] = EPI == GW_COLUMNS ? ((uint32_t)W::column_row(j) * (uint32_t)a.N + W::column_first(j)) * 2
-                                   : (uint32_t)W::piece_row(j) * (uint32_t)(a.K * 2) + W::piece_byte();
-  }
-  __device__ void rows(int k, W::Source& s) const {  // (the launcher checks that the bytes fit 32 bits)
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    s.from(a.x + m0 * a.xs, ((uint32_t)(a.M - 1 - m0) * (uint32_t)a.xs + (uint32_t)a.K) * 2, begin(k) * 128, 128);
-  }
-  __device__ void weights(int k, W::Source& s) const {  // (columns past the last of a row are the next row's first: not stored)
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    if (EPI == GW_COLUMNS)
-      s.from(a.w + n0, ((uint32_t)a.N * (uint32_t)a.K - n0) * 2, begin(k) * (uint32_t)a.N * 128, (uint32_t)a.N * 128);
-    else
-      s.from(a.w + (int64_t)n0 * a.K, (uint32_t)(a.N - n0) * (uint32_t)a.K * 2, begin(k) * 128, 128);
-  }
-  __device__ bool half(int k) const {
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    return a.M - m0 <= W::BM / 2;
-  }
-  template <int M>
-  __device__ int store(int k, const f32x4 (&acc)[W::NW][W::MW]) const {
-    if (k == whole) {  // (nothing comes behind it)
-      float* s = a.slabs + (int64_t)g * GW_SLAB + (W::wave() * W::NW * W::MW * 64 + (threadIdx.x & 63)) * 4;
-#pragma unroll
-      for (int i = 0; i < W::NW; ++i)
-#pragma unroll
-        for (int j = 0; j < M; ++j) {
-          *reinterpret_cast<f32x4*>(s + (i * W::MW + j) * 256) = W::taken(acc[i][j]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      return 0;
-    }
-    int m0, n0;
-    gw_tile(a, id(k), m0, n0);
-    const int nw = n0 + 16 * W::NW * W::wn(), cols = EPI == 1 ? a.N / 2 : a.N;
-    auto go = [&](auto limit) {
-      return W::put<EPI == 1, M>(a.out + (int64_t)m0 * cols, cols, a.M - m0, EPI == 1 ? nw / 2 : nw, acc,
-                                 [&](const f32x4& v, const f32x4& u, float(&y)[4]) { gw_act<EPI, limit.value>(a.limit, v, u, y); });
-    };
-    return EPI == 1 && a.limit > 0.f ? go(W::Int<1>()) : go(W::Int<0>());
-  }
-};
-
-template <int EPI>
-__global__ __launch_bounds__(WideTile::THREADS, 1) void gemm_prompt_kernel(GemmPrompt a) {
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3, step = gridDim.x >> 3;
-  const int per = (a.full + 7) / 8, lo = xcd * per, run = min(per, a.full - lo);  // the XCD's run of whole tiles
-  const int all = a.rest * a.parts, each = (all + 7) / 8, g = xcd * each + at;
-  const int whole = at < run ? (run - at + step - 1) / step : 0, count = whole + (at < each && g < all);
-  if (count == 0) return;
-  WideTile::run<EPI == GW_COLUMNS ? WideTile::COLUMNS : WideTile::ROWS>(smem, count, PromptWork<EPI>{a, lo + at, step, whole, g});
-}
 
 // a left-over tile's parts added and stored; blockIdx.y: two of a wave's eight fragments of weights, two of the eight of rows
 template <int EPI>
@@ -122,7 +23,7 @@ __global__ __launch_bounds__(WideTile::THREADS) void gemm_prompt_close_kernel(Ge
   const int i0 = 2 * (blockIdx.y / (W::MW / 2)), j0 = 2 * (blockIdx.y % (W::MW / 2));
   int m0, n0;
   gw_tile(a, a.full + r, m0, n0);
-  const int frags = a.M - m0 <= W::BM / 2 ? W::MW / 2 : W::MW;
+  const int frags = a.frags == W::MW && a.M - m0 <= W::BM / 2 ? W::MW / 2 : a.frags;
   const int m = m0 + 16 * (frags * W::wm() + j0) + c16, o = n0 + 16 * (W::NW * W::wn() + i0);
   if (j0 >= frags || m - c16 >= a.M || o >= a.N) return;
   f32x4 acc[2][2];
@@ -139,7 +40,7 @@ __global__ __launch_bounds__(WideTile::THREADS) void gemm_prompt_close_kernel(Ge
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    if (m + 16 * j >= a.M) continue;
+    if (m + 16 * j >= a.M || j0 + j >= frags) continue;
 #pragma unroll
     for (int i = 0; i < 2; i += EPI == 1 ? 2 : 1)
       if (o + 16 * i < a.N) {
@@ -151,6 +52,9 @@ __global__ __launch_bounds__(WideTile::THREADS) void gemm_prompt_close_kernel(Ge
   }
 }
 
+// stages that a part has to save: 272 tiles of K 4096 (64 stages, 16 parts) 175 -> 138 us, of K 11008 434 -> 316 us; 112
+// tiles of K 4096 (2 parts, 32 saved) 81 -> 66 us
+constexpr int GW_SPLIT_STAGES = 24;
 // into how many parts the tiles past the last whole wave of CUs are cut (1: they are made whole like the others): where
 // the stages that a CU saves are worth the parts' way through memory
 static int gw_parts(int tiles, int ks) {
@@ -159,14 +63,48 @@ static int gw_parts(int tiles, int ks) {
   const int parts = GW_CUS / rest < ks / 4 ? GW_CUS / rest : ks / 4;  // (at least four stages a part)
   return ks - (ks + parts - 1) / parts >= GW_SPLIT_STAGES ? parts : 1;
 }
+static int gw_tiles(int M, int N, int frags) { return (M + 32 * frags - 1) / (32 * frags) * ((N + 255) / 256); }
+// How high the tiles are: what an estimate in us says.  A stage takes what is listed (a tile of 128 rows 61 % of one of 256), a
+// tile 6.4 more, cut ones 14.7 and their parts' way to memory and back.  Fitted to 48 shapes and row counts whose five heights were
+// timed (6 % off, rms).  At 42 others of 300 to 7000 rows the height that it picks is 0.3 % slower than the best, 256 rows 9 %:
+// 2100 x 4096 x 2048 47 (256 rows), 36 us (160); 4298 x 2048 x 12800 224, 181 (160); columns of 2500 x 4096 x 4096 94, 75 (160).
+static int gw_frags(int M, int N, int K) {
+  const float stage[5] = {0.77f, 0.88f, 1.00f, 1.17f, 1.27f};
+  int best = 8;
+  float least = 1e30f;
+  for (int f = 8; f >= 4; --f) {
+    const int tiles = gw_tiles(M, N, f), ks = K / 64, parts = gw_parts(tiles, ks), rest = parts > 1 ? tiles % GW_CUS : 0;
+    const int turns = (tiles - rest + GW_CUS - 1) / GW_CUS;
+    float t = turns * (ks * stage[f - 4] + 6.4f);
+    if (rest) t += (ks + parts - 1) / parts * stage[f - 4] + 14.7f + 15.8f * rest * parts * f / (8.f * GW_CUS);
+    if (t < least) least = t, best = f;
+  }
+  return best;
+}
+
+template <int EPI>
+static void launch_prompt(const GemmPrompt& a, hipStream_t stream) {
+  if (a.frags == WideTile::MW) launch_prompt<EPI, WideTile::MW>(a, stream);
+  else mp_gemm_prompt_low(&a, EPI, stream);
+  if (a.rest)
+    hipLaunchKernelGGL((gemm_prompt_close_kernel<EPI>), dim3(a.rest, WideTile::MW * WideTile::NW / 4), dim3(WideTile::THREADS), 0,
+                       stream, a);
+}
 
 }  // namespace mp
+
+// fragments of 16 rows of a wave, half a tile's, that a product's tiles have
+extern "C" int mp_gemm_prompt_frags(int M, int N, int K) { return mp::gw_frags(M, N, K); }
 
 // fp32 elements of the workspace
 extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K) {
   using namespace mp;
-  const int tiles = ((M + 255) / 256) * ((N + 255) / 256), parts = gw_parts(tiles, K / 64);
-  return parts > 1 ? parts * (tiles % GW_CUS) * GW_SLAB : 0;
+  int64_t most = 0;
+  for (int f : {gw_frags(M, N, K), WideTile::MW}) {  // (and no less than tiles of 256 rows take, which a caller may have kept)
+    const int tiles = gw_tiles(M, N, f), parts = gw_parts(tiles, K / 64);
+    if (parts > 1) most = std::max(most, parts * (tiles % GW_CUS) * GW_SLAB);
+  }
+  return most;
 }
 
 extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit,
@@ -176,27 +114,16 @@ extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* ou
   if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31))
     return -1;
   if (epi == 1 && N % 32) return -2;
-  GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, (M + 255) / 256, (N + 255) / 256, 0, 0, 1, ws};
-  const int tiles = a.mt * a.nt;
+  const int frags = gw_frags(M, N, K), tiles = gw_tiles(M, N, frags), nt = (N + 255) / 256;
+  GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, tiles / nt, nt, frags, 0, 0, 1, ws};
   a.parts = gw_parts(tiles, K / 64);
   a.rest = a.parts > 1 ? tiles % GW_CUS : 0;
   if (a.rest && ws == nullptr) return -3;
   a.full = tiles - a.rest;
-  // as many workgroups to an XCD as it has tiles or parts, up to its CUs
-  const int per = (a.full + 7) / 8, each = (a.rest * a.parts + 7) / 8, most = per > each ? per : each;
-  const dim3 grid(8 * (most < GW_CUS / 8 ? most : GW_CUS / 8));
-#define MP_GW(E_)                                                                                                          \
-  {                                                                                                                        \
-    (void)hipFuncSetAttribute((const void*)gemm_prompt_kernel<E_>, hipFuncAttributeMaxDynamicSharedMemorySize, WideTile::LDS); \
-    hipLaunchKernelGGL((gemm_prompt_kernel<E_>), grid, dim3(WideTile::THREADS), WideTile::LDS, stream, a);                                  \
-    if (a.rest) hipLaunchKernelGGL((gemm_prompt_close_kernel<E_>), dim3(a.rest, WideTile::MW * WideTile::NW / 4),          \
-                                   dim3(WideTile::THREADS), 0, stream, a);                                               \
-  }
-  if (epi == 0) MP_GW(0)
-  else if (epi == 1) MP_GW(1)
-  else if (epi == 4) MP_GW(4)
-  else if (epi == GW_COLUMNS) MP_GW(GW_COLUMNS)
+  if (epi == 0) launch_prompt<0>(a, stream);
+  else if (epi == 1) launch_prompt<1>(a, stream);
+  else if (epi == 4) launch_prompt<4>(a, stream);
+  else if (epi == GW_COLUMNS) launch_prompt<GW_COLUMNS>(a, stream);
   else return -4;
-#undef MP_GW
   return (int)hipGetLastError();
 }

@@ -765,6 +765,7 @@ struct MoeWork {
   static constexpr int STORES = WideTile::put_stores(GLU);
   static constexpr bool TURNS = false;
   typedef WideTile W;
+  static constexpr int FRAGS = W::MW;
   const MoeGemm& a;
   const MoeLists& l;
   float* ws;

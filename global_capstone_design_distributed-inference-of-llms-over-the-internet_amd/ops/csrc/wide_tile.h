@@ -59,8 +59,8 @@ struct TileLoop {
   static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
   static __device__ __forceinline__ int wm() { return wave() / WN; }
   static __device__ __forceinline__ int wn() { return wave() % WN; }
-  // row of the tile that piece j of this wave reads on this lane, and the byte of it in a stage
-  static __device__ __forceinline__ int piece_row(int j) { return 8 * (PIECES * wave() + j) + ((threadIdx.x & 63) >> 3); }
+  // row of the tile that piece j of this wave reads on this lane (of ``pieces`` a wave), and the byte of it in a stage
+  static __device__ __forceinline__ int piece_row(int j, int pieces = PIECES) { return 8 * (pieces * wave() + j) + ((threadIdx.x & 63) >> 3); }
   static __device__ __forceinline__ int piece_byte() { return 16 * ((threadIdx.x & 7) ^ ((threadIdx.x & 63) >> 3)); }
   // the same of packed weights: 16-row tile and byte
   static __device__ __forceinline__ int packed_tile(int j) { return PIECES / 2 * wave() + (j >> 1); }
@@ -95,17 +95,19 @@ struct TileLoop {
   //   void row_offsets(Source&), weight_offsets(Source&)   the lane's offsets, once
   //   void rows(k, Source&)          tile k's rows (may change the offsets)
   //   void weights(k, Source&)       its weight rows
-  //   bool half(k)                   has it at most half of its rows?
+  //   FRAGS                          the fragments of a wave's rows that all tiles have (of 8: 4 to 8)
+  //   bool half(k)                   where these are all: has tile k at most half of its rows?
   //   TURNS, int turn(k)             does a tile begin with another stage than its first: rows and weights are there, turn(k) stages
   //                                  stand ahead of it and come last
   //   int store<M>(k, acc)           acc[i][j]: weight rows 16 (8 wn + i) .. x rows 16 (M wm + j) .., j < M; lane: row lane % 16,
-  //                                  weight rows 4 (lane / 16) .. + 3.  At least how many stores were issued: 0 or
-  //                                  work.STORES of M = 8, half of them of M = 4.
+  //                                  weight rows 4 (lane / 16) .. + 3.  At least how many stores were issued: 0,
+  //                                  work.STORES of M = FRAGS, half of them of a half tile.
   // Ends with no load in flight.
   template <Weights FORM, class Work>
   static __device__ __forceinline__ void run(char* smem, int count, const Work& work) {
     const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
-    char* mine = smem + wave() * (PIECES * 1024);
+    constexpr int FRAGS = Work::FRAGS;  // loads of a wave and stage of rows, as many as fragments
+    static_assert(FRAGS == MW || (SLOTS == 5 && FRAGS >= 4 && FRAGS < MW));
     Source x, w;
     int lk = 0, left = work.stages(0);  // the tile that is being loaded, its stages left
     int turn = 0;  // how many of them stand ahead of the one it begins with
@@ -117,13 +119,13 @@ struct TileLoop {
     // A load in asm has its place in m0, an operand of it that the compiler sets, and waits five states for scalars that a vector
     // instruction wrote (the compiler may keep some in lanes).  In the loop two MFMAs stand in the place of waits (five waits in
     // front of each load cost 5 % at 1554 x 4096 x 28672).
-    auto place = [&](int j, int slot) { return (lptr_t)(mine + slot * SLOT + j * 1024); };
-    auto load = [&](const Source& s, int j, int slot) {
+    auto place = [&](int pieces, int j, int slot) { return (lptr_t)(smem + slot * SLOT + (wave() * pieces + j) * 1024); };
+    auto load = [&](const Source& s, int pieces, int j, int slot) {
       if constexpr (FORM == COLUMNS)
         asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                     :: "v"(s.off[j]), "s"(s.words), "s"(scalar<Work::TURNS>(s.at)), "{m0}"((uint32_t)(uintptr_t)place(j, slot)) : "memory");
+                     :: "v"(s.off[j]), "s"(s.words), "s"(scalar<Work::TURNS>(s.at)), "{m0}"((uint32_t)(uintptr_t)place(pieces, j, slot)) : "memory");
       else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, place(j, slot), 16, s.off[j], s.at, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(s.base, place(pieces, j, slot), 16, s.off[j], s.at, 0, 0);
     };
     // to the next stage (past the last tile its last stage is loaded again: nothing reads it, and the counts stay what they are)
     auto step = [&] {
@@ -166,16 +168,17 @@ struct TileLoop {
     };
     auto tile = [&](auto fragments, int k) __attribute__((always_inline)) {
       constexpr int M = decltype(fragments)::value;  // fragments of a wave's rows
-      constexpr int R = F == 4 ? 1 : M == MW ? 3 : 2;  // MFMAs to a read
+      constexpr int R = F == 4 ? 1 : M >= 6 ? 3 : 2;  // MFMAs to a read
       constexpr int TURN = 2 * NW;                     // MFMAs of two fragments of rows
       const int xr = (16 * M * wm() + c16) * 128;
       // MFMA q of a half stage: two fragments of rows at a time.  An operand that a vector instruction wrote (a cleared sum, a
       // copy at the loop's head) has to be two wait states old, which nobody counts for asm: a stage's first MFMA has them with it.
       auto weight_of = [](int q) {
+        if (q >= TURN * (M / 2)) return M / 2 % 2 ? NW - 1 - q % TURN : q % TURN;  // (the last fragment of an odd number)
         const int b = q % TURN / 4, s = q % 4, down = q / TURN & 1;
         return 2 * (down ? NW / 2 - 1 - b : b) + ((s == 1 || s == 2) != down);
       };
-      auto row_of = [](int q) { return 2 * (q / TURN) + ((q % 4 >= 2) != (q % TURN / 4 & 1)); };
+      auto row_of = [](int q) { return q >= TURN * (M / 2) ? M - 1 : 2 * (q / TURN) + ((q % 4 >= 2) != (q % TURN / 4 & 1)); };
       auto multiply1 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], bool first) {
         const int i = weight_of(q), j = row_of(q);
         if (first)
@@ -184,9 +187,9 @@ struct TileLoop {
           asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[i]), "v"(xf[j]));
       };
       // MFMAs q - 1 and q and a load in asm behind them (more wait states than a first MFMA needs)
-      auto multiply2 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], const Source& s, int l, int slot) {
+      auto multiply2 = [&](int q, const u16x8(&xf)[MW], const u16x8(&wf)[NW], const Source& s, int pieces, int l, int slot) {
         const int i = weight_of(q - 1), j = row_of(q - 1), i1 = weight_of(q), j1 = row_of(q);
-        const uint32_t to = (uint32_t)(uintptr_t)place(l, slot);
+        const uint32_t to = (uint32_t)(uintptr_t)place(pieces, l, slot);
         asm volatile("s_nop 2\n\tv_mfma_f32_16x16x32_bf16 %0, %2, %3, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %4, %5, %1\n\t"
                      "buffer_load_dwordx4 %6, %7, %8 offen lds"
                      : "+a"(acc[i][j]), "+a"(acc[i1][j1])
@@ -199,10 +202,12 @@ struct TileLoop {
 #pragma unroll
         for (int q = 0; q < NW * M; ++q) {
           constexpr int AT = B || M < 4 ? 1 : M - 3;
-          if (FORM == COLUMNS && q % M == AT) multiply2(q, B ? xb : xa, B ? wb : wa, B ? x : w, q / M, B ? fw : fx);
-          else if (FORM != COLUMNS || q % M != AT - 1) multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
+          constexpr int LOADS = B ? FRAGS : PIECES;  // (group q / M of M MFMAs has one)
+          const bool loads = q / M < LOADS;
+          if (FORM == COLUMNS && loads && q % M == AT) multiply2(q, B ? xb : xa, B ? wb : wa, B ? x : w, LOADS, q / M, B ? fw : fx);
+          else if (FORM != COLUMNS || !loads || q % M != AT - 1) multiply1(q, B ? xb : xa, B ? wb : wa, !B && q == 0);
           if (q % R == R - 1 && q / R < M + NW) take1(!B, q / R, xr, B ? xa : xb, B ? wa : wb, M);
-          if (FORM != COLUMNS && q % M == AT) load(B ? x : w, q / M, B ? fw : fx);
+          if (FORM != COLUMNS && loads && q % M == AT) load(B ? x : w, LOADS, q / M, B ? fw : fx);
           __builtin_amdgcn_sched_barrier(0);
         }
       };
@@ -242,18 +247,19 @@ struct TileLoop {
 #pragma unroll 1
     for (int s = 0; s < AHEAD; ++s) {  // w 0, x 0, w 1, x 1 ..
 #pragma unroll
-      for (int j = 0; j < PIECES; ++j) load(w, j, 2 * s);
+      for (int j = 0; j < PIECES; ++j) load(w, PIECES, j, 2 * s);
 #pragma unroll
-      for (int j = 0; j < PIECES; ++j) load(x, j, 2 * s + 1);
+      for (int j = 0; j < FRAGS; ++j) load(x, FRAGS, j, 2 * s + 1);
       step();
     }
     fx = SLOTS - 1;  // (the next weights)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 * AHEAD - 2) * PIECES) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * (PIECES + FRAGS)) : "memory");
     lds_wait_barrier();
 #pragma unroll
     for (int r = 0; r < NW; ++r) take1(0, r, 0, xa, wa, 0);
     for (int k = 0; k < count; ++k) {
-      if (work.half(k)) tile(Int<MW / 2>(), k);
+      if constexpr (FRAGS < MW) tile(Int<FRAGS>(), k);
+      else if (work.half(k)) tile(Int<MW / 2>(), k);
       else tile(Int<MW>(), k);
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");

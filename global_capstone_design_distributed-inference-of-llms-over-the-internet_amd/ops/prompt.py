@@ -3,12 +3,13 @@
 ``gemm``: y = epilogue(x w^T) over row-major bf16 operands, the gate / relu epilogues of a feed-forward in the same kernel;
 ``gemm_columns``: y = x w, a gradient's way back through a projection.
 The library's rate depends on its choice of solution, from 0.55 to 1.65 PFLOP/s over neighbouring row counts; this kernel's
-on how its 256 x 256 tiles fill 256 CUs, 1.2 to 1.6.  So the choice is measured, as it is for the decode GEMMs, for
+on how its tiles, 256 wide and 128 to 256 high, fill 256 CUs, 1.2 to 1.6.  So the choice is measured, as it is for the decode GEMMs, for
 the callers that ask (``tiles`` of ``ops.linear``: stages and fine-tuning): shapes in the committed table
 (``python -m src.ops.tune --prompt``: every projection of every preset, steps of 257 to 8192 rows, weights that no cache holds,
 as a model's do not stay there from one step to the next) run here at the row-tile
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
-both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close).
+both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close; the
+committed table of more than 256 rows also holds the 56 counts, of 926, that only tiles of 256 rows won, in two sweeps of theirs).
 
 Up to 384 rows there are tiles of 128 x 128 as well (csrc/gemm_mid.hip), by a table of theirs, timed against what runs without
 them: 66 rows of Mistral-7B, forward and backward, 1031 -> 832 us.  The library's call costs the host 25 us, theirs 7, so they stay
