@@ -13,7 +13,7 @@ int mp_train_attn_grad(const void* qkv, int64_t ld, int B, int T, int nh, int nk
 int mp_train_angles(const double* inv, float* out, int n, int64_t T, hipStream_t stream);
 int mp_train_rope(void* x, int64_t ld, const float* cs, int64_t rows, int T, int heads, int D, hipStream_t stream);
 int mp_train_norm(const void* x, const void* y, const void* w, void* sum, void* out, int64_t rows, int H, float eps, int grad,
-                  hipStream_t stream);
+                  const void* deep, int P, int T, int64_t apart, hipStream_t stream);
 int mp_train_glu_grad(void* gu, const void* da, int64_t rows, int F, hipStream_t stream);
 }
 
@@ -92,18 +92,26 @@ void train_rope(at::Tensor& x, const at::Tensor& cs, int64_t heads, int64_t D) {
 }
 
 // forward (res absent): out = norm of x + y, ``sum`` = x + y where y is given; backward (grad): out = sum + norm's gradient
+// deep [1 or sequences, P, H]: added to every sequence's first P rows
 void train_norm(const at::Tensor& x, const opt_tensor& y, const at::Tensor& w, const opt_tensor& sum, at::Tensor& out,
-                double eps, bool grad) {
+                double eps, bool grad, const opt_tensor& deep, int64_t T) {
   MP_CHECK(x.dim() == 2 && x.size(1) % 8 == 0 && x.size(1) >= 8 && x.size(1) <= 16384 && x.size(0) >= 1, "norm width");
-  MP_CHECK(sum.has_value() == y.has_value() && (!grad || y.has_value()), "norm operands");
+  MP_CHECK(sum.has_value() == (y.has_value() || deep.has_value()) && (!grad || (y.has_value() && !deep.has_value())), "norm operands");
   const int64_t R = x.size(0), H = x.size(1);
   const c10::hip::HIPGuard guard(x.device().index());
   MP_CHECK(w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.is_contiguous() && w.numel() == H &&
                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
            "norm weight");
+  const void* first = nullptr;
+  int64_t P = 0, apart = 0;
+  if (deep.has_value()) {
+    MP_CHECK(deep->dim() == 3 && T >= 1 && R % T == 0 && (deep->size(0) == 1 || deep->size(0) == R / T) && deep->size(1) <= T, "deep prompt");
+    P = deep->size(1), apart = deep->size(0) == 1 ? 0 : P * H;
+    first = bf16_rows(deep->view({deep->size(0) * P, deep->size(2)}), deep->size(0) * P, H, "deep");
+  }
   check_launch(mp_train_norm(bf16_rows(x, R, H, "x"), y.has_value() ? bf16_rows(*y, R, H, "y") : nullptr, w.data_ptr(),
                              sum.has_value() ? bf16_rows(*sum, R, H, "sum") : nullptr, bf16_rows(out, R, H, "out"), R, H,
-                             (float)eps, grad, cur_stream()),
+                             (float)eps, grad, first, (int)P, (int)T, apart, cur_stream()),
                "train_norm");
 }
 
@@ -127,7 +135,8 @@ TORCH_LIBRARY_FRAGMENT(mpamd, m) {
   m.def("train_angles(Tensor inv, Tensor(a!) out) -> ()");
   m.def("train_rope(Tensor(a!) x, Tensor cs, int heads, int D) -> ()");
   m.def(
-      "train_norm(Tensor x, Tensor? y, Tensor w, Tensor(a!)? sum, Tensor(b!) out, float eps, bool grad=False) -> ()");
+      "train_norm(Tensor x, Tensor? y, Tensor w, Tensor(a!)? sum, Tensor(b!) out, float eps, bool grad=False, Tensor? deep=None, "
+      "int T=0) -> ()");
   m.def("train_glu_grad(Tensor(a!) gu, Tensor da) -> ()");
 }
 

@@ -31,11 +31,13 @@ def angles(inv: torch.Tensor, T: int) -> torch.Tensor:
     return out
 
 
-def norm(x, w, eps, add=None):
-    """(x + add, its norm times w); without ``add`` the first is ``x`` itself."""
+def norm(x, w, eps, add=None, deep=None, T: int = 0):
+    """(x + add, its norm times w); without ``add`` and ``deep`` the first is ``x`` itself.  ``deep`` [1 or B, P, H]: added as well, to
+    the first P of every ``T`` rows, after that sum was rounded."""
     out = torch.empty_like(x)
-    total = x if add is None else torch.empty_like(x)
-    torch.ops.mpamd.train_norm(x, add, w, None if add is None else total, out, eps)
+    plain = add is None and deep is None
+    total = x if plain else torch.empty_like(x)
+    torch.ops.mpamd.train_norm(x, add, w, None if plain else total, out, eps, False, deep, T)
     return total, out
 
 

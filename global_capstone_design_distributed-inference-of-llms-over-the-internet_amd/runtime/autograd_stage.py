@@ -150,10 +150,13 @@ class AutogradStage:
         nh, nkv, D, eps = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, cfg.rms_norm_eps
         kept, y = [], None
         for i, lay in enumerate(self.w.layers):
+            deep = None
             if prompts is not None and prompts.shape[2]:
-                x, y = (x.clone() if y is None else x + y), None
-                x.view(B, T, -1)[:, :prompts.shape[2]] += prompts[i]
-            x, h = train.norm(x, lay.input_norm, eps, y)
+                deep = prompts[i]
+                if deep.shape[0] not in (1, B) or deep.shape[2] != cfg.hidden_size:  # (what broadcasts, or raises)
+                    deep = deep.expand(B, deep.shape[1], cfg.hidden_size)
+                deep = _rows(deep).view(deep.shape)
+            x, h = train.norm(x, lay.input_norm, eps, y, deep, T)
             qkv = train.rope_(ops.linear(h, lay.qkv, tiles=True), table, nh + nkv, D)
             a, a32, lse = train.attention(qkv, B, nh, nkv, D, keep)
             x2, h = train.norm(x, lay.post_norm, eps, ops.linear(a, lay.o, tiles=True))
