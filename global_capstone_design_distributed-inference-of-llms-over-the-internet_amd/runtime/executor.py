@@ -142,13 +142,14 @@ class _PlanInput:
     """Staging of what a step of several tokens per session takes in (its plan and a changed block table): one pinned buffer, one
     device buffer and one launch a step.  A ring, so that the host runs ahead; an event costs the stream 6 us, so each half
     of the turns has one, and a half is written again when the steps that read it are done.  A buffer that grew is a new one:
-    the launches tell the allocator of pinned memory which work reads the old one."""
+    the launches tell the allocator of pinned memory which work reads the old one.  It holds the largest step that there was: only
+    what did not fit for its size makes it grow."""
 
     TURNS = 4
 
     def __init__(self, device, size: int):
         self.device, self.size = device, 0
-        self.want = 0  # bytes that did not fit a step's buffer, on top of it
+        self.want = 0  # bytes of the largest step that did not fit
         self._grow(size)
 
     def _grow(self, size: int) -> None:
@@ -159,12 +160,12 @@ class _PlanInput:
 
     def open(self, size: int) -> None:
         """``size`` bytes of arrays, up to 15 more for each, and of the table."""
-        if size + self.want > self.size:
-            self._grow(size + self.want)
+        if max(size, self.want) > self.size:
+            self._grow(max(size, self.want))
         half = self.TURNS // 2
         if self._k % half == 0 and self._ev[self._k // half] is not None:
             self._ev[self._k // half].synchronize()
-        self._at = 0
+        self._at = self._over = 0  # bytes of the step that are here, that did not fit
         self._dev = torch.empty(self.size, dtype=torch.uint8, device=self.device)
 
     def room(self, shape, dtype):
@@ -172,7 +173,7 @@ class _PlanInput:
         n = int(np.prod(shape)) * np.dtype(dtype).itemsize
         a = self._at
         if a + n > self.size:
-            self.want += a + n - self.size
+            self._over += -(-n // 16) * 16
             return None
         self._at = a + -(-n // 16) * 16
         return (self._np[self._k, a:a + n].view(dtype).reshape(shape),
@@ -187,15 +188,16 @@ class _PlanInput:
 
     def close(self, sessions: SessionManager) -> None:
         k, n = self._k, min(self._at, self.size)
-        t = sessions.table.nbytes
-        here = t % 8 == 0 and n + t <= self.size
-        if not here:
-            self.want += t
-        table = here and sessions.take_table(self._np[k, n:n + t].view(np.int32))
-        if not here:
+        t = sessions.table_words.nbytes
+        here = n + t <= self.size
+        table = here and sessions.take_table(self._np[k, n:n + t].view(np.int32)[:sessions.table.size])
+        if not here and sessions.stale:
+            self._over += t
             sessions.sync_table()
+        if self._over:
+            self.want = max(self.want, n + self._over)
         if n or table:
-            torch.ops.mpamd.plan_input(self._host[k, :n + t if table else n], self._dev[:n], sessions.table_dev if table else None)
+            torch.ops.mpamd.plan_input(self._host[k, :n + t if table else n], self._dev[:n], sessions.table_words if table else None)
         half = self.TURNS // 2
         if k % half == half - 1:
             self._ev[k // half] = torch.cuda.Event()

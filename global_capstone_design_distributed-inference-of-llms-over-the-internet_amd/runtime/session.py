@@ -44,7 +44,9 @@ class SessionManager:
         self.max_pages = pages_needed(max_seq_len, cache.page_size)
         self.ttl = ttl_seconds
         self.table = np.full((max_sessions, self.max_pages), -1, dtype=np.int32)
-        self.table_dev = torch.from_numpy(self.table.copy()).to(cache.device)
+        n = self.table.size  # (on the device in whole words of 8 bytes, which one launch writes with a step's plan)
+        self.table_words = torch.full((n + n % 2,), -1, dtype=torch.int32, device=cache.device)
+        self.table_dev = self.table_words[:n].view(self.table.shape)
         self._dirty = False
         # double-buffered pinned staging: the H2D copy of a changed table is asynchronous and
         # stream-ordered before the step's kernels (a pageable copy_ would block the host until
@@ -194,6 +196,11 @@ class SessionManager:
             out[...] = self.table.reshape(-1)
             self._dirty = False
             return True
+
+    @property
+    def stale(self) -> bool:
+        """Is the device's block table older?"""
+        return self._dirty
 
     def sync_table(self, stream=None) -> torch.Tensor:
         if self._dirty:

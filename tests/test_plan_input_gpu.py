@@ -76,3 +76,21 @@ def test_plan_on_the_device():
         assert np.array_equal(p.fablocks.cpu().numpy(), fb) and p.fa_waves == waves
         assert (p.qblocks is None) == (T > ops.wide_rows())
         ex.commit(p)
+
+
+def test_tables_of_an_odd_number_of_words(monkeypatch):
+    """5 sessions of 5 pages: the table arrives with the plan, in a buffer that stays as it is."""
+    ops.require_native()
+    cfg = resolve_model("small-llama")
+    w = random_stage_weights(cfg, 0, 1, has_embed=True, has_head=False, device="cuda:0", seed=3)
+    ex = executor.StageExecutor(cfg, w, "cuda:0", max_sessions=5, max_seq_len=320, kv_cache_bytes=16 << 20, warmup=False)
+    assert ex.sessions.table.size == 25
+    copies, sync = [], ex.sessions.sync_table
+    monkeypatch.setattr(ex.sessions, "sync_table", lambda: copies.append(1) or sync())
+    size, at = ex._input.size, ex._input._host.data_ptr()
+    for i in range(200):
+        sid = f"s{i % 5}"
+        ex.forward([(sid, 2 + i)], torch.zeros(2 + i, dtype=torch.long, device="cuda"), reset=[True])
+        if i % 40 == 39:
+            assert np.array_equal(ex.sessions.table_dev.cpu().numpy(), ex.sessions.table)
+    assert ex._input.size == size and ex._input._host.data_ptr() == at and not copies
