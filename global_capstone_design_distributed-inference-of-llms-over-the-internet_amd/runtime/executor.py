@@ -190,14 +190,17 @@ class _PlanInput:
         k, n = self._k, min(self._at, self.size)
         t = sessions.table_words.nbytes
         here = n + t <= self.size
-        table = here and sessions.take_table(self._np[k, n:n + t].view(np.int32)[:sessions.table.size])
-        if not here and sessions.stale:
-            self._over += t
-            sessions.sync_table()
-        if self._over:
-            self.want = max(self.want, n + self._over)
-        if n or table:
-            torch.ops.mpamd.plan_input(self._host[k, :n + t if table else n], self._dev[:n], sessions.table_words if table else None)
+        with sessions.lock:  # (no change of the table between its copy and the mark that it was sent)
+            table = here and sessions.take_table(self._np[k, n:n + t].view(np.int32)[:sessions.table.size])
+            if not here and sessions.stale:
+                self._over += t
+                sessions.sync_table()
+            if self._over:
+                self.want = max(self.want, n + self._over)
+            if n or table:
+                torch.ops.mpamd.plan_input(self._host[k, :n + t if table else n], self._dev[:n], sessions.table_words if table else None)
+            if table:
+                sessions.table_sent()
         half = self.TURNS // 2
         if k % half == half - 1:
             self._ev[k // half] = torch.cuda.Event()

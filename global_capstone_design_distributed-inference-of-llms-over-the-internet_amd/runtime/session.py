@@ -189,13 +189,15 @@ class SessionManager:
         s.last_used = time.monotonic()
 
     def take_table(self, out: np.ndarray) -> bool:
-        """The block table into ``out`` (int32, its size) if the device's is older; the caller brings it there."""
+        """The block table into ``out`` (int32, its size) if the device's is older.  The caller brings it there and says so
+        (``table_sent``), under ``lock``: until then a later step still sends it."""
         with self.lock:
-            if not self._dirty:
-                return False
-            out[...] = self.table.reshape(-1)
-            self._dirty = False
-            return True
+            if self._dirty:
+                out[...] = self.table.reshape(-1)
+            return self._dirty
+
+    def table_sent(self) -> None:
+        self._dirty = False
 
     @property
     def stale(self) -> bool:

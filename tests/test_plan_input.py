@@ -70,3 +70,23 @@ def test_a_buffer_grows_to_the_largest_step(launches):
         assert all(np.array_equal(g.numpy(), a) for g, a in zip(got, arrays))
         sizes.append(inp.size)
     assert sizes[0] == 4096 and sizes[-1] == sizes[8] <= 12288
+
+
+def test_a_table_that_was_not_sent_is_sent_later(launches, monkeypatch):
+    """A launch that raises leaves the device's table old: the next step brings it."""
+    sessions = _sessions(5, 6)
+    inp = executor._PlanInput(torch.device("cpu"), 4096)
+    real = executor.torch.ops.mpamd.plan_input
+
+    def fails(*a):
+        raise RuntimeError("no launch")
+
+    monkeypatch.setattr(executor.torch.ops.mpamd, "plan_input", fails)
+    with pytest.raises(RuntimeError, match="no launch"):
+        _step(inp, sessions, "a", 9)
+    assert not np.array_equal(sessions.table_dev.numpy(), sessions.table)
+    monkeypatch.setattr(executor.torch.ops.mpamd, "plan_input", real)
+    inp.open(4096)
+    inp.put(np.arange(3, dtype=np.int64))
+    inp.close(sessions)
+    assert np.array_equal(sessions.table_dev.numpy(), sessions.table) and not sessions._dirty
