@@ -81,6 +81,9 @@ def test_linear_takes_them(monkeypatch):
     del calls[:]
     ops.linear(x[:90], w, tiles=True)
     assert not calls  # (another range of rows)
+    ss = x.float().pow(2).sum(1)  # (rows of a fused norm: the decode kernels alone scale them)
+    kw = dict(wp=ops.pack_weight(w), ss_in=ss, eps=1e-5)
+    assert torch.equal(ops.linear(x, w, tiles=True, **kw), ops.linear(x, w, **kw)) and not calls
 
 
 def test_which_products(monkeypatch):
