@@ -81,7 +81,8 @@ def test_linear_takes_them(monkeypatch):
     del calls[:]
     ops.linear(x[:90], w, tiles=True)
     assert not calls  # (another range of rows)
-    ss = x.float().pow(2).sum(1)  # (rows of a fused norm: the decode kernels alone scale them)
+    ss = ops.norm_stats_buffer("cuda")[0]  # (rows of a fused norm: the decode kernels alone scale them)
+    ss[0, :100] = (x.double().pow(2).sum(1) * 2 ** 20).long()
     kw = dict(wp=ops.pack_weight(w), ss_in=ss, eps=1e-5)
     assert torch.equal(ops.linear(x, w, tiles=True, **kw), ops.linear(x, w, **kw)) and not calls
 
