@@ -12,9 +12,9 @@ both of two sweeps (one sweep differs from the next in about a third of the shap
 committed table of more than 256 rows also holds the 56 counts, of 926, that only tiles of 256 rows won, in two sweeps of theirs).
 
 Up to 384 rows there are tiles of 128 x 128 as well (csrc/gemm_mid.hip), by a table of theirs, timed against what runs without
-them: 66 rows of Mistral-7B, forward and backward, 1031 -> 832 us.  The library's call costs the host 25 us, theirs 7, so they stay
-where they are up to 3 % slower on the GPU; weights of less than 4M elements always go there: a prompt of 153 tokens of a
-512-wide model, 503 -> 381 us for two blocks.  (Ranges that were timed at 8, 16 and 32 rows hold at 1 to 7 too: 1.0 to 1.7 times as
+them: 66 rows of Mistral-7B, forward and backward, 1031 -> 832 us.  The library's call costs the host 21 us, theirs 13, so they stay
+where they are up to 3 % slower on the GPU.  Weights of less than 4M elements go there by a rule (``mid``): a prompt of 153 tokens
+of a 512-wide model, 503 -> 381 us for two blocks.  (Ranges that were timed at 8, 16 and 32 rows hold at 1 to 7 too: 1.0 to 1.7 times as
 fast as the library's at 33 of 36 shapes, 0.93 at the worst.)
 A third table holds those few of 1 to 256 rows that are best on the large tiles.
 
@@ -39,7 +39,7 @@ EPILOGUES = (0, 1, 4, COLUMNS)
 TILE, MAX_ROWS = 256, 8192
 FEW = (32, 64, 128, TILE)  # (a tile of up to 128 rows takes half the products; the library's times jump at all four)
 MID = (32, 64, 96, 128, 192, 256, 384)
-SMALL = 1 << 22  # elements of a weight below which a product is bound by its call
+SMALL = 1 << 22  # elements of a weight that no table holds
 Shape = Tuple[int, int, int]  # N, K, epilogue
 
 _LOCK = threading.Lock()
@@ -95,7 +95,13 @@ def mid(M: int, N: int, K: int, epilogue: int) -> bool:
     if not shape_ok(M, N, K, epilogue) or M > MAX_ROWS:
         return False
     if N * K < SMALL:
-        return os.environ.get("MPAMD_KERNEL_TABLE") != "0"
+        # Up to 8192 stages of all tiles they take 6 % less than the library's on average, and where they take more (1280 x 1280
+        # of 300 rows 13.7, 7.5 us) no more than its call costs the host beyond theirs; past that only where K is small, or the library's
+        # pass over what it wrote is saved: 8192 x 768 x 4096 65.7, 50.5 us, but 4096 x 16384 x 128 40.4, 39.8 and 8192 x 4064 x 1024
+        # gated 69.4, 113.  That pass moves both lines to twice as much (4096 x 2048 x 1984 gated 34.6, 39.7, of 5000 rows 49.1, 45.7).
+        more = 2 if epilogue in (1, 4) else 1
+        stages = -(-M // 128) * -(-N // 128) * (K // 64)
+        return (K <= 512 * more or stages <= 8192 * more) and os.environ.get("MPAMD_KERNEL_TABLE") != "0"
     return M <= MID[-1] and next(i for i, n in enumerate(MID, 1) if M <= n) in table("mid").get((N, K, epilogue), ())
 
 

@@ -93,6 +93,12 @@ def test_which_products(monkeypatch):
         assert prompt.mid(M, 4096, 4096, 0) == here
     assert not prompt.mid(20, 4096, 4096, 1) and not prompt.mid(20, 4096, 8192, 0)  # (not timed)
     assert prompt.mid(8000, 512, 1024, 0) and not prompt.mid(8193, 512, 1024, 0) and not prompt.mid(100, 512, 1024 + 32, 0)
+    # weights that no table holds: up to 8192 stages of tiles, or K 512; twice as much where the library needs a second pass
+    for M, N, K, epi, here in ((2048, 1008, 4096, 0, True), (2049, 1008, 4096, 0, False), (8192, 768, 4096, 0, False),
+                               (4096, 992, 4096, 1, True), (4097, 992, 4096, 1, False), (4096, 1024, 4032, 4, True), (8192, 1024, 4032, 4, False),
+                               (8192, 4096, 512, 0, True), (8192, 4096, 512, 8, True), (8192, 4096, 576, 0, False), (8192, 4064, 1024, 1, True),
+                               (8192, 2032, 1088, 1, False), (8192, 4096, 768, 8, False), (300, 4080, 1024, 0, True)):
+        assert prompt.mid(M, N, K, epi) == here, (M, N, K, epi)
     x, w = torch.zeros(20, 512, dtype=torch.bfloat16), torch.zeros(512, 512, dtype=torch.bfloat16)
     assert not prompt.ok(x, w, 0) and torch.equal(prompt.gemm_columns(x, w), x @ w)  # the CPU
     monkeypatch.setenv("MPAMD_KERNEL_TABLE", "0")
