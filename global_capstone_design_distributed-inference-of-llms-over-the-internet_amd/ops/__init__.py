@@ -1032,7 +1032,7 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
     N = w.shape[0] if w is not None else 16 * wp.shape[0]
     policy = policy or _GEMM_POLICY
     if tiles and a_rows is None and not out_packed and policy == "auto" and w is not None and ss_in is None and \
-            prompt.mid(M, N, K, epilogue) and prompt.reads(x, w):  # (faster than packing the rows for the decode kernels, too)
+            (wp is None or prompt.ahead(M, N, K)) and prompt.mid(M, N, K, epilogue) and prompt.reads(x, w):
         return prompt.gemm(x, w, out, epilogue, glu_limit, mid=True)
     ok = wp is not None and native_gemm_ok(M, N, K, epilogue, out_packed) and (
         a_rows is not None or (x.stride(0) % 8 == 0 and x.stride(1) == 1))

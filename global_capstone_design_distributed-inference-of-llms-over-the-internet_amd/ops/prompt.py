@@ -105,6 +105,14 @@ def mid(M: int, N: int, K: int, epilogue: int) -> bool:
     return M <= MID[-1] and next(i for i, n in enumerate(MID, 1) if M <= n) in table("mid").get((N, K, epilogue), ())
 
 
+def ahead(M: int, N: int, K: int) -> bool:
+    """Are the 128 x 128 tiles ahead of packing M rows for the decode kernels, where the weights are there packed as well?  Those
+    stream large weights of few rows faster (us of the tiles, of packing and the decode kernel): 8 rows of 4096 x 11008 21.4, 19.3, of
+    6144 x 4096 13.7, 15.2; 16 rows of 8192 x 8192 28.3, 25.3, of 28672 x 4096 gated 41.6, 42.0; 17 rows of 4096 x 11008 22.0, 25.5, of
+    8192 x 8192 28.4, 27.2; 24 rows of 57344 x 8192 gated 163, 146, 32 rows 164, 161, 48 rows 165, 201."""
+    return N * K <= 1 << 25 or M > 32 or (M > 16 and N * K <= 1 << 28)
+
+
 def reads(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Are these operands that the kernel reads (types, strides, alignments), in a call that is not differentiated?"""
     if x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:

@@ -87,6 +87,29 @@ def test_linear_takes_them(monkeypatch):
     assert torch.equal(ops.linear(x, w, tiles=True, **kw), ops.linear(x, w, **kw)) and not calls
 
 
+def test_few_rows_of_large_packed_weights():
+    """Where a step's weights are there packed as well: which rows leave the decode kernels."""
+    for N, K, first in ((512, 512, 1), (6144, 4096, 1), (4096, 11008, 17), (28672, 4096, 17), (8192, 28672, 17), (57344, 8192, 33)):
+        assert [prompt.ahead(M, N, K) for M in (first - 1, first)] == [first == 1, True], (N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,here", [(16, 0), (17, 1)])
+def test_large_packed_weights(M, here, monkeypatch):
+    ops.require_native()
+    monkeypatch.setitem(prompt._STATE, "mid", {(4096, 11008, 0): frozenset({1})})
+    x, w = torch.randn(M, 11008, device="cuda").to(torch.bfloat16), torch.randn(4096, 11008, device="cuda").to(torch.bfloat16)
+    calls, run = [], prompt._run_mid
+    monkeypatch.setattr(prompt, "_run_mid", lambda *a: calls.append(1) or run(*a))
+    want = x.double() @ w.double().t()
+    wp = ops.pack_weight(w)
+    for kw, n in (({"wp": wp}, here), ({}, 1)):
+        del calls[:]
+        y = ops.linear(x, w, tiles=True, **kw)
+        assert float((y.double() - want).norm() / want.norm()) < BF16 and len(calls) == n
+    assert here or torch.equal(ops.linear(x, w, tiles=True, wp=wp), ops.linear(x, w, wp=wp))
+
+
 def test_which_products(monkeypatch):
     monkeypatch.setitem(prompt._STATE, "mid", {(4096, 4096, 0): frozenset({1, 5})})
     for M, here in ((1, True), (32, True), (33, False), (128, False), (129, True), (192, True), (193, False), (385, False)):
