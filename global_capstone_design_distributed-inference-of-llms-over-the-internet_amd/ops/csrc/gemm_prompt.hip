@@ -97,10 +97,10 @@ static void launch_prompt(const GemmPrompt& a, hipStream_t stream) {
 extern "C" int mp_gemm_prompt_frags(int M, int N, int K) { return mp::gw_frags(M, N, K); }
 
 // fp32 elements of the workspace
-extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K) {
+extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K, int frags) {
   using namespace mp;
   int64_t most = 0;
-  for (int f : {gw_frags(M, N, K), WideTile::MW}) {  // (and no less than tiles of 256 rows take, which a caller may have kept)
+  for (int f : {frags ? frags : gw_frags(M, N, K), WideTile::MW}) {  // (and no less than tiles of 256 rows take, which a caller may have kept)
     const int tiles = gw_tiles(M, N, f), parts = gw_parts(tiles, K / 64);
     if (parts > 1) most = std::max(most, parts * (tiles % GW_CUS) * GW_SLAB);
   }
@@ -108,13 +108,15 @@ extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K) {
 }
 
 extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit,
-                            float* ws, hipStream_t stream) {
+                            float* ws, int frags, hipStream_t stream) {
   (void)hipGetLastError();
   using namespace mp;
   if (M < 1 || N < 16 || N % 16 || K < 64 || K % 64 || xs % 8 || (int64_t)M * xs >= (1ll << 31) || (int64_t)N * K >= (1ll << 31))
     return -1;
   if (epi == 1 && N % 32) return -2;
-  const int frags = gw_frags(M, N, K), tiles = gw_tiles(M, N, frags), nt = (N + 255) / 256;
+  if (frags == 0) frags = gw_frags(M, N, K);
+  if (frags < 4 || frags > WideTile::MW) return -5;
+  const int tiles = gw_tiles(M, N, frags), nt = (N + 255) / 256;
   GemmPrompt a{(const bf16_t*)x, xs, (const bf16_t*)w, (bf16_t*)out, M, N, K, limit, tiles / nt, nt, frags, 0, 0, 1, ws};
   a.parts = gw_parts(tiles, K / 64);
   a.rest = a.parts > 1 ? tiles % GW_CUS : 0;

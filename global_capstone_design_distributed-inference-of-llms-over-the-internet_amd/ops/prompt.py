@@ -133,10 +133,11 @@ def ok(x: torch.Tensor, w: Optional[torch.Tensor], epilogue: int) -> bool:
     return (mid(*shape) or chosen(*shape) or few(*shape)) and reads(x, w)
 
 
-def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0):
-    need = torch.ops.mpamd.gemm_prompt_ws(x.shape[0], N, x.shape[1])
+def _run(x, w, y, N: int, epilogue: int, limit: float = 0.0, frags: int = 0):
+    """``frags``: tiles of 32 times as many rows (4 to 8; 0: what the estimate says)."""
+    need = torch.ops.mpamd.gemm_prompt_ws(x.shape[0], N, x.shape[1], frags)
     ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
-    torch.ops.mpamd.gemm_prompt(x, w, y, ws, epilogue, limit)
+    torch.ops.mpamd.gemm_prompt(x, w, y, ws, epilogue, limit, frags)
     return y
 
 

@@ -22,10 +22,18 @@ def _want(z, epi, limit):
     return g * torch.sigmoid(1.702 * g) * (u + 1)
 
 
+@pytest.fixture(params=[0, 8], ids=["estimate", "256rows"])
+def height(request, monkeypatch):
+    """Tiles as high as the estimate says, and of 256 rows, which the sizes below are made for."""
+    run = prompt._run
+    monkeypatch.setattr(prompt, "_run", lambda *a: run(*a, frags=request.param))
+    return request.param
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 64, 65, 255, 256, 257, 640])
 @pytest.mark.parametrize("N,K", [(16, 64), (32, 128), (256, 192), (288, 320), (544, 2048), (4096, 1664)])
-def test_products(M, N, K):
+def test_products(M, N, K, height):
     """One sum of K exact products in 32 bits (in parts or whole), rounded to bf16 once."""
     ops.require_native()
     g = torch.Generator().manual_seed(M + N + K)
@@ -45,9 +53,10 @@ def test_products(M, N, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(4100, 4096, 2048), (300, 4096, 11008), (1030, 4096, 10240), (2049, 2304, 4096)])
-def test_left_over_tiles_in_parts(M, N, K):
+@pytest.mark.parametrize("height", [8], indirect=True)
+def test_left_over_tiles_in_parts(M, N, K, height):
     ops.require_native()
-    assert torch.ops.mpamd.gemm_prompt_ws(M, N, K) > 0
+    assert torch.ops.mpamd.gemm_prompt_ws(M, N, K, height) > 0
     g = torch.Generator(device="cuda").manual_seed(K)
     x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
     w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
@@ -66,7 +75,7 @@ MANY += [(1600, 14336, 192), (1601, 14336, 64), (1664, 14336, 128), (1665, 14336
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", MANY)
-def test_several_tiles_to_a_workgroup(M, N, K):
+def test_several_tiles_to_a_workgroup(M, N, K, height):
     ops.require_native()
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
@@ -86,7 +95,7 @@ def test_several_tiles_to_a_workgroup(M, N, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 40, 130])
-def test_output_rows_of_many_columns(M):
+def test_output_rows_of_many_columns(M, height):
     """A tile's 256 rows of the output are more than 2^31 bytes; K exact products in 32 bits, rounded once."""
     ops.require_native()
     N, K = (1 << 22) + 48, 64
@@ -102,7 +111,7 @@ def test_output_rows_of_many_columns(M):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 100, 129, 250, 300])
 @pytest.mark.parametrize("N", [32, 144, 288])
-def test_nothing_behind_the_output(M, N):
+def test_nothing_behind_the_output(M, N, height):
     """What lies behind the output, up to where a whole tile would end, stays as it was: rows and columns that are not there."""
     ops.require_native()
     K = 128
@@ -141,7 +150,7 @@ def test_gates_far_below_zero():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (65, 272, 192), (257, 240, 64), (640, 528, 1664), (300, 4096, 11008), (2050, 2304, 4096)])
-def test_products_with_columns(M, N, K):
+def test_products_with_columns(M, N, K, height):
     """x w, as a gradient goes back through a projection: ends of tiles and of a wave's columns, tiles in parts."""
     ops.require_native()
     g = torch.Generator(device="cuda").manual_seed(M + N + K)

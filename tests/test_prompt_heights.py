@@ -21,7 +21,6 @@ CASES = [(4, 130, 2496, 64), (4, 2049, 2080, 2048), (4, 1101, 13632, 192), (4, 9
 def test_heights(frags, M, N, K):
     """One sum of K exact products in 32 bits (in parts or whole), rounded to bf16 once; rows behind the output stay."""
     ops.require_native()
-    assert torch.ops.mpamd.gemm_prompt_frags(M, N, K) == frags
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
     w = torch.randn(N, K, device="cuda", generator=g).div(K ** 0.5).to(torch.bfloat16)
@@ -32,11 +31,24 @@ def test_heights(frags, M, N, K):
         cols = N // 2 if epi == 1 else N
         room = torch.full((M + 32, cols), -3.0, dtype=torch.bfloat16, device="cuda")
         v = w.t().contiguous() if epi == prompt.COLUMNS else w
-        prompt._run(x, v, room[:M], N, epi)
+        prompt._run(x, v, room[:M], N, epi, frags=frags)
         want = z if epi == prompt.COLUMNS else _want(z, epi, 0.0)
         assert float((room[:M].double() - want).norm() / want.norm()) < BF16
         assert bool((room[M:] == -3.0).all())
-        assert torch.equal(room[:M], prompt._run(x, v, torch.empty_like(room[:M]), N, epi))
+        assert torch.equal(room[:M], prompt._run(x, v, torch.empty_like(room[:M]), N, epi, frags=frags))
+
+
+@pytest.mark.gpu
+def test_which_height():
+    """Heights that a caller asks for, the estimate's without one, no others."""
+    ops.require_native()
+    x, w = torch.randn(300, 64, device="cuda").to(torch.bfloat16), torch.randn(512, 64, device="cuda").to(torch.bfloat16)
+    y = torch.empty(300, 512, dtype=torch.bfloat16, device="cuda")
+    own = torch.ops.mpamd.gemm_prompt_frags(300, 512, 64)
+    assert 4 <= own <= 8 and torch.ops.mpamd.gemm_prompt_ws(300, 512, 64) == torch.ops.mpamd.gemm_prompt_ws(300, 512, 64, own)
+    for frags in (-1, 1, 3, 9):
+        with pytest.raises(RuntimeError, match="fragments"):
+            prompt._run(x, w, y, 512, 0, frags=frags)
 
 
 @pytest.fixture(scope="module")
