@@ -9,7 +9,6 @@
 // Workgroups of the same part are neighbours, so that an XCD's CUs still walk the same columns of shared rows (ranges that
 // begin anywhere, as many as CUs, lost that: 176 left-over tiles of K 11008 took 310 us, made whole 216 us).
 #include "gemm_prompt.h"
-#include <algorithm>
 
 extern "C" void mp_gemm_prompt_low(const mp::GemmPrompt* a, int epi, hipStream_t stream);
 
@@ -99,12 +98,8 @@ extern "C" int mp_gemm_prompt_frags(int M, int N, int K) { return mp::gw_frags(M
 // fp32 elements of the workspace
 extern "C" int64_t mp_gemm_prompt_ws(int M, int N, int K, int frags) {
   using namespace mp;
-  int64_t most = 0;
-  for (int f : {frags ? frags : gw_frags(M, N, K), WideTile::MW}) {  // (and no less than tiles of 256 rows take, which a caller may have kept)
-    const int tiles = gw_tiles(M, N, f), parts = gw_parts(tiles, K / 64);
-    if (parts > 1) most = std::max(most, parts * (tiles % GW_CUS) * GW_SLAB);
-  }
-  return most;
+  const int tiles = gw_tiles(M, N, frags ? frags : gw_frags(M, N, K)), parts = gw_parts(tiles, K / 64);
+  return parts > 1 ? parts * (tiles % GW_CUS) * GW_SLAB : 0;
 }
 
 extern "C" int mp_gemm_prompt(const void* x, int64_t xs, const void* w, void* out, int M, int N, int K, int epi, float limit,

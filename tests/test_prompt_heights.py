@@ -38,6 +38,15 @@ def test_heights(frags, M, N, K):
         assert torch.equal(room[:M], prompt._run(x, v, torch.empty_like(room[:M]), N, epi, frags=frags))
 
 
+@pytest.mark.skipif(not ops.native_available(), reason="no kernel library")
+@pytest.mark.parametrize("M,N,K,need", [(4100, 4096, 2048, False), (300, 4096, 11008, True), (8000, 4368, 10880, False), (1891, 18704, 28672, False)])
+def test_workspace_is_the_height_s(M, N, K, need):
+    """What the height that runs needs, and nothing where only tiles of 256 rows would be cut."""
+    room = torch.ops.mpamd.gemm_prompt_ws
+    assert room(M, N, K) == room(M, N, K, torch.ops.mpamd.gemm_prompt_frags(M, N, K))
+    assert (room(M, N, K) > 0) == need and room(M, N, K, 8) > 0
+
+
 @pytest.mark.gpu
 def test_which_height():
     """Heights that a caller asks for, the estimate's without one, no others."""
