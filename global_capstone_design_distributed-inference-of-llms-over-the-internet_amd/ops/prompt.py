@@ -9,7 +9,8 @@ the callers that ask (``tiles`` of ``ops.linear``: stages and fine-tuning): shap
 as a model's do not stay there from one step to the next) run here at the row-tile
 counts where this kernel was at least as fast at all three row counts timed inside the tile, and 3 % faster on average, in
 both of two sweeps (one sweep differs from the next in about a third of the shapes, at counts where the two are close; the
-committed table of more than 256 rows also holds the 56 counts, of 926, that only tiles of 256 rows won, in two sweeps of theirs).
+committed table of more than 256 rows also holds 49 counts, of 919, that an earlier pair of sweeps had given to tiles of 256 rows, and
+that were at least as fast at all three row counts when they were timed once more, with the heights that they have now).
 
 Up to 384 rows there are tiles of 128 x 128 as well (csrc/gemm_mid.hip), by a table of theirs, timed against what runs without
 them: 66 rows of Mistral-7B, forward and backward, 1031 -> 832 us.  The library's call costs the host 21 us, theirs 13, so they stay

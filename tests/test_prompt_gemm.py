@@ -1,4 +1,6 @@
 """Prompt products (csrc/gemm_prompt.hip) at the edges of their tiles and parts, and which products take them."""
+import os
+
 import pytest
 import torch
 
@@ -257,3 +259,20 @@ def test_products_of_few_rows(M, N, K, epi):
     want = x.double() @ (w.double() if epi == 8 else w.double().t())
     got = prompt._run(x, w, torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda"), N, epi)
     assert float((got.double() - want).norm() / want.norm()) < BF16
+
+
+def test_counts_that_were_timed_again():
+    """Of the counts that sweeps did not agree on, the table holds those at which the record has the tile kernel no slower."""
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles", "prompt_products", "counts_timed_again.txt")
+    if not os.path.exists(path):
+        pytest.skip("no record")
+    ratios = {}
+    with open(path) as f:
+        for line in f:
+            p = line.split()
+            if line.startswith("N") and len(p) == 7:
+                ratios.setdefault((p[0], int(p[1])), []).append(float(p[6]))
+    table = {prompt._key(s): v for s, v in prompt._load(prompt.TABLE).items()}
+    assert len(ratios) == 56
+    for (shape, m), r in ratios.items():
+        assert (m in table[shape]) == (min(r) >= 1), (shape, m)
