@@ -100,6 +100,10 @@ def run_failover_drill(a, cfg, eng, ex, rank, world, S, R, M, B, device, load_s)
     link = HostLink(store, "bench/all", rank, world, timeout_s=600.0)
     thr = gather_replica_throughput(link, ex, lane, stage, R, batch=min(B, 16))
     link.close()
+    if a.rates:  # (measured rates differ from drill to drill, and with them the replica, micro-batch and row that a session gets)
+        thr = [float(v) for v in a.rates.split(",")]
+        if len(thr) != R or min(thr) <= 0:
+            raise SystemExit(f"--rates {a.rates}: one positive number for each of {R} replicas")
     timeout = float(os.environ.get("MPAMD_DRILL_TIMEOUT", "60"))
     code = 0
     if rank == 0:
@@ -287,6 +291,8 @@ def main(argv=None):
                          "recovery seconds and sessions completed.  Ranks are this launcher's own children")
     ap.add_argument("--drill", action="store_true",
                     help="run the failover drill's front end without killing anyone (the uninterrupted reference)")
+    ap.add_argument("--rates", default=None,
+                    help="drill: place sessions by these rates of the replicas, e.g. 1,1, in place of the measured ones")
     ap.add_argument("--dump-tokens", default=None, help="drill: write every session's tokens (JSON) here")
     ap.add_argument("--channel-data", default=os.environ.get("MPAMD_CHANNEL_DATA", "auto"),
                     choices=["auto", "nccl", "rccl", "gloo"],

@@ -24,8 +24,9 @@ head):
   aborted, see ``engine.PipelineFailure``); a head that dies shows up as a link error or
   timeout.  Either way the replica is marked dead and its unfinished sessions are
   re-placed on the survivors by **re-prefilling prompt + generated tokens** (token history
-  is all a pipeline needs to rebuild KV).  Sampling is seeded by (session seed, position),
-  so the survivors produce exactly the tokens the failed replica would have.
+  is all a pipeline needs to rebuild KV).  Sampling is seeded by (session seed, position): on
+  the CPU the survivors produce exactly the tokens the failed replica would have.  On the GPU
+  a session's row of its micro-batch is mixed in as well (see ``engine``).
 """
 from __future__ import annotations
 

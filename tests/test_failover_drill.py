@@ -5,7 +5,10 @@
   run's (``--drill`` without a kill) - the re-placed sessions included.
 * GPU rehearsal on ONE MI355X (4 ranks on the card, payloads host-staged over gloo: RCCL refuses
   two ranks per device): every session finishes, the failed replica's sessions are re-placed, and
-  every token a session had before the failure equals the uninterrupted run's.  After a
+  every token a session had before the failure equals the uninterrupted run's.  The GPU's sampler mixes
+  a session's row of its micro-batch into its draws, so both drills place by the same rates (--rates):
+  by measured ones a seventh session queued behind a faster replica's six came back in another row, with
+  other tokens from the first on.  After a
   re-placement the GPU logits differ in their last bits (the survivor runs another batch size, so
   another decode GEMM form, and rebuilds the KV by a prefill): the exactness contract there is
   the teacher-forced logit tolerance of ``test_failover_gpu.py``.
@@ -17,6 +20,8 @@ import subprocess
 import sys
 
 import pytest
+
+from src.parallel.failover import ReplicaRouter
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -52,6 +57,24 @@ def _check(ref, ref_dump, rec, dump, exact):
             assert toks == want, rid
 
 
+def _rows(rates, batch=2):
+    """Of the drill's 12 sessions: the row of its micro-batch that each gets (the head fills 3 micro-batches in order, then queues)."""
+    router, on = ReplicaRouter(2, rates), {0: 0, 1: 0}
+    rows = []
+    for i in range(12):
+        r = router.place_one(str(i), [1])
+        rows.append(on[r] % batch if on[r] < 3 * batch else "queued")
+        on[r] += 1
+    return rows
+
+
+def test_rates_decide_rows():
+    """Replicas within a seventh of each other hold six sessions each; past that the last one waits for a row that becomes free."""
+    even = _rows([1.0, 1.0])
+    assert even == [0, 0, 1, 1] * 3 and _rows([0.99, 1.0]) == even and _rows([1.16, 1.0]) == even
+    assert _rows([1.18, 1.0]) == even[:11] + ["queued"]
+
+
 @pytest.mark.timeout(900)
 def test_failover_drill_cpu_exact(tmp_path):
     ref, ref_dump = _drill(tmp_path, "ref", ["--drill"], "cpu", "tiny-llama")
@@ -63,8 +86,9 @@ def test_failover_drill_cpu_exact(tmp_path):
 @pytest.mark.timeout(900)
 def test_failover_drill_one_gpu_rehearsal(tmp_path):
     env = dict(MPAMD_DIST_BACKEND="gloo", MPAMD_CHANNEL_DATA="gloo", MPAMD_KV_GB="1", MPAMD_GEMM_AUTOTUNE="0")
-    ref, ref_dump = _drill(tmp_path, "ref", ["--drill"], "cuda", "small-llama", env)
-    rec, dump = _drill(tmp_path, "kill", ["--kill", "3@10"], "cuda", "small-llama", env)
+    even = ["--rates", "1,1"]
+    ref, ref_dump = _drill(tmp_path, "ref", ["--drill", *even], "cuda", "small-llama", env)
+    rec, dump = _drill(tmp_path, "kill", ["--kill", "3@10", *even], "cuda", "small-llama", env)
     _check(ref, ref_dump, rec, dump, exact=False)
     same = sum(dump["tokens"][k] == ref_dump["tokens"][k] for k in dump["tokens"])
     print(f"failover drill (1-GPU rehearsal): {json.dumps(rec['failover'])}; sessions identical end to end: "
