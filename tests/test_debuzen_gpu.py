@@ -299,6 +299,23 @@ def test_recurrences(dt, kind, H, G, D, V, taps):
     check_gated(a, got, dt)
 
 
+@pytest.mark.parametrize("kind,D,V", [("mamba2", 16, 300), ("mamba2", 16, 301), ("gated_delta", 16, 320), ("gated_delta", 17, 258),
+                                      ("mamba2", 16, 129), ("mamba2", 200, 32)])
+@pytest.mark.parametrize("taps", [4, 16])
+def test_convolutions_of_wide_heads(kind, D, V, taps):
+    """Heads whose channels are four or eight to a lane, neighbours and not, and so two or four rows on their way: ends of rows and
+    of blocks, from nothing and from a ring."""
+    lens = [53, 1, 18]
+    a = U.Gated(kind, lens, 2, 1, D, V, torch.bfloat16, DEV, taps, ranks=(24, 40) if D % 16 == 0 else (5, 7), col=8, pad=8)
+    got = [[] for _ in lens]
+    for ntoks in ([33, 1, 3], [17, 0, 15], [3, 0, 0]):
+        for i, r in enumerate(U.split(a.step(ntoks), ntoks)):
+            if r.numel():
+                got[i].append(r)
+    assert a.at == lens
+    check_gated(a, got, "bf16")
+
+
 @pytest.mark.parametrize("kind,H,G,D,V", [g for g in GATED if g[0] != "gated_delta" and g[3] <= 256])
 def test_long_prompts_in_parts(kind, H, G, D, V):
     """Sequences cut into parts that run at once: from nothing, from an earlier state, beside short ones."""
