@@ -1014,7 +1014,8 @@ def linear(x, w, out=None, epilogue=0, residual=None, policy=None, wp=None, a_ro
     ``tiles``: a prompt's product of row-major operands may run on this package's tile kernel (``prompt``), whose sums end
     in another order than the library's, as far from 64-bit ones or less.  Fine-tuning, hybrid decoders, Mixtral's attention and
     dense stages without a head ask for it: 20 ragged prompts of Llama-2-7B through 2 blocks 5041 -> 4235 us (0.0082 and 0.0073
-    from 64 bits).  With a head they do not: tokens sampled from its logits would be others.
+    from 64 bits).  With a head they do not: a model of one stage would sample other tokens.  Up to 384 rows, and with small
+    weights, the call may run on 128 x 128 tiles ahead of the decode kernels (``prompt.mid``, ``prompt.ahead``), not with ``ss_in``.
     """
     if not _native(x):
         K = 32 * wp.shape[1] if wp is not None else w.shape[1]

@@ -7,16 +7,16 @@
 //     same time, stay in L2).  64 x 28672 x 4096 gated 53.1 -> 43.1 us, 16 x 12288 x 4096 28.0 -> 22.6.
 //   * A CU loads 22 to 29 GB/s, so all of them have to: K is cut into parts, one per workgroup, whose fp32 sums lie as
 //     rows for a second kernel.  How many is an estimate of stages (0.62 us, 0.72 where all CUs load) against the second kernel
-//     and the sums' way (3.5 us and twice their bytes at 5 TB/s); within 10 % of the best number at 34 of 40 shapes and
-//     row counts that were timed with all numbers up to 16.
+//     and the sums' way (3.5 us and twice their bytes at 5 TB/s); within 6 % of the best number at 38 shapes and row counts
+//     that were timed with all numbers up to 16 (at two more it picks 32).
 //   * Nothing is divided on the way to the first load: the grid says tile, row tile and part.  With the divisions of a list of
 //     tiles, 2 us of 13.
 //   * Up to one workgroup per CU has nine slots (56 KB of weights in flight); more of them, where a small model's prompt has many
 //     rows, share CUs with five each: 384 x 12288 x 4096 65, 52 us.
-// us here, of the library and of the 256 x 256 tiles: 64 x 4096 x 14336 27.6, 39.8, 36.4; 192 x 4096 x 4096 17.5, 26.5, 32.0; 128 x
-// 28672 x 4096 gated 49.8, 59.0, 76.9; columns of 64 x 4096 x 6144 18.1, 46.1, 26.0; 1024 x 2048 x 512 gated 8.1, 13.4, 18.7.
-// From about 256 workgroups of 64 stages on the larger tiles or the library are faster: four operands' reads from LDS to 16
-// products, where the larger tiles have two to 16.
+// us here, of the library and of the 256 x 256 tiles: 64 x 4096 x 14336 29.4, 38.9, 36.1; 192 x 4096 x 4096 19.2, 32.5, 32.1; 128 x
+// 28672 x 4096 gated 49.7, 56.9, 65.3; columns of 64 x 4096 x 6144 18.7, 46.5, 26.2; 1024 x 2048 x 512 gated 8.4, 12.8, 18.3.
+// From about 8192 stages of all tiles on (128 workgroups of 64) the larger tiles or the library are mostly faster: four operands' reads
+// from LDS to 16 products, where the larger tiles have two to 16.
 #include "act_io.h"
 #include "gemm_act.h"
 #include "wide_tile.h"

@@ -64,9 +64,10 @@ static int gw_parts(int tiles, int ks) {
 }
 static int gw_tiles(int M, int N, int frags) { return (M + 32 * frags - 1) / (32 * frags) * ((N + 255) / 256); }
 // How high the tiles are: what an estimate in us says.  A stage takes what is listed (a tile of 128 rows 61 % of one of 256), a
-// tile 6.4 more, cut ones 14.7 and their parts' way to memory and back.  Fitted to 48 shapes and row counts whose five heights were
-// timed (6 % off, rms).  At 42 others of 300 to 7000 rows the height that it picks is 0.3 % slower than the best, 256 rows 9 %:
-// 2100 x 4096 x 2048 47 (256 rows), 36 us (160); 4298 x 2048 x 12800 224, 181 (160); columns of 2500 x 4096 x 4096 94, 75 (160).
+// tile 6.4 more, cut ones 14.7 and their parts' way to memory and back.  Fitted to 51 shapes and row counts whose five heights were
+// timed: the height that it picks is 0.6 % slower there than the best, 256 rows 8 %.  At 45 others, of 300 to 7000 rows, 0.3 % (10 at
+// the worst) and 9 %: 2100 x 4096 x 2048 42 (256 rows), 33 us (160); 4298 x 2048 x 12800 226, 177 (160); columns of 2500 x 4096 x 4096
+// 82, 68 (160).
 static int gw_frags(int M, int N, int K) {
   const float stage[5] = {0.77f, 0.88f, 1.00f, 1.17f, 1.27f};
   int best = 8;

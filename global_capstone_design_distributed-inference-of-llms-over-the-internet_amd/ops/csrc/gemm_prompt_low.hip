@@ -1,8 +1,8 @@
 // Prompt products whose tiles are 128, 160, 192 or 224 rows high and 256 weight rows wide: what gemm_prompt.hip asks for where they
 // fill rounds of 256 CUs, or the last tile's rows, better than tiles of 256 rows.  A wave has 4 to 7 fragments of rows to the eight of
 // weights, loads as many pieces of rows, and needs no half tile.  Bound as those are, by MFMA issue and power; with 4 fragments by LDS,
-// whose reads and loads into it take 1280 of a stage's cycles to 1024 of MFMAs.  A stage's time, 256 tiles of K 8192: 1.43 us of
-// 256 rows, 1.27 of 224, 1.11 of 192, 0.97 of 160, 0.90 of 128.
+// whose reads and loads into it take 1280 of a stage's cycles to 1024 of MFMAs.  A stage's time, 256 tiles of K 8192 (128 stages
+// and their ends): 1.36 us of 256 rows, 1.21 of 224, 1.06 of 192, 0.92 of 160, 0.77 of 128.
 #include "gemm_prompt.h"
 
 namespace mp {

@@ -421,8 +421,8 @@ __global__ __launch_bounds__(256) void train_rope_kernel(bf16_t* x, int64_t ld, 
 }
 
 // Norm of a row of the stream, a workgroup a row, the row in registers (one read).  Forward: sum = x + y (y may be
-// absent) + the block's deep prompt in a sequence's first P rows, each sum rounded, out = sum / rms(sum) w.  (The prompt in
-// launches of its own: 13 us a block ahead of this one's 9, at 1554 rows of 4096.)  Backward: out = res + d sum of (norm's gradient ``y``): rms and the row's dot product
+// absent) + the block's deep prompt in a sequence's first P rows, each sum rounded, out = sum / rms(sum) w.  (At
+// 1554 rows of 4096 8.5 us without a prompt, 8.7 with one; the prompt in launches of its own 16.5.)  Backward: out = res + d sum of (norm's gradient ``y``): rms and the row's dot product
 // are made again from ``x``, which is read anyway.
 template <int NC, bool GRAD>
 __global__ __launch_bounds__(256) void train_norm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ y,

@@ -222,7 +222,7 @@ def tune(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS, kernel=None)
 
 def sweep(todo: Iterable[Shape], device="cuda", log=None, rows=ROWS, kernel=None) -> Dict[Shape, list]:
     """Time both products over the row-tile counts of every shape, best of three rounds in turn: the kernel and the library's, or
-    ``_run_mid`` and what would run in its place, where the library's call costs the host 20 us more, which is what the 3 % are for
+    ``_run_mid`` and what would run in its place, where the library's call costs the host 8 us more, which is what the 3 % are for
     elsewhere."""
     from . import hybrid, require_native, swiglu, use_tuned_gemms
 

@@ -854,9 +854,11 @@ class StageExecutor:
             attn = e("attn", (T, cfg.q_dim))
             act = e("act", (T, cfg.intermediate_size))
             fold_native = self._folded_native(T)
-            # products in the tile kernel's order of sums, and gates that are not rounded ahead of their product, leave other last
-            # bits in the cache: of 64 tokens sampled behind a prompt of 10000, 5 to 13 were others.  A stage that has the logits
-            # to sample from keeps the library's, so that its tokens stay what they were; Mixtral's always were on the kernel
+            # The tile kernel's order of sums, and gates that are not rounded ahead of their product, leave other last bits in the
+            # cache, no further from 64-bit ones: of 64 tokens sampled behind a prompt of 10000, 5 to 13 were others.  A stage with
+            # the logits keeps the library's products: where it has all layers its tokens stay what they were, at a sixth of ragged
+            # prompts' time and 3 % of a long one's.  Behind other stages they do not, since its rows come from the tile kernel,
+            # and it takes the longer.  Mixtral's always were on the kernel
             tiles = not self.is_last
             for li, L in self._iter_layers(_DENSE_FIELDS):
                 # W8A16 layers' only weights carry the norm weights folded in (prepare_w8a16).
